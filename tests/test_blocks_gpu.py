@@ -83,6 +83,37 @@ def test_fast_matmul_around_kernel_choices(device, M, N, K):
     assert close(got, want), worst(got, want)
 
 
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("M,N,K", [(5, 8, 4), (16, 24, 32), (17, 40, 36), (16, 4800, 1600), (31, 104, 900), (33, 2304, 768),
+                                   (65, 72, 100), (128, 2304, 768), (128, 3080, 772), (129, 136, 4096), (500, 1032, 96),
+                                   (943, 768, 768), (1000, 3072, 1060)])
+def test_split_matmul_error_bound(device, int8, M, N, K):
+    """The products on the bf16 matrix cores against 64-bit ones: the edges of every tile (16, 32, 64 and 128 rows), partial
+    steps of 32 k and sliced K. The parts of a value add up to it exactly and all six products kept are exact, so the error
+    is that of the fp32 sums: at most six roundings per sixteen k, a few for the slices and waves, each at most 2**-24 of
+    the sum of magnitudes, and 2**-25 of it for the products left out."""
+    rng = np.random.default_rng(M * N + K)
+    A = rng.standard_normal((M, K)).astype(np.float32) * np.exp(rng.standard_normal((M, 1))).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    if int8:
+        q = rng.integers(-128, 128, (K, N))
+        scale = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+        W = q.astype(np.float64) * (scale / np.float32(127.0)).astype(np.float64)
+        inst = FastMatMulBlock.newInt8Instance(M, N, K, init_tensor(A, [M, K]), init_tensor(pack_words(q), [K, N // 4]),
+                                               init_tensor(scale, [N]), init_tensor(bias, [N]))
+    else:
+        w = (rng.standard_normal((K, N)) * np.exp2(rng.integers(-8, 8, (K, N)))).astype(np.float32)
+        W = w.astype(np.float64)
+        inst = FastMatMulBlock.newInstance(M, N, K, init_tensor(A, [M, K]), init_tensor(w, [K, N]), init_tensor(bias, [N]))
+    got = run(inst, (M, N)).astype(np.float64)
+    want = A.astype(np.float64) @ W + bias
+    size = np.abs(A).astype(np.float64) @ np.abs(W) + np.abs(bias)
+    bound = 2.0 ** -24 * (6 * K / 16 + 20) * size
+    assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
+    # and in practice no worse than sums of a few products at a time in fp32
+    assert np.linalg.norm(got - want) <= 2.0 ** -24 * max(4.0, K ** 0.5) * np.linalg.norm(size)
+
+
 def test_fast_matmul_exact_and_preconditions(device):
     A = RNG.integers(-8, 9, (3, 12)).astype(np.float32)
     W = RNG.integers(-8, 9, (12, 16)).astype(np.float32)

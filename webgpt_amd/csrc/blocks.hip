@@ -169,19 +169,11 @@ int wgpt_matmul_bias_i8(int M, int N, int K, wgpt_buf A, wgpt_buf Wq, wgpt_buf s
     int rc = grow_scratch(0, sizeof(float) * gemv_workspace_floats(M, N, K), &ws);
     if (rc) return rc;
     e = launch_gemv_kn_i8(M, N, K, a, K, wq, N / 4, sc, b, c, N, EPI_NONE, nullptr, (float*)ws, rt().stream);
-  } else if (M >= 16) {
-    // Dense contraction on the matrix cores, words dequantised on their way into LDS (same arithmetic).
+  } else {
     void* ws;
     int rc = grow_scratch(0, sizeof(float) * gemm_workspace_floats(M, N), &ws);
     if (rc) return rc;
     e = launch_gemm_i8(M, N, K, a, K, wq, N / 4, sc, b, c, N, EPI_NONE, nullptr, (float*)ws, rt().stream);
-  } else {
-    // A few rows more than the matrix-vector kernel takes: dequantise once (same arithmetic), then the fp32 tile kernel.
-    void* wf;
-    int rc = grow_scratch(1, sizeof(float) * (size_t)K * N, &wf);
-    if (rc) return rc;
-    e = launch_dequant_i8(K, N, wq, N / 4, sc, (float*)wf, N, rt().stream);
-    if (e == hipSuccess) e = launch_gemm(M, N, K, a, K, (const float*)wf, N, b, c, N, EPI_NONE, nullptr, nullptr, rt().stream);
   }
   if (e != hipSuccess) return fail(WGPT_ERR_HIP, "int8 matmul launch: %s", hipGetErrorString(e));
   return WGPT_OK;

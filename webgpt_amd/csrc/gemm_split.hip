@@ -1,0 +1,568 @@
+// FastMatMulBlock (instructions.js:157-319) for prompts, and its int8 weight-only form (other/int8-gemm.js:117-229).
+//
+// The operands are fp32 (the weights perhaps int8), the multiplications run on the bf16 matrix cores: every fp32 value
+// is the exact sum of three bf16 values, x = hi + mid + lo, and of the nine partial products of x y the six largest are
+// taken, all of them exact in the fp32 accumulator's input. The three left out (mid lo, lo mid, lo lo) are together below
+// 2^-25 |x y|, under half an ulp of the product; with sums of sixteen products rounded once instead of two at a time the
+// result is at least as close to the exact one as that of v_mfma_f32_32x32x2_f32. An int8 weight is one bf16 value
+// (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum. Infinities
+// are the one thing that is not carried over: inf = inf + nan + nan, so an infinite operand gives NaN.
+// bf16 runs at 16 times the rate of fp32 here, six products are therefore 2.7 times (int8: 5.3 times) faster.
+#include "gemm_split.h"
+
+#include <cmath>
+
+#include "kernels.h"
+
+namespace wgpt {
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// Two floats as bf16 pairs (round to nearest even): the first in bits 0-15.
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+
+// x = hi + mid + lo exactly (8 + 8 + 8 significand bits, each remainder rounded to nearest and representable), the
+// decomposition of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for
+// higher-precision computations" (2019).
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& hi, unsigned& mid, unsigned& lo) {
+  hi = bf16_pair(a, b);
+  const float ra = a - __builtin_bit_cast(float, hi << 16), rb = b - __builtin_bit_cast(float, hi & 0xffff0000u);
+  mid = bf16_pair(ra, rb);
+  lo = bf16_pair(ra - __builtin_bit_cast(float, mid << 16), rb - __builtin_bit_cast(float, mid & 0xffff0000u));
+}
+
+struct Split8 {  // eight consecutive k of one row or column
+  u32x4 hi, mid, lo;
+};
+__device__ __forceinline__ Split8 split8(const f32x4& a, const f32x4& b) {
+  Split8 r;
+  unsigned h[4], m[4], l[4];
+  split_pair(a[0], a[1], h[0], m[0], l[0]);
+  split_pair(a[2], a[3], h[1], m[1], l[1]);
+  split_pair(b[0], b[1], h[2], m[2], l[2]);
+  split_pair(b[2], b[3], h[3], m[3], l[3]);
+  r.hi = u32x4{h[0], h[1], h[2], h[3]};
+  r.mid = u32x4{m[0], m[1], m[2], m[3]};
+  r.lo = u32x4{l[0], l[1], l[2], l[3]};
+  return r;
+}
+
+template <int R>
+struct SplitBlock;
+template <>
+struct SplitBlock<32> {
+  typedef f32x16 acc_t;
+  static constexpr int NACC = 16;
+  static __device__ __forceinline__ acc_t mfma(const u32x4& w, const u32x4& a, const acc_t& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+  }
+  // column (of W) of the four consecutive ones in accumulator registers 4q..4q+3 of a lane
+  static __device__ __forceinline__ int row4(int q, int lane) { return 8 * q + 4 * (lane >> 5); }
+};
+template <>
+struct SplitBlock<16> {
+  typedef f32x4 acc_t;
+  static constexpr int NACC = 4;
+  static __device__ __forceinline__ acc_t mfma(const u32x4& w, const u32x4& a, const acc_t& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row4(int, int lane) { return 4 * (lane >> 4); }
+};
+
+
+__device__ __forceinline__ float gelu_ref(float x) {
+  const float x3 = x * x * x;
+  const float cdf = 0.5f * (1.0f + tanhf(0.7978845608f * (x + 0.044715f * x3)));
+  float r = x * cdf;
+  r = x < -10.0f ? 0.0f : r;
+  r = x > 10.0f ? x : r;
+  return r;
+}
+
+// ---- operands of one wave: RUN consecutive k per lane and step of 32. Loads are raw buffer loads whose per-lane offset
+// never changes: the step's place is in the scalar offset, so no vector instruction goes into addresses. ----
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes = 0x7fffffffu) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ f32x4 buf_f4(__amdgpu_buffer_rsrc_t b, int v, int s) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, v, s, 0));
+}
+// Lane (c, kg) of a block of R columns supplies k = RUN8 pieces: step s, chunk (STEPS > 1 ? 2 * s + kg : kg) of eight.
+template <int R>
+__device__ __forceinline__ int chunk_of(int s, int kg) { return R == 32 ? 2 * s + kg : kg; }
+
+// [K, N] as the caller's matrices come: one row of 32 (or 16) columns per load
+template <int R, bool I8>
+struct WRaw {
+  static constexpr int STEPS = R == 32 ? 2 : 1;
+  unsigned v[8 * STEPS];
+  static __device__ __forceinline__ int offset(const SplitGemmArgs& a, int n, int kg) { return 4 * ((I8 ? n >> 2 : n) + kg * 8 * a.ldw); }
+  __device__ __forceinline__ void load(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int off, int it) {
+#pragma unroll
+    for (int i = 0; i < 8 * STEPS; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b32(b, off, 4 * (it * 32 + (i >> 3) * 16 + (i & 7)) * a.ldw, 0);
+  }
+  // the step that reaches beyond K: rows past the last one repeat it (their A is zero)
+  __device__ __forceinline__ void load_tail(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int n, int kg, int it) {
+#pragma unroll
+    for (int i = 0; i < 8 * STEPS; ++i) {
+      const int k = it * 32 + chunk_of<R>(i >> 3, kg) * 8 + (i & 7);
+      v[i] = __builtin_amdgcn_raw_buffer_load_b32(b, 4 * ((I8 ? n >> 2 : n) + (k < a.K ? k : a.K - 1) * a.ldw), 0, 0);
+    }
+  }
+  __device__ __forceinline__ Split8 get(int s, int n) const {
+    if constexpr (I8) {
+      const int sh = 24 - 8 * (n & 3);
+      Split8 r;
+      unsigned h[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        h[i] = bf16_pair((float)((int)(v[8 * s + 2 * i] << sh) >> 24), (float)((int)(v[8 * s + 2 * i + 1] << sh) >> 24));
+      r.hi = u32x4{h[0], h[1], h[2], h[3]};
+      return r;
+    } else {
+      const u32x4 a = {v[8 * s], v[8 * s + 1], v[8 * s + 2], v[8 * s + 3]}, b = {v[8 * s + 4], v[8 * s + 5], v[8 * s + 6], v[8 * s + 7]};
+      return split8(__builtin_bit_cast(f32x4, a), __builtin_bit_cast(f32x4, b));
+    }
+  }
+};
+// A of a lane, straight from memory (rows of A, fp32)
+template <int R>
+struct ARaw {
+  static constexpr int STEPS = R == 32 ? 2 : 1;
+  f32x4 v[2 * STEPS];
+  static __device__ __forceinline__ int offset(const SplitGemmArgs& a, int m, int kg) { return 4 * ((m < a.M ? m : a.M - 1) * a.lda + kg * 8); }
+  __device__ __forceinline__ void load(const SplitGemmArgs&, __amdgpu_buffer_rsrc_t b, int off, int it) {
+#pragma unroll
+    for (int i = 0; i < 2 * STEPS; ++i) v[i] = buf_f4(b, off, 128 * it + 64 * (i >> 1) + 16 * (i & 1));
+  }
+  __device__ __forceinline__ void load_tail(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int m, int kg, int it) {
+#pragma unroll
+    for (int i = 0; i < 2 * STEPS; ++i) {
+      const int k = it * 32 + chunk_of<R>(i >> 1, kg) * 8 + 4 * (i & 1);
+      const f32x4 x = buf_f4(b, 4 * ((m < a.M ? m : a.M - 1) * a.lda + (k < a.K ? k : a.K - 4)), 0);
+      v[i] = k < a.K ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  __device__ __forceinline__ Split8 get(int s) const { return split8(v[2 * s], v[2 * s + 1]); }
+};
+
+__device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v, bool i8) {
+  if (m >= a.M || n >= a.N) return;
+  if (i8) {
+    const f32x4 s = *reinterpret_cast<const f32x4*>(a.wscale + n);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] *= s[i] / 127.0f;
+  }
+  if (a.part) {
+    *reinterpret_cast<f32x4*>(a.part + ((size_t)slice * a.M + m) * a.N + n) = v;
+    return;
+  }
+  if (a.bias) v += *reinterpret_cast<const f32x4*>(a.bias + n);
+  if (a.epi == EPI_GELU) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = gelu_ref(v[i]);
+  } else if (a.epi == EPI_RESIDUAL) {
+    v += *reinterpret_cast<const f32x4*>(a.resid + (size_t)m * a.ldc + n);
+  }
+  float* c = a.C + (size_t)m * a.ldc + n;
+  if (a.Kc && n >= a.d) {
+    const bool val = n >= 2 * a.d;
+    const int e = n - (val ? 2 : 1) * a.d, h = e / a.hs;
+    c = (val ? a.Vc : a.Kc) + ((size_t)h * a.ctx + a.pos0 + m) * a.hs + (e - h * a.hs);
+  }
+  *reinterpret_cast<f32x4*>(c) = v;
+}
+
+// position of a workgroup in the grid of tiles: consecutive tiles (m fastest: they share the columns of W) go to one XCD
+__device__ __forceinline__ bool tile_of(const SplitGemmArgs& a, int& m, int& n, int& slice) {
+  const int total = a.mt * a.nt * a.S, per = (total + 7) >> 3;
+  int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || t >= total) return false;
+  m = t % a.mt;
+  t /= a.mt;
+  n = t % a.nt;
+  slice = t / a.nt;
+  return true;
+}
+
+template <int R, int MB, int NB, bool I8>
+__device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Split8 (&xs)[MB], typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
+  typedef SplitBlock<R> B;
+  // smallest products first; the three that are left out are below half an ulp of a product
+#define SPLIT_STEP(wp, xp)                                                                        \
+  _Pragma("unroll") for (int i = 0; i < MB; ++i) _Pragma("unroll") for (int j = 0; j < NB; ++j) \
+      acc[i][j] = B::mfma(ws[j].wp, xs[i].xp, acc[i][j])
+  if constexpr (!I8) SPLIT_STEP(lo, hi);
+  SPLIT_STEP(hi, lo);
+  if constexpr (!I8) SPLIT_STEP(mid, mid);
+  if constexpr (!I8) SPLIT_STEP(mid, hi);
+  SPLIT_STEP(hi, mid);
+  SPLIT_STEP(hi, hi);
+#undef SPLIT_STEP
+}
+
+// sum of NP partial tiles (LDS, 64 float4 per entry) and epilogue
+template <int R, int MB, int NB, int NP, int THREADS, bool I8>
+__device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4* red, int m0, int n0, int slice) {
+  typedef SplitBlock<R> B;
+  constexpr int Q = B::NACC / 4, ENT = MB * NB * Q;
+  for (int e = threadIdx.x; e < ENT * 64; e += THREADS) {
+    f32x4 v = red[e];
+#pragma unroll
+    for (int u = 1; u < NP; ++u) v += red[u * ENT * 64 + e];
+    const int ln = e & 63, b = e >> 6, q = b % Q, ij = b / Q;
+    split_epilogue(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v, I8);
+  }
+}
+
+// The waves of a workgroup split K, each holds the whole tile and takes its operands straight from memory: no barrier and no
+// LDS until the sums meet. Bound by the load instructions of a compute unit up to ~100 rows (10-15 ns each whatever their
+// width), beyond that by matrix and vector instructions one after the other (six products per pair against eleven vector
+// instructions per two values split). Dependent launches, cold weights: 13x2304x768 5.5 us, 13x768x3072 in four slices 5.1 us
+// (219 and 193 us with the fp32 tile kernel that served 5 to 15 rows before); 64x64 tiles: 512x4096x1024 32.4 us = 132
+// TFLOP/s (39.9 us with v_mfma_f32_32x32x2_f32), int8 300x6400x1600 38.8 us (73).
+template <int R, int MB, int NB, int NW, bool I8>
+__global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
+  typedef SplitBlock<R> B;
+  constexpr int STEPS = WRaw<R, I8>::STEPS, Q = B::NACC / 4, ENT = MB * NB * Q;
+  extern __shared__ __attribute__((aligned(16))) float gs_lds[];
+  int m0, n0, slice;
+  if (!tile_of(a, m0, n0, slice)) return;
+  m0 *= MB * R;
+  n0 *= NB * R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & (R - 1), kg = lane / R;
+  const int iters = a.K >> 5, part = slice * NW + wave, parts = a.S * NW;
+  const int it0 = (int)((long)iters * part / parts), it1 = (int)((long)iters * (part + 1) / parts);
+  const __amdgpu_buffer_rsrc_t wb = buffer_of(a.W), xb = buffer_of(a.A);
+  int nn[NB], wo[NB], xo[MB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    nn[j] = n0 + j * R + r < a.N ? n0 + j * R + r : a.N - 1;
+    wo[j] = WRaw<R, I8>::offset(a, nn[j], kg);
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i) xo[i] = ARaw<R>::offset(a, m0 + i * R + r, kg);
+  typename B::acc_t acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < B::NACC; ++e) acc[i][j][e] = 0.f;
+  WRaw<R, I8> w[NB];
+  ARaw<R> x[MB];
+  Split8 ws[STEPS][NB], xs[STEPS][MB];
+  auto fetch = [&](int it) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w[j].load(a, wb, wo[j], it);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) x[i].load(a, xb, xo[i], it);
+  };
+  auto convert = [&] {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) ws[s][j] = w[j].get(s, nn[j]);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) xs[s][i] = x[i].get(s);
+    }
+  };
+  if (it0 < it1) fetch(it0);
+  for (int it = it0; it < it1; ++it) {
+    convert();
+    fetch(it + 1 < it1 ? it + 1 : it);
+    __builtin_amdgcn_sched_barrier(0);  // the requests leave before the products, not where their values are first needed
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) split_products<R, MB, NB, I8>(ws[s], xs[s], acc);
+  }
+  if ((a.K & 31) && part == parts - 1) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w[j].load_tail(a, wb, nn[j], kg, iters);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) x[i].load_tail(a, xb, m0 + i * R + r, kg, iters);
+    convert();
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) split_products<R, MB, NB, I8>(ws[s], xs[s], acc);
+  }
+  f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        red[(wave * ENT + (i * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  __syncthreads();
+  finish_tile<R, MB, NB, NW, NW * 64, I8>(a, red, m0, n0, slice);
+}
+
+__device__ __forceinline__ void lds_barrier() {  // orders LDS accesses only: loads from memory stay in flight
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// KG groups of NWN waves; a group takes every KG-th step of 32 k. Its waves own 32 * NB columns each, for all rows of the
+// tile: W goes straight from memory into registers, A through LDS, split once per workgroup on its way in; the products of a
+// step have the splitting of the next one between them. Half the traffic from L2 of the kernel above per product (a
+// compute unit takes 58 KB/us from there): 1024x4096x1024 in 128x128 tiles 54.4 us = 158 TFLOP/s, where 64x64 tiles of the
+// other take 61; 32x64 tiles for 65 to 128 rows: 100x3072x768 10.9 us against 12.5.
+template <int MB, int NB, int NWN, int KG, bool I8, int OCC, int D>
+__global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmArgs a) {
+  constexpr int R = 32;
+  typedef SplitBlock<R> B;
+  constexpr int MT = MB * R, GT = NWN * 64, Q = 4;
+  constexpr int CH = MT + 2;               // units of 16 bytes between chunks of eight k: conflict-free writes and reads
+  constexpr int BUF = 3 * 4 * CH;          // units of one buffer: planes x chunks
+  constexpr int AV = MT * 4 / GT;          // runs of eight k that a thread stages per step
+  static_assert(AV >= 1 && MT * 4 % GT == 0, "staging");
+  extern __shared__ __attribute__((aligned(16))) float gs_lds[];
+  int m0, n0, slice;
+  if (!tile_of(a, m0, n0, slice)) return;
+  m0 *= MT;
+  n0 *= NB * NWN * R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave / NWN, wn = wave % NWN, gt = threadIdx.x % GT;
+  const int r = lane & 31, kg = lane >> 5;
+  u32x4* abuf = reinterpret_cast<u32x4*>(gs_lds) + grp * 2 * BUF;
+  const int full = a.K >> 5;
+  const int s0 = (int)((long)full * slice / a.S), s1 = (int)((long)full * (slice + 1) / a.S);
+  const int rounds = (s1 - s0 + KG - 1) / KG;
+  const __amdgpu_buffer_rsrc_t wb = buffer_of(a.W), xb = buffer_of(a.A);
+  int nn[NB], wo[NB], xo[AV], xl[AV];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int n = n0 + (wn * NB + j) * R + r;
+    nn[j] = n < a.N ? n : a.N - 1;
+    wo[j] = WRaw<R, I8>::offset(a, nn[j], kg);
+  }
+#pragma unroll
+  for (int v = 0; v < AV; ++v) {
+    const int row = (gt + v * GT) >> 2, c = gt & 3;
+    xo[v] = 4 * ((m0 + row < a.M ? m0 + row : a.M - 1) * a.lda + c * 8);
+    xl[v] = c * CH + row;
+  }
+  typename B::acc_t acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < B::NACC; ++e) acc[i][j][e] = 0.f;
+  static_assert(D % 2 == 0, "the buffer of a step is a constant of the unrolled loop");
+  WRaw<R, I8> w[D][NB];
+  f32x4 x[D][AV][2];
+  Split8 ws[2][2][NB];
+  const auto clamp_step = [&](int i) { const int t = s0 + i * KG + grp; return t < s1 ? t : s1 - 1; };
+  const auto fetch_w = [&](int u, int i) {
+    const int t = clamp_step(i);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w[u][j].load(a, wb, wo[j], t);
+  };
+  // steps beyond the slice's end are asked for out of the buffer's range and come back as zeros
+  const auto fetch_x = [&](int u, int i) {
+    const int t = s0 + i * KG + grp;
+#pragma unroll
+    for (int v = 0; v < AV; ++v) {
+      const int o = t < s1 ? xo[v] : -32;
+      x[u][v][0] = buf_f4(xb, o, t < s1 ? 128 * t : 0);
+      x[u][v][1] = buf_f4(xb, o + 16, t < s1 ? 128 * t : 0);
+    }
+  };
+  const auto stage = [&](int u, int buf) {
+#pragma unroll
+    for (int v = 0; v < AV; ++v) {
+      const Split8 p = split8(x[u][v][0], x[u][v][1]);
+      u32x4* d = abuf + buf * BUF + xl[v];
+      d[0] = p.hi;
+      d[4 * CH] = p.mid;
+      d[8 * CH] = p.lo;
+    }
+  };
+  const auto convert = [&](int u, int c) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) ws[c][s][j] = w[u][j].get(s, nn[j]);
+  };
+  const auto multiply = [&](int buf, int c) {
+    Split8 xs[2][MB];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const u32x4* p = abuf + buf * BUF + (2 * s + kg) * CH + i * R + r;
+        xs[s][i].hi = p[0];
+        xs[s][i].mid = p[4 * CH];
+        xs[s][i].lo = p[8 * CH];
+      }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) split_products<R, MB, NB, I8>(ws[c][s], xs[s], acc);
+  };
+  if (rounds > 0) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      fetch_x(u, u);
+      fetch_w(u, u);
+    }
+    stage(0, 0);
+    fetch_x(0, D);
+    convert(0, 0);
+    fetch_w(0, D);
+    lds_barrier();
+    for (int i = 0; i < rounds; i += D) {
+#pragma unroll
+      for (int u = 0; u < D; ++u) {
+        if (u > 0 && i + u >= rounds) break;
+        // the products of step i + u; between them, so that the vector units work while the matrix units do, the
+        // splitting of the next step's W and A
+        multiply(u & 1, u & 1);
+        convert((u + 1) % D, (u + 1) & 1);
+        stage((u + 1) % D, (u + 1) & 1);
+        fetch_w((u + 1) % D, i + u + 1 + D);
+        fetch_x((u + 1) % D, i + u + 1 + D);
+        constexpr int NMF = MB * NB * 2 * (I8 ? 3 : 6), NVAL = (NB * 2 * (I8 ? 14 : 46) + AV * 48) / NMF + 1;
+        __builtin_amdgcn_sched_group_barrier(0x100, 3 * MB, 0);
+#pragma unroll
+        for (int m = 0; m < NMF; ++m) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, NVAL, 0);
+          if (m == 1) __builtin_amdgcn_sched_group_barrier(0x100, 3 * MB, 0);
+        }
+        lds_barrier();
+      }
+    }
+  }
+  if ((a.K & 31) && slice == a.S - 1) {  // the last, partial step: group 0
+    if (grp == 0) {
+#pragma unroll
+      for (int v = 0; v < AV; ++v) {
+        const int row = (gt + v * GT) >> 2, m = m0 + row < a.M ? m0 + row : a.M - 1;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = full * 32 + (gt & 3) * 8 + 4 * h;
+          const f32x4 t = buf_f4(xb, 4 * (m * a.lda + (k < a.K ? k : a.K - 4)), 0);
+          x[0][v][h] = k < a.K ? t : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      stage(0, 0);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) w[0][j].load_tail(a, wb, nn[j], kg, full);
+    }
+    lds_barrier();
+    if (grp == 0) {
+      convert(0, 0);
+      multiply(0, 0);
+    }
+    lds_barrier();
+  }
+  f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
+  constexpr int NBW = NWN * NB, ENT = MB * NBW * Q;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        red[(grp * ENT + (i * NBW + wn * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  __syncthreads();
+  finish_tile<R, MB, NBW, KG, NWN * KG * 64, I8>(a, red, m0, n0, slice);
+}
+
+// ---- launches ----
+// A launch takes about fixed + rounds * (one + more * (ceil(workgroups / 256) - 1)) us, where a workgroup needs
+// ceil(steps of its slice / kpar) rounds: a compute unit that gets a second workgroup determines the launch. The numbers
+// are least-squares fits to 2700 launches on MI355X (8 to 943 rows, 384 to 6400 columns, K from 384 to 6400, 1 to 8 slices;
+// 6-13 % rms); the shape that they choose is within 1.3 % of the best one of nine tried (geometric mean; 2.9 % where K may
+// be sliced).
+struct Shape {
+  int mtile, ntile, kpar;  // tile; steps of 32 k that a workgroup works on at a time
+  struct { float fixed, one, more; } f32, i8;
+};
+constexpr Shape SHAPES[] = {
+    {16, 16, 8, {2.78f, 0.77f, 0.92f}, {2.99f, 0.52f, 0.60f}},   // gemm_split_rows<16, 1, 1, 8>
+    {16, 32, 8, {3.11f, 0.90f, 1.31f}, {3.10f, 0.68f, 0.82f}},   // gemm_split_rows<16, 1, 2, 8>
+    {32, 32, 8, {3.09f, 1.27f, 1.75f}, {3.39f, 1.26f, 1.29f}},   // gemm_split_rows<32, 1, 1, 8>
+    {64, 64, 4, {4.56f, 1.45f, 2.06f}, {5.30f, 1.05f, 1.56f}},   // gemm_split_rows<32, 2, 2, 4>
+    {64, 64, 8, {4.58f, 2.58f, 4.77f}, {5.05f, 2.11f, 3.49f}},   // gemm_split_rows<32, 2, 2, 8>
+    {32, 64, 4, {4.70f, 1.03f, 2.41f}, {4.84f, 0.87f, 1.04f}},   // gemm_split_tile<1, 1, 2, 4>
+    {128, 128, 2, {7.97f, 2.00f, 4.69f}, {8.00f, 1.56f, 3.06f}}, // gemm_split_tile<4, 1, 4, 2>
+};
+constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
+
+constexpr size_t rows_lds(int R, int MB, int NB, int NW) { return (size_t)NW * MB * NB * R * R * sizeof(float); }
+constexpr size_t tile_lds(int MB, int NB, int NWN, int KG) {
+  const size_t red = (size_t)KG * MB * NB * NWN * 32 * 32 * sizeof(float), stage = (size_t)KG * 2 * 3 * 4 * (MB * 32 + 2) * 16;
+  return red > stage ? red : stage;
+}
+
+template <typename K>
+hipError_t launch_kernel(K kernel, const SplitGemmArgs& a, int threads, size_t lds, hipStream_t s) {
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  const long grid = ((long)a.mt * a.nt * a.S + 7) / 8 * 8;
+  if (grid > 0x7fffffffL) return hipErrorInvalidValue;
+  kernel<<<(unsigned)grid, threads, lds, s>>>(a);
+  return hipGetLastError();
+}
+
+template <bool I8>
+hipError_t launch_shape(int kind, const SplitGemmArgs& a, hipStream_t s) {
+  switch (kind) {
+    case 0: return launch_kernel(gemm_split_rows<16, 1, 1, 8, I8>, a, 512, rows_lds(16, 1, 1, 8), s);
+    case 1: return launch_kernel(gemm_split_rows<16, 1, 2, 8, I8>, a, 512, rows_lds(16, 1, 2, 8), s);
+    case 2: return launch_kernel(gemm_split_rows<32, 1, 1, 8, I8>, a, 512, rows_lds(32, 1, 1, 8), s);
+    case 3: return launch_kernel(gemm_split_rows<32, 2, 2, 4, I8>, a, 256, rows_lds(32, 2, 2, 4), s);
+    case 4: return launch_kernel(gemm_split_rows<32, 2, 2, 8, I8>, a, 512, rows_lds(32, 2, 2, 8), s);
+    case 5: return launch_kernel(gemm_split_tile<1, 1, 2, 4, I8, 2, 2>, a, 512, tile_lds(1, 1, 2, 4), s);
+    case 6: return launch_kernel(gemm_split_tile<4, 1, 4, 2, I8, 2, 2>, a, 512, tile_lds(4, 1, 4, 2), s);
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+SplitPlan plan_gemm_split(int M, int N, int K, bool i8, bool with_pass, bool may_slice) {
+  SplitPlan best = {0, 1};
+  double best_t = 1e30;
+  const int steps = (K + 31) / 32;
+  for (int c = 0; c < NSHAPES; ++c) {
+    const Shape& sh = SHAPES[c];
+    const auto& f = i8 ? sh.i8 : sh.f32;
+    const double tiles = (double)((M + sh.mtile - 1) / sh.mtile) * ((N + sh.ntile - 1) / sh.ntile);
+    for (int S = 1; S <= (may_slice ? 8 : 1); ++S) {
+      if (S > 1 && steps < 4 * S) break;
+      const double load = std::ceil(tiles * S / 256.0);
+      const double rounds = ((steps + S - 1) / S + sh.kpar - 1) / sh.kpar;
+      double t = f.fixed + rounds * (f.one + f.more * (load - 1));
+      if (S > 1) t += (with_pass ? 0.0 : 4.0) + (double)S * M * N * 8.0 / 5.0e6;  // the pass over the partial sums, at 5 TB/s
+      if (t < best_t) {
+        best_t = t;
+        best = {c, S};
+      }
+    }
+  }
+  return best;
+}
+
+hipError_t launch_gemm_split(const SplitPlan& p, SplitGemmArgs a, bool i8, hipStream_t s) {
+  a.mt = (a.M + SHAPES[p.kind].mtile - 1) / SHAPES[p.kind].mtile;
+  a.nt = (a.N + SHAPES[p.kind].ntile - 1) / SHAPES[p.kind].ntile;
+  a.S = p.S;
+  return i8 ? launch_shape<true>(p.kind, a, s) : launch_shape<false>(p.kind, a, s);
+}
+
+}  // namespace wgpt

@@ -22,8 +22,8 @@ size_t gemv_workspace_floats(int M, int N, int K);
 hipError_t launch_gemv_kn(int M, int N, int K, const float* A, int lda, const float* W, int ldw, const float* bias,
                           float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s);
 
-// Same contraction for any M through the tiled GEMM kernels (matrix cores for M >= 16).
-// workspace (gemm_workspace_floats(M, N) floats, may be null) enables split-K for
+// Same contraction for any M on the matrix cores (gemm_split.hip).
+// workspace (gemm_workspace_floats(M, N) floats, may be null) enables slices of K for
 // shapes with too few output tiles to fill the GPU.
 size_t gemm_workspace_floats(int M, int N);
 // A LayerNormBlock applied to the finished rows of C right after the product (out may not alias C). Where the
@@ -44,8 +44,7 @@ struct KvAfter {
 hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float* W, int ldw, const float* bias,
                        float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
                        const LnAfter* ln = nullptr, const KvAfter* kv = nullptr);
-// Same with the packed int8 weights of other/int8-gemm.js (Wq[K, ldwq] words, scale[N]), dequantised inside
-// the kernel; M >= 16.
+// Same with the packed int8 weights of other/int8-gemm.js (Wq[K, ldwq] words, scale[N]).
 hipError_t launch_gemm_i8(int M, int N, int K, const float* A, int lda, const int32_t* Wq, int ldwq, const float* scale,
                           const float* bias, float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
                           const LnAfter* ln = nullptr, const KvAfter* kv = nullptr);

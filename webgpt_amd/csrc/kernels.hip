@@ -4,7 +4,10 @@
 // reduction and combine by wave shuffles), which stays inside the fp32 tolerance.
 #include "kernels.h"
 
+#include <algorithm>
 #include <type_traits>
+
+#include "gemm_split.h"
 
 namespace wgpt {
 
@@ -313,498 +316,6 @@ __global__ __launch_bounds__(WG) void dequant_i8_kernel(int K, int N, const int3
   if (idx >= (size_t)K * n4) return;
   const int k = (int)(idx / n4), w = (int)(idx - (size_t)k * n4);
   st4(W + (size_t)k * ldw + 4 * w, unpack_i8x4(Wq[(size_t)k * ldwq + w], ld4(scale + 4 * w)));
-}
-
-// ---------------------------------------------------------------------------
-// FastMatMulBlock for any M (prefill): 64x64 output tile per workgroup, 4x4 per
-// thread, K in steps of 16 through LDS. Same contraction and bias-last order of
-// operations per element as instructions.js:248-314 up to fp32 reassociation.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(WG) void gemm_tile64(int M, int N, int K, const float* __restrict__ A, int lda,
-                                                   const float* __restrict__ W, int ldw, const float* __restrict__ bias,
-                                                   float* C, int ldc, int epi, const float* resid) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Bs[16][64];
-  const int tid = threadIdx.x;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int tm = tid >> 4, tn = tid & 15;
-  const int arow = tid >> 2, akq = (tid & 3) * 4;
-  const int brow = tid >> 4, bnq = (tid & 15) * 4;
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    float4 av = make_float4(0.f, 0.f, 0.f, 0.f), bv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (m0 + arow < M && k0 + akq < K) av = ld4(A + (size_t)(m0 + arow) * lda + k0 + akq);
-    if (k0 + brow < K && n0 + bnq < N) bv = ld4(W + (size_t)(k0 + brow) * ldw + n0 + bnq);
-    As[akq + 0][arow] = av.x;
-    As[akq + 1][arow] = av.y;
-    As[akq + 2][arow] = av.z;
-    As[akq + 3][arow] = av.w;
-    st4(&Bs[brow][bnq], bv);
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const float4 a = ld4(&As[kk][tm * 4]);
-      const float4 b = ld4(&Bs[kk][tn * 4]);
-      const float aa[4] = {a.x, a.y, a.z, a.w};
-      const float bb[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += aa[i] * bb[j];
-    }
-    __syncthreads();
-  }
-  const int n = n0 + tn * 4;
-  if (n >= N) return;
-  float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (bias) b = ld4(bias + n);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + tm * 4 + i;
-    if (m >= M) break;
-    float4 v = make_float4(acc[i][0] + b.x, acc[i][1] + b.y, acc[i][2] + b.z, acc[i][3] + b.w);
-    if (epi == EPI_GELU) {
-      v.x = gelu_ref(v.x); v.y = gelu_ref(v.y); v.z = gelu_ref(v.z); v.w = gelu_ref(v.w);
-    } else if (epi == EPI_RESIDUAL) {
-      const float4 q = ld4(resid + (size_t)m * ldc + n);
-      v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
-    }
-    st4(C + (size_t)m * ldc + n, v);
-  }
-}
-
-
-// ---------------------------------------------------------------------------
-// FastMatMulBlock as a dense contraction on the matrix cores (prefill, M >= 16):
-// C = epi(A . W + bias). fp32 MFMA v_mfma_f32_32x32x2_f32: per instruction a wave
-// multiplies a 32x2 slice of A by a 2x32 slice of W into a 32x32 fp32 accumulator
-// (16 VGPRs per lane). Workgroup tile TM x TN (64 or 128 each), four waves in a 2x2
-// arrangement, each owning (TM/2) x (TN/2) of C as RB x CB accumulator blocks, so an
-// operand fragment read from LDS feeds CB (or RB) instructions. K advances in steps
-// of BK = 32 through two LDS stages (one barrier per step); inside a step every wave
-// interleaves its matrix instructions with the LDS reads of the next quarter-step, the
-// global loads of a later step and the move of the next step into the other stage.
-// A is staged as [m][BK + 4] with the k of a step permuted to (k odd, k / 2), so the
-// values a lane feeds to four consecutive instructions are one 128-bit read; W as
-// [k][n], odd k with the two 32-column halves of a row swapped so that the two half-waves
-// of an operand read (k and k + 1) use different LDS banks.
-// Operand lane mapping of the instruction: lane l supplies A[row l%32][k l/32] and
-// W[k l/32][col l%32]; accumulator register r of lane l is
-// C[row (r/4)*8 + (l/32)*4 + r%4][col l%32].
-// ---------------------------------------------------------------------------
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// With kchunk < K (split-K) slice blockIdx.z covers k in [z*kchunk, (z+1)*kchunk) and
-// writes its raw partial sums to C + z*M*ldc (bias, epilogue: gemv_reduce afterwards).
-// I8W: W is the packed int8 matrix of other/int8-gemm.js:36-43 (`Wv` points to [K, ldw] words of four
-// consecutive columns, `wscale` to the per-column scales); a thread's word of a step is
-// dequantised on its way into LDS with the arithmetic of unpackInt8x4, so the matrix cores
-// see exactly the weights wgpt_dequant_i8 would write, without the trip through memory.
-template <int TM, int TN, int BK, bool I8W, bool EXACT>
-__global__ __launch_bounds__(WG) void gemm_mfma(int M, int N, int K, int kchunk, const float* __restrict__ A, int lda,
-                                                 const void* __restrict__ Wv, int ldw, const float* __restrict__ wscale,
-                                                 const float* __restrict__ bias, float* C, int ldc, int epi, const float* resid) {
-  const float* W = static_cast<const float*>(Wv);
-  const int32_t* Wq = static_cast<const int32_t*>(Wv);
-  constexpr int AST = BK + 4;                // floats per staged A row (16-byte aligned, odd multiple of 4 banks)
-  constexpr int RB = TM / 64, CB = TN / 64;  // 32x32 accumulator blocks per wave
-  constexpr int KQ = BK / 4;                 // float4 per A row of a step
-  constexpr int AROWS = WG / KQ;             // A rows covered by one pass of the workgroup
-  constexpr int NA = TM / AROWS;             // float4 per thread of the A tile of a step
-  constexpr int BROWS = WG / (TN / 4);       // W rows covered by one pass of the workgroup
-  constexpr int NB = BK / BROWS;             // float4 per thread of the W tile of a step
-  constexpr int HK = BK / 2;                 // MFMA instructions per step and accumulator block
-  constexpr int NQ = HK / 4;                 // quarters of a step: four k pairs each
-  constexpr int BST = TN;                    // floats per staged W row (odd rows swap their 32-column halves)
-  __shared__ __attribute__((aligned(16))) float As[2][TM * AST];
-  __shared__ __attribute__((aligned(16))) float Bs[2][BK * BST];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
-  const int arow = tid / KQ, akq = (tid % KQ) * 4;
-  const int brow = tid / (TN / 4), bnq = (tid % (TN / 4)) * 4;
-  // D register sets of global data: a step's tile is fetched D steps ahead of its use and moves into
-  // LDS one step ahead; with two sets, set p holds the steps of parity p
-  constexpr int D = RB * CB == 1 ? 2 : 1;  // the large tile has registers for one set only
-  float4 ga[D][NA], gb[D][I8W ? 1 : NB];
-  int32_t gq[D][I8W ? NB : 1];  // packed words of the step, unpacked when they are staged
-  float4 sc4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (I8W && n0 + bnq < N) sc4 = ld4(wscale + n0 + bnq);
-  // Every global load is unconditional and in bounds: rows beyond M and columns beyond N repeat the
-  // last valid ones (their results are never stored), k beyond the slice repeats its last values and is
-  // zeroed when the step is staged. (A load under a bounds branch makes the compiler wait for it on
-  // the spot, which exposes the whole memory latency in every step.) EXACT: every K slice is whole
-  // steps, so there is nothing to clamp or zero along k, and a step's addresses are a uniform base
-  // plus per-thread offsets: vector-ALU instructions of a step queue behind the matrix instructions
-  // of the other waves of the SIMD, so the fewer the better.
-  const int kbeg = blockIdx.z * kchunk;
-  const int kend = kbeg + kchunk < K ? kbeg + kchunk : K;
-  C += (size_t)blockIdx.z * M * ldc;
-  K = kend;
-  const int ncl = n0 + bnq < N ? n0 + bnq : N - 4;
-  unsigned aoff[NA], boff[NB];  // element offsets from the step's first k (A) / first row (W)
-#pragma unroll
-  for (int r = 0; r < NA; ++r) {
-    const int m = m0 + arow + r * AROWS;
-    aoff[r] = (unsigned)((size_t)(m < M ? m : M - 1) * lda + akq);
-  }
-#pragma unroll
-  for (int r = 0; r < NB; ++r) boff[r] = (unsigned)((size_t)(brow + r * BROWS) * ldw + (I8W ? ncl >> 2 : ncl));
-  int kf[D] = {};  // first k of the step held by each set
-  auto fetch = [&](auto P, int k0) {
-    constexpr int p = decltype(P)::value;
-    kf[p] = k0;
-    if (EXACT) {
-      const float* at = A + k0;
-      const size_t wrow = (size_t)k0 * ldw;
-#pragma unroll
-      for (int r = 0; r < NA; ++r) ga[p][r] = ld4(at + aoff[r]);
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        if (I8W) gq[p][I8W ? r : 0] = (Wq + wrow)[boff[r]];
-        else gb[p][I8W ? 0 : r] = ld4(W + wrow + boff[r]);
-      }
-    } else {
-      const int ka = k0 + akq < K ? k0 : K - 4 - akq;
-#pragma unroll
-      for (int r = 0; r < NA; ++r) ga[p][r] = ld4(A + ka + aoff[r]);
-#pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        const int k = k0 + brow + r * BROWS;
-        const size_t wrow = (size_t)(k < K ? k0 : K - 1 - brow - r * BROWS) * ldw;
-        if (I8W) gq[p][I8W ? r : 0] = (Wq + wrow)[boff[r]];
-        else gb[p][I8W ? 0 : r] = ld4(W + wrow + boff[r]);
-      }
-    }
-  };
-  // LDS layouts: A tile as [m][BK + 4], W tile as [k][TN] with the two 32-column halves of every 64 columns
-  // swapped in rows with bit 2 set. Matrix instruction i of quarter q takes k = 8q + 4h + i from half-wave h, so
-  // a lane's four A values of a quarter are one 128-bit read of the unpermuted row, and the two half-waves of
-  // a W read (rows 8q + i and 8q + 4 + i) use different banks.
-  auto stage = [&](auto P, int st) {
-    constexpr int p = decltype(P)::value;
-    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    const bool ain = EXACT || kf[p] + akq < K;
-#pragma unroll
-    for (int r = 0; r < NA; ++r) st4(As[st] + (arow + r * AROWS) * AST + akq, ain ? ga[p][r] : z);
-#pragma unroll
-    for (int r = 0; r < NB; ++r) {
-      const int row = brow + r * BROWS;
-      const bool bin = EXACT || kf[p] + row < K;
-      const float4 v = I8W ? unpack_i8x4(gq[p][I8W ? r : 0], sc4) : gb[p][I8W ? 0 : r];
-      st4(Bs[st] + row * BST + (bnq ^ (((row >> 2) & 1) << 5)), bin ? v : z);
-    }
-  };
-  f32x16 acc[RB][CB];
-#pragma unroll
-  for (int r = 0; r < RB; ++r)
-#pragma unroll
-    for (int c = 0; c < CB; ++c)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[r][c][i] = 0.f;
-
-  const int h = lane >> 5, l32 = lane & 31;
-  // operands of quarter q of the step in LDS stage st: four k pairs per accumulator row / column block
-  auto operands = [&](float (&av)[RB][4], float (&bv)[CB][4], int st, int q) {
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const float4 v = ld4(As[st] + (wm + r * 32 + l32) * AST + 8 * q + 4 * h);
-      av[r][0] = v.x; av[r][1] = v.y; av[r][2] = v.z; av[r][3] = v.w;
-    }
-#pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      const float* bp = Bs[st] + (8 * q + 4 * h) * BST + ((wn + c * 32 + l32) ^ (h << 5));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bv[c][i] = bp[i * BST];
-    }
-  };
-  auto multiply = [&](const float (&av)[RB][4], const float (&bv)[CB][4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-#pragma unroll
-        for (int c = 0; c < CB; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[r][i], bv[c][i], acc[r][c], 0, 0, 0);
-  };
-
-  // requested before the main loop so that the epilogue does not wait for it
-  float biasv[CB];
-#pragma unroll
-  for (int c = 0; c < CB; ++c) {
-    const int n = n0 + wn + c * 32 + l32;
-    biasv[c] = (bias && n < N) ? bias[n] : 0.f;
-  }
-  typedef std::integral_constant<int, 0> P0;
-  typedef std::integral_constant<int, 1> P1;
-  fetch(P0(), kbeg);
-  stage(P0(), 0);
-  if constexpr (D == 2) {
-    if (kbeg + BK < kend) fetch(P1(), kbeg + BK);
-  }
-  __syncthreads();
-  float av[2][RB][4], bv[2][CB][4];  // operands of the quarter being multiplied and of the next one
-  operands(av[0], bv[0], 0, 0);
-  int st = 0;
-  // One K step. A wave keeps its own matrix pipe fed: while the instructions of a quarter run, the
-  // operands of the next quarter are on their way from LDS, the global loads of a later step (D steps
-  // ahead) are in flight, and the next step's tile moves from registers into the other LDS stage. The
-  // last quarter is multiplied after the barrier, behind the request for the next step's first
-  // operands. (Leaving the overlap to a second wave of the SIMD does not work: the workgroups of a
-  // compute unit fall into step with each other and stall together.)
-  // FETCH / STAGE are compile-time so that the steady state is straight-line code: with a branch
-  // around the loads the compiler can no longer tell which of them are outstanding and waits early.
-  auto kstep = [&](auto P, auto FETCH, auto STAGE, int k0) {
-    constexpr int p = decltype(P)::value;
-    static_assert(NQ % 2 == 0, "the last quarter of a step must sit in operand set 1");
-    if (decltype(FETCH)::value) {
-      fetch(std::integral_constant<int, D == 2 ? p : 0>(), k0 + D * BK);  // that set was staged a step ago
-      __builtin_amdgcn_sched_barrier(0);  // keep the loads here, at the head of the step
-    }
-#pragma unroll
-    for (int q = 0; q < NQ - 1; ++q) {
-      operands(av[(q + 1) & 1], bv[(q + 1) & 1], st, q + 1);
-      multiply(av[q & 1], bv[q & 1]);
-    }
-    if (decltype(STAGE)::value) {
-      __builtin_amdgcn_sched_barrier(0);  // nothing of the move into LDS (it waits for the loads) drifts up
-      stage(std::integral_constant<int, D == 2 ? 1 - p : 0>(), st ^ 1);
-      __syncthreads();
-      st ^= 1;
-      operands(av[0], bv[0], st, 0);
-    }
-    multiply(av[1], bv[1]);
-  };
-  const std::true_type yes;
-  const std::false_type no;
-  int k0 = kbeg;
-  if constexpr (D == 2) {
-    for (; k0 + 3 * BK < kend; k0 += 2 * BK) {
-      kstep(P0(), yes, yes, k0);
-      kstep(P1(), yes, yes, k0 + BK);
-    }
-    if (k0 + 2 * BK < kend) {  // three steps left
-      kstep(P0(), yes, yes, k0);
-      kstep(P1(), no, yes, k0 + BK);
-      kstep(P0(), no, no, k0 + 2 * BK);
-    } else if (k0 + BK < kend) {  // two
-      kstep(P0(), no, yes, k0);
-      kstep(P1(), no, no, k0 + BK);
-    } else if (k0 < kend) {  // one
-      kstep(P0(), no, no, k0);
-    }
-  } else {
-    for (; k0 + BK < kend; k0 += BK) kstep(P0(), yes, yes, k0);
-    if (k0 < kend) kstep(P0(), no, no, k0);
-  }
-#pragma unroll
-  for (int c = 0; c < CB; ++c) {
-    const int n = n0 + wn + c * 32 + l32;
-    if (n >= N) continue;
-    const float bvs = biasv[c];
-#pragma unroll
-    for (int r = 0; r < RB; ++r)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = m0 + wm + r * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-        if (m < M) {
-          float v = acc[r][c][i] + bvs;
-          if (epi == EPI_GELU) v = gelu_ref(v);
-          else if (epi == EPI_RESIDUAL) v += resid[(size_t)m * ldc + n];
-          C[(size_t)m * ldc + n] = v;
-        }
-      }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The same contraction for problems that give every compute unit one 64 x 128 tile: 512 threads, two
-// groups of four waves (one wave of each group per SIMD); group g owns columns [64g, 64g + 64) of the
-// tile, its waves a 32 x 32 block each. The groups alternate: while one issues the 16 matrix
-// instructions of a K step from registers, the other does its memory work (operands of its next
-// step from LDS into registers, its share of a later tile from registers into LDS, global loads two
-// steps ahead of that), then they swap at a barrier. A SIMD's matrix pipe therefore always has
-// exactly one wave feeding it, and no wave waits for memory between matrix instructions. (With
-// independent workgroups the waves of a SIMD run in step, want the pipe at the same time and stall
-// at the same time.) Tiles of K steps 0, 1, ... alternate between two LDS stages; group 0 multiplies
-// step k in the first half of iteration k, group 1 in the second half. Every load and LDS write is
-// unconditional: tiles beyond the K range are fetched from clamped addresses and staged as zeros.
-// ---------------------------------------------------------------------------
-constexpr int PP_THREADS = 512;
-constexpr int PP_BK = 32;  // K step (64 measured 3-5 % slower)
-constexpr size_t PP_LDS = sizeof(float) * 2 * (64 * (PP_BK + 4) + PP_BK * 128);
-template <int BK>
-__global__ __launch_bounds__(PP_THREADS) void gemm_pingpong(int M, int N, int K, int kchunk, const float* __restrict__ A, int lda,
-                                                            const float* __restrict__ W, int ldw, const float* __restrict__ bias,
-                                                            float* C, int ldc, int epi, const float* resid) {
-  constexpr int TM = 64, TN = 128, AST = BK + 4, HK = BK / 2;
-  constexpr int NA = BK / 32, NB = BK / 16;  // float4 of A and of W per thread and tile
-  extern __shared__ __attribute__((aligned(16))) float pp_lds[];
-  float* const As = pp_lds;                  // [2][TM * AST]
-  float* const Bs = pp_lds + 2 * TM * AST;   // [2][BK * TN]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = wave >> 2, wq = wave & 3, t = tid & 255;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int wm = (wq >> 1) * 32, wn = g * 64 + (wq & 1) * 32;
-  const int h = lane >> 5, l32 = lane & 31;
-  // this thread's share of a tile: NA float4 of A (row 32g + t / 8, float4 t % 8 + 8j of the row), NB of W (the
-  // group's own columns, rows t / 16 + 16r). Rows beyond M and columns beyond N repeat the last valid ones
-  // (their results are never stored).
-  const int arow = g * 32 + (t >> 3), akq = (t & 7) * 4;
-  const int brow = t >> 4, bnq = g * 64 + (t & 15) * 4;
-  const int ncl = n0 + bnq < N ? n0 + bnq : N - 4;
-  // byte offsets of the thread inside a tile; the tile's own address is uniform and advances with the step,
-  // so that a memory phase issues almost no vector-ALU instructions: those queue behind the other group's
-  // matrix instructions on the same SIMD, LDS and global-memory instructions do not
-  unsigned aoff[NA], boff[NB];
-#pragma unroll
-  for (int j = 0; j < NA; ++j) aoff[j] = (unsigned)(((size_t)(m0 + arow < M ? m0 + arow : M - 1) * lda + akq + 32 * j) * sizeof(float));
-#pragma unroll
-  for (int j = 0; j < NB; ++j) boff[j] = (unsigned)(((size_t)(brow + 16 * j) * ldw + ncl) * sizeof(float));
-
-  const int kbeg = blockIdx.z * kchunk;
-  const int kend = kbeg + kchunk < K ? kbeg + kchunk : K;
-  C += (size_t)blockIdx.z * M * ldc;
-  const int nsteps = (kend - kbeg) / BK;  // the launcher guarantees whole steps
-  const char* Abase = reinterpret_cast<const char*>(A + kbeg);
-  const char* Wbase = reinterpret_cast<const char*>(W + (size_t)kbeg * ldw);
-  const size_t wstep = (size_t)BK * ldw * sizeof(float);
-
-  struct Share {
-    float4 a[NA], b[NB];
-  };
-  auto load_share = [&](int tile) {  // this thread's share of tile `tile` (tiles past the end repeat the last one)
-    const int tc = tile < nsteps ? tile : nsteps - 1;
-    // the tile addresses are uniform: keep them in scalar registers
-    const unsigned long long wo = (unsigned long long)tc * wstep;
-    const unsigned wlo = __builtin_amdgcn_readfirstlane((unsigned)wo), whi = __builtin_amdgcn_readfirstlane((unsigned)(wo >> 32));
-    const char* at = Abase + __builtin_amdgcn_readfirstlane(tc * (int)(BK * sizeof(float)));
-    const char* wt = Wbase + (((unsigned long long)whi << 32) | wlo);
-    Share r;
-#pragma unroll
-    for (int j = 0; j < NA; ++j) r.a[j] = *reinterpret_cast<const float4*>(at + aoff[j]);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) r.b[j] = *reinterpret_cast<const float4*>(wt + boff[j]);
-    return r;
-  };
-  Share set[2];
-  auto fetch = [&](auto P, int tile) { set[decltype(P)::value] = load_share(tile); };
-  // LDS layouts: A tile as [m][BK + 4], W tile as [k][TN] with the two 32-column halves of a 64-column group
-  // swapped in rows with bit 2 set. Matrix instruction i of quarter q takes k = 8q + 4h + i from half-wave h, so a
-  // lane's four A values of a quarter are one 128-bit read of the unpermuted row, and the two half-waves of a W
-  // read (rows 8q + i and 8q + 4 + i) use different banks.
-  float* const adst = As + arow * AST + akq;
-  float* const bdst = Bs + brow * TN + (bnq ^ (((brow >> 2) & 1) << 5));  // rows + 16r have the same bit 2
-  auto stage = [&](auto P, int st) {  // set p -> LDS stage st
-    constexpr int p = decltype(P)::value;
-#pragma unroll
-    for (int j = 0; j < NA; ++j) st4(adst + st * (TM * AST) + 32 * j, set[p].a[j]);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) st4(bdst + st * (BK * TN) + 16 * j * TN, set[p].b[j]);
-  };
-  float av[HK], bv[HK];
-  const float* const asrc = As + (wm + l32) * AST + 4 * h;
-  const float* const bsrc = Bs + 4 * h * TN + ((wn + l32) ^ (h << 5));
-  auto operands = [&](int st) {  // the wave's operands of a whole K step
-#pragma unroll
-    for (int q = 0; q < HK / 4; ++q) {
-      const float4 v = ld4(asrc + st * (TM * AST) + 8 * q);
-      av[4 * q] = v.x; av[4 * q + 1] = v.y; av[4 * q + 2] = v.z; av[4 * q + 3] = v.w;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bv[4 * q + i] = bsrc[st * (BK * TN) + (8 * q + i) * TN];
-    }
-  };
-  f32x16 acc;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-  auto multiply = [&]() {
-#pragma unroll
-    for (int i = 0; i < HK; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], acc, 0, 0, 0);
-  };
-  const int n = n0 + wn + l32;
-  const float bvs = (bias && n < N) ? bias[n] : 0.f;  // requested early: the epilogue does not wait for it
-
-  typedef std::integral_constant<int, 0> P0;
-  typedef std::integral_constant<int, 1> P1;
-  // the matrix instructions touch registers only, so the scheduler would move them across a barrier into the
-  // memory phase and undo the alternation: pin both sides
-  auto phase_barrier = [&]() {
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // Tile j lives in LDS stage j & 1 and travels through register set j & 1. The two groups run separate
-  // loops with the same number of barriers (1 + 2 * nsteps), so that no value has to be merged between
-  // their code paths.
-  if (g == 0) {
-    // multiplies step k in the first half of iteration k; leads by two tiles: 0 and 1 staged, 2 and 3 in flight
-    fetch(P0(), 0);
-    fetch(P1(), 1);
-    const Share t2 = load_share(2), t3 = load_share(3);  // requested before the first two are waited for
-    stage(P0(), 0);
-    stage(P1(), 1);
-    set[0] = t2;
-    set[1] = t3;
-    phase_barrier();
-    operands(0);
-    auto iteration = [&](auto parity, int k) {
-      typedef decltype(parity) P;
-      multiply();  // step k
-      phase_barrier();
-      operands(1 - P::value);  // step k + 1
-      stage(P(), P::value);    // tile k + 2
-      fetch(P(), k + 4);
-      phase_barrier();
-    };
-    int k = 0;
-    for (; k + 1 < nsteps; k += 2) {
-      iteration(P0(), k);
-      iteration(P1(), k + 1);
-    }
-    if (k < nsteps) iteration(P0(), k);
-  } else {
-    // multiplies step k in the second half of iteration k; leads by one tile: 0 staged, 1 and 2 in flight
-    fetch(P0(), 0);
-    fetch(P1(), 1);
-    const Share t2 = load_share(2);
-    stage(P0(), 0);
-    set[0] = t2;
-    phase_barrier();
-    auto iteration = [&](auto parity, int k) {
-      typedef decltype(parity) P;
-      typedef std::integral_constant<int, 1 - P::value> Q;
-      operands(P::value);      // step k
-      stage(Q(), Q::value);    // tile k + 1
-      fetch(Q(), k + 3);
-      phase_barrier();
-      multiply();  // step k
-      phase_barrier();
-    };
-    int k = 0;
-    for (; k + 1 < nsteps; k += 2) {
-      iteration(P0(), k);
-      iteration(P1(), k + 1);
-    }
-    if (k < nsteps) iteration(P0(), k);
-  }
-
-  if (n < N) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = m0 + wm + (i >> 2) * 8 + h * 4 + (i & 3);
-      if (m < M) {
-        float v = acc[i] + bvs;
-        if (epi == EPI_GELU) v = gelu_ref(v);
-        else if (epi == EPI_RESIDUAL) v += resid[(size_t)m * ldc + n];
-        C[(size_t)m * ldc + n] = v;
-      }
-    }
-  }
 }
 
 // ResidualBlock, instructions.js:381-382
@@ -1132,6 +643,8 @@ constexpr int AMK = 32;        // keys per tile
 constexpr int AMKST = AHS + 4; // row stride of a staged K tile (conflict-free 128-bit reads by 32 rows)
 constexpr int AM_WAVE_FLOATS = AMK * AMKST + AMK * AHS;  // K tile + V tile of one wave
 constexpr int AMOST = AMQ + 1; // row stride of a wave's O^T[dim][query] in the merge
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int NWV>
 __global__ __launch_bounds__(NWV * 64) void attention_mfma_kernel(int Tq, int pos0, float scale, const float* __restrict__ q, int ldq,
@@ -2044,112 +1557,65 @@ void finish_split(int M, int N, int S, const float* workspace, const float* bias
   if (ln) layernorm_kernel<<<M, WG, 0, s>>>(N, C, ldc, ln->gamma, ln->beta, ln->out, ln->ldo);
 }
 
-// The same two follow-ups after a product that wrote C itself.
-void finish_direct(int M, int N, const float* C, int ldc, const LnAfter* ln, const KvAfter* kv, hipStream_t s) {
-  if (kv) kv_append_kernel<<<M, WG, 0, s>>>(kv->d, kv->hs, kv->ctx, kv->pos0, C, kv->Kc, kv->Vc);
-  if (ln) layernorm_kernel<<<M, WG, 0, s>>>(N, C, ldc, ln->gamma, ln->beta, ln->out, ln->ldo);
-}
-
-template <int TM, int TN, int BK, bool I8W>
-void run_gemm_mfma(int M, int N, int K, int S, const float* A, int lda, const void* W, int ldw, const float* wscale,
-                   const float* bias, float* C, int ldc, int epi, const float* resid, float* workspace, const LnAfter* ln,
-                   const KvAfter* kv, hipStream_t s) {
-  const dim3 grid(cdiv(N, TN), cdiv(M, TM), S);
-  // partial sums of the K slices are combined in ascending order by gemv_reduce (deterministic), bias last
-  const int kchunk = S == 1 ? K : (int)cdiv(cdiv(K, S), BK) * BK;
-  const bool exact = K % BK == 0;  // then every slice is whole steps (kchunk is a multiple of BK)
-  const float* kb = S == 1 ? bias : nullptr;
-  float* kc = S == 1 ? C : workspace;
-  const int kldc = S == 1 ? ldc : N, kepi = S == 1 ? epi : EPI_NONE;
-  const float* kres = S == 1 ? resid : nullptr;
-  if (exact) gemm_mfma<TM, TN, BK, I8W, true><<<grid, WG, 0, s>>>(M, N, K, kchunk, A, lda, W, ldw, wscale, kb, kc, kldc, kepi, kres);
-  else gemm_mfma<TM, TN, BK, I8W, false><<<grid, WG, 0, s>>>(M, N, K, kchunk, A, lda, W, ldw, wscale, kb, kc, kldc, kepi, kres);
-  if (S > 1) finish_split(M, N, S, workspace, bias, C, ldc, epi, resid, ln, kv, s);
-  else finish_direct(M, N, C, ldc, ln, kv, s);
-}
-
-// 128x128 tiles when they alone fill the 256 compute units twice over, else 64x64 (measured
-// best or within 3 % of it from 128 to 1024 rows); then split K (at most 8 ways, slices of
-// at least 128) until there are two workgroups per compute unit.
-template <bool I8W>
-void run_gemm(int M, int N, int K, const float* A, int lda, const void* W, int ldw, const float* wscale, const float* bias,
-              float* C, int ldc, int epi, const float* resid, float* workspace, const LnAfter* ln, const KvAfter* kv,
-              hipStream_t s) {
-  // 64 x 128 tiles of the two-group kernel when, with K split at most 4 ways, they give each of the 256
-  // compute units one workgroup (and at most two)
-  const size_t pp = (size_t)cdiv(M, 64) * cdiv(N, 128);
-  if (!I8W && K % PP_BK == 0 && pp >= 64) {
-    int S = 1;
-    while (workspace && S < 4 && pp * S < 256 && K / (2 * S) >= 128 && (K / (2 * S)) % PP_BK == 0) S *= 2;
-    // whole rounds of 256 workgroups, or nearly: a last round that leaves compute units idle costs as much as a full one
-    const size_t wgs = pp * S, rounds = cdiv(wgs, 256);
-    if (wgs * 100 >= rounds * 256 * 85 && wgs <= 1024) {
-      static const bool raised = [] {
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_pingpong<PP_BK>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)PP_LDS) == hipSuccess;
-      }();
-      if (raised) {
-        const dim3 grid(cdiv(N, 128), cdiv(M, 64), S);
-        const float* Wf = static_cast<const float*>(W);
-        if (S == 1) {
-          gemm_pingpong<PP_BK><<<grid, PP_THREADS, PP_LDS, s>>>(M, N, K, K, A, lda, Wf, ldw, bias, C, ldc, epi, resid);
-          finish_direct(M, N, C, ldc, ln, kv, s);
-        } else {
-          gemm_pingpong<PP_BK><<<grid, PP_THREADS, PP_LDS, s>>>(M, N, K, K / S, A, lda, Wf, ldw, nullptr, workspace, N, EPI_NONE, nullptr);
-          finish_split(M, N, S, workspace, bias, C, ldc, epi, resid, ln, kv, s);
-        }
-        return;
-      }
-    }
+// C = epi(A . W + bias) on the matrix cores; W fp32 [K, ldw], or words of four int8 with a scale per column.
+hipError_t run_gemm(int M, int N, int K, const float* A, int lda, const void* W, int ldw, const float* wscale, const float* bias,
+                    float* C, int ldc, int epi, const float* resid, float* workspace, const LnAfter* ln, const KvAfter* kv, hipStream_t s) {
+  const bool i8 = wscale != nullptr;
+  SplitGemmArgs a{};
+  a.N = N; a.K = K; a.lda = lda; a.W = W; a.ldw = ldw; a.wscale = wscale; a.bias = bias; a.epi = epi; a.ldc = ldc;
+  if (kv) { a.Kc = kv->Kc; a.Vc = kv->Vc; a.d = kv->d; a.hs = kv->hs; a.ctx = kv->ctx; }
+  // the kernels address A with 32-bit offsets: very tall matrices go in runs of rows
+  const int rows = (int)std::min<size_t>((size_t)M, (((size_t)1 << 31) - 4096) / (sizeof(float) * (size_t)lda));
+  if (rows < 1) return hipErrorInvalidValue;
+  for (int m0 = 0; m0 < M; m0 += rows) {
+    const int m = std::min(rows, M - m0);
+    const SplitPlan p = plan_gemm_split(m, N, K, i8, ln != nullptr, workspace != nullptr);
+    a.M = m;
+    a.A = A + (size_t)m0 * lda;
+    a.C = C + (size_t)m0 * ldc;
+    a.resid = resid ? resid + (size_t)m0 * ldc : nullptr;
+    a.pos0 = kv ? kv->pos0 + m0 : 0;
+    a.part = p.S > 1 ? workspace : nullptr;
+    const hipError_t e = launch_gemm_split(p, a, i8, s);
+    if (e != hipSuccess) return e;
+    KvAfter kv2;
+    if (kv) { kv2 = *kv; kv2.pos0 = a.pos0; }
+    LnAfter ln2;
+    if (ln) { ln2 = *ln; ln2.out = ln->out + (size_t)m0 * ln->ldo; }
+    if (p.S > 1) finish_split(m, N, p.S, workspace, bias, a.C, ldc, epi, a.resid, ln ? &ln2 : nullptr, kv ? &kv2 : nullptr, s);
+    else if (ln) layernorm_kernel<<<m, WG, 0, s>>>(N, a.C, ldc, ln2.gamma, ln2.beta, ln2.out, ln2.ldo);
   }
-  const bool big = (size_t)cdiv(M, 128) * cdiv(N, 128) >= 512;
-  const int t = big ? 128 : 64;
-  constexpr int BKS = 32;  // K step of gemm_mfma
-  int S = 1;
-  const size_t tiles = (size_t)cdiv(M, t) * cdiv(N, t);
-  while (workspace && S < 8 && tiles * S < 512 && K / (2 * S) >= 128) S *= 2;
-  if (workspace && M <= 448 && tiles <= 256) {
-    // Few rows: the workgroups of a launch all start together, one to a compute unit and a second one on some once
-    // there are more than 256 of them, and the launch lasts as long as the busiest unit. Any slice count that
-    // leaves whole K steps will do (three slices of c_attn at 128 rows are 216 workgroups of 8 steps, where four
-    // are 288 of 6, two of them on 32 units): the cheapest of rounds x (steps per slice + 4 for a round's prologue
-    // and epilogue). 117M T = 128: 0.895 -> 0.86 ms, T = 192: 1.07 -> 0.97; 1.5B T = 128: 6.67 -> 5.96; beyond
-    // ~450 rows several workgroups share a unit anyway and the doubling rule above measures better (T = 960:
-    // 2.56 against 2.63 ms).
-    long best = -1;
-    for (int c = 1; c <= 8; ++c) {
-      if (K % (BKS * c) != 0 || (c > 1 && K / c < 96)) continue;
-      const long cost = (long)cdiv(tiles * c, 256) * (K / (BKS * c) + 4);
-      if (best < 0 || cost < best) {
-        best = cost;
-        S = c;
-      }
-    }
-  }
-  if (big) run_gemm_mfma<128, 128, 32, I8W>(M, N, K, S, A, lda, W, ldw, wscale, bias, C, ldc, epi, resid, workspace, ln, kv, s);
-  else run_gemm_mfma<64, 64, 32, I8W>(M, N, K, S, A, lda, W, ldw, wscale, bias, C, ldc, epi, resid, workspace, ln, kv, s);
+  return hipGetLastError();
 }
 }  // namespace
 
 hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float* W, int ldw, const float* bias,
                        float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s, const LnAfter* ln,
                        const KvAfter* kv) {
-  if (M < 16) {
-    // too few rows for a matrix-core tile: scalar-FMA tile kernel
-    gemm_tile64<<<dim3(cdiv(N, 64), cdiv(M, 64)), WG, 0, s>>>(M, N, K, A, lda, W, ldw, bias, C, ldc, epi, resid);
-    finish_direct(M, N, C, ldc, ln, kv, s);
-    return hipGetLastError();
+  // the kernels address W with 32-bit offsets: a larger matrix goes in runs of rows whose products are added up
+  const int rows = (int)std::min<size_t>((size_t)K, (((size_t)1 << 31) - 4096) / (sizeof(float) * (size_t)ldw) / 4 * 4);
+  if (rows >= K) return run_gemm(M, N, K, A, lda, W, ldw, nullptr, bias, C, ldc, epi, resid, workspace, ln, kv, s);
+  if (rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  for (int k0 = 0; k0 < K; k0 += rows) {
+    const hipError_t e = run_gemm(M, N, std::min(rows, K - k0), A + k0, lda, W + (size_t)k0 * ldw, ldw, nullptr,
+                                  k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, s);
+    if (e != hipSuccess) return e;
   }
-  run_gemm<false>(M, N, K, A, lda, W, ldw, nullptr, bias, C, ldc, epi, resid, workspace, ln, kv, s);
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 hipError_t launch_gemm_i8(int M, int N, int K, const float* A, int lda, const int32_t* Wq, int ldwq, const float* scale,
                           const float* bias, float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
                           const LnAfter* ln, const KvAfter* kv) {
-  if (M < 16 || (N & 3)) return hipErrorInvalidValue;
-  run_gemm<true>(M, N, K, A, lda, Wq, ldwq, scale, bias, C, ldc, epi, resid, workspace, ln, kv, s);
-  return hipGetLastError();
+  const int rows = (int)std::min<size_t>((size_t)K, (((size_t)1 << 31) - 4096) / (sizeof(int32_t) * (size_t)ldwq) / 4 * 4);
+  if (rows >= K) return run_gemm(M, N, K, A, lda, Wq, ldwq, scale, bias, C, ldc, epi, resid, workspace, ln, kv, s);
+  if (rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  for (int k0 = 0; k0 < K; k0 += rows) {
+    const hipError_t e = run_gemm(M, N, std::min(rows, K - k0), A + k0, lda, Wq + (size_t)k0 * ldwq, ldwq, scale,
+                                  k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_residual(size_t n4, const float* a, const float* b, float* out, hipStream_t s) {

@@ -41,8 +41,7 @@ struct Model {
   // activations for up to maxT rows
   float *x = nullptr, *ln = nullptr, *qkv = nullptr, *att = nullptr, *tmp = nullptr, *h = nullptr;
   float* logits = nullptr;       // [V]
-  float* part = nullptr;         // GEMV partial sums
-  float* dq = nullptr;           // fp32 scratch for a dequantised int8 matrix (prefill)
+  float* part = nullptr;         // partial sums of the prefill products
   float* taps = nullptr;         // [(2+6L)][maxT][d]
   int32_t* tok_dev = nullptr;    // [maxT] token ids of the current call
   int32_t* out_tok_dev = nullptr;  // [ctx] ids chosen by the greedy loop

@@ -92,29 +92,8 @@ static bool parse_name(Model* m, const std::string& name, Slot* slot) {
 // With `ln` the LayerNorm that follows in the forward is applied to the finished rows as part of the product.
 static int linear(Model* m, int M, int N, int K, const float* A, int lda, const LinW& w, const float* bias, float* C,
                   int ldc, int epi, const float* resid, const LnAfter* ln = nullptr, const KvAfter* kv = nullptr) {
-  hipStream_t s = rt().stream;
-  hipError_t e;
-  bool ln_done = true;
-  if (w.q) {
-    if (M <= GEMV_MAX_ROWS) {
-      e = launch_gemv_kn_i8(M, N, K, A, lda, w.q, N / 4, w.s, bias, C, ldc, epi, resid, m->part, s);
-      ln_done = false;
-    } else if (M >= 16) {
-      e = launch_gemm_i8(M, N, K, A, lda, w.q, N / 4, w.s, bias, C, ldc, epi, resid, m->part, s, ln, kv);
-    } else {
-      e = launch_dequant_i8(K, N, w.q, N / 4, w.s, m->dq, N, s);
-      if (e == hipSuccess) e = launch_gemm(M, N, K, A, lda, m->dq, N, bias, C, ldc, epi, resid, m->part, s, ln, kv);
-    }
-  } else if (M <= GEMV_MAX_ROWS) {
-    e = launch_gemv_kn(M, N, K, A, lda, w.w, N, bias, C, ldc, epi, resid, m->part, s);
-    ln_done = false;
-  } else {
-    e = launch_gemm(M, N, K, A, lda, w.w, N, bias, C, ldc, epi, resid, m->part, s, ln, kv);
-  }
-  if (e == hipSuccess && !ln_done) {  // the matrix-vector kernels take no follow-ups
-    if (kv) e = launch_kv_append(M, kv->d, kv->hs, kv->ctx, kv->pos0, C, kv->Kc, kv->Vc, s);
-    if (e == hipSuccess && ln) e = launch_layernorm(M, N, C, ldc, ln->gamma, ln->beta, ln->out, ln->ldo, s);
-  }
+  const hipError_t e = w.q ? launch_gemm_i8(M, N, K, A, lda, w.q, N / 4, w.s, bias, C, ldc, epi, resid, m->part, rt().stream, ln, kv)
+                           : launch_gemm(M, N, K, A, lda, w.w, N, bias, C, ldc, epi, resid, m->part, rt().stream, ln, kv);
   if (e != hipSuccess) return fail(WGPT_ERR_HIP, "linear layer launch: %s", hipGetErrorString(e));
   return WGPT_OK;
 }
@@ -683,13 +662,8 @@ int wgpt_model_finalize(wgpt_model h) {
   if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(int32_t), (void**)&m->out_tok_dev))) return rc;
   if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(int32_t), (void**)&m->out_samp_dev))) return rc;
   if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(double), (void**)&m->u_dev))) return rc;
-  size_t ws = gemv_workspace_floats(GEMV_MAX_ROWS, 4 * (int)d, (int)d);
-  const size_t ws2 = gemv_workspace_floats(GEMV_MAX_ROWS, (int)d, 4 * (int)d);
-  if (ws2 > ws) ws = ws2;
-  const size_t ws3 = gemm_workspace_floats((int)T, 4 * (int)d);  // split-K partial sums of the prefill GEMMs
-  if (ws3 > ws) ws = ws3;
+  const size_t ws = gemm_workspace_floats((int)T, 4 * (int)d);  // partial sums of the prefill products
   if ((rc = dev_alloc(m, ws * f, (void**)&m->part))) return rc;
-  if (i8 && (rc = dev_alloc(m, d * 4 * d * f, (void**)&m->dq))) return rc;
   if ((m->p.flags & WGPT_FLAG_TAPS) && (rc = dev_alloc(m, (size_t)(2 + 6 * m->L) * T * d * f, (void**)&m->taps))) return rc;
   WGPT_HIP(hipMemsetAsync(m->kv, 0, (size_t)m->L * 2 * m->ctx * d * f, rt().stream));
   WGPT_HIP(hipEventCreate(&m->ev0));
