@@ -77,6 +77,56 @@ def test_device_selection_matches_oracle(device):
         buf.destroy()
 
 
+def hard_cases():
+    """Inputs on which the bound by the threads' maxima is weak or the candidates are many: equal values, values in order,
+    large values all with one thread, both zeros, infinities, more candidates than the fast sort takes."""
+    rng = np.random.default_rng(12)
+    n = lambda V: rng.standard_normal(V).astype(np.float32)
+    one = n(50257)
+    one[np.arange(0, 50257, 4096)] += 50.0                       # thread 0 holds the twelve largest
+    zeros = np.where(rng.random(5000) < 0.5, np.float32(0.0), np.float32(-0.0)).astype(np.float32)
+    inf = n(3000)
+    inf[[5, 7, 2000]] = np.inf
+    inf[[1, 2999]] = -np.inf
+    return [("equal", np.full(50257, 1.5, np.float32), 40), ("equal long", np.zeros(262144, np.float32), 7),
+            ("ascending", np.arange(50257, dtype=np.float32), 40), ("descending", -np.arange(65536, dtype=np.float32), 1024),
+            ("one thread", one, 40), ("two values", np.where(rng.random(50257) < 0.5, 1.0, 2.0).astype(np.float32), 1024),
+            ("zeros", zeros, 33), ("infinities", inf, 2998), ("k = 1024", n(50257), 1024), ("V = 4097", n(4097), 1023),
+            ("V = 65537", n(65537), 100), ("V = 262144", n(262144), 1024), ("k = V", n(700), 700), ("V = 3", n(3), 3)]
+
+
+def test_host_selection_is_a_stable_sort():
+    from webgpt_amd import sampling
+    for name, x, k in hard_cases() + [("short", np.array([1.0, 3.0, 3.0, 2.0], np.float32), 3)]:
+        want = np.argsort(-x.astype(np.float64), kind="stable")[:k]
+        got = sampling.selectTopK(x, k)
+        assert got["topKIndices"] == [int(i) for i in want], name
+        assert got["topKProbs"] == [float(v) for v in x[want]], name
+    assert sampling.selectTopK([0.5, 2, 1], 2) == {"topKIndices": [1, 2], "topKProbs": [2.0, 1.0]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,x,k", hard_cases(), ids=[c[0] for c in hard_cases()])
+def test_device_selection_of_hard_inputs(device, name, x, k):
+    from webgpt_amd import _lib, blocks
+    k = min(k, 1024)
+    buf = blocks.init_tensor(x, [x.size])
+    cid, ids, p = C.c_int32(-1), np.empty(k, np.int32), np.empty(k, np.float64)
+    for u in (0.0, 0.63):
+        _lib.call("wgpt_sample_topk", x.size, k, 0.9, u, buf.handle, C.byref(cid), ids.ctypes.data_as(C.POINTER(C.c_int32)),
+                  p.ctypes.data_as(C.POINTER(C.c_double)))
+        order = np.argsort(-x.astype(np.float64), kind="stable")[:k]
+        assert np.array_equal(ids, order)
+        if np.isfinite(x).all():
+            want_id, _, want_p = brute(x, k, 0.9, u)
+            # brute divides by the temperature before it subtracts the maximum: its exponents are off by a rounding of
+            # x / T each, 2**-53 of it; the rest is a few ulp of exp between libraries
+            rtol = 1e-12 + 4 * 2.0 ** -53 * float(np.abs(x[order]).max()) / 0.9
+            assert np.allclose(p, want_p, rtol=rtol, atol=0)
+            assert cid.value == want_id
+    buf.destroy()
+
+
 @pytest.mark.gpu
 def test_device_selection_rejects_bad_arguments(device):
     from webgpt_amd import _lib, blocks

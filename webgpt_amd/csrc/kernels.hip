@@ -1316,129 +1316,200 @@ __global__ __launch_bounds__(WG) void kv_append_kernel(int d, int hs, int ctx, i
   }
 }
 
-// Token selection of GPT.generate (model.js:81-85) on the device, one workgroup:
+// Token selection of GPT.generate (model.js:81-85) on the device:
 //   selectTopK (globals.js:66-74): stable descending sort of (value, index), first k;
-//     here k rounds of arg-max with the lowest index among equal values;
 //   cpuSoftmax (globals.js:59-64) of those k logits in float64:
 //     exp((x - max) / temperature), summed left to right, divided by the sum;
 //   sampleFromDistribution (globals.js:47-57): first i with u < p_0 + .. + p_i, else k - 1;
 //     u is the caller's uniform draw in [0, 1) (the reference's Math.random()).
 // The chosen id goes to tok[0] (input of the next decode step) and out[slot]; ids/probs
 // (optional) receive the k selected indices and their probabilities.
-__device__ __forceinline__ bool better(float ov, int oi, float cv, int ci) {
-  return oi != 0x7fffffff && (ci == 0x7fffffff || ov > cv || (ov == cv && oi < ci));
+// A logit and its index as one number whose order is the selection's: larger value first, lower index among equals
+// (-0 and 0 are equal; NaN comes last).
+typedef unsigned long long sel_key;
+__device__ __forceinline__ unsigned order_bits(float v) {
+  const unsigned b = __float_as_uint(v + 0.0f);
+  return v != v ? 0u : (b & 0x80000000u ? ~b : b | 0x80000000u);
+}
+__device__ __forceinline__ sel_key make_key(float v, int i) { return (sel_key)order_bits(v) << 32 | (0xffffffffu - (unsigned)i); }
+__device__ __forceinline__ float key_value(sel_key k) {
+  const unsigned b = (unsigned)(k >> 32);
+  return b == 0u ? NAN : __uint_as_float(b & 0x80000000u ? b & 0x7fffffffu : ~b);
+}
+__device__ __forceinline__ int key_index(sel_key k) { return (int)(0xffffffffu - (unsigned)k); }
+
+// x[lane] of the wave, lane uniform
+__device__ __forceinline__ double wave_read(double x, int lane) {
+  const unsigned long long b = __double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
+  return __longlong_as_double((unsigned long long)hi << 32 | lo);
 }
 
-// REG: the logits of a thread's stride (V <= 65536: at most 64 of them) stay in registers, so the
-// owner's search for its next candidate after a selection touches no memory.
-template <bool REG>
+// One workgroup. A bound below which the k largest logits cannot lie is the k-th largest of the threads' maxima, or a little
+// less; the logits not below it are k candidates or some more (normal logits, V = 50257, k = 40: about 60), and only they are
+// sorted: by counting, for each, the larger ones, or with a bitonic network when they are many. Reading the logits is 4 us of
+// a launch (58 KB/us is what a compute unit gets): 13 us for V = 50257 and k = 40, where k rounds of a workgroup-wide arg-max
+// took 165.
+// Logits that leave more candidates than LDS holds (long runs of equal values) get the exact bound first, one bit at a time.
+constexpr int SAMPLE_CAND = 8192, SAMPLE_RANK = 256;
+template <bool REG>  // REG: V <= 65536, a thread's logits stay in registers between the two looks at them
 __global__ __launch_bounds__(1024) void sample_topk_kernel(int V, int k, double temperature, const double* __restrict__ u,
                                                             const float* __restrict__ logits, int32_t* tok, int32_t* out, int slot,
                                                             int32_t* ids, double* probs) {
-  __shared__ unsigned taken[SAMPLE_MAX_V / 32];
-  __shared__ float wv[16];
-  __shared__ int wi[16];
-  __shared__ float sel_v[SAMPLE_MAX_K];
-  __shared__ int sel_i[SAMPLE_MAX_K];
+  extern __shared__ __attribute__((aligned(16))) sel_key cand[];  // [SAMPLE_CAND]
   __shared__ double ev[SAMPLE_MAX_K];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (!REG)
-    for (int i = tid; i < (V + 31) / 32; i += 1024) taken[i] = 0u;
+  __shared__ double total;
+  __shared__ float bound;
+  __shared__ int count;
+  const int tid = threadIdx.x, lane = tid & 63;
   if (k > V) k = V;
-  float mine[REG ? 64 : 1];
-  unsigned long long gone = 0ull;  // REG: bit j set once element tid + 1024 j has been selected
-  if (REG) {
+  constexpr int RJ = REG ? 16 : 1;
+  float4 mine[RJ];
+  const auto fetch = [&](int j) {  // logits 4 (tid + 1024 j) ..
+    const int i = 4 * (tid + 1024 * j);
+    if (i + 3 < V) return ld4(logits + i);
+    return make_float4(i < V ? logits[i] : NAN, i + 1 < V ? logits[i + 1] : NAN, i + 2 < V ? logits[i + 2] : NAN, NAN);
+  };
+  // f(value, index) for every logit of this thread (and NAN for places beyond the last)
+  const auto each = [&](auto f) {
+    const auto four = [&](const float4& v, int j) {
+      const int i = 4 * (tid + 1024 * j);
+      f(v.x, i);
+      f(v.y, i + 1);
+      f(v.z, i + 2);
+      f(v.w, i + 3);
+    };
+    if constexpr (REG) {
 #pragma unroll
-    for (int j = 0; j < 64; ++j) mine[j] = tid + 1024 * j < V ? logits[tid + 1024 * j] : -INFINITY;
-  }
-  // this thread's candidate: the best not yet taken element of its stride
-  auto scan = [&](float& best, int& besti) {
-    best = -INFINITY;
-    besti = 0x7fffffff;
-    if (REG) {
-#pragma unroll
-      for (int j = 0; j < 64; ++j) {
-        const int i = tid + 1024 * j;
-        if (i < V && !((gone >> j) & 1ull) && (mine[REG ? j : 0] > best || besti == 0x7fffffff)) {
-          best = mine[REG ? j : 0];
-          besti = i;
-        }
-      }
-      return;
-    }
-    for (int i = tid; i < V; i += 1024) {
-      if (taken[i >> 5] & (1u << (i & 31))) continue;
-      const float v = logits[i];
-      if (v > best || besti == 0x7fffffff) {
-        best = v;
-        besti = i;
-      }
+      for (int j = 0; j < RJ; ++j) four(mine[j], j);
+    } else {
+      for (int j = 0; 4096 * j < V; ++j) four(fetch(j), j);
     }
   };
-  __syncthreads();
-  float best;
-  int besti;
-  scan(best, besti);
-  for (int r = 0; r < k; ++r) {
-    float cv = best;
-    int ci = besti;
+  if constexpr (REG) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(cv, off);
-      const int oi = __shfl_xor(ci, off);
-      if (better(ov, oi, cv, ci)) {
-        cv = ov;
-        ci = oi;
-      }
+    for (int j = 0; j < RJ; ++j) mine[j] = fetch(j);
+  }
+  if (tid == 0) count = 0;
+  float top = -INFINITY;
+  each([&](float v, int) { top = fmaxf(top, v); });
+  unsigned* tops = reinterpret_cast<unsigned*>(cand);
+  tops[tid] = order_bits(top);
+  __syncthreads();
+  if (tid < 64) {
+    unsigned m[16], least = 0u;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) m[j] = tops[lane + 64 * j];
+    for (int bit = 31; bit >= 0; --bit) {
+      const unsigned trial = least | 1u << bit;
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) n += __popcll(__ballot(m[j] >= trial));
+      if (n < k) continue;
+      least = trial;
+      if (n <= k + k / 2 + 16 && n < 512) break;  // near enough
     }
-    if (lane == 0) {
-      wv[wave] = cv;
-      wi[wave] = ci;
+    // (the bits of -infinity are the least that a maximum has; with a shorter prefix every logit is a candidate)
+    const unsigned low = order_bits(-INFINITY);
+    if (tid == 0) bound = key_value((sel_key)(least < low ? low : least) << 32);
+  }
+  __syncthreads();
+  const float least = bound;
+  each([&](float v, int i) {
+    if (v >= least) {
+      const int at = atomicAdd(&count, 1);
+      if (at < SAMPLE_CAND) cand[at] = make_key(v, i);
+    }
+  });
+  __syncthreads();
+  if (count > SAMPLE_CAND || count < k) {  // (fewer than k: NaN among the logits)
+    // the exact k-th largest key, from its highest bit down: keys are distinct, so exactly k are not below it
+    sel_key exact = 0;
+    for (int bit = 63; bit >= 0; --bit) {
+      const sel_key trial = exact | (sel_key)1 << bit;
+      int n = 0;
+      each([&](float v, int i) { n += i < V && make_key(v, i) >= trial; });
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+      __syncthreads();
+      if (tid == 0) count = 0;
+      __syncthreads();
+      if (lane == 0) atomicAdd(&count, n);
+      __syncthreads();
+      if (count >= k) exact = trial;
     }
     __syncthreads();
-    cv = wv[0];
-    ci = wi[0];
-#pragma unroll
-    for (int w = 1; w < 16; ++w)
-      if (better(wv[w], wi[w], cv, ci)) {
-        cv = wv[w];
-        ci = wi[w];
-      }
-    // every thread knows the winner; its owner marks it and looks for its next candidate
-    if (tid == 0) {
-      sel_v[r] = cv;
-      sel_i[r] = ci;
-    }
-    if ((ci & 1023) == tid) {
-      if (REG) gone |= 1ull << (ci >> 10);
-      else taken[ci >> 5] |= 1u << (ci & 31);
-      scan(best, besti);
-    }
+    if (tid == 0) count = 0;
+    __syncthreads();
+    each([&](float v, int i) {
+      if (i < V && make_key(v, i) >= exact) cand[atomicAdd(&count, 1)] = make_key(v, i);
+    });
     __syncthreads();
   }
-  if (tid == 0) {
-    const double mx = (double)sel_v[0];
+  const int n = count;
+  if (n <= SAMPLE_RANK) {
+    const sel_key x = tid < n ? cand[tid] : 0;
+    int rank = 0;
+    if (tid < n)
+      for (int i = 0; i < n; ++i) rank += cand[i] > x;
+    __syncthreads();
+    if (tid < n) cand[rank] = x;
+  } else {
+    int size2 = 512;
+    while (size2 < n) size2 <<= 1;
+    for (int i = n + tid; i < size2; i += 1024) cand[i] = 0;
+    __syncthreads();
+    for (int size = 2; size <= size2; size <<= 1)
+      for (int j = size >> 1; j > 0; j >>= 1) {
+        for (int p = tid; p < size2 / 2; p += 1024) {
+          const int a = 2 * p - (p & (j - 1)), b = a + j;
+          const sel_key x = cand[a], y = cand[b];
+          if ((y > x) == ((a & size) == 0)) {
+            cand[a] = y;
+            cand[b] = x;
+          }
+        }
+        __syncthreads();
+      }
+  }
+  __syncthreads();
+  const double mx = (double)key_value(cand[0]);
+  if (tid < k) ev[tid] = exp(((double)key_value(cand[tid]) - mx) / temperature);
+  __syncthreads();
+  if (tid < 64) {  // left to right, as cpuSoftmax adds them
     double sum = 0.0;
-    for (int i = 0; i < k; ++i) {
-      ev[i] = exp(((double)sel_v[i] - mx) / temperature);
-      sum += ev[i];
+    for (int base = 0; base < k; base += 64) {
+      const double mine64 = base + lane < k ? ev[base + lane] : 0.0;
+      const int m = k - base < 64 ? k - base : 64;
+      for (int i = 0; i < m; ++i) sum += wave_read(mine64, i);
     }
+    if (tid == 0) total = sum;
+  }
+  __syncthreads();
+  if (tid < k) {
+    const double p = ev[tid] / total;
+    ev[tid] = p;
+    if (probs) probs[tid] = p;
+    if (ids) ids[tid] = key_index(cand[tid]);
+  }
+  __syncthreads();
+  if (tid < 64) {
     const double rnd = *u;
     double cum = 0.0;
-    int pick = k - 1;
-    bool found = false;
-    for (int i = 0; i < k; ++i) {
-      const double p = ev[i] / sum;
-      if (probs) probs[i] = p;
-      if (ids) ids[i] = sel_i[i];
-      cum += p;
-      if (!found && rnd < cum) {
-        pick = i;
-        found = true;
+    int pick = -1;
+    for (int base = 0; base < k && pick < 0; base += 64) {
+      const double mine64 = base + lane < k ? ev[base + lane] : 0.0;
+      const int m = k - base < 64 ? k - base : 64;
+      for (int i = 0; i < m && pick < 0; ++i) {
+        cum += wave_read(mine64, i);
+        if (rnd < cum) pick = base + i;
       }
     }
-    tok[0] = sel_i[pick];
-    if (out) out[slot] = sel_i[pick];
+    if (pick < 0) pick = k - 1;
+    if (tid == 0) {
+      tok[0] = key_index(cand[pick]);
+      if (out) out[slot] = key_index(cand[pick]);
+    }
   }
 }
 
@@ -1705,8 +1776,11 @@ hipError_t launch_kv_append(int T, int d, int hs, int ctx, int pos0, const float
 hipError_t launch_sample_topk(int V, int k, double temperature, const double* u, const float* logits, int32_t* tok,
                               int32_t* out, int slot, int32_t* ids, double* probs, hipStream_t s) {
   if (V < 1 || V > SAMPLE_MAX_V || k < 1 || k > SAMPLE_MAX_K) return hipErrorInvalidValue;
-  if (V <= 65536) sample_topk_kernel<true><<<1, 1024, 0, s>>>(V, k, temperature, u, logits, tok, out, slot, ids, probs);
-  else sample_topk_kernel<false><<<1, 1024, 0, s>>>(V, k, temperature, u, logits, tok, out, slot, ids, probs);
+  constexpr size_t lds = sizeof(sel_key) * SAMPLE_CAND;
+  const auto kernel = V <= 65536 ? sample_topk_kernel<true> : sample_topk_kernel<false>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  kernel<<<1, 1024, lds, s>>>(V, k, temperature, u, logits, tok, out, slot, ids, probs);
   return hipGetLastError();
 }
 
