@@ -114,6 +114,37 @@ def test_split_matmul_error_bound(device, int8, M, N, K):
     assert np.linalg.norm(got - want) <= 2.0 ** -24 * max(4.0, K ** 0.5) * np.linalg.norm(size)
 
 
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("M,N,K", [(5, 8, 4), (17, 40, 100), (33, 768, 3072), (130, 136, 256)])
+def test_split_matmul_not_finite(device, int8, M, N, K):
+    """Operands without a three-way bf16 split (infinite ones, and those within half a bf16 ulp of the largest float) give
+    what fp32 products give; all other values stay small integers, whose sums are exact."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(1, 5, (M, K)).astype(np.float32)
+    q = rng.integers(1, 5, (K, N)) * rng.choice([-1, 1], (1, N))
+    q[1], q[:, 5] = np.sign(q[1]), np.abs(q[:, 5])  # the large values meet ones, and each other with one sign: one reading
+    A[:, K - 1] = 1
+    w = q.astype(np.float32)
+    A[0, K - 1], A[1, 0], A[2, K // 2], A[3, 1] = np.inf, -np.inf, np.nan, np.float32(3.4e38)
+    if int8:
+        q[0, 3] = 0  # inf times zero
+        w = q.astype(np.float32)
+        inst = FastMatMulBlock.newInt8Instance(M, N, K, init_tensor(A, [M, K]), init_tensor(pack_words(q), [K, N // 4]),
+                                               init_tensor(np.full(N, 127, np.float32), [N]), init_tensor(np.zeros(N, np.float32), [N]))
+    else:
+        w[1, 2], w[K - 1, 5] = -np.inf, np.float32(3.4e38)
+        inst = FastMatMulBlock.newInstance(M, N, K, init_tensor(A, [M, K]), init_tensor(w, [K, N]), init_tensor(np.zeros(N, np.float32), [N]))
+    got = run(inst, (M, N))
+    with np.errstate(all="ignore"):
+        want = np.zeros((M, N), np.float32)  # products and sums rounded to fp32, as far as infinities go
+        for k in range(K):
+            want = (want + A[:, k:k + 1] * w[k:k + 1]).astype(np.float32)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    assert np.allclose(got[fin], want[fin], rtol=1e-6, atol=0)
+
+
 def test_fast_matmul_exact_and_preconditions(device):
     A = RNG.integers(-8, 9, (3, 12)).astype(np.float32)
     W = RNG.integers(-8, 9, (12, 16)).astype(np.float32)

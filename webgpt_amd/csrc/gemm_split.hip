@@ -5,8 +5,9 @@
 // taken, all of them exact in the fp32 accumulator's input. The three left out (mid lo, lo mid, lo lo) are together below
 // 2^-25 |x y|, under half an ulp of the product; with sums of sixteen products rounded once instead of two at a time the
 // result is at least as close to the exact one as that of v_mfma_f32_32x32x2_f32. An int8 weight is one bf16 value
-// (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum. Infinities
-// are the one thing that is not carried over: inf = inf + nan + nan, so an infinite operand gives NaN.
+// (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum. A value that is
+// infinite, or rounds to an infinite bf16, has no such split (inf + nan + nan): every sum it takes part in comes out as NaN
+// or infinite, and sums that do are taken again without the split (plain_products).
 // bf16 runs at 16 times the rate of fp32 here, six products are therefore 2.7 times (int8: 5.3 times) faster.
 #include "gemm_split.h"
 
@@ -156,9 +157,34 @@ struct ARaw {
   __device__ __forceinline__ Split8 get(int s) const { return split8(v[2 * s], v[2 * s + 1]); }
 };
 
-__device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v, bool i8) {
+// Row m times columns n..n+3 over the k of a slice, one fp32 product after the other: for sums with operands that cannot be
+// split. Slow (a thread reads everything itself), and only they pay for it.
+template <bool I8>
+__device__ __attribute__((noinline)) f32x4 plain_products(const SplitGemmArgs& a, int m, int n, int slice) {
+  const int steps = a.K >> 5;
+  const int k0 = 32 * (int)((long)steps * slice / a.S), k1 = slice == a.S - 1 ? a.K : 32 * (int)((long)steps * (slice + 1) / a.S);
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  for (int k = k0; k < k1; ++k) {
+    const float x = a.A[(size_t)m * a.lda + k];
+    f32x4 w;
+    if constexpr (I8) {
+      const int word = static_cast<const int*>(a.W)[(size_t)k * a.ldw + (n >> 2)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = (float)((int)((unsigned)word << (24 - 8 * i)) >> 24);
+    } else {
+      w = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.W) + (size_t)k * a.ldw + n);
+    }
+    v += x * w;
+  }
+  return v;
+}
+
+template <bool I8>
+__device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v) {
   if (m >= a.M || n >= a.N) return;
-  if (i8) {
+  const float check = (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]);  // 0, or NaN if one is not finite
+  if (check != 0.f) v = plain_products<I8>(a, m, n, slice);
+  if constexpr (I8) {
     const f32x4 s = *reinterpret_cast<const f32x4*>(a.wscale + n);
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] *= s[i] / 127.0f;
@@ -221,7 +247,7 @@ __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4*
 #pragma unroll
     for (int u = 1; u < NP; ++u) v += red[u * ENT * 64 + e];
     const int ln = e & 63, b = e >> 6, q = b % Q, ij = b / Q;
-    split_epilogue(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v, I8);
+    split_epilogue<I8>(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v);
   }
 }
 
