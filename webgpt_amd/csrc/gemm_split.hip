@@ -102,32 +102,71 @@ __device__ __forceinline__ f32x4 buf_f4(__amdgpu_buffer_rsrc_t b, int v, int s) 
 template <int R>
 __device__ __forceinline__ int chunk_of(int s, int kg) { return R == 32 ? 2 * s + kg : kg; }
 
-// [K, N] as the caller's matrices come: one row of 32 (or 16) columns per load
-template <int R, bool I8>
+// W as the caller's matrices come, [K, N]: one row of 32 (or 16) columns per load. BLK: as a model keeps it (block_weights),
+// [K / 4][N][4] floats or [K / 8][N][8] int8: a lane's eight consecutive k in two (one) loads of 16 (8) bytes, neighbours
+// next to each other. A compute unit takes a load instruction every 10-15 ns whatever its width; a step of 32 k is four (two)
+// of them instead of sixteen. Cold weights, best shape of each: int8 300x6400x1600 37.9 -> 25.8 us, 943x6400x1600 97.0 ->
+// 64.8 us, 16x4800x1600 8.7 -> 7.4 us; fp32, where the splitting of W costs more than its loads, 128x3072x768 11.5 -> 10.2 us,
+// 16x3072x1024 8.9 -> 7.0 us, 943x3072x768 37.2 -> 36.9 us.
+template <int R, bool I8, bool BLK>
 struct WRaw {
   static constexpr int STEPS = R == 32 ? 2 : 1;
-  unsigned v[8 * STEPS];
-  static __device__ __forceinline__ int offset(const SplitGemmArgs& a, int n, int kg) { return 4 * ((I8 ? n >> 2 : n) + kg * 8 * a.ldw); }
-  __device__ __forceinline__ void load(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int off, int it) {
-#pragma unroll
-    for (int i = 0; i < 8 * STEPS; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b32(b, off, 4 * (it * 32 + (i >> 3) * 16 + (i & 7)) * a.ldw, 0);
+  unsigned v[BLK && I8 ? 2 * STEPS : 8 * STEPS];
+  static __device__ __forceinline__ int offset(const SplitGemmArgs& a, int n, int kg) {
+    if constexpr (BLK) return I8 ? 8 * (n + kg * a.N) : 16 * (n + kg * 2 * a.N);
+    else return 4 * ((I8 ? n >> 2 : n) + kg * 8 * a.ldw);
   }
-  // the step that reaches beyond K: rows past the last one repeat it (their A is zero)
-  __device__ __forceinline__ void load_tail(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int n, int kg, int it) {
+  __device__ __forceinline__ void load(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int off, int it) {
+    if constexpr (BLK && I8) {
 #pragma unroll
-    for (int i = 0; i < 8 * STEPS; ++i) {
-      const int k = it * 32 + chunk_of<R>(i >> 3, kg) * 8 + (i & 7);
-      v[i] = __builtin_amdgcn_raw_buffer_load_b32(b, 4 * ((I8 ? n >> 2 : n) + (k < a.K ? k : a.K - 1) * a.ldw), 0, 0);
+      for (int s = 0; s < STEPS; ++s) put2(s, __builtin_amdgcn_raw_buffer_load_b64(b, off, 8 * (it * 4 + 2 * s) * a.N, 0));
+    } else if constexpr (BLK) {
+#pragma unroll
+      for (int i = 0; i < 2 * STEPS; ++i) put4(i, __builtin_amdgcn_raw_buffer_load_b128(b, off, 16 * (it * 8 + (i >> 1) * 4 + (i & 1)) * a.N, 0));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8 * STEPS; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b32(b, off, 4 * (it * 32 + (i >> 3) * 16 + (i & 7)) * a.ldw, 0);
     }
   }
+  // the step that reaches beyond K: rows (runs of eight, K a multiple of eight) past the last one repeat it (their A is zero)
+  __device__ __forceinline__ void load_tail(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t b, int n, int kg, int it) {
+    if constexpr (BLK) {
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        const int c = it * 4 + chunk_of<R>(s, kg), last = (a.K >> 3) - 1, u = c < last ? c : last;
+        if constexpr (I8) {
+          put2(s, __builtin_amdgcn_raw_buffer_load_b64(b, 8 * (u * a.N + n), 0, 0));
+        } else {
+          put4(2 * s, __builtin_amdgcn_raw_buffer_load_b128(b, 16 * (2 * u * a.N + n), 0, 0));
+          put4(2 * s + 1, __builtin_amdgcn_raw_buffer_load_b128(b, 16 * ((2 * u + 1) * a.N + n), 0, 0));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8 * STEPS; ++i) {
+        const int k = it * 32 + chunk_of<R>(i >> 3, kg) * 8 + (i & 7);
+        v[i] = __builtin_amdgcn_raw_buffer_load_b32(b, 4 * ((I8 ? n >> 2 : n) + (k < a.K ? k : a.K - 1) * a.ldw), 0, 0);
+      }
+    }
+  }
+  __device__ __forceinline__ void put2(int i, u32x2 x) { v[2 * i] = x[0], v[2 * i + 1] = x[1]; }
+  __device__ __forceinline__ void put4(int i, u32x4 x) { v[4 * i] = x[0], v[4 * i + 1] = x[1], v[4 * i + 2] = x[2], v[4 * i + 3] = x[3]; }
   __device__ __forceinline__ Split8 get(int s, int n) const {
     if constexpr (I8) {
-      const int sh = 24 - 8 * (n & 3);
       Split8 r;
       unsigned h[4];
+      if constexpr (BLK) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        h[i] = bf16_pair((float)((int)(v[8 * s + 2 * i] << sh) >> 24), (float)((int)(v[8 * s + 2 * i + 1] << sh) >> 24));
+        for (int i = 0; i < 4; ++i) {
+          const unsigned x = v[2 * s + (i >> 1)], sh = 16 * (i & 1);
+          h[i] = bf16_pair((float)((int)(x << (24 - sh)) >> 24), (float)((int)(x << (16 - sh)) >> 24));
+        }
+      } else {
+        const int sh = 24 - 8 * (n & 3);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          h[i] = bf16_pair((float)((int)(v[8 * s + 2 * i] << sh) >> 24), (float)((int)(v[8 * s + 2 * i + 1] << sh) >> 24));
+      }
       r.hi = u32x4{h[0], h[1], h[2], h[3]};
       return r;
     } else {
@@ -159,15 +198,22 @@ struct ARaw {
 
 // Row m times columns n..n+3 over the k of a slice, one fp32 product after the other: for sums with operands that cannot be
 // split. Slow (a thread reads everything itself), and only they pay for it.
-template <bool I8>
-__device__ __attribute__((noinline)) f32x4 plain_products(const SplitGemmArgs& a, int m, int n, int slice) {
+// (Inlined: a call would cost every launch of these kernels 5 us, for the stack that it needs.)
+template <bool I8, bool BLK>
+__device__ __forceinline__ f32x4 plain_products(const SplitGemmArgs& a, int m, int n, int slice) {
   const int steps = a.K >> 5;
   const int k0 = 32 * (int)((long)steps * slice / a.S), k1 = slice == a.S - 1 ? a.K : 32 * (int)((long)steps * (slice + 1) / a.S);
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
   for (int k = k0; k < k1; ++k) {
     const float x = a.A[(size_t)m * a.lda + k];
     f32x4 w;
-    if constexpr (I8) {
+    if constexpr (BLK) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        w[i] = I8 ? (float)static_cast<const signed char*>(a.W)[((size_t)(k >> 3) * a.N + n + i) * 8 + (k & 7)]
+                  : static_cast<const float*>(a.W)[((size_t)(k >> 2) * a.N + n + i) * 4 + (k & 3)];
+    } else if constexpr (I8) {
       const int word = static_cast<const int*>(a.W)[(size_t)k * a.ldw + (n >> 2)];
 #pragma unroll
       for (int i = 0; i < 4; ++i) w[i] = (float)((int)((unsigned)word << (24 - 8 * i)) >> 24);
@@ -179,11 +225,11 @@ __device__ __attribute__((noinline)) f32x4 plain_products(const SplitGemmArgs& a
   return v;
 }
 
-template <bool I8>
+template <bool I8, bool BLK>
 __device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v) {
   if (m >= a.M || n >= a.N) return;
   const float check = (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]);  // 0, or NaN if one is not finite
-  if (check != 0.f) v = plain_products<I8>(a, m, n, slice);
+  if (check != 0.f) v = plain_products<I8, BLK>(a, m, n, slice);
   if constexpr (I8) {
     const f32x4 s = *reinterpret_cast<const f32x4*>(a.wscale + n);
 #pragma unroll
@@ -238,7 +284,7 @@ __device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Spl
 }
 
 // sum of NP partial tiles (LDS, 64 float4 per entry) and epilogue
-template <int R, int MB, int NB, int NP, int THREADS, bool I8>
+template <int R, int MB, int NB, int NP, int THREADS, bool I8, bool BLK>
 __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4* red, int m0, int n0, int slice) {
   typedef SplitBlock<R> B;
   constexpr int Q = B::NACC / 4, ENT = MB * NB * Q;
@@ -247,7 +293,7 @@ __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4*
 #pragma unroll
     for (int u = 1; u < NP; ++u) v += red[u * ENT * 64 + e];
     const int ln = e & 63, b = e >> 6, q = b % Q, ij = b / Q;
-    split_epilogue<I8>(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v);
+    split_epilogue<I8, BLK>(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v);
   }
 }
 
@@ -257,10 +303,10 @@ __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4*
 // instructions per two values split). Dependent launches, cold weights: 13x2304x768 5.5 us, 13x768x3072 in four slices 5.1 us
 // (219 and 193 us with the fp32 tile kernel that served 5 to 15 rows before); 64x64 tiles: 512x4096x1024 32.4 us = 132
 // TFLOP/s (39.9 us with v_mfma_f32_32x32x2_f32), int8 300x6400x1600 38.8 us (73).
-template <int R, int MB, int NB, int NW, bool I8>
+template <int R, int MB, int NB, int NW, bool I8, bool BLK>
 __global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
   typedef SplitBlock<R> B;
-  constexpr int STEPS = WRaw<R, I8>::STEPS, Q = B::NACC / 4, ENT = MB * NB * Q;
+  constexpr int STEPS = WRaw<R, I8, BLK>::STEPS, Q = B::NACC / 4, ENT = MB * NB * Q;
   extern __shared__ __attribute__((aligned(16))) float gs_lds[];
   int m0, n0, slice;
   if (!tile_of(a, m0, n0, slice)) return;
@@ -275,7 +321,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
     nn[j] = n0 + j * R + r < a.N ? n0 + j * R + r : a.N - 1;
-    wo[j] = WRaw<R, I8>::offset(a, nn[j], kg);
+    wo[j] = WRaw<R, I8, BLK>::offset(a, nn[j], kg);
   }
 #pragma unroll
   for (int i = 0; i < MB; ++i) xo[i] = ARaw<R>::offset(a, m0 + i * R + r, kg);
@@ -286,7 +332,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < B::NACC; ++e) acc[i][j][e] = 0.f;
-  WRaw<R, I8> w[NB];
+  WRaw<R, I8, BLK> w[NB];
   ARaw<R> x[MB];
   Split8 ws[STEPS][NB], xs[STEPS][MB];
   auto fetch = [&](int it) {
@@ -330,7 +376,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
       for (int q = 0; q < Q; ++q)
         red[(wave * ENT + (i * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  finish_tile<R, MB, NB, NW, NW * 64, I8>(a, red, m0, n0, slice);
+  finish_tile<R, MB, NB, NW, NW * 64, I8, BLK>(a, red, m0, n0, slice);
 }
 
 __device__ __forceinline__ void lds_barrier() {  // orders LDS accesses only: loads from memory stay in flight
@@ -344,7 +390,7 @@ __device__ __forceinline__ void lds_barrier() {  // orders LDS accesses only: lo
 // step have the splitting of the next one between them. Half the traffic from L2 of the kernel above per product (a
 // compute unit takes 58 KB/us from there): 1024x4096x1024 in 128x128 tiles 54.4 us = 158 TFLOP/s, where 64x64 tiles of the
 // other take 61; 32x64 tiles for 65 to 128 rows: 100x3072x768 10.9 us against 12.5.
-template <int MB, int NB, int NWN, int KG, bool I8, int OCC, int D>
+template <int MB, int NB, int NWN, int KG, bool I8, bool BLK, int OCC, int D>
 __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmArgs a) {
   constexpr int R = 32;
   typedef SplitBlock<R> B;
@@ -371,7 +417,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
   for (int j = 0; j < NB; ++j) {
     const int n = n0 + (wn * NB + j) * R + r;
     nn[j] = n < a.N ? n : a.N - 1;
-    wo[j] = WRaw<R, I8>::offset(a, nn[j], kg);
+    wo[j] = WRaw<R, I8, BLK>::offset(a, nn[j], kg);
   }
 #pragma unroll
   for (int v = 0; v < AV; ++v) {
@@ -387,7 +433,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
 #pragma unroll
       for (int e = 0; e < B::NACC; ++e) acc[i][j][e] = 0.f;
   static_assert(D % 2 == 0, "the buffer of a step is a constant of the unrolled loop");
-  WRaw<R, I8> w[D][NB];
+  WRaw<R, I8, BLK> w[D][NB];
   f32x4 x[D][AV][2];
   Split8 ws[2][2][NB];
   const auto clamp_step = [&](int i) { const int t = s0 + i * KG + grp; return t < s1 ? t : s1 - 1; };
@@ -503,29 +549,48 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
       for (int q = 0; q < Q; ++q)
         red[(grp * ENT + (i * NBW + wn * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  finish_tile<R, MB, NBW, KG, NWN * KG * 64, I8>(a, red, m0, n0, slice);
+  finish_tile<R, MB, NBW, KG, NWN * KG * 64, I8, BLK>(a, red, m0, n0, slice);
+}
+
+// [K, N] to the order that WRaw<.., BLK> reads; a thread makes one run of four (int8: eight) k of a column.
+__global__ __launch_bounds__(256) void block_weights_f32(int K, int N, const float* __restrict__ W, f32x4* __restrict__ out) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)(K >> 2) * N) return;
+  const size_t k = i / N * 4, n = i % N;
+  out[i] = f32x4{W[k * N + n], W[(k + 1) * N + n], W[(k + 2) * N + n], W[(k + 3) * N + n]};
+}
+__global__ __launch_bounds__(256) void block_weights_i8(int K, int N, const signed char* __restrict__ W, u32x2* __restrict__ out) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)(K >> 3) * N) return;
+  const size_t k = i / N * 8, n = i % N;
+  u32x2 v = {0, 0};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j >> 2] |= (unsigned)(unsigned char)W[(k + j) * N + n] << (8 * (j & 3));
+  out[i] = v;
 }
 
 // ---- launches ----
 // A launch takes about fixed + rounds * (one + more * (ceil(workgroups / 256) - 1)) us, where a workgroup needs
 // ceil(steps of its slice / kpar) rounds: a compute unit that gets a second workgroup determines the launch. The numbers
-// are least-squares fits to 2700 launches on MI355X (8 to 943 rows, 384 to 6400 columns, K from 384 to 6400, 1 to 8 slices;
-// 6-13 % rms); the shape that they choose is within 1.3 % of the best one of nine tried (geometric mean; 2.9 % where K may
-// be sliced).
+// are least-squares fits to launches on MI355X (8 to 943 rows, 384 to 6400 columns, K from 384 to 6400, 1 to 8 slices):
+// 2700 of them for rows of W (6-13 % rms), 5700 for blocked W (8-19 %). The shape that they choose is within 1.4 % of the best
+// one (geometric mean; 2.9 % where K may be sliced).
 struct Shape {
   int mtile, ntile, kpar;  // tile; steps of 32 k that a workgroup works on at a time
-  struct { float fixed, one, more; } f32, i8;
+  struct Fit { float fixed, one, more; } f32, i8, f32_blk, i8_blk;
 };
 constexpr Shape SHAPES[] = {
-    {16, 16, 8, {2.78f, 0.77f, 0.92f}, {2.99f, 0.52f, 0.60f}},   // gemm_split_rows<16, 1, 1, 8>
-    {16, 32, 8, {3.11f, 0.90f, 1.31f}, {3.10f, 0.68f, 0.82f}},   // gemm_split_rows<16, 1, 2, 8>
-    {32, 32, 8, {3.09f, 1.27f, 1.75f}, {3.39f, 1.26f, 1.29f}},   // gemm_split_rows<32, 1, 1, 8>
-    {64, 64, 4, {4.56f, 1.45f, 2.06f}, {5.30f, 1.05f, 1.56f}},   // gemm_split_rows<32, 2, 2, 4>
-    {64, 64, 8, {4.58f, 2.58f, 4.77f}, {5.05f, 2.11f, 3.49f}},   // gemm_split_rows<32, 2, 2, 8>
-    {32, 64, 4, {4.70f, 1.03f, 2.41f}, {4.84f, 0.87f, 1.04f}},   // gemm_split_tile<1, 1, 2, 4>
-    {128, 128, 2, {7.97f, 2.00f, 4.69f}, {8.00f, 1.56f, 3.06f}}, // gemm_split_tile<4, 1, 4, 2>
+    {16, 16, 8, {2.78f, 0.77f, 0.92f}, {2.99f, 0.52f, 0.60f}, {3.37f, 0.57f, 0.74f}, {3.11f, 0.45f, 0.62f}},    // gemm_split_rows<16, 1, 1, 8>
+    {16, 32, 8, {3.11f, 0.90f, 1.31f}, {3.10f, 0.68f, 0.82f}, {3.51f, 0.71f, 0.98f}, {3.31f, 0.51f, 0.72f}},    // gemm_split_rows<16, 1, 2, 8>
+    {32, 32, 8, {3.09f, 1.27f, 1.75f}, {3.39f, 1.26f, 1.29f}, {3.46f, 1.07f, 1.55f}, {3.44f, 0.78f, 1.38f}},    // gemm_split_rows<32, 1, 1, 8>
+    {64, 64, 4, {4.56f, 1.45f, 2.06f}, {5.30f, 1.05f, 1.56f}, {4.63f, 1.38f, 1.82f}, {4.71f, 0.95f, 1.51f}},    // gemm_split_rows<32, 2, 2, 4>
+    {64, 64, 8, {4.58f, 2.58f, 4.77f}, {5.05f, 2.11f, 3.49f}, {4.35f, 2.39f, 4.31f}, {4.34f, 1.73f, 3.71f}},    // gemm_split_rows<32, 2, 2, 8>
+    {32, 64, 4, {4.70f, 1.03f, 2.41f}, {4.84f, 0.87f, 1.04f}, {4.64f, 0.88f, 1.16f}, {4.29f, 0.49f, 0.73f}},    // gemm_split_tile<1, 1, 2, 4>
+    {128, 128, 2, {7.97f, 2.00f, 4.69f}, {8.00f, 1.56f, 3.06f}, {7.74f, 2.27f, 3.73f}, {8.61f, 1.22f, 2.48f}},  // gemm_split_tile<4, 1, 4, 2>
+    {64, 128, 2, {0, 0, 0}, {0, 0, 0}, {5.36f, 1.24f, 2.09f}, {5.45f, 0.67f, 0.96f}},                         // gemm_split_tile<2, 1, 4, 2>
 };
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
+constexpr int NSHAPES_ROWS = NSHAPES - 1;  // with rows of W the last one is never the best
 
 constexpr size_t rows_lds(int R, int MB, int NB, int NW) { return (size_t)NW * MB * NB * R * R * sizeof(float); }
 constexpr size_t tile_lds(int MB, int NB, int NWN, int KG) {
@@ -545,29 +610,31 @@ hipError_t launch_kernel(K kernel, const SplitGemmArgs& a, int threads, size_t l
   return hipGetLastError();
 }
 
-template <bool I8>
+template <bool I8, bool BLK>
 hipError_t launch_shape(int kind, const SplitGemmArgs& a, hipStream_t s) {
   switch (kind) {
-    case 0: return launch_kernel(gemm_split_rows<16, 1, 1, 8, I8>, a, 512, rows_lds(16, 1, 1, 8), s);
-    case 1: return launch_kernel(gemm_split_rows<16, 1, 2, 8, I8>, a, 512, rows_lds(16, 1, 2, 8), s);
-    case 2: return launch_kernel(gemm_split_rows<32, 1, 1, 8, I8>, a, 512, rows_lds(32, 1, 1, 8), s);
-    case 3: return launch_kernel(gemm_split_rows<32, 2, 2, 4, I8>, a, 256, rows_lds(32, 2, 2, 4), s);
-    case 4: return launch_kernel(gemm_split_rows<32, 2, 2, 8, I8>, a, 512, rows_lds(32, 2, 2, 8), s);
-    case 5: return launch_kernel(gemm_split_tile<1, 1, 2, 4, I8, 2, 2>, a, 512, tile_lds(1, 1, 2, 4), s);
-    case 6: return launch_kernel(gemm_split_tile<4, 1, 4, 2, I8, 2, 2>, a, 512, tile_lds(4, 1, 4, 2), s);
+    case 0: return launch_kernel(gemm_split_rows<16, 1, 1, 8, I8, BLK>, a, 512, rows_lds(16, 1, 1, 8), s);
+    case 1: return launch_kernel(gemm_split_rows<16, 1, 2, 8, I8, BLK>, a, 512, rows_lds(16, 1, 2, 8), s);
+    case 2: return launch_kernel(gemm_split_rows<32, 1, 1, 8, I8, BLK>, a, 512, rows_lds(32, 1, 1, 8), s);
+    case 3: return launch_kernel(gemm_split_rows<32, 2, 2, 4, I8, BLK>, a, 256, rows_lds(32, 2, 2, 4), s);
+    case 4: return launch_kernel(gemm_split_rows<32, 2, 2, 8, I8, BLK>, a, 512, rows_lds(32, 2, 2, 8), s);
+    case 5: return launch_kernel(gemm_split_tile<1, 1, 2, 4, I8, BLK, 2, 2>, a, 512, tile_lds(1, 1, 2, 4), s);
+    case 6: return launch_kernel(gemm_split_tile<4, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(4, 1, 4, 2), s);
+    case 7:
+      if constexpr (BLK) return launch_kernel(gemm_split_tile<2, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(2, 1, 4, 2), s);
   }
   return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-SplitPlan plan_gemm_split(int M, int N, int K, bool i8, bool with_pass, bool may_slice) {
+SplitPlan plan_gemm_split(int M, int N, int K, bool i8, bool blocked, bool with_pass, bool may_slice) {
   SplitPlan best = {0, 1};
   double best_t = 1e30;
   const int steps = (K + 31) / 32;
-  for (int c = 0; c < NSHAPES; ++c) {
+  for (int c = 0; c < (blocked ? NSHAPES : NSHAPES_ROWS); ++c) {
     const Shape& sh = SHAPES[c];
-    const auto& f = i8 ? sh.i8 : sh.f32;
+    const Shape::Fit& f = blocked ? (i8 ? sh.i8_blk : sh.f32_blk) : i8 ? sh.i8 : sh.f32;
     const double tiles = (double)((M + sh.mtile - 1) / sh.mtile) * ((N + sh.ntile - 1) / sh.ntile);
     for (int S = 1; S <= (may_slice ? 8 : 1); ++S) {
       if (S > 1 && steps < 4 * S) break;
@@ -584,11 +651,20 @@ SplitPlan plan_gemm_split(int M, int N, int K, bool i8, bool with_pass, bool may
   return best;
 }
 
+hipError_t launch_block_weights(int K, int N, bool i8, const void* src, void* dst, hipStream_t s) {
+  if ((K & 7) || (N & 3)) return hipErrorInvalidValue;
+  const size_t n = (size_t)(i8 ? K >> 3 : K >> 2) * N;
+  if (i8) block_weights_i8<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(K, N, static_cast<const signed char*>(src), static_cast<u32x2*>(dst));
+  else block_weights_f32<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(K, N, static_cast<const float*>(src), static_cast<f32x4*>(dst));
+  return hipGetLastError();
+}
+
 hipError_t launch_gemm_split(const SplitPlan& p, SplitGemmArgs a, bool i8, hipStream_t s) {
   a.mt = (a.M + SHAPES[p.kind].mtile - 1) / SHAPES[p.kind].mtile;
   a.nt = (a.N + SHAPES[p.kind].ntile - 1) / SHAPES[p.kind].ntile;
   a.S = p.S;
-  return i8 ? launch_shape<true>(p.kind, a, s) : launch_shape<false>(p.kind, a, s);
+  if (a.blocked) return i8 ? launch_shape<true, true>(p.kind, a, s) : launch_shape<false, true>(p.kind, a, s);
+  return i8 ? launch_shape<true, false>(p.kind, a, s) : launch_shape<false, false>(p.kind, a, s);
 }
 
 }  // namespace wgpt

@@ -24,7 +24,7 @@ hipError_t launch_gemv_kn(int M, int N, int K, const float* A, int lda, const fl
 
 // Same contraction for any M on the matrix cores (gemm_split.hip).
 // workspace (gemm_workspace_floats(M, N) floats, may be null) enables slices of K for
-// shapes with too few output tiles to fill the GPU.
+// shapes with too few output tiles to fill the GPU. blocked: W is in the order of launch_block_weights.
 size_t gemm_workspace_floats(int M, int N);
 // A LayerNormBlock applied to the finished rows of C right after the product (out may not alias C). Where the
 // product ends in a split-K reduction pass, that pass normalises the rows it has just finished.
@@ -43,11 +43,11 @@ struct KvAfter {
 };
 hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float* W, int ldw, const float* bias,
                        float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
-                       const LnAfter* ln = nullptr, const KvAfter* kv = nullptr);
+                       const LnAfter* ln = nullptr, const KvAfter* kv = nullptr, bool blocked = false);
 // Same with the packed int8 weights of other/int8-gemm.js (Wq[K, ldwq] words, scale[N]).
 hipError_t launch_gemm_i8(int M, int N, int K, const float* A, int lda, const int32_t* Wq, int ldwq, const float* scale,
                           const float* bias, float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
-                          const LnAfter* ln = nullptr, const KvAfter* kv = nullptr);
+                          const LnAfter* ln = nullptr, const KvAfter* kv = nullptr, bool blocked = false);
 
 // int8 weight-only variants: Wq is [K, ldwq] words holding 4 columns each.
 hipError_t launch_gemv_kn_i8(int M, int N, int K, const float* A, int lda, const int32_t* Wq, int ldwq,

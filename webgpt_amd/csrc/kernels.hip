@@ -1628,19 +1628,20 @@ void finish_split(int M, int N, int S, const float* workspace, const float* bias
   if (ln) layernorm_kernel<<<M, WG, 0, s>>>(N, C, ldc, ln->gamma, ln->beta, ln->out, ln->ldo);
 }
 
-// C = epi(A . W + bias) on the matrix cores; W fp32 [K, ldw], or words of four int8 with a scale per column.
+// C = epi(A . W + bias) on the matrix cores; W fp32 [K, ldw], or words of four int8 with a scale per column
+// (blocked: in the order of launch_block_weights).
 hipError_t run_gemm(int M, int N, int K, const float* A, int lda, const void* W, int ldw, const float* wscale, const float* bias,
-                    float* C, int ldc, int epi, const float* resid, float* workspace, const LnAfter* ln, const KvAfter* kv, hipStream_t s) {
+                    float* C, int ldc, int epi, const float* resid, float* workspace, const LnAfter* ln, const KvAfter* kv, bool blocked, hipStream_t s) {
   const bool i8 = wscale != nullptr;
   SplitGemmArgs a{};
-  a.N = N; a.K = K; a.lda = lda; a.W = W; a.ldw = ldw; a.wscale = wscale; a.bias = bias; a.epi = epi; a.ldc = ldc;
+  a.N = N; a.K = K; a.lda = lda; a.W = W; a.ldw = ldw; a.blocked = blocked; a.wscale = wscale; a.bias = bias; a.epi = epi; a.ldc = ldc;
   if (kv) { a.Kc = kv->Kc; a.Vc = kv->Vc; a.d = kv->d; a.hs = kv->hs; a.ctx = kv->ctx; }
   // the kernels address A with 32-bit offsets: very tall matrices go in runs of rows
   const int rows = (int)std::min<size_t>((size_t)M, (((size_t)1 << 31) - 4096) / (sizeof(float) * (size_t)lda));
   if (rows < 1) return hipErrorInvalidValue;
   for (int m0 = 0; m0 < M; m0 += rows) {
     const int m = std::min(rows, M - m0);
-    const SplitPlan p = plan_gemm_split(m, N, K, i8, ln != nullptr, workspace != nullptr);
+    const SplitPlan p = plan_gemm_split(m, N, K, i8, blocked, ln != nullptr, workspace != nullptr);
     a.M = m;
     a.A = A + (size_t)m0 * lda;
     a.C = C + (size_t)m0 * ldc;
@@ -1662,14 +1663,14 @@ hipError_t run_gemm(int M, int N, int K, const float* A, int lda, const void* W,
 
 hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float* W, int ldw, const float* bias,
                        float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s, const LnAfter* ln,
-                       const KvAfter* kv) {
+                       const KvAfter* kv, bool blocked) {
   // the kernels address W with 32-bit offsets: a larger matrix goes in runs of rows whose products are added up
   const int rows = (int)std::min<size_t>((size_t)K, (((size_t)1 << 31) - 4096) / (sizeof(float) * (size_t)ldw) / 4 * 4);
-  if (rows >= K) return run_gemm(M, N, K, A, lda, W, ldw, nullptr, bias, C, ldc, epi, resid, workspace, ln, kv, s);
-  if (rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  if (rows >= K) return run_gemm(M, N, K, A, lda, W, ldw, nullptr, bias, C, ldc, epi, resid, workspace, ln, kv, blocked, s);
+  if (blocked || rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
   for (int k0 = 0; k0 < K; k0 += rows) {
     const hipError_t e = run_gemm(M, N, std::min(rows, K - k0), A + k0, lda, W + (size_t)k0 * ldw, ldw, nullptr,
-                                  k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, s);
+                                  k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, false, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1677,13 +1678,13 @@ hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float
 
 hipError_t launch_gemm_i8(int M, int N, int K, const float* A, int lda, const int32_t* Wq, int ldwq, const float* scale,
                           const float* bias, float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
-                          const LnAfter* ln, const KvAfter* kv) {
+                          const LnAfter* ln, const KvAfter* kv, bool blocked) {
   const int rows = (int)std::min<size_t>((size_t)K, (((size_t)1 << 31) - 4096) / (sizeof(int32_t) * (size_t)ldwq) / 4 * 4);
-  if (rows >= K) return run_gemm(M, N, K, A, lda, Wq, ldwq, scale, bias, C, ldc, epi, resid, workspace, ln, kv, s);
-  if (rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  if (rows >= K) return run_gemm(M, N, K, A, lda, Wq, ldwq, scale, bias, C, ldc, epi, resid, workspace, ln, kv, blocked, s);
+  if (blocked || rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
   for (int k0 = 0; k0 < K; k0 += rows) {
     const hipError_t e = run_gemm(M, N, std::min(rows, K - k0), A + k0, lda, Wq + (size_t)k0 * ldwq, ldwq, scale,
-                                  k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, s);
+                                  k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, false, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

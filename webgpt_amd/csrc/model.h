@@ -12,7 +12,8 @@
 
 namespace wgpt {
 
-// One linear layer's weight: fp32 [K,N], or int8 words [K,N/4] + per-column scale [N].
+// One linear layer's weight: fp32 [K,N], or int8 words [K,N/4] + per-column scale [N]; once the model is finalised in the
+// order of launch_block_weights.
 struct LinW {
   float* w = nullptr;
   int32_t* q = nullptr;

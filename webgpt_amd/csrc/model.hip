@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "common.h"
+#include "gemm_split.h"
 #include "kernels.h"
 #include "model.h"
 
@@ -92,8 +93,8 @@ static bool parse_name(Model* m, const std::string& name, Slot* slot) {
 // With `ln` the LayerNorm that follows in the forward is applied to the finished rows as part of the product.
 static int linear(Model* m, int M, int N, int K, const float* A, int lda, const LinW& w, const float* bias, float* C,
                   int ldc, int epi, const float* resid, const LnAfter* ln = nullptr, const KvAfter* kv = nullptr) {
-  const hipError_t e = w.q ? launch_gemm_i8(M, N, K, A, lda, w.q, N / 4, w.s, bias, C, ldc, epi, resid, m->part, rt().stream, ln, kv)
-                           : launch_gemm(M, N, K, A, lda, w.w, N, bias, C, ldc, epi, resid, m->part, rt().stream, ln, kv);
+  const hipError_t e = w.q ? launch_gemm_i8(M, N, K, A, lda, w.q, N / 4, w.s, bias, C, ldc, epi, resid, m->part, rt().stream, ln, kv, true)
+                           : launch_gemm(M, N, K, A, lda, w.w, N, bias, C, ldc, epi, resid, m->part, rt().stream, ln, kv, true);
   if (e != hipSuccess) return fail(WGPT_ERR_HIP, "linear layer launch: %s", hipGetErrorString(e));
   return WGPT_OK;
 }
@@ -555,6 +556,29 @@ static int finish_steps(Model* m, int32_t* out_tokens, const int32_t* ids_dev, i
   return WGPT_OK;
 }
 
+// Puts the linear weights, which the decode layouts have been built from, into the order that the prefill products read
+// (in place, through a buffer of the largest one).
+static int block_linear_weights(Model* m) {
+  const int d = m->d;
+  const bool i8 = m->p.weight_dtype == 1;
+  const size_t elem = i8 ? 1 : sizeof(float);
+  void* tmp = nullptr;
+  hipError_t e = hipMalloc(&tmp, (size_t)4 * d * d * elem);
+  if (e != hipSuccess) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): %s", (size_t)4 * d * d * elem, hipGetErrorString(e));
+  for (const LayerW& l : m->layers) {
+    const struct { const LinW* w; int K, N; } lins[4] = {{&l.attn, d, 3 * d}, {&l.proj, d, d}, {&l.fc, d, 4 * d}, {&l.fc2, 4 * d, d}};
+    for (const auto& t : lins) {
+      void* w = i8 ? (void*)t.w->q : (void*)t.w->w;
+      if (e == hipSuccess) e = launch_block_weights(t.K, t.N, i8, w, tmp, rt().stream);
+      if (e == hipSuccess) e = hipMemcpyAsync(w, tmp, (size_t)t.K * t.N * elem, hipMemcpyDeviceToDevice, rt().stream);
+    }
+  }
+  const hipError_t es = hipStreamSynchronize(rt().stream), ef = hipFree(tmp);
+  if (e == hipSuccess) e = es != hipSuccess ? es : ef;
+  if (e != hipSuccess) return fail(WGPT_ERR_HIP, "layout of the linear weights: %s", hipGetErrorString(e));
+  return WGPT_OK;
+}
+
 static void destroy_model(Model* m) {
   if (m->token_graph_exec) (void)hipGraphExecDestroy(m->token_graph_exec);
   if (m->token_graph) (void)hipGraphDestroy(m->token_graph);
@@ -670,6 +694,7 @@ int wgpt_model_finalize(wgpt_model h) {
   WGPT_HIP(hipEventCreate(&m->ev1));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   if ((rc = setup_persistent(m))) return rc;
+  if ((rc = block_linear_weights(m))) return rc;
   m->decode_mode = m->persist_ok ? 1 : 0;
   m->pos = 0;
   m->finalized = true;
