@@ -277,6 +277,39 @@ def test_attention(device, T, H, hs):
     assert close(got, want), worst(got, want)
 
 
+@pytest.mark.parametrize("T,H,hs", [(192, 2, 4), (193, 2, 20), (320, 5, 32), (257, 2, 36), (700, 2, 64), (225, 2, 68), (331, 4, 96),
+                                    (256, 2, 100), (1023, 2, 128)])
+def test_attention_split_operands(device, T, H, hs):
+    """Prompts long enough for the split operands: the edges of a block of 32 queries, keys or dimensions. With the identity as
+    every weight, q = k = v = x; scores reach 20 (the diagonal), so that maxima move from tile to tile. Products and sums of
+    the scores are rounded like fp32 ones: an error of a few ulp of the largest score, 2**-20 of the weights at most, and
+    2**-23 for each of the few roundings behind them. Infinite and other special values reach the rows that see them, and no others."""
+    d = H * hs
+    rng = np.random.default_rng(T + d)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    special = x.copy()
+    special[T - 2, 0], special[T - 1, 1] = np.inf, np.nan
+    eye, zero = np.eye(d, dtype=np.float32), np.zeros(d, np.float32)
+    scale = 1 / math.sqrt(hs)
+    got = []
+    for values in (x, special):
+        bufs = [init_tensor(values, [T, d])]
+        for i in range(4):
+            bufs += [init_tensor(eye, [d, d]), init_tensor(zero, [d])]
+        got.append(run(AttentionBlock.newFusedInstance(T, d, scale, H, hs, *bufs, FastMatMulBlock, SoftmaxBlock), (T, d)))
+    v = x.astype(np.float64).reshape(T, H, hs).transpose(1, 0, 2)
+    s = v @ v.transpose(0, 2, 1) * np.float64(np.float32(scale))
+    s[:, np.triu(np.ones((T, T), bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = (p @ v).transpose(1, 0, 2).reshape(T, d)
+    size = (p @ np.abs(v)).transpose(1, 0, 2).reshape(T, d)
+    bound = (2.0 ** -20 * max(1.0, np.abs(s[np.isfinite(s)]).max() / 16) + 2.0 ** -21) * size
+    assert np.all(np.abs(got[0] - want) <= bound)
+    assert np.all(np.abs(got[1] - want)[:T - 2] <= bound[:T - 2])  # (a block with such rows is taken again without splits: other roundings)
+    assert not np.isfinite(got[1][T - 2]).any() and not np.isfinite(got[1][T - 1]).any()
+
+
 def test_attention_values_known_answer(device):
     # other/test.js:370-388 through the attention block: with Wq = Wk = 0 every score is 0, so the
     # softmax is uniform over j <= i: P = 1/(i+1). V = c // hs + 1 (via bv, Wv = 0), Wo = I:

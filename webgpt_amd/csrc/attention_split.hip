@@ -1,0 +1,305 @@
+// Causal attention of a prompt (AttentionBlock: formatQ, fusedWeights, softmax and attentionValues of
+// instructions.js:1129-1212) on the bf16 matrix cores, for head sizes up to 128.
+//
+// Operands are split into three bf16 values each and the six largest partial products taken, as in gemm_split.hip: an error
+// no larger than that of fp32 products at 2.7 times their rate. q, K and V are split once, by a pass in front
+// (attention_operands), which also lays them out so that every operand of a matrix instruction is one load of 1 KB of
+// neighbouring bytes per wave: no LDS, no transposition and no conversion in the loop over the keys, where only the weights
+// are split. Everything is computed transposed, S^T = K Q^T and O^T = V^T P^T: an accumulator then holds 16 keys of ONE query
+// per lane, so that the softmax needs one exchange between lanes and the weights are where the second product wants them.
+// A workgroup owns 32 queries of a head, its waves share the keys in runs of 32-key tiles and are merged at the end.
+// Bound by what a compute unit takes from L2 (12 KB per 32 keys at head size 64, read by every block of 32 queries).
+#include <cmath>
+
+#include "kernels.h"
+#include "split_bf16.h"
+
+namespace wgpt {
+namespace {
+
+constexpr int ASQ = 32;         // queries per workgroup, keys per tile
+constexpr int AS_MERGE = ASQ + 1;  // row stride of a wave's O^T[dim][query] in the merge
+
+struct AttnSplitArgs {
+  int Tq, pos0, H, hs, nq, nt;  // nq, nt: blocks of 32 queries, tiles of 32 keys
+  float scale;
+  const float* q;
+  int ldq;
+  const float *Kc, *Vc;
+  size_t hstride;
+  int ldkv;
+  float* out;
+  int ldo;
+  u32x4 *Q3, *K3, *V3;  // [H][block or tile][KS steps][3 parts][64 lanes]
+};
+
+// Operands of one block of queries or tile of keys: unit (step, part, lane) of 16 bytes holds the eight values that the lane
+// supplies to the step. q and K: row lane % 32, dimensions 16 step + 8 (lane / 32) ..; V: dimension 32 (step / 2) + lane % 32,
+// and of the sixteen keys of step % 2 the eight that the accumulator of S^T leaves in this half of the wave.
+// Values beyond the head size, the last query or the last key are zeros.
+__global__ void attention_operands(AttnSplitArgs a) {
+  const int lane = threadIdx.x & 63, step = threadIdx.x >> 6, steps = blockDim.x >> 6;
+  const int h = blockIdx.y, r = lane & 31, half = lane >> 5, nkeys = a.pos0 + a.Tq;
+  int t = blockIdx.x;
+  f32x4 v[2];
+  u32x4* dst;
+  if (t < a.nq + a.nt) {
+    const bool isq = t < a.nq;
+    if (!isq) t -= a.nq;
+    const int row = t * ASQ + r;
+    const bool live = row < (isq ? a.Tq : nkeys);
+    const float* p = isq ? a.q + (size_t)row * a.ldq + (size_t)h * a.hs : a.Kc + h * a.hstride + (size_t)row * a.ldkv;
+    const int d0 = 16 * step + 8 * half;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      v[i] = live && d0 + 4 * i < a.hs ? *reinterpret_cast<const f32x4*>(p + d0 + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+    dst = isq ? a.Q3 + (size_t)(h * a.nq + t) * steps * 192 : a.K3 + (size_t)(h * a.nt + t) * steps * 192;
+  } else {
+    t -= a.nq + a.nt;
+    const int dim = 32 * (step >> 1) + r, k0 = t * ASQ + 16 * (step & 1) + 4 * half;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int key = k0 + 8 * (j >> 2) + (j & 3);
+      v[j >> 2][j & 3] = dim < a.hs && key < nkeys ? a.Vc[h * a.hstride + (size_t)key * a.ldkv + dim] : 0.f;
+    }
+    dst = a.V3 + (size_t)(h * a.nt + t) * steps * 192;
+  }
+  const Split8 s = split8(v[0], v[1]);
+  dst += step * 192 + lane;
+  dst[0] = s.hi;
+  dst[64] = s.mid;
+  dst[128] = s.lo;
+}
+
+// exp(x) for x <= 0 with the rounding of x * log2(e) made up for: as exact as expf down to its smallest normal result
+__device__ __forceinline__ float exp_neg(float x) {
+  const float t = x * 1.44269504f;
+  const float r = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t));  // log2(e) = 1.44269502162933 + 1.92596303e-8
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, r * 0.693147181f, e);
+}
+
+__device__ __forceinline__ f32x16 mfma(const u32x4& p, const u32x4& q, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, p), __builtin_bit_cast(bf16x8, q), c, 0, 0, 0);
+}
+// The product of the leading parts goes to its own sum: what the other five, 2^-8 of it and less, add up to meets it once
+// per tile, and the sum of a tile is rounded three times instead of twelve.
+__device__ __forceinline__ void split_mfma(const u32x4 (&w)[3], const u32x4 (&x)[3], f32x16& lead, f32x16& rest) {
+  rest = mfma(w[2], x[0], rest);
+  lead = mfma(w[0], x[0], lead);
+  rest = mfma(w[0], x[2], rest);
+  rest = mfma(w[1], x[1], rest);
+  rest = mfma(w[1], x[0], rest);
+  rest = mfma(w[0], x[1], rest);
+}
+
+// One output with plain fp32 products: for operands that have no split (infinite ones, see gemm_split.hip) and for NaN.
+__device__ __forceinline__ float plain_attention(const AttnSplitArgs& a, int h, int i, int dim) {
+  const float* q = a.q + (size_t)i * a.ldq + (size_t)h * a.hs;
+  const float* K = a.Kc + h * a.hstride;
+  float m = -3.402823e+38f, num = 0.f, den = 0.f;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass)
+#pragma unroll 1
+    for (int j = 0; j <= a.pos0 + i; ++j) {
+      float s = 0.f;
+#pragma unroll 1
+      for (int k = 0; k < a.hs; ++k) s = fmaf(q[k], K[(size_t)j * a.ldkv + k], s);
+      s *= a.scale;
+      if (pass == 0) {
+        m = fmaxf(m, s);
+      } else {
+        const float e = s - m <= 0.f ? exp_neg(fmaxf(s - m, -200.f)) : s - m;  // (not a number stays that)
+        num = fmaf(e, a.Vc[h * a.hstride + (size_t)j * a.ldkv + dim], num);
+        den += e;
+      }
+    }
+  return num / den;
+}
+
+// DB: blocks of 32 dimensions that hold a head. Registers: the operands of a tile's K and V (24 DB each), O (16 DB) and the
+// sums; q fits beside them for DB = 1 only and waits in LDS otherwise. From three blocks on a wave needs more than half a
+// SIMD's registers, so four waves fill the compute unit.
+template <int DB, int NWV>
+__global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(AttnSplitArgs a) {
+  constexpr int KS = 2 * DB, DIMS = 32 * DB, WAVE_FLOATS = DIMS * AS_MERGE + 2 * ASQ;
+  constexpr bool QREG = DB == 1;
+  extern __shared__ __attribute__((aligned(16))) float as_lds[];
+  // consecutive blocks go to one XCD, whose L2 then holds the K and V of few heads; the longest rows of keys first
+  const int total = a.H * a.nq, per = (total + 7) >> 3, item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || item >= total) return;
+  const int h = item / a.nq, qb = a.nq - 1 - item % a.nq, q0 = qb * ASQ;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int qpos = a.pos0 + q0 + l32;  // keys 0..qpos are visible to this lane's query (which may be beyond the last one)
+  const int nt = (a.pos0 + min(q0 + ASQ, a.Tq) + ASQ - 1) / ASQ;
+  const int tb = nt * wave / NWV, te = nt * (wave + 1) / NWV;
+
+  const u32x4* qsrc = a.Q3 + (size_t)(h * a.nq + qb) * KS * 192;
+  u32x4* qlds = reinterpret_cast<u32x4*>(as_lds);
+  u32x4 qr[QREG ? KS : 1][3];
+  if constexpr (QREG) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) qr[s][p] = qsrc[(s * 3 + p) * 64 + lane];
+  } else {
+    for (int i = threadIdx.x; i < KS * 192; i += NWV * 64) qlds[i] = qsrc[i];
+    __syncthreads();
+  }
+  f32x16 o[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
+  float m = -INFINITY, lsum = 0.f;
+  u32x4 kf[KS][3], vf[KS][3];
+  const auto fetch = [&](u32x4 (&f)[KS][3], const u32x4* base, int t) {
+    const u32x4* src = base + (size_t)(h * a.nt + t) * KS * 192 + lane;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) f[s][p] = src[(s * 3 + p) * 64];
+  };
+  if (tb < te) fetch(kf, a.K3, tb);
+  for (int t = tb; t < te; ++t) {
+    fetch(vf, a.V3, t);
+    f32x16 sacc, rest;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sacc[r] = rest[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if constexpr (QREG) {
+        split_mfma(kf[s], qr[s], sacc, rest);
+      } else {
+        const u32x4 x[3] = {qlds[(s * 3 + 0) * 64 + lane], qlds[(s * 3 + 1) * 64 + lane], qlds[(s * 3 + 2) * 64 + lane]};
+        split_mfma(kf[s], x, sacc, rest);
+      }
+    }
+    fetch(kf, a.K3, t + 1 < te ? t + 1 : t);
+    float tmax = -INFINITY;
+    if (t * ASQ + ASQ - 1 > a.pos0 + q0) {  // keys that not all queries see
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = t * ASQ + (r >> 2) * 8 + hh * 4 + (r & 3);
+        sacc[r] = key <= qpos ? (sacc[r] + rest[r]) * a.scale : -INFINITY;
+        tmax = fmaxf(tmax, sacc[r]);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        sacc[r] = (sacc[r] + rest[r]) * a.scale;
+        tmax = fmaxf(tmax, sacc[r]);
+      }
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+    const float mnew = fmaxf(m, tmax);
+    // a query with no visible key so far keeps m = -inf: guard the exponentials
+    const float corr = m > -INFINITY ? exp_neg(m - mnew) : 0.f;
+    float psum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      sacc[r] = sacc[r] == -INFINITY ? 0.f : exp_neg(sacc[r] - mnew);  // (not a number stays that: plain_attention)
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) psum += (sacc[r] + sacc[r + 1]) + (sacc[r + 2] + sacc[r + 3]);
+    lsum = lsum * corr + psum;
+    m = mnew;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[b][r] *= corr;
+    u32x4 pf[2][3];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const Split8 w = split8(f32x4{sacc[8 * s], sacc[8 * s + 1], sacc[8 * s + 2], sacc[8 * s + 3]},
+                              f32x4{sacc[8 * s + 4], sacc[8 * s + 5], sacc[8 * s + 6], sacc[8 * s + 7]});
+      pf[s][0] = w.hi;
+      pf[s][1] = w.mid;
+      pf[s][2] = w.lo;
+    }
+#pragma unroll
+    for (int b = 0; b < DB; ++b) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) rest[r] = 0.f;
+      split_mfma(vf[2 * b], pf[0], o[b], rest);
+      split_mfma(vf[2 * b + 1], pf[1], o[b], rest);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[b][r] += rest[r];
+    }
+  }
+  lsum += __shfl_xor(lsum, 32);  // the two halves of a column saw disjoint keys, the same maximum
+
+  if constexpr (!QREG) __syncthreads();
+  float* Om = as_lds + wave * WAVE_FLOATS;  // [DIMS][AS_MERGE], then maxima and sums of the 32 queries
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) Om[(b * 32 + (r >> 2) * 8 + hh * 4 + (r & 3)) * AS_MERGE + l32] = o[b][r];
+  if (hh == 0) {
+    Om[DIMS * AS_MERGE + l32] = m;
+    Om[DIMS * AS_MERGE + ASQ + l32] = lsum;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < ASQ * DIMS; e += NWV * 64) {
+    const int qi = e / DIMS, dim = e % DIMS;
+    if (q0 + qi >= a.Tq || dim >= a.hs) continue;
+    float mw[NWV], M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      mw[w] = as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + qi];
+      M = fmaxf(M, mw[w]);
+    }
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      const float f = mw[w] > -INFINITY ? exp_neg(mw[w] - M) : 0.f;
+      num += as_lds[w * WAVE_FLOATS + dim * AS_MERGE + qi] * f;
+      den += as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + ASQ + qi] * f;
+    }
+    float v = num / den;
+    if (!(v - v == 0.f)) v = plain_attention(a, h, q0 + qi, dim);
+    a.out[(size_t)(q0 + qi) * a.ldo + (size_t)h * a.hs + dim] = v;
+  }
+}
+
+template <int DB, int NWV>
+hipError_t launch_waves(const AttnSplitArgs& a, hipStream_t s) {
+  const size_t merge = sizeof(float) * NWV * (32 * DB * AS_MERGE + 2 * ASQ), ql = DB > 1 ? (size_t)2 * DB * 192 * 16 : 0;
+  const size_t lds = merge > ql ? merge : ql;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_split_kernel<DB, NWV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  const long grid = ((long)a.H * a.nq + 7) / 8 * 8;
+  if (grid > 0x7fffffffL) return hipErrorInvalidValue;
+  attention_split_kernel<DB, NWV><<<(unsigned)grid, NWV * 64, lds, s>>>(a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+size_t attention_split_bytes(int Tq, int pos0, int H, int hs) {
+  const size_t per = (size_t)2 * ((hs + 31) / 32) * 192 * 16;
+  return per * H * ((Tq + ASQ - 1) / ASQ + 2 * (size_t)((pos0 + Tq + ASQ - 1) / ASQ));
+}
+
+hipError_t launch_attention_split(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc, const float* Vc,
+                                  size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s) {
+  if (hs > 128 || (hs & 3) || H > 65535) return hipErrorInvalidValue;
+  AttnSplitArgs a{Tq, pos0, H, hs, (Tq + ASQ - 1) / ASQ, (pos0 + Tq + ASQ - 1) / ASQ, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, nullptr, nullptr, nullptr};
+  const int DB = (hs + 31) / 32;
+  const size_t unit = (size_t)2 * DB * 192;
+  a.Q3 = static_cast<u32x4*>(ws);
+  a.K3 = a.Q3 + unit * H * a.nq;
+  a.V3 = a.K3 + unit * H * a.nt;
+  attention_operands<<<dim3(a.nq + 2 * a.nt, H), 2 * DB * 64, 0, s>>>(a);
+  switch (DB) {
+    case 1: return launch_waves<1, 8>(a, s);
+    case 2: return launch_waves<2, 8>(a, s);
+    case 3: return launch_waves<3, 4>(a, s);
+    default: return launch_waves<4, 4>(a, s);
+  }
+}
+
+}  // namespace wgpt

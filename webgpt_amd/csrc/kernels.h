@@ -68,8 +68,14 @@ hipError_t launch_vocab_gemv(int V, int d, const float* x, const float* wte, flo
 // Causal attention of Tq query rows (absolute positions pos0..pos0+Tq-1) against
 // keys/values 0..pos. q row i is at q + i*ldq + h*hs; key row j of head h is at
 // Kc + h*hstride + j*ldkv (likewise values).
+// ws: attention_workspace_bytes of memory (may be null where that is 0).
+size_t attention_workspace_bytes(int Tq, int pos0, int H, int hs);
 hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc,
-                            const float* Vc, size_t hstride, int ldkv, float* out, int ldo, hipStream_t s);
+                            const float* Vc, size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s);
+// The same on the bf16 matrix cores (attention_split.hip), hs a multiple of 4 up to 128; ws: attention_split_bytes.
+size_t attention_split_bytes(int Tq, int pos0, int H, int hs);
+hipError_t launch_attention_split(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc, const float* Vc,
+                                  size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s);
 // Appends the K and V columns of qkv[T,3d] at positions pos0.. of a head-major cache [H][ctx][hs].
 hipError_t launch_kv_append(int T, int d, int hs, int ctx, int pos0, const float* qkv, float* Kc, float* Vc, hipStream_t s);
 // Copies rows of src (row stride lds, `cols` floats wide) to dst (row stride ldd).

@@ -1728,8 +1728,23 @@ hipError_t launch_vocab_gemv(int V, int d, const float* x, const float* wte, flo
   return hipGetLastError();
 }
 
+// Where the split operands pay for the pass that makes them (two launches; MI355X, us of a call, this kernel against the ones
+// below): head size 64 has a matrix kernel of its own, 12 heads x 512 rows 18.5 against 17.8, x 943 33.8 against 37.6, 25 x 943
+// 57.7 against 60.1; the other sizes have a workgroup per query, which reads all keys: 12 x 48 at 128 rows 10.6 against
+// 9.1, at 200 11.9 against 17.0, at 943 32.3 against 128; 8 x 128 at 200 rows 19.6 against 20.8, 2 x 128 18.0 against 16.8
+// and at 300 21.2 against 22.1.
+static bool attention_splits(int Tq, int pos0, int H, int hs) {
+  if (hs > 128 || (hs & 3) || H > 65535 || pos0 + Tq > 12288) return false;
+  return Tq >= (hs == AHS ? 700 : hs > 96 ? 256 : 192);
+}
+
+size_t attention_workspace_bytes(int Tq, int pos0, int H, int hs) {
+  return attention_splits(Tq, pos0, H, hs) ? attention_split_bytes(Tq, pos0, H, hs) : 0;
+}
+
 hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc,
-                            const float* Vc, size_t hstride, int ldkv, float* out, int ldo, hipStream_t s) {
+                            const float* Vc, size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s) {
+  if (ws && attention_splits(Tq, pos0, H, hs)) return launch_attention_split(Tq, pos0, H, hs, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, ws, s);
   // a block of 32 queries per workgroup on the matrix cores
   if (hs == AHS && Tq >= AMQ) {
     static_assert(AHS * AMOST + 2 * AMQ <= AM_WAVE_FLOATS, "merge area must fit a wave's tile area");

@@ -43,6 +43,7 @@ struct Model {
   float *x = nullptr, *ln = nullptr, *qkv = nullptr, *att = nullptr, *tmp = nullptr, *h = nullptr;
   float* logits = nullptr;       // [V]
   float* part = nullptr;         // partial sums of the prefill products
+  void* att_ws = nullptr;        // workspace of the prefill attention
   float* taps = nullptr;         // [(2+6L)][maxT][d]
   int32_t* tok_dev = nullptr;    // [maxT] token ids of the current call
   int32_t* out_tok_dev = nullptr;  // [ctx] ids chosen by the greedy loop

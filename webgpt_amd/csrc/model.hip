@@ -134,7 +134,7 @@ static int forward_blocks(Model* m, int T, int pos0, bool want_taps) {
     ++ti;
     const KvAfter kva = {Kc, Vc, d, hs, m->ctx, pos0};  // the new keys and values join the cache with the product
     if ((rc = linear(m, T, 3 * d, d, m->ln, d, l.attn, l.attn_b, m->qkv, 3 * d, EPI_NONE, nullptr, nullptr, &kva))) return rc;
-    LAUNCH(launch_attention(T, pos0, H, hs, scale, m->qkv, 3 * d, Kc, Vc, (size_t)m->ctx * hs, hs, m->att, d, s));
+    LAUNCH(launch_attention(T, pos0, H, hs, scale, m->qkv, 3 * d, Kc, Vc, (size_t)m->ctx * hs, hs, m->att, d, m->att_ws, s));
     if (taps) {
       if ((rc = linear(m, T, d, d, m->att, d, l.proj, l.proj_b, m->tmp, d, EPI_NONE, nullptr))) return rc;
       if ((rc = tap(m, T, ti, m->tmp))) return rc;
@@ -688,6 +688,8 @@ int wgpt_model_finalize(wgpt_model h) {
   if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(double), (void**)&m->u_dev))) return rc;
   const size_t ws = gemm_workspace_floats((int)T, 4 * (int)d);  // partial sums of the prefill products
   if ((rc = dev_alloc(m, ws * f, (void**)&m->part))) return rc;
+  const size_t att_ws = attention_workspace_bytes((int)T, 0, m->H, m->hs);
+  if (att_ws && (rc = dev_alloc(m, att_ws, &m->att_ws))) return rc;
   if ((m->p.flags & WGPT_FLAG_TAPS) && (rc = dev_alloc(m, (size_t)(2 + 6 * m->L) * T * d * f, (void**)&m->taps))) return rc;
   WGPT_HIP(hipMemsetAsync(m->kv, 0, (size_t)m->L * 2 * m->ctx * d * f, rt().stream));
   WGPT_HIP(hipEventCreate(&m->ev0));
