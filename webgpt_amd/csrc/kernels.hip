@@ -130,6 +130,27 @@ __global__ __launch_bounds__(WG) void gemv_kn_partial(int N, int K, const float*
   }
 }
 
+// Sum of S partial sums, `stride` floats apart, in ascending order, U of them requested at a time: one after the other each is
+// a memory round trip (reduce_ln_kernel, 128 rows of 768 in 8 slices: 5.6 -> 5.2 us; 345M prompt of 512: 3.47 -> 3.25 ms).
+template <int U>
+__device__ __forceinline__ float4 sum_slices_by(const float* p, size_t stride, int S) {
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int s0 = 0; s0 < S; s0 += U) {
+    float4 v[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) v[j] = ld4(p + (size_t)(s0 + j < S ? s0 + j : S - 1) * stride);
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+      if (s0 + j < S) {
+        s.x += v[j].x; s.y += v[j].y; s.z += v[j].z; s.w += v[j].w;
+      }
+  }
+  return s;
+}
+__device__ __forceinline__ float4 sum_slices(const float* p, size_t stride, int S) {
+  return S <= 2 ? sum_slices_by<2>(p, stride, S) : S <= 4 ? sum_slices_by<4>(p, stride, S) : sum_slices_by<8>(p, stride, S);
+}
+
 // With kv.Kc set, C is a [M, 3d] q/k/v matrix whose key and value columns also go to the head-major cache
 // (kv_append_kernel's layout).
 __global__ __launch_bounds__(WG) void gemv_reduce(int M, int N, int S, const float* __restrict__ part,
@@ -139,11 +160,7 @@ __global__ __launch_bounds__(WG) void gemv_reduce(int M, int N, int S, const flo
   const int idx = blockIdx.x * WG + threadIdx.x;
   if (idx >= M * n4) return;
   const int r = idx / n4, n0 = (idx - r * n4) * 4;
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int sp = 0; sp < S; ++sp) {
-    const float4 v = ld4(part + ((size_t)sp * M + r) * N + n0);
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-  }
+  float4 s = sum_slices(part + (size_t)r * N + n0, (size_t)M * N, S);
   if (bias) {
     const float4 b = ld4(bias + n0);
     s.x += b.x; s.y += b.y; s.z += b.z; s.w += b.w;
@@ -224,11 +241,7 @@ __global__ __launch_bounds__(WG) void reduce_ln_kernel(int M, int N, int S, cons
       // (requested with the partial sums: behind the two reductions they would be a memory round trip of their own)
       gpre[j] = ld4(gamma + n0);
       bpre[j] = ld4(beta + n0);
-      float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int sp = 0; sp < S; ++sp) {
-        const float4 p = ld4(part + ((size_t)sp * M + r) * N + n0);
-        a.x += p.x; a.y += p.y; a.z += p.z; a.w += p.w;
-      }
+      float4 a = sum_slices(part + (size_t)r * N + n0, (size_t)M * N, S);
       if (bias) {
         const float4 b = ld4(bias + n0);
         a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
