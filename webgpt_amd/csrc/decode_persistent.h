@@ -48,6 +48,8 @@ __host__ __device__ inline LayerParamOffsets layer_param_offsets(int d) {
   return o;
 }
 
+constexpr int PD_U_ARG = 8;  // draws that travel with a launch: the tokens that GPT.generate makes per call
+
 struct PersistentArgs {
   int L, H, d, ctx, V;
   float scale;
@@ -83,15 +85,18 @@ struct PersistentArgs {
   // (model.js:81-85) with u[step] for the step's Math.random() and the float64 temperature
   int top_k;
   double temperature;
-  const double* u;  // [nsteps], device memory (unused for top_k == 1)
+  const double* u;  // [nsteps], device memory (unused for top_k == 1); null: u_arg holds the draws (a call of a few steps saves a copy)
+  double u_arg[PD_U_ARG];
   unsigned ebase;      // epoch of the last word published by earlier launches
   int pos0, nsteps;
-  // Results written straight into pinned host memory, so that a call of one step needs no copy behind the kernel
-  // (both may be null). host_logits[V]: the logits of the last step (shapes persistent_writes_host_logits names;
+  // Results written straight into pinned host memory, so that a call needs no copy behind the kernel
+  // (each may be null). host_logits[V]: the logits of the last step (shapes persistent_writes_host_logits names;
   // needs rows_per_wg <= 4 d). host_done: workgroup 0 stores *err there once it has finished the last step, which
   // it can only after every workgroup has published its last word; a launch that gave up leaves the word alone.
+  // host_ids[nsteps]: the ids of out_tok once more.
   float* host_logits;
   int* host_done;
+  int32_t* host_ids;
 };
 
 PhaseGeom make_geom(int N, int K);

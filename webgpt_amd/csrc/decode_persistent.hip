@@ -1869,7 +1869,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
     // ======================= arg-max over the workgroups, finished by everyone =======================
     double ustep = 0.0;
     if (SAMPLE) {
-      ustep = a.u[step];
+      ustep = a.u ? a.u[step] : a.u_arg[step];
       poll_words<2 * PD_TOPK * C::G>(a.bufAM, ep, attp, a.err, a.delay[6], a.spin_limit);
     } else {
       poll_words<2 * C::G>(a.bufAM, ep, attp, a.err, a.delay[6], a.spin_limit);
@@ -1936,7 +1936,10 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
         }
       }
       tok = pick != NOCAND ? pick : lastsel;
-      if (wg == 0 && tid == 0) a.out_tok[step] = tok;
+      if (wg == 0 && tid == 0) {
+        a.out_tok[step] = tok;
+        if (a.host_ids) a.host_ids[step] = tok;
+      }
     } else {
       float b = -INFINITY;
       int bi = 0x7fffffff;
@@ -1958,7 +1961,10 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
         }
       }
       tok = bi;  // every wave of every workgroup holds the same result
-      if (wg == 0 && tid == 0) a.out_tok[step] = tok;
+      if (wg == 0 && tid == 0) {
+        a.out_tok[step] = tok;
+        if (a.host_ids) a.host_ids[step] = tok;
+      }
     }
     __syncthreads();
   }

@@ -373,15 +373,16 @@ static int setup_persistent(Model* m) {
     // curves are flat within a few percent around them and over context length);
     // wgpt_model_tune_poll_delays searches around them on the GPU at hand,
     // WEBGPT_AMD_POLL_DELAYS="a,b,c,d,e,f,g" overrides them for experiments
-    static const int tuned[5][7] = {{16, 4, 22, 78, 24, 28, 48},    // d <= 768
+    static const int tuned[6][7] = {{16, 4, 22, 78, 24, 28, 48},    // d = 768
                                     {36, 0, 26, 82, 40, 40, 4},     // d = 1024
                                     {20, 0, 34, 100, 16, 16, 52},   // d = 1280
                                     {8, 12, 22, 84, 20, 12, 44},    // d = 1600, int8
-                                    {32, 0, 48, 96, 4, 20, 40}};    // d = 1600, fp32
+                                    {32, 0, 48, 96, 4, 20, 40},     // d = 1600, fp32
+                                    {20, 4, 22, 78, 16, 16, 32}};   // d = 384: 51.1 us per token against 55.0 with d = 768's
     // growth of [2] and [3] per 1024 positions of context (the best values at contexts of 100, 350, 650 and 900
     // positions lie on a line: 117M 80, 88, 88, 104 for [3]; int8 88, 104, 128, 136)
-    static const int slopes[5][2] = {{11, 28}, {0, 46}, {9, 70}, {20, 61}, {0, 0}};
-    const int row = d <= 768 ? 0 : d == 1024 ? 1 : d == 1280 ? 2 : i8 ? 3 : 4;
+    static const int slopes[6][2] = {{11, 28}, {0, 46}, {9, 70}, {20, 61}, {0, 0}, {11, 28}};
+    const int row = d <= 384 ? 5 : d <= 768 ? 0 : d == 1024 ? 1 : d == 1280 ? 2 : i8 ? 3 : 4;
     const int* dflt = tuned[row];
     for (int i = 0; i < 7; ++i) a.delay[i] = dflt[i];
     a.att_slope[0] = slopes[row][0];
@@ -432,21 +433,30 @@ static int setup_persistent(Model* m) {
 
 // Runs `steps` greedy decode steps from position m->pos with the persistent kernel.
 // The first token is in m->tok_dev[0]; chosen ids land in m->out_tok_dev.
-// top_k == 1: greedy. Otherwise u_dev holds the steps' uniform draws.
-// host_results: the call ends with a read-back (finish_timed, finish_steps): the kernel then reports its error word, and
-// where the shape allows the last step's logits, in pinned host memory itself instead of through copies behind it.
-static int decode_persistent(Model* m, int steps, int top_k = 1, double temperature = 1.0, const double* u_dev = nullptr, int token = -1,
+// top_k == 1: greedy. Otherwise u holds the steps' uniform draws (on the host; up to PD_U_ARG of them travel with the launch).
+// host_results: the call ends with a read-back (finish_timed, finish_steps): the kernel then reports its error word and the
+// ids, and where the shape allows the last step's logits, in pinned host memory itself instead of through copies behind it.
+// (generate() at the toy model's size: three copies and a synchronisation less per eight tokens, see finish_steps.)
+static int decode_persistent(Model* m, int steps, int top_k = 1, double temperature = 1.0, const double* u = nullptr, int token = -1,
                              bool host_results = false) {
   PersistentArgs a = m->pa;
   a.host_logits = nullptr;
   a.host_done = nullptr;
+  a.host_ids = host_results ? m->ids_pin : nullptr;
   if (token >= 0) {  // the first token travels with the launch instead of through tok_dev
     a.tok = nullptr;
     a.tok_value = token;
   }
   a.top_k = top_k;
   a.temperature = temperature;
-  a.u = u_dev;
+  a.u = nullptr;
+  if (u && steps <= PD_U_ARG) {
+    for (int i = 0; i < steps; ++i) a.u_arg[i] = u[i];
+  } else if (u) {
+    memcpy(m->u_pin, u, sizeof(double) * (size_t)steps);  // (every earlier use has completed: each call ends with a synchronisation)
+    WGPT_HIP(hipMemcpyAsync(m->u_dev, m->u_pin, sizeof(double) * (size_t)steps, hipMemcpyHostToDevice, rt().stream));
+    a.u = m->u_dev;
+  }
   const unsigned per_step = persistent_epochs_per_step(m->L);
   if (m->epoch > 0x7fffffffu - per_step * (unsigned)steps - 8u) {
     // epoch counter about to leave the positive ints (the kernel's error word is the epoch of the wait that
@@ -470,6 +480,8 @@ static int decode_persistent(Model* m, int steps, int top_k = 1, double temperat
     a.tok = a.out_tok + short_steps - 1;
     a.out_tok += short_steps;
     if (a.u) a.u += short_steps;
+    for (int i = 0; i + short_steps < PD_U_ARG; ++i) a.u_arg[i] = a.u_arg[i + short_steps];
+    if (a.host_ids) a.host_ids += short_steps;
     a.nsteps = steps - short_steps;
   }
   if (host_results) {  // (the last launch of the call only)
@@ -479,6 +491,7 @@ static int decode_persistent(Model* m, int steps, int top_k = 1, double temperat
   }
   LAUNCH(launch_decode_persistent(a, rt().stream));
   m->res_host_done = a.host_done != nullptr;
+  m->res_host_ids = a.host_ids != nullptr;
   m->res_host_logits = a.host_logits != nullptr;
   m->epoch += per_step * (unsigned)steps;
   return WGPT_OK;
@@ -517,7 +530,7 @@ static int check_persistent(Model* m) {
 // memory itself (res_host_done, res_host_logits) is not copied again.
 static int read_back(Model* m, float* logits) {
   const bool host_done = m->res_host_done, host_logits = m->res_host_logits;
-  m->res_host_done = m->res_host_logits = false;
+  m->res_host_done = m->res_host_logits = m->res_host_ids = false;
   const bool copy_logits = logits && !host_logits, copy_err = m->perr && !host_done;
   if (copy_logits && copy_err) {
     WGPT_HIP(hipMemcpyAsync(m->logits_pin, m->logits, sizeof(float) * ((size_t)m->V + 1), hipMemcpyDeviceToHost, rt().stream));
@@ -548,7 +561,7 @@ static int finish_timed(Model* m, float* logits) {
 // staged by the runtime and costs tens of microseconds per call. Ends with the stream drained.
 static int finish_steps(Model* m, int32_t* out_tokens, const int32_t* ids_dev, int steps, float* logits) {
   WGPT_HIP(hipEventRecord(m->ev1, rt().stream));
-  WGPT_HIP(hipMemcpyAsync(m->ids_pin, ids_dev, sizeof(int32_t) * (size_t)steps, hipMemcpyDeviceToHost, rt().stream));
+  if (!m->res_host_ids) WGPT_HIP(hipMemcpyAsync(m->ids_pin, ids_dev, sizeof(int32_t) * (size_t)steps, hipMemcpyDeviceToHost, rt().stream));
   const int rc = read_back(m, logits);
   if (rc) return rc;
   memcpy(out_tokens, m->ids_pin, sizeof(int32_t) * (size_t)steps);
@@ -556,26 +569,21 @@ static int finish_steps(Model* m, int32_t* out_tokens, const int32_t* ids_dev, i
   return WGPT_OK;
 }
 
-// Puts the linear weights, which the decode layouts have been built from, into the order that the prefill products read
-// (in place, through a buffer of the largest one).
-static int block_linear_weights(Model* m) {
+// Puts the linear weights, which the decode layouts have been built from, into the order that the prefill products read. Each
+// matrix goes where the one before it was, the first into free_buf, of the largest size: largest matrices first.
+static int block_linear_weights(Model* m, void* free_buf) {
   const int d = m->d;
   const bool i8 = m->p.weight_dtype == 1;
-  const size_t elem = i8 ? 1 : sizeof(float);
-  void* tmp = nullptr;
-  hipError_t e = hipMalloc(&tmp, (size_t)4 * d * d * elem);
-  if (e != hipSuccess) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): %s", (size_t)4 * d * d * elem, hipGetErrorString(e));
-  for (const LayerW& l : m->layers) {
-    const struct { const LinW* w; int K, N; } lins[4] = {{&l.attn, d, 3 * d}, {&l.proj, d, d}, {&l.fc, d, 4 * d}, {&l.fc2, 4 * d, d}};
-    for (const auto& t : lins) {
-      void* w = i8 ? (void*)t.w->q : (void*)t.w->w;
-      if (e == hipSuccess) e = launch_block_weights(t.K, t.N, i8, w, tmp, rt().stream);
-      if (e == hipSuccess) e = hipMemcpyAsync(w, tmp, (size_t)t.K * t.N * elem, hipMemcpyDeviceToDevice, rt().stream);
+  const struct { LinW LayerW::*w; int K, N; } lins[4] = {{&LayerW::fc, d, 4 * d}, {&LayerW::fc2, 4 * d, d}, {&LayerW::attn, d, 3 * d}, {&LayerW::proj, d, d}};
+  for (const auto& t : lins)
+    for (LayerW& l : m->layers) {
+      LinW& w = l.*t.w;
+      void* old = i8 ? (void*)w.q : (void*)w.w;
+      LAUNCH(launch_block_weights(t.K, t.N, i8, old, free_buf, rt().stream));
+      if (i8) w.q = (int32_t*)free_buf;
+      else w.w = (float*)free_buf;
+      free_buf = old;
     }
-  }
-  const hipError_t es = hipStreamSynchronize(rt().stream), ef = hipFree(tmp);
-  if (e == hipSuccess) e = es != hipSuccess ? es : ef;
-  if (e != hipSuccess) return fail(WGPT_ERR_HIP, "layout of the linear weights: %s", hipGetErrorString(e));
   return WGPT_OK;
 }
 
@@ -585,7 +593,7 @@ static void destroy_model(Model* m) {
   for (void* p : m->allocs) (void)hipFree(p);
   if (m->pin) (void)hipHostFree(m->pin);
   if (m->logits_pin) (void)hipHostFree(m->logits_pin);
-  if (m->ids_pin) (void)hipHostFree(m->ids_pin);
+  if (m->u_pin) (void)hipHostFree(m->u_pin);
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
   delete m;
@@ -663,40 +671,49 @@ int wgpt_model_finalize(wgpt_model h) {
   }
   const size_t d = m->d, T = m->maxT, f = sizeof(float);
   int rc;
-  if ((rc = dev_alloc(m, (size_t)m->L * 2 * m->ctx * d * f, (void**)&m->kv))) return rc;
-  if ((rc = dev_alloc(m, T * d * f, (void**)&m->x))) return rc;
-  if ((rc = dev_alloc(m, T * d * f, (void**)&m->ln))) return rc;
-  if ((rc = dev_alloc(m, T * 3 * d * f, (void**)&m->qkv))) return rc;
-  if ((rc = dev_alloc(m, T * d * f, (void**)&m->att))) return rc;
-  if ((rc = dev_alloc(m, T * d * f, (void**)&m->tmp))) return rc;
-  if ((rc = dev_alloc(m, T * 4 * d * f, (void**)&m->h))) return rc;
-  // the error word of the persistent kernel lives right behind the logits, so that one copy brings both back
-  if ((rc = dev_alloc(m, ((size_t)m->V + 1) * f, (void**)&m->logits))) return rc;
-  if ((rc = dev_alloc(m, T * sizeof(int32_t), (void**)&m->tok_dev))) return rc;
+  m->att_nslice = attention_decode_slices(m->hs, m->ctx);
+  const size_t part_bytes = gemm_workspace_floats((int)T, 4 * (int)d) * f;  // partial sums of the prefill products
+  const size_t att_ws = attention_workspace_bytes((int)T, 0, m->H, m->hs);
+  void* block_buf = nullptr;
+  // everything in one allocation: each costs a model's load tenths of a millisecond
+  const struct { void** dst; size_t bytes; } bufs[] = {
+      {(void**)&m->kv, (size_t)m->L * 2 * m->ctx * d * f},
+      {(void**)&m->x, T * d * f}, {(void**)&m->ln, T * d * f}, {(void**)&m->qkv, T * 3 * d * f}, {(void**)&m->att, T * d * f},
+      {(void**)&m->tmp, T * d * f}, {(void**)&m->h, T * 4 * d * f},
+      // the error word of the persistent kernel lives right behind the logits, so that one copy brings both back
+      {(void**)&m->logits, ((size_t)m->V + 1) * f},
+      {(void**)&m->tok_dev, T * sizeof(int32_t)}, {(void**)&m->pos_dev, sizeof(int)},
+      {(void**)&m->att_part, m->att_nslice > 1 ? (size_t)m->H * m->att_nslice * (m->hs + 4) * f : 0},
+      {(void**)&m->out_tok_dev, (size_t)m->ctx * sizeof(int32_t)}, {(void**)&m->out_samp_dev, (size_t)m->ctx * sizeof(int32_t)},
+      {(void**)&m->u_dev, (size_t)m->ctx * sizeof(double)}, {(void**)&m->part, part_bytes},
+      {(void**)&m->att_ws, att_ws > part_bytes ? att_ws : 0},
+      {(void**)&m->taps, m->p.flags & WGPT_FLAG_TAPS ? (size_t)(2 + 6 * m->L) * T * d * f : 0},
+      {&block_buf, (size_t)4 * d * d * (i8 ? 1 : f)}};
+  const auto room = [](size_t bytes) { return (bytes + 16 + 255) / 256 * 256; };
+  size_t total = 0;
+  for (const auto& b : bufs) total += room(b.bytes);
+  char* base;
+  if ((rc = dev_alloc(m, total, (void**)&base))) return rc;
+  for (const auto& b : bufs) {
+    if (b.bytes) *b.dst = base;
+    base += room(b.bytes);
+  }
+  // the attention's workspace is in use while no product's partial sums are
+  if (att_ws && att_ws <= part_bytes) m->att_ws = m->part;
   if (!m->pin) {
     WGPT_HIP(hipHostMalloc((void**)&m->pin, 4 * sizeof(int32_t), hipHostMallocDefault));
     m->pin[0] = m->pin[1] = m->pin[2] = m->pin[3] = 0;
     WGPT_HIP(hipHostMalloc((void**)&m->logits_pin, sizeof(float) * ((size_t)m->V + 1), hipHostMallocDefault));
-    WGPT_HIP(hipHostMalloc((void**)&m->ids_pin, sizeof(int32_t) * (size_t)m->ctx, hipHostMallocDefault));
+    WGPT_HIP(hipHostMalloc((void**)&m->u_pin, (sizeof(double) + sizeof(int32_t)) * (size_t)m->ctx, hipHostMallocDefault));
+    m->ids_pin = reinterpret_cast<int32_t*>(m->u_pin + m->ctx);
   }
-  if ((rc = dev_alloc(m, sizeof(int), (void**)&m->pos_dev))) return rc;
-  m->att_nslice = attention_decode_slices(m->hs, m->ctx);
-  if (m->att_nslice > 1 && (rc = dev_alloc(m, (size_t)m->H * m->att_nslice * (m->hs + 4) * f, (void**)&m->att_part))) return rc;
   WGPT_HIP(hipMemsetAsync(m->pos_dev, 0, sizeof(int), rt().stream));
-  if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(int32_t), (void**)&m->out_tok_dev))) return rc;
-  if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(int32_t), (void**)&m->out_samp_dev))) return rc;
-  if ((rc = dev_alloc(m, (size_t)m->ctx * sizeof(double), (void**)&m->u_dev))) return rc;
-  const size_t ws = gemm_workspace_floats((int)T, 4 * (int)d);  // partial sums of the prefill products
-  if ((rc = dev_alloc(m, ws * f, (void**)&m->part))) return rc;
-  const size_t att_ws = attention_workspace_bytes((int)T, 0, m->H, m->hs);
-  if (att_ws && (rc = dev_alloc(m, att_ws, &m->att_ws))) return rc;
-  if ((m->p.flags & WGPT_FLAG_TAPS) && (rc = dev_alloc(m, (size_t)(2 + 6 * m->L) * T * d * f, (void**)&m->taps))) return rc;
   WGPT_HIP(hipMemsetAsync(m->kv, 0, (size_t)m->L * 2 * m->ctx * d * f, rt().stream));
   WGPT_HIP(hipEventCreate(&m->ev0));
   WGPT_HIP(hipEventCreate(&m->ev1));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   if ((rc = setup_persistent(m))) return rc;
-  if ((rc = block_linear_weights(m))) return rc;
+  if ((rc = block_linear_weights(m, block_buf))) return rc;
   m->decode_mode = m->persist_ok ? 1 : 0;
   m->pos = 0;
   m->finalized = true;
@@ -708,7 +725,7 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
   WGPT_REQUIRE_INIT();
   Model* m = find_model(h);
   if (!m) return WGPT_ERR_ARG;
-  m->res_host_done = m->res_host_logits = false;  // (left set by a call that failed between its launch and its read-back)
+  m->res_host_done = m->res_host_logits = m->res_host_ids = false;  // (left set by a call that failed between its launch and its read-back)
   if (!m->finalized) return fail(WGPT_ERR_STATE, "wgpt_prefill: model not finalised");
   if (!tokens || T < 1) return fail(WGPT_ERR_ARG, "wgpt_prefill: tokens and T >= 1 required");
   if (T > m->maxT) return fail(WGPT_ERR_ARG, "wgpt_prefill: T = %d exceeds max_prefill = %d", T, m->maxT);
@@ -734,7 +751,7 @@ int wgpt_decode(wgpt_model h, int32_t token, float* logits) {
   WGPT_REQUIRE_INIT();
   Model* m = find_model(h);
   if (!m) return WGPT_ERR_ARG;
-  m->res_host_done = m->res_host_logits = false;  // (left set by a call that failed between its launch and its read-back)
+  m->res_host_done = m->res_host_logits = m->res_host_ids = false;  // (left set by a call that failed between its launch and its read-back)
   m->x_rows = 0;
   if (!m->finalized) return fail(WGPT_ERR_STATE, "wgpt_decode: model not finalised");
   if (token < 0 || token >= m->V) return fail(WGPT_ERR_ARG, "wgpt_decode: token id %d outside [0, %d)", token, m->V);
@@ -759,7 +776,7 @@ int wgpt_decode_greedy(wgpt_model h, int32_t token, int steps, int32_t* out_toke
   WGPT_REQUIRE_INIT();
   Model* m = find_model(h);
   if (!m) return WGPT_ERR_ARG;
-  m->res_host_done = m->res_host_logits = false;  // (left set by a call that failed between its launch and its read-back)
+  m->res_host_done = m->res_host_logits = m->res_host_ids = false;  // (left set by a call that failed between its launch and its read-back)
   m->x_rows = 0;
   if (!m->finalized) return fail(WGPT_ERR_STATE, "wgpt_decode_greedy: model not finalised");
   if (token < 0 || token >= m->V) return fail(WGPT_ERR_ARG, "wgpt_decode_greedy: token id %d outside [0, %d)", token, m->V);
@@ -801,7 +818,7 @@ int wgpt_decode_sample(wgpt_model h, int32_t token, int steps, int top_k, double
   WGPT_REQUIRE_INIT();
   Model* m = find_model(h);
   if (!m) return WGPT_ERR_ARG;
-  m->res_host_done = m->res_host_logits = false;  // (left set by a call that failed between its launch and its read-back)
+  m->res_host_done = m->res_host_logits = m->res_host_ids = false;  // (left set by a call that failed between its launch and its read-back)
   m->x_rows = 0;
   if (!m->finalized) return fail(WGPT_ERR_STATE, "wgpt_decode_sample: model not finalised");
   if (token < 0 || token >= m->V) return fail(WGPT_ERR_ARG, "wgpt_decode_sample: token id %d outside [0, %d)", token, m->V);
@@ -813,25 +830,26 @@ int wgpt_decode_sample(wgpt_model h, int32_t token, int steps, int top_k, double
     if (!(u[i] >= 0.0 && u[i] < 1.0)) return fail(WGPT_ERR_ARG, "wgpt_decode_sample: u[%d] must be in [0, 1)", i);
   if (m->pos + steps > m->ctx)
     return fail(WGPT_ERR_STATE, "wgpt_decode_sample: %d steps from position %d exceed the context of %d", steps, m->pos, m->ctx);
-  WGPT_HIP(hipMemcpyAsync(m->tok_dev, &token, sizeof(int32_t), hipMemcpyHostToDevice, rt().stream));
-  WGPT_HIP(hipMemcpyAsync(m->u_dev, u, sizeof(double) * (size_t)steps, hipMemcpyHostToDevice, rt().stream));
   const bool persistent = m->decode_mode == 1;
-  if (!persistent) {
-    int rc0 = upload_position(m);
-    if (rc0) return rc0;
-  }
-  WGPT_HIP(hipStreamSynchronize(rt().stream));
-  WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
   const int k = top_k < m->V ? top_k : m->V;
   // up to PD_TOPK candidates the persistent kernel selects and samples itself, all steps in one launch
   const bool in_kernel = persistent && k <= PD_TOPK;
+  if (!in_kernel) {  // (that launch brings the token and the draws along)
+    m->pin[0] = token;  // every earlier use of the pinned words has completed: each call ends with a synchronisation
+    memcpy(m->u_pin, u, sizeof(double) * (size_t)steps);
+    WGPT_HIP(hipMemcpyAsync(m->tok_dev, &m->pin[0], sizeof(int32_t), hipMemcpyHostToDevice, rt().stream));
+    WGPT_HIP(hipMemcpyAsync(m->u_dev, m->u_pin, sizeof(double) * (size_t)steps, hipMemcpyHostToDevice, rt().stream));
+    int rc0;
+    if (!persistent && (rc0 = upload_position(m))) return rc0;
+  }
+  WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
   // The cache position is committed only when the whole call has succeeded (as wgpt_decode and
   // wgpt_decode_greedy do): after a failure the caller's history is unchanged, so a retry must find the
   // model where the call started. A step of the loop below reads m->pos; it is restored on every error path.
   const int pos_before = m->pos;
   int rc = WGPT_OK;
   if (in_kernel) {
-    rc = decode_persistent(m, steps, k, temperature, m->u_dev, token, true);
+    rc = decode_persistent(m, steps, k, temperature, u, token, true);
   } else {
     for (int i = 0; i < steps && rc == WGPT_OK; ++i) {
       // one token per launch: the sampled id in tok_dev[0] is the next launch's input
@@ -883,7 +901,7 @@ int wgpt_model_tune_poll_delays(wgpt_model h, int rounds, int32_t* chosen, float
     return fail(WGPT_ERR_STATE, "wgpt_model_tune_poll_delays: the persistent decode kernel is not in use for this model");
   if (m->pos != 0) return fail(WGPT_ERR_STATE, "wgpt_model_tune_poll_delays: a context is in use (position %d); call it before the first prefill or after wgpt_model_reset_cache", m->pos);
   if (rounds < 0 || rounds > 8) return fail(WGPT_ERR_ARG, "wgpt_model_tune_poll_delays: rounds must be in [0, 8]");
-  m->res_host_done = m->res_host_logits = false;
+  m->res_host_done = m->res_host_logits = m->res_host_ids = false;
   m->x_rows = 0;
   // a trial is two launches, at three tenths and at three quarters of the context (the attention exchange's best
   // delays move with the context length: a row found at one length loses at another), together long enough (about
