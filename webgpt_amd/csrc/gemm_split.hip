@@ -7,7 +7,7 @@
 // result is at least as close to the exact one as that of v_mfma_f32_32x32x2_f32. An int8 weight is one bf16 value
 // (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum. A value that is
 // infinite, or rounds to an infinite bf16, has no such split (inf + nan + nan): every sum it takes part in comes out as NaN
-// or infinite, and sums that do are taken again without the split (plain_products).
+// or infinite, and a wave that finds one among its sums takes them again with fp32 matrix instructions (plain_sums).
 // bf16 runs at 16 times the rate of fp32 here, six products are therefore 2.7 times (int8: 5.3 times) faster.
 #include "gemm_split.h"
 
@@ -28,6 +28,8 @@ struct SplitBlock<32> {
   static __device__ __forceinline__ acc_t mfma(const u32x4& w, const u32x4& a, const acc_t& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
   }
+  // fp32 operands: one k for each half of the wave
+  static __device__ __forceinline__ acc_t plain(float w, float a, const acc_t& c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(w, a, c, 0, 0, 0); }
   // column (of W) of the four consecutive ones in accumulator registers 4q..4q+3 of a lane
   static __device__ __forceinline__ int row4(int q, int lane) { return 8 * q + 4 * (lane >> 5); }
 };
@@ -38,6 +40,7 @@ struct SplitBlock<16> {
   static __device__ __forceinline__ acc_t mfma(const u32x4& w, const u32x4& a, const acc_t& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
   }
+  static __device__ __forceinline__ acc_t plain(float w, float a, const acc_t& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, c, 0, 0, 0); }
   static __device__ __forceinline__ int row4(int, int lane) { return 4 * (lane >> 4); }
 };
 
@@ -135,6 +138,12 @@ struct WRaw {
       return split8(__builtin_bit_cast(f32x4, a), __builtin_bit_cast(f32x4, b));
     }
   }
+  // value e of the eight of step s
+  __device__ __forceinline__ float plain(int s, int e, int n) const {
+    if constexpr (!I8) return __builtin_bit_cast(float, v[8 * s + e]);
+    else if constexpr (BLK) return (float)((int)(v[2 * s + (e >> 2)] << (24 - 8 * (e & 3))) >> 24);
+    else return (float)((int)(v[8 * s + e] << (24 - 8 * (n & 3))) >> 24);
+  }
 };
 // A of a lane, straight from memory (rows of A, fp32)
 template <int R>
@@ -155,42 +164,12 @@ struct ARaw {
     }
   }
   __device__ __forceinline__ Split8 get(int s) const { return split8(v[2 * s], v[2 * s + 1]); }
+  __device__ __forceinline__ float plain(int s, int e) const { return v[2 * s + (e >> 2)][e & 3]; }
 };
 
-// Row m times columns n..n+3 over the k of a slice, one fp32 product after the other: for sums with operands that cannot be
-// split. Slow (a thread reads everything itself), and only they pay for it.
-// (Inlined: a call would cost every launch of these kernels 5 us, for the stack that it needs.)
-template <bool I8, bool BLK>
-__device__ __forceinline__ f32x4 plain_products(const SplitGemmArgs& a, int m, int n, int slice) {
-  const int steps = a.K >> 5;
-  const int k0 = 32 * (int)((long)steps * slice / a.S), k1 = slice == a.S - 1 ? a.K : 32 * (int)((long)steps * (slice + 1) / a.S);
-  f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int k = k0; k < k1; ++k) {
-    const float x = a.A[(size_t)m * a.lda + k];
-    f32x4 w;
-    if constexpr (BLK) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        w[i] = I8 ? (float)static_cast<const signed char*>(a.W)[((size_t)(k >> 3) * a.N + n + i) * 8 + (k & 7)]
-                  : static_cast<const float*>(a.W)[((size_t)(k >> 2) * a.N + n + i) * 4 + (k & 3)];
-    } else if constexpr (I8) {
-      const int word = static_cast<const int*>(a.W)[(size_t)k * a.ldw + (n >> 2)];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = (float)((int)((unsigned)word << (24 - 8 * i)) >> 24);
-    } else {
-      w = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.W) + (size_t)k * a.ldw + n);
-    }
-    v += x * w;
-  }
-  return v;
-}
-
-template <bool I8, bool BLK>
+template <bool I8>
 __device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v) {
   if (m >= a.M || n >= a.N) return;
-  const float check = (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]);  // 0, or NaN if one is not finite
-  if (check != 0.f) v = plain_products<I8, BLK>(a, m, n, slice);
   if constexpr (I8) {
     const f32x4 s = *reinterpret_cast<const f32x4*>(a.wscale + n);
 #pragma unroll
@@ -244,8 +223,70 @@ __device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Spl
 #undef SPLIT_STEP
 }
 
+// Is there a sum in the wave's tile that is not finite? (One instruction per two registers: the maximum lets NaN through.)
+template <int R, int MB, int NB>
+__device__ __forceinline__ bool not_finite(const typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
+  float most = 0.f;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < SplitBlock<R>::NACC; ++e) most = __builtin_elementwise_maximum(most, fabsf(acc[i][j][e]));
+  return __builtin_amdgcn_ballot_w64(!(most < INFINITY)) != 0;
+}
+
+// The sums of a wave's tile from row m0 of A over its steps it0, it0 + by, .. below it1 (and the one that reaches beyond K) with
+// fp32 matrix instructions, for operands that cannot be split: 2.7 times (int8: 5.3 times) the matrix time of the sums that they
+// replace, and only the waves with such operands pay it: 943x3072x768 with nothing but NaN 37 -> about 92 us (1.7 ms with one
+// product after the other).
+// (Inlined: a call would cost every launch of these kernels 5 us, for the stack that it needs.)
+template <int R, int MB, int NB, bool I8, bool BLK>
+__device__ __forceinline__ void plain_sums(const SplitGemmArgs& a, __amdgpu_buffer_rsrc_t wb, __amdgpu_buffer_rsrc_t xb, int m0, const int (&nn)[NB],
+                                           int it0, int it1, int by, bool tail, typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
+  typedef SplitBlock<R> B;
+  const int lane = threadIdx.x & 63, r = lane & (R - 1), kg = lane / R;
+  WRaw<R, I8, BLK> w[NB];
+  ARaw<R> x[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < B::NACC; ++e) acc[i][j][e] = 0.f;
+  const auto multiply = [&](int kend) {  // kend: how many of a chunk's eight k there are
+#pragma unroll
+    for (int s = 0; s < WRaw<R, I8, BLK>::STEPS; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          // (beyond K the loads repeat the last row of W, which may be infinite, and A is zero)
+          const float wv = chunk_of<R>(s, kg) * 8 + e < kend ? w[j].plain(s, e, nn[j]) : 0.f;
+#pragma unroll
+          for (int i = 0; i < MB; ++i) acc[i][j] = B::plain(wv, x[i].plain(s, e), acc[i][j]);
+        }
+  };
+#pragma unroll 1
+  for (int it = it0; it < it1; it += by) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w[j].load(a, wb, WRaw<R, I8, BLK>::offset(a, nn[j], kg), it);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) x[i].load(a, xb, ARaw<R>::offset(a, m0 + i * R + r, kg), it);
+    multiply(32);
+  }
+  if (tail) {
+    const int it = a.K >> 5;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w[j].load_tail(a, wb, nn[j], kg, it);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) x[i].load_tail(a, xb, m0 + i * R + r, kg, it);
+    multiply(a.K & 31);
+  }
+}
+
 // sum of NP partial tiles (LDS, 64 float4 per entry) and epilogue
-template <int R, int MB, int NB, int NP, int THREADS, bool I8, bool BLK>
+template <int R, int MB, int NB, int NP, int THREADS, bool I8>
 __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4* red, int m0, int n0, int slice) {
   typedef SplitBlock<R> B;
   constexpr int Q = B::NACC / 4, ENT = MB * NB * Q;
@@ -254,7 +295,7 @@ __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4*
 #pragma unroll
     for (int u = 1; u < NP; ++u) v += red[u * ENT * 64 + e];
     const int ln = e & 63, b = e >> 6, q = b % Q, ij = b / Q;
-    split_epilogue<I8, BLK>(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v);
+    split_epilogue<I8>(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v);
   }
 }
 
@@ -265,7 +306,7 @@ __device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4*
 // (219 and 193 us with the fp32 tile kernel that served 5 to 15 rows before); 64x64 tiles: 512x4096x1024 32.4 us = 132
 // TFLOP/s (39.9 us with v_mfma_f32_32x32x2_f32), int8 300x6400x1600 38.8 us (73).
 template <int R, int MB, int NB, int NW, bool I8, bool BLK>
-__global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
+__global__ __launch_bounds__(NW * 64, MB == 2 ? 2 : 4) void gemm_split_rows(SplitGemmArgs a) {
   typedef SplitBlock<R> B;
   constexpr int STEPS = WRaw<R, I8, BLK>::STEPS, Q = B::NACC / 4, ENT = MB * NB * Q;
   extern __shared__ __attribute__((aligned(16))) float gs_lds[];
@@ -328,6 +369,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) split_products<R, MB, NB, I8>(ws[s], xs[s], acc);
   }
+  if (not_finite<R, MB, NB>(acc)) plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, it0, it1, 1, (a.K & 31) && part == parts - 1, acc);
   f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
 #pragma unroll
   for (int i = 0; i < MB; ++i)
@@ -337,7 +379,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_split_rows(SplitGemmArgs a) {
       for (int q = 0; q < Q; ++q)
         red[(wave * ENT + (i * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  finish_tile<R, MB, NB, NW, NW * 64, I8, BLK>(a, red, m0, n0, slice);
+  finish_tile<R, MB, NB, NW, NW * 64, I8>(a, red, m0, n0, slice);
 }
 
 __device__ __forceinline__ void lds_barrier() {  // orders LDS accesses only: loads from memory stay in flight
@@ -500,6 +542,8 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
     }
     lds_barrier();
   }
+  if (not_finite<R, MB, NB>(acc))
+    plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, s0 + grp, s1, KG, grp == 0 && (a.K & 31) && slice == a.S - 1, acc);
   f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
   constexpr int NBW = NWN * NB, ENT = MB * NBW * Q;
 #pragma unroll
@@ -510,7 +554,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
       for (int q = 0; q < Q; ++q)
         red[(grp * ENT + (i * NBW + wn * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  finish_tile<R, MB, NBW, KG, NWN * KG * 64, I8, BLK>(a, red, m0, n0, slice);
+  finish_tile<R, MB, NBW, KG, NWN * KG * 64, I8>(a, red, m0, n0, slice);
 }
 
 // [K, N] to the order that WRaw<.., BLK> reads; a thread makes one run of four (int8: eight) k of a column.
