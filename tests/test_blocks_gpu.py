@@ -368,6 +368,78 @@ def test_attention_split_operands(device, T, H, hs):
     assert not np.isfinite(got[1][T - 2]).any() and not np.isfinite(got[1][T - 1]).any()
 
 
+@pytest.mark.parametrize("T,H,hs,where", [(943, 12, 48, "key"), (943, 12, 48, "value"), (300, 8, 128, "key"), (943, 4, 32, "last")])
+def test_attention_split_not_finite_in_time(device, T, H, hs, where):
+    """A NaN in the first key, an infinity in the first value (every query takes its output again, to the end) and a NaN in the
+    last key: less than eight times the time of a call without (measured: 2.0 to 3.2; 100 to 710 with a loop over the keys
+    for each output)."""
+    d = H * hs
+    x = rnd(T, d)
+    eye, zero = np.eye(d, dtype=np.float32), np.zeros(d, np.float32)
+    ms = []
+    for special in (False, True):
+        v = x.copy()
+        bias = zero
+        if special and where == "value":  # (scores stay finite: the infinity comes in with the values' bias)
+            bias = zero.copy()
+            bias[::hs] = np.inf
+        elif special:
+            v[0 if where == "key" else T - 1, 0] = np.nan
+        bufs = [init_tensor(v, [T, d])]
+        for b in (zero, zero, bias, zero):
+            bufs += [init_tensor(eye, [d, d]), init_tensor(b, [d])]
+        inst = AttentionBlock.newFusedInstance(T, d, 1 / math.sqrt(hs), H, hs, *bufs, FastMatMulBlock, SoftmaxBlock)
+        ms.append(_launch_ms(inst, 10))
+        blocks.clearOperationCache()
+    assert ms[1] < 8 * ms[0], ms
+
+
+@pytest.mark.parametrize("T,H,hs", [(300, 4, 20), (2200, 3, 64), (2300, 4, 36), (400, 3, 96), (400, 2, 128)])
+def test_attention_split_infinite_values(device, T, H, hs):
+    """Operands that have no split although the outputs are finite: a key whose scores are -inf (its weight is zero), values next
+    to the largest float; and an infinite value, for the queries from its own on. Context of more than 2048 keys among
+    them. They come out of the projections: the last three columns of x are zero but for one row each, and meet 2**70."""
+    d = H * hs
+    rng = np.random.default_rng(T + d)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    x[:, 0] = np.abs(x[:, 0]) + 0.1
+    x[:, d - 3:] = 0
+    x[5, d - 3], x[9, d - 2], x[T - 2, d - 1] = 2.0 ** 70, np.float32(3.4e38) * np.float32(2.0 ** -70), 2.0 ** 70
+    wq, wo, zero = np.eye(d, dtype=np.float32), np.eye(d, dtype=np.float32), np.zeros(d, np.float32)
+    wq[d - 3:] = 0
+    wk, wv = wq.copy(), wq.copy()
+    wk[d - 3, 0] = -2.0 ** 70       # key 5 of head 0: -inf in dimension 0
+    wv[d - 2, hs + 2] = 2.0 ** 70   # value 9 of head 1: 3.4e38 in dimension 2
+    wv[d - 1, hs + 3] = 2.0 ** 70   # value T - 2 of head 1: inf in dimension 3
+    bufs = [init_tensor(x, [T, d])]
+    for w in (wq, wk, wv, wo):
+        bufs += [init_tensor(w, [d, d]), init_tensor(zero, [d])]
+    scale = 1 / math.sqrt(hs)
+    got = run(AttentionBlock.newFusedInstance(T, d, scale, H, hs, *bufs, FastMatMulBlock, SoftmaxBlock), (T, d))
+    with np.errstate(all="ignore"):
+        heads = lambda w: (x.astype(np.float64) @ w).reshape(T, H, hs).transpose(1, 0, 2)
+        q, k, v = heads(wq), heads(wk), heads(wv)
+        v[1, 9, 2] = np.float32(3.4e38)
+        k[0, 5, 0] = 0
+        s = q @ k.transpose(0, 2, 1) * np.float64(np.float32(scale))
+        s[0, :, 5] = -np.inf
+        s[:, np.triu(np.ones((T, T), bool), 1)] = -np.inf
+        p = np.exp(s - s.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        v[1, T - 2, 3] = 0
+        want = (p @ v).transpose(1, 0, 2).reshape(T, d)
+        size = (p @ np.abs(v)).transpose(1, 0, 2).reshape(T, d)
+        # a score is a sum of hs products in any order of up to eight roundings, and is rounded once more with the scale and the
+        # maximum: an absolute error e, which is the relative one of its weight; value 9 makes single weights visible. The
+        # sums over the keys: a run of at most T / 32 additions in a lane, and a few between lanes.
+        e = 2.0 ** -24 * (8 * (np.abs(q) @ np.abs(k).transpose(0, 2, 1)) * scale + 2 * np.abs(np.where(np.isfinite(s), s, 0)) + 8)
+        pe = p * e
+        bound = (pe @ np.abs(v) + pe.sum(-1, keepdims=True) * (p @ np.abs(v))).transpose(1, 0, 2).reshape(T, d) + 2.0 ** -24 * (T / 32 + 16) * size + 1e-30
+    ratio = (np.abs(got - want) / bound)[:T - 2]
+    assert np.all(ratio <= 1), (float(ratio.max()), np.unravel_index(ratio.argmax(), ratio.shape))
+    assert not np.isfinite(got[T - 2:]).any()  # (the projection behind it spreads an infinite output over its row)
+
+
 def test_attention_values_known_answer(device):
     # other/test.js:370-388 through the attention block: with Wq = Wk = 0 every score is 0, so the
     # softmax is uniform over j <= i: P = 1/(i+1). V = c // hs + 1 (via bv, Wv = 0), Wo = I:
