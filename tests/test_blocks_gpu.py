@@ -171,6 +171,33 @@ def test_split_matmul_not_finite_in_every_kernel(device, int8, M, N, K):
     assert np.array_equal(got, want.astype(np.float32), equal_nan=True)
 
 
+@pytest.mark.parametrize("big", ["all", "row", "value"])
+@pytest.mark.parametrize("M,N,K", [(5, 8, 100), (17, 568, 1872), (33, 2816, 1836), (33, 2744, 2148), (17, 4280, 2068), (100, 3240, 40), (300, 3528, 900),
+                                   (449, 4552, 260)])
+def test_int8_matmul_large_activations(device, M, N, K, big):
+    """Activations whose product with the bare int8 weights leaves the range of fp32, while that with scaled weights does not:
+    everywhere, in one row and in one value (whose wave's sums are then scaled apart from the others'). Error: that of
+    test_split_matmul_error_bound, and two roundings for the scaled weights."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    if big == "all":
+        A *= np.float32(3e36)
+    elif big == "row":
+        A[M // 2] *= np.float32(3e36)
+    else:
+        A[M // 2, K // 3] = 3e37
+    q = rng.integers(-128, 128, (K, N))
+    scale = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    got = run(FastMatMulBlock.newInt8Instance(M, N, K, init_tensor(A, [M, K]), init_tensor(pack_words(q), [K, N // 4]), init_tensor(scale, [N]),
+                                              init_tensor(bias, [N])), (M, N)).astype(np.float64)
+    W = q * (scale / np.float32(127.0)).astype(np.float64)
+    want = A.astype(np.float64) @ W + bias
+    size = np.abs(A).astype(np.float64) @ np.abs(W) + np.abs(bias)
+    assert np.abs(size).max() < 1e38
+    assert np.all(np.abs(got - want) <= 2.0 ** -24 * (K + 24) * size), float(np.max(np.abs(got - want) / size))
+
+
 def _launch_ms(inst, launches=40):
     """Milliseconds of a launch, the best of three runs of them (the copy of the result that ends a run is in it)."""
     best = math.inf

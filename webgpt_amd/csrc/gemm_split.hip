@@ -5,8 +5,9 @@
 // taken, all of them exact in the fp32 accumulator's input. The three left out (mid lo, lo mid, lo lo) are together below
 // 2^-25 |x y|, under half an ulp of the product; with sums of sixteen products rounded once instead of two at a time the
 // result is at least as close to the exact one as that of v_mfma_f32_32x32x2_f32. An int8 weight is one bf16 value
-// (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum. A value that is
-// infinite, or rounds to an infinite bf16, has no such split (inf + nan + nan): every sum it takes part in comes out as NaN
+// (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum; where that sum
+// leaves the range of fp32, which the scaled one need not, it is taken again with weights that are scaled first (plain_sums).
+// A value that is infinite, or rounds to an infinite bf16, has no such split (inf + nan + nan): every sum it takes part in comes out as NaN
 // or infinite, and a wave that finds one among its sums takes them again with fp32 matrix instructions (plain_sums).
 // bf16 runs at 16 times the rate of fp32 here, six products are therefore 2.7 times (int8: 5.3 times) faster.
 #include "gemm_split.h"
@@ -168,13 +169,16 @@ struct ARaw {
 };
 
 template <bool I8>
-__device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v) {
-  if (m >= a.M || n >= a.N) return;
+__device__ __forceinline__ f32x4 scaled(const SplitGemmArgs& a, int n, f32x4 v) {
   if constexpr (I8) {
     const f32x4 s = *reinterpret_cast<const f32x4*>(a.wscale + n);
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] *= s[i] / 127.0f;
   }
+  return v;
+}
+
+__device__ __forceinline__ void split_epilogue(const SplitGemmArgs& a, int m, int n, int slice, f32x4 v) {
   if (a.part) {
     *reinterpret_cast<f32x4*>(a.part + ((size_t)slice * a.M + m) * a.N + n) = v;
     return;
@@ -223,8 +227,9 @@ __device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Spl
 #undef SPLIT_STEP
 }
 
-// Is there a sum in the wave's tile that is not finite? (One instruction per two registers: the maximum lets NaN through.)
-template <int R, int MB, int NB>
+// Is there a sum in the wave's tile that is not finite? (One instruction per two registers: the maximum lets NaN through.) Unscaled
+// int8 sums have to stay below 2^124, so that the eight of a workgroup have a finite sum.
+template <int R, int MB, int NB, bool I8>
 __device__ __forceinline__ bool not_finite(const typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
   float most = 0.f;
 #pragma unroll
@@ -233,11 +238,11 @@ __device__ __forceinline__ bool not_finite(const typename SplitBlock<R>::acc_t (
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < SplitBlock<R>::NACC; ++e) most = __builtin_elementwise_maximum(most, fabsf(acc[i][j][e]));
-  return __builtin_amdgcn_ballot_w64(!(most < INFINITY)) != 0;
+  return __builtin_amdgcn_ballot_w64(!(most < (I8 ? 0x1p124f : INFINITY))) != 0;
 }
 
 // The sums of a wave's tile from row m0 of A over its steps it0, it0 + by, .. below it1 (and the one that reaches beyond K) with
-// fp32 matrix instructions, for operands that cannot be split: 2.7 times (int8: 5.3 times) the matrix time of the sums that they
+// fp32 matrix instructions (and int8 weights scaled), for operands that cannot be split: 2.7 times (int8: 5.3 times) the matrix time of the sums that they
 // replace, and only the waves with such operands pay it: 943x3072x768 with nothing but NaN 37 -> about 92 us (1.7 ms with one
 // product after the other).
 // (Inlined: a call would cost every launch of these kernels 5 us, for the stack that it needs.)
@@ -248,6 +253,11 @@ __device__ __forceinline__ void plain_sums(const SplitGemmArgs& a, __amdgpu_buff
   const int lane = threadIdx.x & 63, r = lane & (R - 1), kg = lane / R;
   WRaw<R, I8, BLK> w[NB];
   ARaw<R> x[MB];
+  float scale[NB];
+  if constexpr (I8) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) scale[j] = a.wscale[nn[j]] / 127.0f;
+  }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -262,7 +272,8 @@ __device__ __forceinline__ void plain_sums(const SplitGemmArgs& a, __amdgpu_buff
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
           // (beyond K the loads repeat the last row of W, which may be infinite, and A is zero)
-          const float wv = chunk_of<R>(s, kg) * 8 + e < kend ? w[j].plain(s, e, nn[j]) : 0.f;
+          float wv = chunk_of<R>(s, kg) * 8 + e < kend ? w[j].plain(s, e, nn[j]) : 0.f;
+          if constexpr (I8) wv *= scale[j];
 #pragma unroll
           for (int i = 0; i < MB; ++i) acc[i][j] = B::plain(wv, x[i].plain(s, e), acc[i][j]);
         }
@@ -285,17 +296,38 @@ __device__ __forceinline__ void plain_sums(const SplitGemmArgs& a, __amdgpu_buff
   }
 }
 
-// sum of NP partial tiles (LDS, 64 float4 per entry) and epilogue
-template <int R, int MB, int NB, int NP, int THREADS, bool I8>
-__device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4* red, int m0, int n0, int slice) {
+// Sum of NP partial tiles (LDS, 64 float4 per entry) and epilogue. A tile's columns belong to NWN waves; `plain`, int8 only: a
+// flag for each wave, partial tile by partial tile, whose sums are scaled already.
+template <int R, int MB, int NB, int NP, int NWN, int THREADS, bool I8>
+__device__ __forceinline__ void finish_tile(const SplitGemmArgs& a, const f32x4* red, const int* plain, int m0, int n0, int slice) {
   typedef SplitBlock<R> B;
   constexpr int Q = B::NACC / 4, ENT = MB * NB * Q;
-  for (int e = threadIdx.x; e < ENT * 64; e += THREADS) {
-    f32x4 v = red[e];
+  int some = 0;
+  if constexpr (I8) {
 #pragma unroll
-    for (int u = 1; u < NP; ++u) v += red[u * ENT * 64 + e];
+    for (int u = 0; u < NP * NWN; ++u) some |= plain[u];
+  }
+  for (int e = threadIdx.x; e < ENT * 64; e += THREADS) {
     const int ln = e & 63, b = e >> 6, q = b % Q, ij = b / Q;
-    split_epilogue<I8>(a, m0 + (ij / NB) * R + (ln & (R - 1)), n0 + (ij % NB) * R + B::row4(q, ln), slice, v);
+    const int m = m0 + (ij / NB) * R + (ln & (R - 1)), n = n0 + (ij % NB) * R + B::row4(q, ln);
+    if (m >= a.M || n >= a.N) continue;
+    f32x4 v;
+    if (I8 && some) {
+      f32x4 done = {0.f, 0.f, 0.f, 0.f};
+      v = done;
+#pragma unroll 1
+      for (int u = 0; u < NP; ++u) {
+        if (plain[u * NWN + (ij % NB) / (NB / NWN)]) done += red[u * ENT * 64 + e];
+        else v += red[u * ENT * 64 + e];
+      }
+      v = scaled<I8>(a, n, v) + done;
+    } else {
+      v = red[e];
+#pragma unroll
+      for (int u = 1; u < NP; ++u) v += red[u * ENT * 64 + e];
+      v = scaled<I8>(a, n, v);
+    }
+    split_epilogue(a, m, n, slice, v);
   }
 }
 
@@ -369,7 +401,10 @@ __global__ __launch_bounds__(NW * 64, MB == 2 ? 2 : 4) void gemm_split_rows(Spli
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) split_products<R, MB, NB, I8>(ws[s], xs[s], acc);
   }
-  if (not_finite<R, MB, NB>(acc)) plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, it0, it1, 1, (a.K & 31) && part == parts - 1, acc);
+  __shared__ int plain[NW];
+  const bool again = not_finite<R, MB, NB, I8>(acc);
+  if (again) plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, it0, it1, 1, (a.K & 31) && part == parts - 1, acc);
+  if constexpr (I8) plain[wave] = again;
   f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
 #pragma unroll
   for (int i = 0; i < MB; ++i)
@@ -379,7 +414,7 @@ __global__ __launch_bounds__(NW * 64, MB == 2 ? 2 : 4) void gemm_split_rows(Spli
       for (int q = 0; q < Q; ++q)
         red[(wave * ENT + (i * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  finish_tile<R, MB, NB, NW, NW * 64, I8>(a, red, m0, n0, slice);
+  finish_tile<R, MB, NB, NW, 1, NW * 64, I8>(a, red, plain, m0, n0, slice);
 }
 
 __device__ __forceinline__ void lds_barrier() {  // orders LDS accesses only: loads from memory stay in flight
@@ -542,8 +577,11 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
     }
     lds_barrier();
   }
-  if (not_finite<R, MB, NB>(acc))
+  __shared__ int plain[KG * NWN];
+  const bool again = not_finite<R, MB, NB, I8>(acc);
+  if (again)
     plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, s0 + grp, s1, KG, grp == 0 && (a.K & 31) && slice == a.S - 1, acc);
+  if constexpr (I8) plain[wave] = again;
   f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
   constexpr int NBW = NWN * NB, ENT = MB * NBW * Q;
 #pragma unroll
@@ -554,7 +592,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
       for (int q = 0; q < Q; ++q)
         red[(grp * ENT + (i * NBW + wn * NB + j) * Q + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  finish_tile<R, MB, NBW, KG, NWN * KG * 64, I8>(a, red, m0, n0, slice);
+  finish_tile<R, MB, NBW, KG, NWN, NWN * KG * 64, I8>(a, red, plain, m0, n0, slice);
 }
 
 // [K, N] to the order that WRaw<.., BLK> reads; a thread makes one run of four (int8: eight) k of a column.
