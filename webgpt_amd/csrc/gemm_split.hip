@@ -1,7 +1,7 @@
 // FastMatMulBlock (instructions.js:157-319) for prompts, and its int8 weight-only form (other/int8-gemm.js:117-229).
 //
-// The operands are fp32 (the weights perhaps int8), the multiplications run on the bf16 matrix cores: every fp32 value
-// is the exact sum of three bf16 values, x = hi + mid + lo, and of the nine partial products of x y the six largest are
+// The operands are fp32 (the weights perhaps int8), the multiplications run on the bf16 matrix cores: an fp32 value from
+// 2^-110 on is the exact sum of three bf16 values, x = hi + mid + lo (smaller ones: spoilt), and of the nine partial products of x y the six largest are
 // taken, all of them exact in the fp32 accumulator's input. The three left out (mid lo, lo mid, lo lo) are together below
 // 2^-25 |x y|, under half an ulp of the product; with sums of sixteen products rounded once instead of two at a time the
 // result is at least as close to the exact one as that of v_mfma_f32_32x32x2_f32. An int8 weight is one bf16 value
@@ -227,18 +227,23 @@ __device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Spl
 #undef SPLIT_STEP
 }
 
-// Is there a sum in the wave's tile that is not finite? (One instruction per two registers: the maximum lets NaN through.) Unscaled
-// int8 sums have to stay below 2^124, so that the eight of a workgroup have a finite sum.
+// Are there sums in the wave's tile that the split may have spoilt? Those that are not finite; unscaled int8 ones of 2^124 and
+// more, so that the eight of a workgroup have a finite sum; and a row of nothing but tiny ones: a value under 2^-110 loses
+// what its third part would hold under the smallest bf16 subnormal, 2^-134 at most, which shows where the whole row is
+// that small. (One instruction per two registers: the maximum lets NaN through.)
 template <int R, int MB, int NB, bool I8>
-__device__ __forceinline__ bool not_finite(const typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
-  float most = 0.f;
+__device__ __forceinline__ bool spoilt(const typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
+  bool bad = false;
 #pragma unroll
-  for (int i = 0; i < MB; ++i)
+  for (int i = 0; i < MB; ++i) {
+    float most = 0.f;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < SplitBlock<R>::NACC; ++e) most = __builtin_elementwise_maximum(most, fabsf(acc[i][j][e]));
-  return __builtin_amdgcn_ballot_w64(!(most < (I8 ? 0x1p124f : INFINITY))) != 0;
+    bad = bad || !(most < (I8 ? 0x1p124f : INFINITY)) || (most < 0x1p-100f && most > 0.f);
+  }
+  return __builtin_amdgcn_ballot_w64(bad) != 0;
 }
 
 // The sums of a wave's tile from row m0 of A over its steps it0, it0 + by, .. below it1 (and the one that reaches beyond K) with
@@ -402,7 +407,7 @@ __global__ __launch_bounds__(NW * 64, MB == 2 ? 2 : 4) void gemm_split_rows(Spli
     for (int s = 0; s < STEPS; ++s) split_products<R, MB, NB, I8>(ws[s], xs[s], acc);
   }
   __shared__ int plain[NW];
-  const bool again = not_finite<R, MB, NB, I8>(acc);
+  const bool again = spoilt<R, MB, NB, I8>(acc);
   if (again) plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, it0, it1, 1, (a.K & 31) && part == parts - 1, acc);
   if constexpr (I8) plain[wave] = again;
   f32x4* red = reinterpret_cast<f32x4*>(gs_lds);
@@ -578,7 +583,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
     lds_barrier();
   }
   __shared__ int plain[KG * NWN];
-  const bool again = not_finite<R, MB, NB, I8>(acc);
+  const bool again = spoilt<R, MB, NB, I8>(acc);
   if (again)
     plain_sums<R, MB, NB, I8, BLK>(a, wb, xb, m0, nn, s0 + grp, s1, KG, grp == 0 && (a.K & 31) && slice == a.S - 1, acc);
   if constexpr (I8) plain[wave] = again;
