@@ -92,7 +92,8 @@ def test_split_matmul_error_bound(device, int8, M, N, K):
     """The products on the bf16 matrix cores against 64-bit ones: the edges of every tile (16, 32, 64 and 128 rows), partial
     steps of 32 k and sliced K. The parts of a value add up to it exactly and all six products kept are exact, so the error
     is that of the fp32 sums: at most six roundings per sixteen k, a few for the slices and waves, each at most 2**-24 of
-    the sum of magnitudes, and 2**-25 of it for the products left out."""
+    the sum of magnitudes, and 2**-24 of it for the products left out (a value's second and third parts are at most 2**-8
+    and 2**-17 of it, and two such products are left out)."""
     rng = np.random.default_rng(M * N + K)
     A = rng.standard_normal((M, K)).astype(np.float32) * np.exp(rng.standard_normal((M, 1))).astype(np.float32)
     bias = rng.standard_normal(N).astype(np.float32)
@@ -113,6 +114,18 @@ def test_split_matmul_error_bound(device, int8, M, N, K):
     assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
     # and in practice no worse than sums of a few products at a time in fp32
     assert np.linalg.norm(got - want) <= 2.0 ** -24 * max(4.0, K ** 0.5) * np.linalg.norm(size)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 64, 4), (33, 72, 64), (65, 136, 1024), (130, 264, 260)])
+def test_split_matmul_largest_part_left_out(device, M, N, K):
+    """Every value 1 + 2**-8 - 2**-17, whose parts are 1, 2**-8 and -2**-17: the products left out are 1.98 * 2**-25 of each
+    product, all of one sign. Bound of test_split_matmul_error_bound."""
+    x = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    inst = FastMatMulBlock.newInstance(M, N, K, init_tensor(np.full((M, K), x), [M, K]), init_tensor(np.full((K, N), x), [K, N]),
+                                       init_tensor(np.zeros(N, np.float32), [N]))
+    got = run(inst, (M, N)).astype(np.float64)
+    want = K * np.float64(x) ** 2
+    assert np.all(np.abs(got - want) <= 2.0 ** -24 * (6 * K / 16 + 2) * want), float(np.abs(got / want - 1).max()) * 2.0 ** 24
 
 
 @pytest.mark.parametrize("int8", [False, True])

@@ -1,14 +1,16 @@
 // FastMatMulBlock (instructions.js:157-319) for prompts, and its int8 weight-only form (other/int8-gemm.js:117-229).
 //
-// The operands are fp32 (the weights perhaps int8), the multiplications run on the bf16 matrix cores: an fp32 value from
-// 2^-110 on is the exact sum of three bf16 values, x = hi + mid + lo (smaller ones: spoilt), and of the nine partial products of x y the six largest are
-// taken, all of them exact in the fp32 accumulator's input. The three left out (mid lo, lo mid, lo lo) are together below
-// 2^-25 |x y|, under half an ulp of the product; with sums of sixteen products rounded once instead of two at a time the
-// result is at least as close to the exact one as that of v_mfma_f32_32x32x2_f32. An int8 weight is one bf16 value
-// (8 significand bits), so three products do, and the column's scale[n] / 127 is applied to the finished sum; where that sum
-// leaves the range of fp32, which the scaled one need not, it is taken again with weights that are scaled first (plain_sums).
-// A value that is infinite, or rounds to an infinite bf16, has no such split (inf + nan + nan): every sum it takes part in comes out as NaN
-// or infinite, and a wave that finds one among its sums takes them again with fp32 matrix instructions (plain_sums).
+// The operands are fp32 (the weights perhaps int8), the multiplications run on the bf16 matrix cores: an fp32 value of 2^-110
+// and more is the exact sum of three bf16 values, x = hi + mid + lo with |mid| <= 2^-8 |x| and |lo| <= 2^-17 |x| (smaller
+// values: spoilt), and of the nine partial products of x y the six largest are taken, all of them exact in the fp32
+// accumulator's input. The three left out (mid lo, lo mid, lo lo) are together at most 2^-24 |x y|, an fp32 rounding of one
+// product; with sums of sixteen products rounded once instead of two at a time the sum of four products and more is at least
+// as close to the exact one as that of v_mfma_f32_32x32x2_f32 (emulated, norm of the errors: K = 4 2.6e-8 against 3.1e-8,
+// K = 768 3.1e-7 against 3.7e-7). An int8 weight is one bf16 value (8 significand bits), so three products do, and
+// the column's scale[n] / 127 is applied to the finished sum; where that sum leaves the range of fp32, which the scaled
+// one need not, it is taken again with weights that are scaled first (plain_sums). A value that is infinite, or rounds to an
+// infinite bf16, has no such split (inf + nan + nan): every sum it takes part in comes out as NaN or infinite, and a wave that
+// finds one among its sums takes them again with fp32 matrix instructions (plain_sums).
 // bf16 runs at 16 times the rate of fp32 here, six products are therefore 2.7 times (int8: 5.3 times) faster.
 #include "gemm_split.h"
 
@@ -214,7 +216,7 @@ __device__ __forceinline__ bool tile_of(const SplitGemmArgs& a, int& m, int& n, 
 template <int R, int MB, int NB, bool I8>
 __device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Split8 (&xs)[MB], typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
   typedef SplitBlock<R> B;
-  // smallest products first; the three that are left out are below half an ulp of a product
+  // smallest products first; the three that are left out are at most 2^-24 of a product
 #define SPLIT_STEP(wp, xp)                                                                        \
   _Pragma("unroll") for (int i = 0; i < MB; ++i) _Pragma("unroll") for (int j = 0; j < NB; ++j) \
       acc[i][j] = B::mfma(ws[j].wp, xs[i].xp, acc[i][j])

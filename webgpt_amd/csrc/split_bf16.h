@@ -21,7 +21,8 @@ __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
 }
 
-// x = hi + mid + lo exactly (8 + 8 + 8 significand bits, each remainder rounded to nearest and representable), the
+// x = hi + mid + lo exactly for |x| >= 2^-110 (8 + 8 + 8 significand bits, each remainder rounded to nearest and
+// representable; below, lo falls under the smallest bf16 subnormal, 2^-133, and the sum is off by 2^-134 at most), the
 // decomposition of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for
 // higher-precision computations" (2019).
 __device__ __forceinline__ void split_pair(float a, float b, unsigned& hi, unsigned& mid, unsigned& lo) {
