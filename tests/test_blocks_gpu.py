@@ -212,32 +212,43 @@ def test_int8_matmul_large_activations(device, M, N, K, big):
 
 
 @pytest.mark.parametrize("int8", [False, True])
-@pytest.mark.parametrize("small", ["A", "row", "W"])
+@pytest.mark.parametrize("small", ["A", "row", "W", "column", "value"])
 @pytest.mark.parametrize("M,N,K", [(5, 8, 100), (17, 568, 1872), (33, 4200, 1048), (33, 2744, 2148), (100, 3240, 40), (300, 3400, 648), (449, 4552, 36)])
 def test_split_matmul_tiny_values(device, int8, M, N, K, small):
-    """Operands around 2**-119, whose third bf16 part is too small for bf16: the same relative error as at any other size. The
-    fp32 sums have a quantum of 2**-149."""
+    """Operands around 2**-119, whose third bf16 part is too small for bf16: the same relative error as at any other size, also
+    where a single row, column or output is that small. The fp32 sums have a quantum of 2**-149."""
     rng = np.random.default_rng(M + N + K)
     A = rng.standard_normal((M, K)).astype(np.float32)
     tiny = np.float32(2.0 ** -119)
     if small == "A" or (int8 and small == "W"):
         A *= tiny
-    elif small == "row":
+    elif small in ("row", "value"):
         A[M // 2] *= tiny
+        if small == "value":  # (the first column of W takes that row's only value that is not tiny)
+            A[M // 2, 0] = 1
     if int8:
         q = rng.integers(-128, 128, (K, N))
+        if small == "value":
+            q[0, 1:] = 1
+            q[0, 0] = 0
         scale = rng.uniform(100, 200, N).astype(np.float32)
         inst = FastMatMulBlock.newInt8Instance(M, N, K, init_tensor(A, [M, K]), init_tensor(pack_words(q), [K, N // 4]), init_tensor(scale, [N]),
                                                init_tensor(np.zeros(N, np.float32), [N]))
         W = q * (scale / np.float32(127.0)).astype(np.float64)
     else:
         w = rng.standard_normal((K, N)).astype(np.float32) * (tiny if small == "W" else np.float32(1))
+        if small == "column":
+            w[:, N // 3] *= tiny
+        elif small == "value":
+            w[0, 0] = 0
         inst = FastMatMulBlock.newInstance(M, N, K, init_tensor(A, [M, K]), init_tensor(w, [K, N]), init_tensor(np.zeros(N, np.float32), [N]))
         W = w.astype(np.float64)
     got = run(inst, (M, N)).astype(np.float64)
     want = A.astype(np.float64) @ W
     bound = 2.0 ** -24 * (K + 24) * (np.abs(A).astype(np.float64) @ np.abs(W)) + K * 2.0 ** -149
-    assert np.linalg.norm((got - want) / bound) <= 0.25 * math.sqrt(M * N), float(np.linalg.norm((got - want) / bound) / math.sqrt(M * N))
+    if small == "value":
+        got, want, bound = got[M // 2, :1], want[M // 2, :1], bound[M // 2, :1]
+    assert np.linalg.norm((got - want) / bound) <= 0.25 * math.sqrt(got.size), float(np.linalg.norm((got - want) / bound) / math.sqrt(got.size))
     assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
 
 
