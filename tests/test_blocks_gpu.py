@@ -521,6 +521,37 @@ def test_attention_split_infinite_values(device, T, H, hs):
     assert not np.isfinite(got[T - 2:]).any()  # (the projection behind it spreads an infinite output over its row)
 
 
+@pytest.mark.parametrize("small", ["all", "dimension"])
+@pytest.mark.parametrize("T,H,hs", [(193, 2, 20), (700, 2, 64), (331, 4, 96), (1023, 2, 128)])
+def test_attention_split_tiny_values(device, T, H, hs, small):
+    """Values around 2**-119, all of them or those of one dimension, whose third bf16 part is too small for bf16: the relative
+    error of test_attention_split_operands, and for each key a quantum of 2**-149."""
+    d = H * hs
+    rng = np.random.default_rng(T + d)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    eye, zero = np.eye(d, dtype=np.float32), np.zeros(d, np.float32)
+    wv = eye.copy()
+    if small == "all":
+        wv *= np.float32(2.0 ** -119)
+    else:
+        wv[hs + 3, hs + 3] = 2.0 ** -119
+    bufs = [init_tensor(x, [T, d])]
+    for w in (eye, eye, wv, eye):
+        bufs += [init_tensor(w, [d, d]), init_tensor(zero, [d])]
+    scale = 1 / math.sqrt(hs)
+    got = run(AttentionBlock.newFusedInstance(T, d, scale, H, hs, *bufs, FastMatMulBlock, SoftmaxBlock), (T, d)).astype(np.float64)
+    k = x.astype(np.float64).reshape(T, H, hs).transpose(1, 0, 2)
+    v = (x.astype(np.float64) * np.diag(wv)).reshape(T, H, hs).transpose(1, 0, 2)
+    s = k @ k.transpose(0, 2, 1) * np.float64(np.float32(scale))
+    s[:, np.triu(np.ones((T, T), bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = (p @ v).transpose(1, 0, 2).reshape(T, d)
+    size = (p @ np.abs(v)).transpose(1, 0, 2).reshape(T, d)
+    bound = (2.0 ** -20 * max(1.0, np.abs(s[np.isfinite(s)]).max() / 16) + 2.0 ** -21) * size + T * 2.0 ** -149
+    assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
+
+
 def test_attention_values_known_answer(device):
     # other/test.js:370-388 through the attention block: with Wq = Wk = 0 every score is 0, so the
     # softmax is uniform over j <= i: P = 1/(i+1). V = c // hs + 1 (via bv, Wv = 0), Wo = I:

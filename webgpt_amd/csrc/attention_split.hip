@@ -114,7 +114,8 @@ __device__ __forceinline__ f32x4 over_workgroup(f32x4 v, f32x4* sh) {
 }
 
 // The outputs of the queries q0 + (bits of `left`) with plain fp32 products, four at a time by the whole workgroup, over runs of
-// AS_RUN keys: for operands that have no split (infinite ones, see gemm_split.hip) and for NaN. Scores that are not numbers end
+// AS_RUN keys: for operands that have no split (infinite ones, see gemm_split.hip), for NaN, and for values so small that their
+// third part is lost (under 2^-110: outputs under 2^-100 are taken again). Scores that are not numbers end
 // it, as nothing else can come out. An attention block of 12 heads x 48 at 943 rows takes 325 us where every output is taken
 // again (128 us where none is; 21.6 ms with a loop over the keys per output).
 constexpr int AS_RUN = 1024;
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
   constexpr bool QREG = DB == 1;
   static_assert(4 * AS_RUN + 4 * NWV * 64 + 4 * NWV + 4 * 128 <= NWV * WAVE_FLOATS, "plain_rows' memory");
   extern __shared__ __attribute__((aligned(16))) float as_lds[];
-  __shared__ unsigned again;  // queries whose output is not finite
+  __shared__ unsigned again;  // queries with an output that the split may have spoilt
   // consecutive blocks go to one XCD, whose L2 then holds the K and V of few heads; the longest rows of keys first
   const int total = a.H * a.nq, per = (total + 7) >> 3, item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || item >= total) return;
@@ -373,8 +374,11 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
       den += as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + ASQ + qi] * f;
     }
     const float v = num / den;
-    if (fabsf(v) < INFINITY) a.out[(size_t)(q0 + qi) * a.ldo + (size_t)h * a.hs + dim] = v;
-    else atomicOr(&again, 1u << qi);
+    a.out[(size_t)(q0 + qi) * a.ldo + (size_t)h * a.hs + dim] = v;
+    // twice the bits, so without the sign: under 2^-100 and no zero, or not finite
+    constexpr unsigned LO = (127 - 100) << 24, HI = 0xff000000u;
+    const unsigned v2 = __float_as_uint(v) << 1;
+    if (v2 - LO >= HI - LO && v2 != 0u) atomicOr(&again, 1u << qi);
   }
   __syncthreads();
   const unsigned left = __builtin_amdgcn_readfirstlane(again);
