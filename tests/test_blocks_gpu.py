@@ -416,7 +416,7 @@ def test_attention(device, T, H, hs):
     assert close(got, want), worst(got, want)
 
 
-@pytest.mark.parametrize("T,H,hs", [(192, 2, 4), (193, 2, 20), (320, 5, 32), (257, 2, 36), (700, 2, 64), (225, 2, 68), (331, 4, 96),
+@pytest.mark.parametrize("T,H,hs", [(192, 2, 4), (192, 12, 4), (191, 14, 8), (1152, 2, 16), (193, 2, 20), (320, 5, 32), (257, 2, 36), (700, 2, 64), (225, 2, 68), (331, 4, 96),
                                     (256, 2, 100), (1023, 2, 128)])
 def test_attention_split_operands(device, T, H, hs):
     """Prompts long enough for the split operands: the edges of a block of 32 queries, keys or dimensions. With the identity as

@@ -1741,13 +1741,15 @@ hipError_t launch_vocab_gemv(int V, int d, const float* x, const float* wte, flo
   return hipGetLastError();
 }
 
-// Where the split operands pay for the pass that makes them (two launches; MI355X, us of a call, this kernel against the ones
-// below): head size 64 has a matrix kernel of its own, 12 heads x 512 rows 18.5 against 17.8, x 943 33.8 against 37.6, 25 x 943
-// 57.7 against 60.1; the other sizes have a workgroup per query, which reads all keys: 12 x 48 at 128 rows 10.6 against
-// 9.1, at 200 11.9 against 17.0, at 943 32.3 against 128; 8 x 128 at 200 rows 19.6 against 20.8, 2 x 128 18.0 against 16.8
-// and at 300 21.2 against 22.1.
+// Where the split operands pay for the pass that makes them (two launches; MI355X, us saved per call against the kernels
+// below). Head size 64 has a matrix kernel of its own: from 700 rows 4 to 8 us at 2 to 25 heads, at 600 rows 4 at 2 heads but
+// -0.3 at 25. The other sizes have a workgroup per query, which reads all keys: 12 heads x 48 at 128 rows -2.5, at 192 4.1, at
+// 943 98; 12 x 32 at 192 3.4, 2 x 32 -0.4; above 96 the operands of a wave take half the registers: 1 x 128 at 192 rows -2.3,
+// at 256 0.1, at 320 0.8, 8 x 128 -2.8, 3.1, 9.5. Sizes up to 16 are padded to 32 dimensions and need several heads for their
+// work to be more than the launches: 12 x 8 at 192 rows 1.8, 2 x 8 -0.7, at 1024 -2.0, at 2048 4.4.
 static bool attention_splits(int Tq, int pos0, int H, int hs) {
   if (hs > 128 || (hs & 3) || H > 65535 || pos0 + Tq > 12288) return false;
+  if (hs <= 16 && (size_t)H * Tq < 12 * 192) return false;
   return Tq >= (hs == AHS ? 700 : hs > 96 ? 256 : 192);
 }
 
