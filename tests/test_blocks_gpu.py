@@ -284,6 +284,36 @@ def test_split_matmul_not_finite_in_time(device, int8, M, N, K):
     assert ms[1] < 5 * ms[0], ms
 
 
+@pytest.mark.parametrize("M,N,K,int8", [(5, 2 ** 20 + 8, 516, False), (17, 2 ** 22 + 32, 516, True), (530000, 8, 1024, False), (5, 2 ** 27 + 8, 4, False)])
+def test_matmul_beyond_two_gib(device, M, N, K, int8):
+    """Operands beyond the reach of 32-bit offsets: W in runs of rows (fp32 and int8), A in runs of rows, and rows of W of which
+    not even four are in reach. Small integers, repeated with a prime period: every sum is exact."""
+    rng = np.random.default_rng(N)
+    A = np.tile(rng.integers(-3, 4, (min(M, 4099), K)).astype(np.float32), ((M + 4098) // 4099, 1))[:M]
+    base = rng.integers(-3, 4, (K, min(N, 4099))).astype(np.int8 if int8 else np.float32)
+    W = np.tile(base, (1, (N + 4098) // 4099))[:, :N]
+    bias = np.tile(rng.integers(-3, 4, base.shape[1]).astype(np.float32), (N + 4098) // 4099)[:N]
+    if int8:
+        W = np.ascontiguousarray(W).view(np.int32)
+    bufs = [init_tensor(A, [M, K]), init_tensor(W, W.shape), init_tensor(bias, [N])]
+    try:
+        if int8:
+            bufs.append(init_tensor(np.full(N, 127, np.float32), [N]))
+            inst = FastMatMulBlock.newInt8Instance(M, N, K, bufs[0], bufs[1], bufs[3], bufs[2])
+        else:
+            inst = FastMatMulBlock.newInstance(M, N, K, *bufs)
+        got = run(inst, (M, N))
+    finally:
+        for b in bufs:
+            b.destroy()
+        FastMatMulBlock.destroyBuffers()  # (up to 2.7 GB of result)
+    want = A[:4099] @ base.astype(np.float32) + bias[:base.shape[1]]
+    for m in range(0, M, len(want)):
+        for n in range(0, N, want.shape[1]):
+            part = got[m:m + len(want), n:n + want.shape[1]]
+            assert np.array_equal(part, want[:part.shape[0], :part.shape[1]]), (m, n)
+
+
 def test_fast_matmul_exact_and_preconditions(device):
     A = RNG.integers(-8, 9, (3, 12)).astype(np.float32)
     W = RNG.integers(-8, 9, (12, 16)).astype(np.float32)

@@ -1641,17 +1641,22 @@ void finish_split(int M, int N, int S, const float* workspace, const float* bias
   if (ln) layernorm_kernel<<<M, WG, 0, s>>>(N, C, ldc, ln->gamma, ln->beta, ln->out, ln->ldo);
 }
 
+constexpr size_t GEMM_BYTES = ((size_t)1 << 31) - 4096;  // of A or W that a launch reaches: its offsets have 32 bits and a sign
+// Rows of W that a launch takes (a multiple of four, or all K), ldw words of four bytes apart; 0: not even four
+int gemm_rows_of_w(int K, int ldw) {
+  return (int)std::min<size_t>((size_t)K, std::min(GEMM_BYTES / (sizeof(float) * (size_t)ldw), GEMM_BYTES / sizeof(float)) / 4 * 4);
+}
+
 // C = epi(A . W + bias) on the matrix cores; W fp32 [K, ldw], or words of four int8 with a scale per column
-// (blocked: in the order of launch_block_weights).
+// (blocked: in the order of launch_block_weights). K from gemm_rows_of_w.
 hipError_t run_gemm(int M, int N, int K, const float* A, int lda, const void* W, int ldw, const float* wscale, const float* bias,
                     float* C, int ldc, int epi, const float* resid, float* workspace, const LnAfter* ln, const KvAfter* kv, bool blocked, hipStream_t s) {
   const bool i8 = wscale != nullptr;
   SplitGemmArgs a{};
   a.N = N; a.K = K; a.lda = lda; a.W = W; a.ldw = ldw; a.blocked = blocked; a.wscale = wscale; a.bias = bias; a.epi = epi; a.ldc = ldc;
   if (kv) { a.Kc = kv->Kc; a.Vc = kv->Vc; a.d = kv->d; a.hs = kv->hs; a.ctx = kv->ctx; }
-  // the kernels address A with 32-bit offsets: very tall matrices go in runs of rows
-  const int rows = (int)std::min<size_t>((size_t)M, (((size_t)1 << 31) - 4096) / (sizeof(float) * (size_t)lda));
-  if (rows < 1) return hipErrorInvalidValue;
+  // the kernels address A with 32-bit offsets: very tall matrices go in runs of rows, of which the last has K columns
+  const int rows = (int)std::min<size_t>((size_t)M, 1 + (GEMM_BYTES - sizeof(float) * (size_t)K) / (sizeof(float) * (size_t)lda));
   for (int m0 = 0; m0 < M; m0 += rows) {
     const int m = std::min(rows, M - m0);
     const SplitPlan p = plan_gemm_split(m, N, K, i8, blocked, ln != nullptr, workspace != nullptr);
@@ -1672,15 +1677,31 @@ hipError_t run_gemm(int M, int N, int K, const float* A, int lda, const void* W,
   }
   return hipGetLastError();
 }
+
+// Rows of W so long that not even four are in reach (134 M columns, four times as many of int8): the matrix-vector kernels, a
+// few rows of A at a time, in the workspace of the product.
+template <typename F>
+hipError_t gemv_by_rows(int M, int N, int K, const float* workspace, F launch) {
+  const int most = std::min(M, GEMV_MAX_ROWS);
+  if (!workspace || gemv_workspace_floats(most, N, K) > gemm_workspace_floats(M, N)) return hipErrorInvalidValue;
+  for (int m0 = 0; m0 < M; m0 += most) {
+    const hipError_t e = launch(m0, std::min(most, M - m0));
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 }  // namespace
 
 hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float* W, int ldw, const float* bias,
                        float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s, const LnAfter* ln,
                        const KvAfter* kv, bool blocked) {
-  // the kernels address W with 32-bit offsets: a larger matrix goes in runs of rows whose products are added up
-  const int rows = (int)std::min<size_t>((size_t)K, (((size_t)1 << 31) - 4096) / (sizeof(float) * (size_t)ldw) / 4 * 4);
+  // a larger W goes in runs of rows whose products are added up
+  const int rows = gemm_rows_of_w(K, ldw);
   if (rows >= K) return run_gemm(M, N, K, A, lda, W, ldw, nullptr, bias, C, ldc, epi, resid, workspace, ln, kv, blocked, s);
-  if (blocked || rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  if (blocked || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  if (rows == 0) return gemv_by_rows(M, N, K, workspace, [&](int m0, int m) {
+    return launch_gemv_kn(m, N, K, A + (size_t)m0 * lda, lda, W, ldw, bias, C + (size_t)m0 * ldc, ldc, EPI_NONE, nullptr, workspace, s);
+  });
   for (int k0 = 0; k0 < K; k0 += rows) {
     const hipError_t e = run_gemm(M, N, std::min(rows, K - k0), A + k0, lda, W + (size_t)k0 * ldw, ldw, nullptr,
                                   k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, false, s);
@@ -1692,9 +1713,12 @@ hipError_t launch_gemm(int M, int N, int K, const float* A, int lda, const float
 hipError_t launch_gemm_i8(int M, int N, int K, const float* A, int lda, const int32_t* Wq, int ldwq, const float* scale,
                           const float* bias, float* C, int ldc, int epi, const float* resid, float* workspace, hipStream_t s,
                           const LnAfter* ln, const KvAfter* kv, bool blocked) {
-  const int rows = (int)std::min<size_t>((size_t)K, (((size_t)1 << 31) - 4096) / (sizeof(int32_t) * (size_t)ldwq) / 4 * 4);
+  const int rows = gemm_rows_of_w(K, ldwq);
   if (rows >= K) return run_gemm(M, N, K, A, lda, Wq, ldwq, scale, bias, C, ldc, epi, resid, workspace, ln, kv, blocked, s);
-  if (blocked || rows < 4 || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  if (blocked || epi != EPI_NONE || ln || kv) return hipErrorInvalidValue;
+  if (rows == 0) return gemv_by_rows(M, N, K, workspace, [&](int m0, int m) {
+    return launch_gemv_kn_i8(m, N, K, A + (size_t)m0 * lda, lda, Wq, ldwq, scale, bias, C + (size_t)m0 * ldc, ldc, EPI_NONE, nullptr, workspace, s);
+  });
   for (int k0 = 0; k0 < K; k0 += rows) {
     const hipError_t e = run_gemm(M, N, std::min(rows, K - k0), A + k0, lda, Wq + (size_t)k0 * ldwq, ldwq, scale,
                                   k0 + rows >= K ? bias : nullptr, C, ldc, k0 ? EPI_RESIDUAL : EPI_NONE, k0 ? C : nullptr, workspace, nullptr, nullptr, false, s);
