@@ -252,6 +252,21 @@ def test_split_matmul_tiny_values(device, int8, M, N, K, small):
     assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 8, 100), (17, 568, 1872), (33, 4200, 1048), (33, 2744, 2148), (100, 3240, 40), (300, 3400, 648), (449, 4552, 36)])
+@pytest.mark.parametrize("small", ["A", "W"])
+def test_split_matmul_tiny_times_large(device, small, M, N, K):
+    """One operand around 2**-119, the other around 2**30: the outputs are not tiny themselves. Independent roundings of K
+    additions, each 2**-25 of a partial sum in the mean square and none larger than the outputs: sqrt(K) 2**-25 in norm, of
+    which four times is allowed (2**-15.7 with the third parts lost)."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.standard_normal((M, K)).astype(np.float32) * np.float32(2.0 ** (-119 if small == "A" else 30))
+    w = rng.standard_normal((K, N)).astype(np.float32) * np.float32(2.0 ** (30 if small == "A" else -119))
+    inst = FastMatMulBlock.newInstance(M, N, K, init_tensor(A, [M, K]), init_tensor(w, [K, N]), init_tensor(np.zeros(N, np.float32), [N]))
+    got = run(inst, (M, N)).astype(np.float64)
+    want = A.astype(np.float64) @ w.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 4 * math.sqrt(K) * 2.0 ** -25 * np.linalg.norm(want), float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
 def _launch_ms(inst, launches=40):
     """Milliseconds of a launch, the best of three runs of them (the copy of the result that ends a run is in it)."""
     best = math.inf

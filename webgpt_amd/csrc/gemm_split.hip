@@ -231,8 +231,10 @@ __device__ __forceinline__ void split_products(const Split8 (&ws)[NB], const Spl
 
 // Are there sums in the wave's tile that the split may have spoilt? Those that are not finite; unscaled int8 ones of 2^124 and
 // more, so that the eight of a workgroup have a finite sum; and tiny ones: a value under 2^-110 loses what its third part
-// would hold under the smallest bf16 subnormal, 2^-134 at most, which shows in sums under 2^-100. (One instruction per two
-// registers for the largest and one for the smallest; the largest lets NaN through. Zeros are no tiny sums.)
+// would hold under the smallest bf16 subnormal, 2^-134 at most, which shows in sums under SPLIT_TINY unless the other operand
+// has values of about 2^50 and more. (One instruction per two registers for the largest and one for the smallest; the largest
+// lets NaN through. Zeros are no tiny sums.)
+constexpr float SPLIT_TINY = 0x1p-60f;
 template <int R, int MB, int NB, bool I8>
 __device__ __forceinline__ bool spoilt(const typename SplitBlock<R>::acc_t (&acc)[MB][NB]) {
   float most = 0.f, least = INFINITY;
@@ -246,7 +248,7 @@ __device__ __forceinline__ bool spoilt(const typename SplitBlock<R>::acc_t (&acc
         least = __builtin_elementwise_minimum(least, fabsf(acc[i][j][e]));
       }
   bool bad = !(most < (I8 ? 0x1p124f : INFINITY));
-  if (least < 0x1p-100f) {
+  if (least < SPLIT_TINY) {
     unsigned tiny = ~0u;  // (twice the bits, less one: the sign is gone and a zero is the largest)
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -254,7 +256,7 @@ __device__ __forceinline__ bool spoilt(const typename SplitBlock<R>::acc_t (&acc
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int e = 0; e < SplitBlock<R>::NACC; ++e) tiny = min(tiny, (__float_as_uint(acc[i][j][e]) << 1) - 1u);
-    bad = bad || tiny < (__float_as_uint(0x1p-100f) << 1) - 1u;
+    bad = bad || tiny < (__float_as_uint(SPLIT_TINY) << 1) - 1u;
   }
   return __builtin_amdgcn_ballot_w64(bad) != 0;
 }
