@@ -146,7 +146,8 @@ int wgpt_model_create(const wgpt_params* params, wgpt_model* out);
  * given as `<stem>.weight.q` (int32 words [K, N/4]) and `<stem>.weight.scale` (fp32 [N]).
  * The Q/K/V split of c_attn (model.js:456-482) happens inside. data is copied. */
 int wgpt_model_set_tensor(wgpt_model m, const char* name, const void* data, size_t bytes);
-/* Checks that every tensor arrived and prepares the device-side layouts. */
+/* Checks that every tensor arrived and prepares the device-side layouts. A call that fails may be made again (with the
+ * missing tensors, or more memory), unless it had begun to re-order the weights: then WGPT_ERR_STATE, load the model again. */
 int wgpt_model_finalize(wgpt_model m);
 /* run(idx) for a whole window (model.js:104): resets the KV cache, processes T tokens
  * at positions 0..T-1, writes logits[V] of the last one. logits may be NULL. */

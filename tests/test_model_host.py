@@ -1,0 +1,76 @@
+"""Host code of the model entry points on tests/host_hip.cc, which stands in for the HIP runtime: kernels do not run, so only
+error paths and the order of calls are looked at. A process of its own per test: the stand-in has to be loaded first."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, sys
+hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+launches, fail_at, unwaited = (C.c_int.in_dll(hip, "host_hip_" + n) for n in ("launches", "fail_at", "unwaited"))
+import numpy as np
+from webgpt_amd import WgptError, _lib, synth
+from helpers import make_model, small_cfg
+_lib.init(0)
+cfg = small_cfg(dtype=sys.argv[2])
+tensors = make_model(cfg, 1)
+
+def refused(name, *args):
+    try:
+        _lib.call(name, *args)
+    except WgptError as e:
+        return str(e) or "refused"
+    return None
+
+def model():
+    m = C.c_uint64(0)
+    _lib.call("wgpt_model_create", C.byref(_lib.Params(**synth.model_params(cfg), weight_dtype=int(sys.argv[2] == "int8"))), C.byref(m))
+    for n, t in tensors.items():
+        _lib.call("wgpt_model_set_tensor", m, n.encode(), np.ascontiguousarray(t).ctypes.data, t.nbytes)
+    return m
+"""
+
+
+@pytest.fixture(scope="module")
+def host_hip(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host_hip") / "host_hip.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-Wno-deprecated-declarations",
+                    os.path.join(HERE, "host_hip.cc"), "-o", out], check=True)
+    return out
+
+
+def run(host_hip, dtype, body):
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.dirname(HERE), HERE]))
+    p = subprocess.run([sys.executable, "-c", PRELUDE + body, host_hip, dtype], env=env, capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout + p.stderr
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_finalize_after_a_failed_launch(host_hip, dtype):
+    """Whichever launch of wgpt_model_finalize fails: the call fails, and a later one either has everything left as it needs it
+    or is refused. After the first matrix was put into the order of the prefill products (the last 4 n_layer launches) the
+    decode layouts can no longer be built from it."""
+    run(host_hip, dtype, """
+m = model()
+at = launches.value
+_lib.call("wgpt_model_finalize", m)
+total, moves = launches.value - at, 4 * cfg["n_layer"]
+assert total > moves
+for i in range(1, total + 1):
+    m = model()
+    fail_at.value = launches.value + i
+    assert refused("wgpt_model_finalize", m)
+    fail_at.value = 0
+    assert refused("wgpt_prefill", m, np.zeros(2, np.int32).ctypes.data_as(C.POINTER(C.c_int32)), 2, None)
+    again = refused("wgpt_model_finalize", m)
+    assert (again is not None) == (i > total - moves), (i, total, again)
+    t = tensors["transformer.wpe.weight"]
+    if again:
+        assert "load the model again" in again
+        assert refused("wgpt_model_set_tensor", m, b"transformer.wpe.weight", t.ctypes.data, t.nbytes)
+    _lib.call("wgpt_model_destroy", m)
+""")

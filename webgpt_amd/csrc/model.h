@@ -30,6 +30,7 @@ struct Model {
   wgpt_params p{};
   int L = 0, H = 0, d = 0, hs = 0, ctx = 0, V = 0, maxT = 0;
   bool finalized = false;
+  bool weights_moved = false;  // finalising has begun to re-order the linear weights: the decode layouts cannot be built from them again
   int decode_mode = 0;
   int pos = 0;     // positions held by the KV cache
   int tap_T = 0;   // rows of the recorded taps (0 = none)

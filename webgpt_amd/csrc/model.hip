@@ -642,6 +642,7 @@ int wgpt_model_set_tensor(wgpt_model h, const char* name, const void* data, size
   Model* m = find_model(h);
   if (!m) return WGPT_ERR_ARG;
   if (m->finalized) return fail(WGPT_ERR_STATE, "wgpt_model_set_tensor: model already finalised");
+  if (m->weights_moved) return fail(WGPT_ERR_STATE, "wgpt_model_set_tensor: wgpt_model_finalize failed half-way; load the model again");
   if (!name || !data) return fail(WGPT_ERR_ARG, "wgpt_model_set_tensor: NULL argument");
   Slot slot;
   if (!parse_name(m, name, &slot)) return fail(WGPT_ERR_ARG, "wgpt_model_set_tensor: unknown tensor name '%s'", name);
@@ -660,6 +661,7 @@ int wgpt_model_finalize(wgpt_model h) {
   Model* m = find_model(h);
   if (!m) return WGPT_ERR_ARG;
   if (m->finalized) return WGPT_OK;
+  if (m->weights_moved) return fail(WGPT_ERR_STATE, "wgpt_model_finalize: an earlier call failed half-way; load the model again");
   const bool i8 = m->p.weight_dtype == 1;
   if (!m->wte || !m->wpe || !m->lnf_g || !m->lnf_b) return fail(WGPT_ERR_STATE, "wgpt_model_finalize: embeddings or final layer norm missing");
   for (int i = 0; i < m->L; ++i) {
@@ -713,6 +715,7 @@ int wgpt_model_finalize(wgpt_model h) {
   WGPT_HIP(hipEventCreate(&m->ev1));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   if ((rc = setup_persistent(m))) return rc;
+  m->weights_moved = true;
   if ((rc = block_linear_weights(m, block_buf))) return rc;
   m->decode_mode = m->persist_ok ? 1 : 0;
   m->pos = 0;
