@@ -74,3 +74,12 @@ for i in range(1, total + 1):
         assert refused("wgpt_model_set_tensor", m, b"transformer.wpe.weight", t.ctypes.data, t.nbytes)
     _lib.call("wgpt_model_destroy", m)
 """)
+
+
+def test_finalize_waits_for_its_launches(host_hip):
+    """An error of the re-ordering belongs to wgpt_model_finalize, not to the first prefill: it returns with nothing in flight."""
+    run(host_hip, "f32", """
+m = model()
+_lib.call("wgpt_model_finalize", m)
+assert unwaited.value == 0, unwaited.value
+""")

@@ -717,6 +717,7 @@ int wgpt_model_finalize(wgpt_model h) {
   if ((rc = setup_persistent(m))) return rc;
   m->weights_moved = true;
   if ((rc = block_linear_weights(m, block_buf))) return rc;
+  WGPT_HIP(hipStreamSynchronize(rt().stream));  // (its errors are this call's)
   m->decode_mode = m->persist_ok ? 1 : 0;
   m->pos = 0;
   m->finalized = true;
