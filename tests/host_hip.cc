@@ -1,5 +1,5 @@
 // The HIP calls that libwebgpt_amd.so makes, on host memory: allocations and copies are the host's, a kernel launch does
-// nothing but count, and launch `host_hip_fail_at` (from 1; 0: none) fails instead. Loaded in front of the library
+// nothing but count, and launch `host_hip_fail_at` (from 1; 0: none) or allocation `host_hip_alloc_fail_at` fails instead. Loaded in front of the library
 // (RTLD_GLOBAL) it takes the place of the HIP runtime in that process, so that the library's host code can be tested
 // without a GPU, its error paths among them.
 #include <cstdlib>
@@ -9,6 +9,7 @@
 
 extern "C" {
 int host_hip_launches = 0, host_hip_fail_at = 0;
+int host_hip_allocs = 0, host_hip_alloc_fail_at = 0;
 int host_hip_unwaited = 0;  // launches since the last wait for the stream
 
 static dim3 cfg_grid, cfg_block;
@@ -48,9 +49,13 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
 }
 hipError_t hipGetSymbolAddress(void** p, const void*) { return *p = symbol, hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
-hipError_t hipMalloc(void** p, size_t n) { return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+static hipError_t allocate(void** p, size_t n) {
+  if (++host_hip_allocs == host_hip_alloc_fail_at) return hipErrorOutOfMemory;
+  return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipMalloc(void** p, size_t n) { return allocate(p, n); }
 hipError_t hipFree(void* p) { return free(p), hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return allocate(p, n); }
 hipError_t hipHostFree(void* p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
@@ -60,5 +65,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = rein
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return host_hip_unwaited = 0, hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(symbol), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 }

@@ -12,6 +12,7 @@ PRELUDE = """
 import ctypes as C, sys
 hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 launches, fail_at, unwaited = (C.c_int.in_dll(hip, "host_hip_" + n) for n in ("launches", "fail_at", "unwaited"))
+allocs, alloc_fail_at = (C.c_int.in_dll(hip, "host_hip_" + n) for n in ("allocs", "alloc_fail_at"))
 import numpy as np
 from webgpt_amd import WgptError, _lib, synth
 from helpers import make_model, small_cfg
@@ -82,4 +83,24 @@ def test_finalize_waits_for_its_launches(host_hip):
 m = model()
 _lib.call("wgpt_model_finalize", m)
 assert unwaited.value == 0, unwaited.value
+""")
+
+
+def test_finalize_after_a_failed_allocation(host_hip):
+    """Whichever allocation of wgpt_model_finalize fails, a second call succeeds and the model runs."""
+    run(host_hip, "f32", """
+m = model()
+at = allocs.value
+_lib.call("wgpt_model_finalize", m)
+total = allocs.value - at
+tokens, logits = np.zeros(2, np.int32), np.zeros(cfg["vocab_size"], np.float32)
+for i in range(1, total + 1):
+    m = model()
+    alloc_fail_at.value = allocs.value + i
+    assert refused("wgpt_model_finalize", m)
+    alloc_fail_at.value = 0
+    _lib.call("wgpt_model_finalize", m)
+    _lib.call("wgpt_prefill", m, tokens.ctypes.data_as(C.POINTER(C.c_int32)), 2, logits.ctypes.data_as(C.POINTER(C.c_float)))
+    _lib.call("wgpt_decode_sample", m, 1, 2, 12, 1.0, np.zeros(2).ctypes.data_as(C.POINTER(C.c_double)), tokens.ctypes.data_as(C.POINTER(C.c_int32)), None)
+    _lib.call("wgpt_model_destroy", m)
 """)

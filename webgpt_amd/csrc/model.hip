@@ -702,17 +702,18 @@ int wgpt_model_finalize(wgpt_model h) {
   }
   // the attention's workspace is in use while no product's partial sums are
   if (att_ws && att_ws <= part_bytes) m->att_ws = m->part;
+  // (each unless an earlier call, which failed behind it, has it already)
   if (!m->pin) {
     WGPT_HIP(hipHostMalloc((void**)&m->pin, 4 * sizeof(int32_t), hipHostMallocDefault));
     m->pin[0] = m->pin[1] = m->pin[2] = m->pin[3] = 0;
-    WGPT_HIP(hipHostMalloc((void**)&m->logits_pin, sizeof(float) * ((size_t)m->V + 1), hipHostMallocDefault));
-    WGPT_HIP(hipHostMalloc((void**)&m->u_pin, (sizeof(double) + sizeof(int32_t)) * (size_t)m->ctx, hipHostMallocDefault));
-    m->ids_pin = reinterpret_cast<int32_t*>(m->u_pin + m->ctx);
   }
+  if (!m->logits_pin) WGPT_HIP(hipHostMalloc((void**)&m->logits_pin, sizeof(float) * ((size_t)m->V + 1), hipHostMallocDefault));
+  if (!m->u_pin) WGPT_HIP(hipHostMalloc((void**)&m->u_pin, (sizeof(double) + sizeof(int32_t)) * (size_t)m->ctx, hipHostMallocDefault));
+  m->ids_pin = reinterpret_cast<int32_t*>(m->u_pin + m->ctx);
   WGPT_HIP(hipMemsetAsync(m->pos_dev, 0, sizeof(int), rt().stream));
   WGPT_HIP(hipMemsetAsync(m->kv, 0, (size_t)m->L * 2 * m->ctx * d * f, rt().stream));
-  WGPT_HIP(hipEventCreate(&m->ev0));
-  WGPT_HIP(hipEventCreate(&m->ev1));
+  if (!m->ev0) WGPT_HIP(hipEventCreate(&m->ev0));
+  if (!m->ev1) WGPT_HIP(hipEventCreate(&m->ev1));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   if ((rc = setup_persistent(m))) return rc;
   m->weights_moved = true;
