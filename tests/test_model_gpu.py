@@ -70,6 +70,81 @@ def test_short_prompt_prefill_against_oracle(device, name, n_layer, T):
     gpt.unloadBuffers()
 
 
+# Widths that are no multiple of 32 (a partial step of every product but the second MLP matrix's), and lengths that take each
+# tile shape of the prefill products, with and without slices of K, as far as the launch times let a model of that dtype have it.
+BLOCKED_SHAPES = [(200, 5, 5), (200, 5, 37), (200, 5, 129), (200, 5, 300), (200, 5, 943), (1000, 25, 5), (1000, 25, 17), (1000, 25, 37), (1000, 25, 100),
+                  (1000, 25, 129), (1000, 25, 300), (1000, 25, 513), (1240, 31, 37), (1240, 31, 200), (1240, 31, 943), (2056, 257, 37), (2056, 257, 513)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head,T", BLOCKED_SHAPES)
+def test_prefill_products_of_other_widths(device, dtype, d, n_head, T):
+    """The products on weights in the order that a model keeps them (rows of W are what the block tests have). Two layers: the
+    cache rows of the second hold every row of all products of the first."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=max(T, 16), vocab_size=40, dtype=dtype)
+    gpt, tensors = load(cfg, seed=d + T)
+    tokens = synth.tokens(3, "prompt", T, cfg["vocab_size"])
+    want, _, want_kv = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens, want_taps=True, want_kv=True)
+    got = gpt.prefill(tokens)
+    for i in range(2):
+        assert close(gpt.tap(f"kv{i}_k"), want_kv[i, 0]), (i, worst(gpt.tap(f"kv{i}_k"), want_kv[i, 0]))
+        assert close(gpt.tap(f"kv{i}_v"), want_kv[i, 1]), (i, worst(gpt.tap(f"kv{i}_v"), want_kv[i, 1]))
+    assert close(got, want), worst(got, want)
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head,T", [(200, 5, 37), (1000, 25, 37), (1000, 25, 129), (1000, 25, 300), (1240, 31, 300), (1240, 31, 943), (2056, 257, 513)])
+def test_prefill_of_an_infinite_embedding(device, dtype, d, n_head, T):
+    """An infinite value in one position's embedding: that position and what attends to it is NaN, every other row as the oracle
+    has it, although the tiles around are taken again with fp32 products."""
+    at = T // 2
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=T, vocab_size=40, dtype=dtype)
+    tensors = make_model(cfg, d + T)
+    tokens = synth.tokens(3, "prompt", T, cfg["vocab_size"])
+    _, _, want = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens, want_taps=True, want_kv=True)
+    tensors["transformer.wpe.weight"] = tensors["transformer.wpe.weight"].copy()
+    tensors["transformer.wpe.weight"][at, d // 3] = np.inf
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg))
+    gpt.initialize()
+    logits = gpt.prefill(tokens)
+    assert np.isnan(logits).all()
+    for i in range(2):
+        for j, name in enumerate("kv"):
+            got, exp = gpt.tap(f"kv{i}_{name}"), want[i, j]
+            lost = np.arange(T) == at if i == 0 else np.arange(T) >= at
+            assert np.isnan(got[lost]).all()
+            assert close(got[~lost], exp[~lost]), (i, name, worst(got[~lost], exp[~lost]))
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("d,n_head,T", [(200, 5, 37), (1000, 25, 37), (1000, 25, 129), (1000, 25, 300), (1240, 31, 943), (2056, 257, 513)])
+def test_prefill_of_an_infinite_weight(device, d, n_head, T):
+    """An infinite weight in one of the last eight rows of the first MLP matrix, the one whose input has both signs most evenly:
+    GELU gives zero where it makes -inf and inf otherwise, so some rows are lost and the others as the oracle has them."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=T, vocab_size=40)
+    tensors = make_model(cfg, d + T)
+    tokens = synth.tokens(3, "prompt", T, cfg["vocab_size"])
+    _, taps, _ = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens, want_taps=True, want_kv=True)
+    positive = (taps[ref.tap_names(2).index("block0_ln2")][:, d - 8:] > 0).mean(0)
+    name = "transformer.h.0.mlp.c_fc.weight"
+    tensors[name] = tensors[name].copy()
+    tensors[name].reshape(d, 4 * d)[d - 8 + np.argmin(abs(positive - 0.5)), 2 * d + 5] = np.inf
+    with np.errstate(all="ignore"):
+        _, _, want = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens, want_taps=True, want_kv=True)
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg))
+    gpt.initialize()
+    gpt.prefill(tokens)
+    for i in range(2):
+        for j, name in enumerate("kv"):
+            got, exp = gpt.tap(f"kv{i}_{name}"), want[i, j]
+            lost = ~np.isfinite(exp)
+            assert np.array_equal(~np.isfinite(got), lost)
+            assert 0 < lost.any(1).sum() < T if i else not lost.any()
+            assert close(got[~lost], exp[~lost]), (i, name, worst(got[~lost], exp[~lost]))
+    gpt.unloadBuffers()
+
+
 def test_decode_equals_last_row_of_full_forward(device):
     # decode(t) with the KV cache must equal the reference's full-window recompute of tokens [0..t]
     cfg = dict(synth.CONFIGS["toy"])
