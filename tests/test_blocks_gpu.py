@@ -89,8 +89,9 @@ def test_fast_matmul_around_kernel_choices(device, M, N, K):
                                    (65, 72, 100), (128, 2304, 768), (128, 3080, 772), (129, 136, 4096), (500, 1032, 96),
                                    (943, 768, 768), (1000, 3072, 1060)])
 def test_split_matmul_error_bound(device, int8, M, N, K):
-    """The products on the bf16 matrix cores against 64-bit ones: the edges of every tile (16, 32, 64 and 128 rows), partial
-    steps of 32 k and sliced K. The parts of a value add up to it exactly and all six products kept are exact, so the error
+    """The products on the bf16 matrix cores against 64-bit ones: the edges of every tile that rows of W have (16, 32, 64
+    and 128 rows; the 64x128 one is for a model's order of the weights), partial steps of 32 k and sliced K. The parts of a
+    value of 2**-110 and more add up to it exactly and all six products kept are exact, so the error
     is that of the fp32 sums: at most six roundings per sixteen k, a few for the slices and waves, each at most 2**-24 of
     the sum of magnitudes, and 2**-24 of it for the products left out (a value's second and third parts are at most 2**-8
     and 2**-17 of it, and two such products are left out)."""

@@ -214,7 +214,7 @@ def test_int8_model(device):
     gpt, tensors = load(cfg, seed=13)
     w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
     tokens = synth.tokens(3, "prompt", 12, cfg["vocab_size"])
-    for T in (3, 9):      # GEMV path (<= 4 rows) and the dequantise + GEMM path
+    for T in (3, 9):
         got = gpt.prefill(tokens[:T])
         want = ref.forward(p, w, tokens[:T])
         assert close(got, want), worst(got, want)

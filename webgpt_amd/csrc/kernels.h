@@ -10,7 +10,7 @@ namespace wgpt {
 
 enum Epilogue { EPI_NONE = 0, EPI_GELU = 1, EPI_RESIDUAL = 2 };
 
-// Rows handled per pass of the GEMV path; a matmul with M <= this is a GEMV.
+// Rows of A that the matrix-vector kernels take; a block's matmul with M <= this runs on them (a model's prefill never does).
 constexpr int GEMV_MAX_ROWS = 4;
 constexpr int GEMV_KCHUNK = 64;
 
@@ -35,7 +35,7 @@ struct LnAfter {
   int ldo;
 };
 // For a product that yields a [M, 3d] q/k/v matrix: the key and value columns of row i also go to row pos0 + i of
-// the head-major cache (launch_kv_append's layout), by the pass that finishes C where there is one.
+// the cache [H][ctx][hs], by the pass that finishes C where there is one.
 struct KvAfter {
   float* Kc;
   float* Vc;
@@ -76,10 +76,6 @@ hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const 
 size_t attention_split_bytes(int Tq, int pos0, int H, int hs);
 hipError_t launch_attention_split(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc, const float* Vc,
                                   size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s);
-// Appends the K and V columns of qkv[T,3d] at positions pos0.. of a head-major cache [H][ctx][hs].
-hipError_t launch_kv_append(int T, int d, int hs, int ctx, int pos0, const float* qkv, float* Kc, float* Vc, hipStream_t s);
-// Copies rows of src (row stride lds, `cols` floats wide) to dst (row stride ldd).
-hipError_t launch_copy_rows(int rows, int cols, const float* src, int lds, float* dst, int ldd, hipStream_t s);
 // Top-k / temperature / inverse-CDF selection of one token on the device (globals.js:47-74,
 // model.js:81-85); *u is the uniform draw, device memory. tok[0] and out[slot] (optional) get
 // the id, ids[k] / probs[k] (optional) the selected indices and their probabilities.

@@ -151,8 +151,7 @@ __device__ __forceinline__ float4 sum_slices(const float* p, size_t stride, int 
   return S <= 2 ? sum_slices_by<2>(p, stride, S) : S <= 4 ? sum_slices_by<4>(p, stride, S) : sum_slices_by<8>(p, stride, S);
 }
 
-// With kv.Kc set, C is a [M, 3d] q/k/v matrix whose key and value columns also go to the head-major cache
-// (kv_append_kernel's layout).
+// With kv.Kc set, C is a [M, 3d] q/k/v matrix whose key and value columns also go to the cache [H][ctx][hs].
 __global__ __launch_bounds__(WG) void gemv_reduce(int M, int N, int S, const float* __restrict__ part,
                                                    const float* __restrict__ bias, float* C, int ldc, int epi,
                                                    const float* resid, KvAfter kv = KvAfter{nullptr, nullptr, 0, 0, 0, 0}) {
@@ -1308,27 +1307,6 @@ __global__ __launch_bounds__(WG) void vocab_gemv_ln_kernel(int V, int d, const f
   if (pos && blockIdx.x == 0 && threadIdx.x == 0) *pos += 1;
 }
 
-
-__global__ __launch_bounds__(WG) void copy_rows_kernel(int cols4, const float* __restrict__ src, int lds,
-                                                        float* __restrict__ dst, int ldd) {
-  const int r = blockIdx.y;
-  const int c = blockIdx.x * WG + threadIdx.x;
-  if (c < cols4) st4(dst + (size_t)r * ldd + 4 * c, ld4(src + (size_t)r * lds + 4 * c));
-}
-
-// Appends T rows of keys and values (columns d..2d and 2d..3d of qkv[T,3d]) to the
-// head-major cache: row (h, pos0+i) of K at Kc + (h*ctx + pos0+i)*hs.
-__global__ __launch_bounds__(WG) void kv_append_kernel(int d, int hs, int ctx, int pos0, const float* __restrict__ qkv,
-                                                        float* __restrict__ Kc, float* __restrict__ Vc) {
-  const int i = blockIdx.x;
-  for (int c4 = threadIdx.x; c4 < (d >> 2); c4 += WG) {
-    const int c = c4 * 4, h = c / hs, e = c - h * hs;
-    const size_t dst = ((size_t)h * ctx + pos0 + i) * hs + e;
-    st4(Kc + dst, ld4(qkv + (size_t)i * 3 * d + d + c));
-    st4(Vc + dst, ld4(qkv + (size_t)i * 3 * d + 2 * d + c));
-  }
-}
-
 // Token selection of GPT.generate (model.js:81-85) on the device:
 //   selectTopK (globals.js:66-74): stable descending sort of (value, index), first k;
 //   cpuSoftmax (globals.js:59-64) of those k logits in float64:
@@ -1815,16 +1793,6 @@ hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const 
   const size_t smem = sizeof(float) * (size_t)(pos0 + Tq);
   if (smem > 48 * 1024) return hipErrorInvalidValue;
   attention_kernel<<<dim3(H, Tq), WG, smem, s>>>(pos0, hs, lpk, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo);
-  return hipGetLastError();
-}
-
-hipError_t launch_copy_rows(int rows, int cols, const float* src, int lds, float* dst, int ldd, hipStream_t s) {
-  copy_rows_kernel<<<dim3(cdiv(cols >> 2, WG), rows), WG, 0, s>>>(cols >> 2, src, lds, dst, ldd);
-  return hipGetLastError();
-}
-
-hipError_t launch_kv_append(int T, int d, int hs, int ctx, int pos0, const float* qkv, float* Kc, float* Vc, hipStream_t s) {
-  kv_append_kernel<<<T, WG, 0, s>>>(d, hs, ctx, pos0, qkv, Kc, Vc);
   return hipGetLastError();
 }
 
