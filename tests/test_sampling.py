@@ -105,6 +105,21 @@ def test_host_selection_is_a_stable_sort():
     assert sampling.selectTopK([0.5, 2, 1], 2) == {"topKIndices": [1, 2], "topKProbs": [2.0, 1.0]}
 
 
+def test_host_selection_takes_what_a_sort_takes():
+    """Any sequence of values that are floats or become ones, and every top_k that cuts a list."""
+    import array
+    import torch
+    from webgpt_amd import sampling
+    x = np.random.default_rng(3).permutation(np.repeat(np.arange(100), 2)).astype(np.float32)
+    forms = [x, x.tolist(), tuple(x), array.array("d", x), x.astype(np.int64), x.astype(np.longdouble), x.astype(object), x[::-1], x.astype(">f4"),
+             torch.tensor(x), torch.tensor(x).to(torch.bfloat16), dict(enumerate(x))]
+    for form in forms:
+        for k in (None, -195, 0, 1, 2, 7, 200, 300, True):
+            values = [float(form[i]) for i in range(len(form))]
+            order = sorted(range(len(values)), key=lambda i: -values[i])[:k]
+            assert sampling.selectTopK(form, k) == {"topKIndices": order, "topKProbs": [values[i] for i in order]}, (type(form), k)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,x,k", hard_cases(), ids=[c[0] for c in hard_cases()])
 def test_device_selection_of_hard_inputs(device, name, x, k):

@@ -9,12 +9,13 @@ def selectTopK(probs, top_k):
     """Stable descending sort by value, first top_k (globals.js:66-74): ties keep the
     lower index first. Of a long array only what can be among the first top_k is sorted: the values not below
     the top_k-th largest of the maxima of runs of 64 (50257 values, top_k = 40: 8 ms for all of them in a list, 0.1 ms so)."""
-    a = np.asarray(probs)
-    if a.dtype.kind != "f":
-        a = a.astype(np.float64)
+    if isinstance(probs, np.ndarray) and probs.ndim == 1 and probs.dtype in (np.float16, np.float32, np.float64):
+        a = probs
+    else:  # any sequence of what float() takes
+        a = np.array([float(probs[i]) for i in range(len(probs))], np.float64)
     runs = a.size // 64
     order = None
-    if 0 < top_k < runs:
+    if top_k is not None and 0 < top_k < runs:
         tops = a[:64 * runs].reshape(runs, 64).max(axis=1)
         order = np.flatnonzero(a >= np.partition(tops, runs - top_k)[runs - top_k])
         if order.size < top_k:  # NaN among them
