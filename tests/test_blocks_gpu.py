@@ -598,6 +598,31 @@ def test_attention_split_tiny_values(device, T, H, hs, small):
     assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
 
 
+@pytest.mark.parametrize("T,H,hs", [(193, 2, 20), (700, 2, 64), (331, 4, 96), (1023, 2, 128)])
+def test_attention_split_tiny_weights(device, T, H, hs):
+    """Weights of 2**-124 to 2**-119 (scores 83 to 86 below the first key's, whose value is zero), whose third bf16 part is too
+    small for bf16, on values around 2**30: the outputs are not tiny themselves. Scores are exact here and all terms positive: a
+    few roundings for a weight and the quotient, and one for each of the at most T / 8 keys that are added up in a row (2**-12 with
+    the third parts lost)."""
+    d = H * hs
+    rng = np.random.default_rng(T + d)
+    x = (rng.uniform(1, 2, (T, d)) * 2.0 ** 30).astype(np.float32)
+    x[0] = 0
+    x[1:, ::hs] = -rng.integers(83 * 64, 86 * 64, (T - 1, H)) / np.float32(64)  # the scores: q is 1 in the first dimension, else 0
+    eye, none, zero = np.eye(d, dtype=np.float32), np.zeros((d, d), np.float32), np.zeros(d, np.float32)
+    bq = zero.copy()
+    bq[::hs] = 1
+    bufs = [init_tensor(x, [T, d])]
+    for w, b in ((none, bq), (eye, zero), (eye, zero), (eye, zero)):
+        bufs += [init_tensor(w, [d, d]), init_tensor(b, [d])]
+    got = run(AttentionBlock.newFusedInstance(T, d, 1.0, H, hs, *bufs, FastMatMulBlock, SoftmaxBlock), (T, d)).astype(np.float64)
+    weights = np.exp(x[:, ::hs].astype(np.float64))
+    for h in range(H):
+        want = np.cumsum(weights[:, h:h + 1] * x[:, h * hs + 1:(h + 1) * hs], 0) / np.cumsum(weights[:, h:h + 1], 0)
+        error = np.abs(got[:, h * hs + 1:(h + 1) * hs] - want)
+        assert np.all(error <= 2.0 ** -24 * (T / 8 + 16) * want), float(np.max(error[1:] / want[1:]))
+
+
 def test_attention_values_known_answer(device):
     # other/test.js:370-388 through the attention block: with Wq = Wk = 0 every score is 0, so the
     # softmax is uniform over j <= i: P = 1/(i+1). V = c // hs + 1 (via bv, Wv = 0), Wo = I:

@@ -115,9 +115,10 @@ __device__ __forceinline__ f32x4 over_workgroup(f32x4 v, f32x4* sh) {
 
 // The outputs of the queries q0 + (bits of `left`) with plain fp32 products, four at a time by the whole workgroup, over runs of
 // AS_RUN keys: for operands that have no split (infinite ones, see gemm_split.hip), for NaN, and for values so small that their
-// third part is lost (under 2^-110: outputs under 2^-100 are taken again). Scores that are not numbers end
-// it, as nothing else can come out. An attention block of 12 heads x 48 at 943 rows takes 325 us where every output is taken
-// again (128 us where none is; 21.6 ms with a loop over the keys per output).
+// third part is lost (under 2^-110: outputs under 2^-60 are taken again, as sums are in gemm_split.hip, which leaves out such
+// values times others of about 2^50 and more). Scores that are not numbers end it, as nothing else can come out. An attention
+// block of 12 heads x 48 at 943 rows takes 325 us where every output is taken again (128 us where none is; 21.6 ms with a loop
+// over the keys per output).
 constexpr int AS_RUN = 1024;
 template <int NT>
 __device__ __forceinline__ void plain_rows(const AttnSplitArgs& a, int h, int q0, unsigned left, float* lds) {
@@ -375,8 +376,8 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
     }
     const float v = num / den;
     a.out[(size_t)(q0 + qi) * a.ldo + (size_t)h * a.hs + dim] = v;
-    // twice the bits, so without the sign: under 2^-100 and no zero, or not finite
-    constexpr unsigned LO = (127 - 100) << 24, HI = 0xff000000u;
+    // twice the bits, so without the sign: under 2^-60 and no zero, or not finite
+    constexpr unsigned LO = (127 - 60) << 24, HI = 0xff000000u;
     const unsigned v2 = __float_as_uint(v) << 1;
     if (v2 - LO >= HI - LO && v2 != 0u) atomicOr(&again, 1u << qi);
   }
