@@ -1,4 +1,4 @@
-// Device code: an fp32 value as the exact sum of three bf16 values, the operands of gemm_split.hip and attention_split.hip.
+// Device code: an fp32 value as the sum of three bf16 values (exact from 2^-110 on), the operands of gemm_split.hip and attention_split.hip.
 #ifndef WGPT_SPLIT_BF16_H
 #define WGPT_SPLIT_BF16_H
 
