@@ -598,17 +598,18 @@ def test_attention_split_tiny_values(device, T, H, hs, small):
     assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
 
 
+@pytest.mark.parametrize("below,exponent", [(83, 30), (83, 80), (88, 40), (88, 100)])
 @pytest.mark.parametrize("T,H,hs", [(193, 2, 20), (700, 2, 64), (331, 4, 96), (1023, 2, 128)])
-def test_attention_split_tiny_weights(device, T, H, hs):
+def test_attention_split_tiny_weights(device, T, H, hs, below, exponent):
     """Weights of 2**-124 to 2**-119 (scores 83 to 86 below the first key's, whose value is zero), whose third bf16 part is too
-    small for bf16, on values around 2**30: the outputs are not tiny themselves. Scores are exact here and all terms positive: a
-    few roundings for a weight and the quotient, and one for each of the at most T / 8 keys that are added up in a row (2**-12 with
-    the third parts lost)."""
+    small for bf16, on values around 2**30 and 2**80: the outputs are not tiny themselves. Scores are exact here and all terms
+    positive: a few roundings for a weight and the quotient, and one for each of the at most T / 8 keys that are added up in a row
+    (2**-12 with the third parts lost). Scores 88 to 91 below: weights are subnormal, within 2**-149 (2**-17 of them), and not zero."""
     d = H * hs
     rng = np.random.default_rng(T + d)
-    x = (rng.uniform(1, 2, (T, d)) * 2.0 ** 30).astype(np.float32)
+    x = (rng.uniform(1, 2, (T, d)) * 2.0 ** exponent).astype(np.float32)
     x[0] = 0
-    x[1:, ::hs] = -rng.integers(83 * 64, 86 * 64, (T - 1, H)) / np.float32(64)  # the scores: q is 1 in the first dimension, else 0
+    x[1:, ::hs] = -rng.integers(below * 64, (below + 3) * 64, (T - 1, H)) / np.float32(64)  # the scores: q is 1 in the first dimension, else 0
     eye, none, zero = np.eye(d, dtype=np.float32), np.zeros((d, d), np.float32), np.zeros(d, np.float32)
     bq = zero.copy()
     bq[::hs] = 1
@@ -620,7 +621,7 @@ def test_attention_split_tiny_weights(device, T, H, hs):
     for h in range(H):
         want = np.cumsum(weights[:, h:h + 1] * x[:, h * hs + 1:(h + 1) * hs], 0) / np.cumsum(weights[:, h:h + 1], 0)
         error = np.abs(got[:, h * hs + 1:(h + 1) * hs] - want)
-        assert np.all(error <= 2.0 ** -24 * (T / 8 + 16) * want), float(np.max(error[1:] / want[1:]))
+        assert np.all(error <= (2.0 ** -24 * (T / 8 + 16) + (2.0 ** -17 if below > 87 else 0)) * want), float(np.max(error[1:] / want[1:]))
 
 
 def test_attention_values_known_answer(device):

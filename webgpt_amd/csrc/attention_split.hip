@@ -115,11 +115,13 @@ __device__ __forceinline__ f32x4 over_workgroup(f32x4 v, f32x4* sh) {
 
 // The outputs of the queries q0 + (bits of `left`) with plain fp32 products, four at a time by the whole workgroup, over runs of
 // AS_RUN keys: for operands that have no split (infinite ones, see gemm_split.hip), for NaN, and for values so small that their
-// third part is lost (under 2^-110: outputs under 2^-60 are taken again, as sums are in gemm_split.hip, which leaves out such
-// values times others of about 2^50 and more). Scores that are not numbers end it, as nothing else can come out. An attention
-// block of 12 heads x 48 at 943 rows takes 325 us where every output is taken again (128 us where none is; 21.6 ms with a loop
+// third part is lost (under 2^-110: outputs under 2^-60 are taken again, as sums are in gemm_split.hip). Weights are as small
+// for keys whose scores are AS_FAR below the largest one, and exp_neg has none under 2^-126: queries with such keys have their
+// outputs under 2^-20 taken again, zeros among them, which leaves out such weights on values of about 2^80 and more. Scores
+// that are not numbers end it, as nothing else can come out. An attention block of 12 heads x 48 at 943 rows takes 325 us where every output is taken again (128 us where none is; 21.6 ms with a loop
 // over the keys per output).
 constexpr int AS_RUN = 1024;
+constexpr float AS_FAR = 76.f;  // exp(-76) is 2^-109.6
 template <int NT>
 __device__ __forceinline__ void plain_rows(const AttnSplitArgs& a, int h, int q0, unsigned left, float* lds) {
   float* const scores = lds;  // [4][AS_RUN]
@@ -236,7 +238,7 @@ __device__ __forceinline__ void plain_rows(const AttnSplitArgs& a, int h, int q0
 // SIMD's registers, so four waves fill the compute unit.
 template <int DB, int NWV>
 __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(AttnSplitArgs a) {
-  constexpr int KS = 2 * DB, DIMS = 32 * DB, WAVE_FLOATS = DIMS * AS_MERGE + 2 * ASQ;
+  constexpr int KS = 2 * DB, DIMS = 32 * DB, WAVE_FLOATS = DIMS * AS_MERGE + 3 * ASQ;
   constexpr bool QREG = DB == 1;
   static_assert(4 * AS_RUN + 4 * NWV * 64 + 4 * NWV + 4 * 128 <= NWV * WAVE_FLOATS, "plain_rows' memory");
   extern __shared__ __attribute__((aligned(16))) float as_lds[];
@@ -268,7 +270,7 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
   for (int b = 0; b < DB; ++b)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
-  float m = -INFINITY, lsum = 0.f;
+  float m = -INFINITY, lsum = 0.f, least = INFINITY;
   u32x4 kf[KS][3], vf[KS][3];
   const auto fetch = [&](u32x4 (&f)[KS][3], const u32x4* base, int t) {
     const u32x4* src = base + (size_t)(h * a.nt + t) * KS * 192 + lane;
@@ -299,12 +301,14 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
       for (int r = 0; r < 16; ++r) {
         const int key = t * ASQ + (r >> 2) * 8 + hh * 4 + (r & 3);
         sacc[r] = key <= qpos ? (sacc[r] + rest[r]) * a.scale : -INFINITY;
+        least = fminf(least, key <= qpos ? sacc[r] : INFINITY);
         tmax = fmaxf(tmax, sacc[r]);
       }
     } else {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sacc[r] = (sacc[r] + rest[r]) * a.scale;
+        least = fminf(least, sacc[r]);
         tmax = fmaxf(tmax, sacc[r]);
       }
     }
@@ -345,9 +349,10 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
     }
   }
   lsum += __shfl_xor(lsum, 32);  // the two halves of a column saw disjoint keys, the same maximum
+  least = fminf(least, __shfl_xor(least, 32));
 
   if constexpr (!QREG) __syncthreads();
-  float* Om = as_lds + wave * WAVE_FLOATS;  // [DIMS][AS_MERGE], then maxima and sums of the 32 queries
+  float* Om = as_lds + wave * WAVE_FLOATS;  // [DIMS][AS_MERGE], then maxima, sums and least scores of the 32 queries
 #pragma unroll
   for (int b = 0; b < DB; ++b)
 #pragma unroll
@@ -355,6 +360,7 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
   if (hh == 0) {
     Om[DIMS * AS_MERGE + l32] = m;
     Om[DIMS * AS_MERGE + ASQ + l32] = lsum;
+    Om[DIMS * AS_MERGE + 2 * ASQ + l32] = least;
   }
   if (threadIdx.x == 0) again = 0u;
   __syncthreads();
@@ -367,19 +373,21 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
       mw[w] = as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + qi];
       M = fmaxf(M, mw[w]);
     }
-    float num = 0.f, den = 0.f;
+    float num = 0.f, den = 0.f, lo = INFINITY;
 #pragma unroll
     for (int w = 0; w < NWV; ++w) {
       const float f = mw[w] > -INFINITY ? exp_neg(mw[w] - M) : 0.f;
       num += as_lds[w * WAVE_FLOATS + dim * AS_MERGE + qi] * f;
       den += as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + ASQ + qi] * f;
+      lo = fminf(lo, as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + 2 * ASQ + qi]);
     }
     const float v = num / den;
     a.out[(size_t)(q0 + qi) * a.ldo + (size_t)h * a.hs + dim] = v;
-    // twice the bits, so without the sign: under 2^-60 and no zero, or not finite
-    constexpr unsigned LO = (127 - 60) << 24, HI = 0xff000000u;
-    const unsigned v2 = __float_as_uint(v) << 1;
-    if (v2 - LO >= HI - LO && v2 != 0u) atomicOr(&again, 1u << qi);
+    // twice the bits, so without the sign: not finite, or under 2^-60 and no zero (far keys: under 2^-20, or zero)
+    constexpr unsigned HI = 0xff000000u;
+    const bool far = lo < M - AS_FAR;
+    const unsigned v2 = __float_as_uint(v) << 1, limit = (far ? 127 - 20 : 127 - 60) << 24;
+    if (v2 >= HI || (v2 < limit && (far || v2 != 0u))) atomicOr(&again, 1u << qi);
   }
   __syncthreads();
   const unsigned left = __builtin_amdgcn_readfirstlane(again);
@@ -388,7 +396,7 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
 
 template <int DB, int NWV>
 hipError_t launch_waves(const AttnSplitArgs& a, hipStream_t s) {
-  const size_t merge = sizeof(float) * NWV * (32 * DB * AS_MERGE + 2 * ASQ), ql = DB > 1 ? (size_t)2 * DB * 192 * 16 : 0;
+  const size_t merge = sizeof(float) * NWV * (32 * DB * AS_MERGE + 3 * ASQ), ql = DB > 1 ? (size_t)2 * DB * 192 * 16 : 0;
   const size_t lds = merge > ql ? merge : ql;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_split_kernel<DB, NWV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
