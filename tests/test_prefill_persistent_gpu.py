@@ -1,0 +1,104 @@
+"""Prompts that run as one persistent launch (wgpt_prefill, csrc/prefill_persistent.hip) against the CPU oracle: edges of the
+sixteen rows of a row group, of the steps of 32 of a contraction and of the tiles of sixteen columns, head sizes, both weight
+dtypes, and what the host does when the launch gives up."""
+import numpy as np
+import pytest
+
+from oracle import ref
+from webgpt_amd import _lib, synth
+from webgpt_amd.model import GPT
+
+from helpers import close, make_model, oracle_weights, small_cfg, worst
+
+pytestmark = pytest.mark.gpu
+
+# (width, heads): the smallest, widths of no whole step or slice, more heads than column groups, head sizes up to 128, the widest
+SHAPES = [(8, 1), (40, 2), (200, 5), (256, 2), (576, 12), (640, 40), (1240, 31), (1280, 10), (1600, 25), (1792, 14)]
+
+
+def load(cfg, tensors, flags=0):
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg), flags=flags)
+    gpt.initialize()
+    return gpt
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head", SHAPES)
+def test_prompts_against_oracle(device, dtype, d, n_head):
+    """Logits, cache rows of both layers and the residual rows, of one model in turn: a launch meets what the one before it left."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=130, vocab_size=301, dtype=dtype)
+    tensors = make_model(cfg, d)
+    gpt = load(cfg, tensors)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (1, 16, 128, 17, 2, 61, 64, 65, 113, 129):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        want, taps, kv = ref.forward(p, w, tokens, want_taps=True, want_kv=True)
+        got = gpt.prefill(tokens)
+        assert close(got, want), (T, worst(got, want))
+        for i in range(2):
+            for j, name in enumerate("kv"):
+                rows = gpt.tap(f"kv{i}_{name}")
+                assert close(rows, kv[i, j]), (T, i, name, worst(rows, kv[i, j]))
+        # a residual value is the sum of an embedding and four products of the rows' size: near zero its error is that of its
+        # terms (d = 1600: 1e-5 of their root mean square, of which the oracle's ascending fp32 sums have the larger half)
+        rows, exp = gpt.tap("residual", T), taps[ref.tap_names(2).index("block1_r2")]
+        assert close(rows, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_expired_wait_falls_back_to_launches(device, monkeypatch, dtype):
+    """Waits that give up at their first look (forced from the host; every kernel drains): the call's results are those of the
+    launches, bit for bit, and so are those of the next call."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 3)
+    launches = load(cfg, tensors, flags=_lib.FLAG_TAPS)  # (with taps a prompt always takes them)
+    monkeypatch.setenv("WEBGPT_AMD_SPIN_LIMIT", "0")
+    gpt = load(cfg, tensors)
+    monkeypatch.delenv("WEBGPT_AMD_SPIN_LIMIT")
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (40, 12):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        got = gpt.prefill(tokens)
+        assert close(got, ref.forward(p, w, tokens)), T
+        assert close(got, launches.prefill(tokens))
+    gpt.unloadBuffers()
+    launches.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("what", ["value", "scale", "weight"])
+def test_values_that_are_not_finite(device, dtype, what):
+    """A bias of the values that is infinite, an infinite column scale (int8) or weight (fp32), tiny embeddings: rows that the
+    launches lose are lost and all others as they give them."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    T = 50
+    tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+    if what == "value":  # one position's embedding: its keys and values are NaN, queries before it must not see them
+        tensors["transformer.wpe.weight"] = tensors["transformer.wpe.weight"].copy()
+        tensors["transformer.wpe.weight"][37, 5] = np.inf
+    else:
+        name = "transformer.h.1.mlp.c_fc." + ("weight" if dtype == "f32" else "weight.scale")
+        if what == "weight":
+            name = "transformer.wpe.weight"  # products of nothing but tiny values behind a LayerNorm that divides by sqrt(1e-5)
+            tensors["transformer.wte.weight"] = tensors["transformer.wte.weight"] * np.float32(0)
+            tensors[name] = tensors[name] * np.float32(1e-30)
+        else:
+            tensors[name] = tensors[name].copy()
+            tensors[name].reshape(-1)[7] = np.inf
+    launches = load(cfg, tensors, flags=_lib.FLAG_TAPS)
+    gpt = load(cfg, tensors)
+    with np.errstate(all="ignore"):
+        got, want = gpt.prefill(tokens), launches.prefill(tokens)
+        for i in range(2):
+            for name in "kv":
+                a, b = gpt.tap(f"kv{i}_{name}"), launches.tap(f"kv{i}_{name}")
+                assert (np.isfinite(a) == np.isfinite(b)).all(), (i, name)
+                ok = np.isfinite(b)
+                assert close(a[ok], b[ok]), (i, name)
+        assert (np.isfinite(got) == np.isfinite(want)).all()
+        ok = np.isfinite(want)
+        assert close(got[ok], want[ok])
+    gpt.unloadBuffers()
+    launches.unloadBuffers()

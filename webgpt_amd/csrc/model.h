@@ -9,6 +9,7 @@
 
 #include "../../include/webgpt_amd.h"
 #include "decode_persistent.h"
+#include "prefill_persistent.h"
 
 namespace wgpt {
 
@@ -68,6 +69,12 @@ struct Model {
   // ids_pin the ids
   bool res_host_done = false, res_host_logits = false, res_host_ids = false;
   unsigned epoch = 0;        // last epoch published by earlier launches
+
+  // persistent prefill of prompts of up to pp_rows tokens (any decode mode)
+  int pp_rows = 0;
+  PrefillArgs pp{};
+  unsigned pp_epoch = 0;       // last epoch of its earlier launches
+  int32_t* tok_pin = nullptr;  // pinned (behind ids_pin's): [PP_MAX_T] the prompt, then the word that a launch leaves its error in
 
   // decode with one launch per block (decode_mode 0): the token's launches read the cache position from pos_dev and
   // are recorded once as a HIP graph that every later token replays

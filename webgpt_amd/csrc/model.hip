@@ -271,6 +271,18 @@ static int decode_token_blocks(Model* m, int pos) {
   return token_launches(m, pos);
 }
 
+// A wait of a persistent kernel that takes this many poll rounds (a quarter of a second) means a workgroup is not running;
+// WEBGPT_AMD_SPIN_LIMIT lowers it (tests of the fallback force an expiry this way: with 0 a wait gives up when its first look
+// finds a word missing, which without poll delays is certain).
+static unsigned spin_limit() {
+  if (const char* e = getenv("WEBGPT_AMD_SPIN_LIMIT")) {
+    char* end = nullptr;
+    const long v = strtol(e, &end, 10);
+    if (end != e && v >= 0 && v < (1l << 30)) return (unsigned)v;
+  }
+  return 1u << 18;
+}
+
 // Prepares the decode paths: slab-layout copies of the linear weights and the per-layer parameter blocks
 // (any shape), then, for the shapes the persistent whole-token kernel is built for, its per-workgroup
 // parameter blocks and exchange buffers. Leaves m->persist_ok false (and the per-block path in charge) for
@@ -398,15 +410,7 @@ static int setup_persistent(Model* m) {
         for (int i = 0; i < 2; ++i) a.att_slope[i] = v[i] < 0 ? 0 : (v[i] > 1024 ? 1024 : v[i]);
     }
   }
-  // a wait that takes this many poll rounds (a quarter of a second) means a workgroup is not running;
-  // WEBGPT_AMD_SPIN_LIMIT lowers it (tests of the fallback force an expiry this way: with 0 a wait
-  // gives up when its first look finds a word missing, which without poll delays is certain)
-  a.spin_limit = 1u << 18;
-  if (const char* e = getenv("WEBGPT_AMD_SPIN_LIMIT")) {
-    char* end = nullptr;
-    const long v = strtol(e, &end, 10);
-    if (end != e && v >= 0 && v < (1l << 30)) a.spin_limit = (unsigned)v;
-  }
+  a.spin_limit = spin_limit();
   // context length from which a launch uses twice the attention slices per head (WEBGPT_AMD_SHORT_KEYS for tuning)
   a.short_keys = PD_SHORT_KEYS;
   if (const char* e = getenv("WEBGPT_AMD_SHORT_KEYS")) {
@@ -587,6 +591,60 @@ static int block_linear_weights(Model* m, void* free_buf) {
   return WGPT_OK;
 }
 
+// Prepares the persistent prefill in the buffers that wgpt_model_finalize has allocated for it; after block_linear_weights.
+static int setup_prefill(Model* m) {
+  const bool i8 = m->p.weight_dtype == 1;
+  std::vector<PrefillLayer> layers(m->L);
+  for (int i = 0; i < m->L; ++i) {
+    const LayerW& l = m->layers[i];
+    const LinW* w[4] = {&l.attn, &l.proj, &l.fc, &l.fc2};
+    const void* p[4];
+    for (int j = 0; j < 4; ++j) p[j] = i8 ? (const void*)w[j]->q : (const void*)w[j]->w;
+    layers[i] = {p[0], p[1], p[2], p[3], w[0]->s, w[1]->s, w[2]->s, w[3]->s, l.attn_b, l.proj_b, l.fc_b, l.fc2_b,
+                 l.ln1_g, l.ln1_b, l.ln2_g, l.ln2_b};
+  }
+  PrefillArgs& a = m->pp;
+  WGPT_HIP(hipMemcpyAsync((void*)a.layers, layers.data(), sizeof(PrefillLayer) * (size_t)m->L, hipMemcpyHostToDevice, rt().stream));
+  WGPT_HIP(hipMemsetAsync(a.flags, 0, PP_FLAGS * sizeof(unsigned), rt().stream));
+  WGPT_HIP(hipStreamSynchronize(rt().stream));
+  a.L = m->L; a.H = m->H; a.hs = m->hs; a.d = m->d; a.ctx = m->ctx; a.V = m->V;
+  a.scale = (float)(1.0 / std::sqrt((double)m->hs));
+  a.tok = m->tok_pin;
+  a.wte = m->wte; a.wpe = m->wpe; a.lnf_g = m->lnf_g; a.lnf_b = m->lnf_b;
+  a.x = m->x;
+  const size_t row_floats = (size_t)prefill_rows(m->pp_rows) * m->d;
+  a.xe = a.q + row_floats; a.x1 = a.xe + row_floats; a.att = a.x1 + row_floats; a.h = a.att + row_floats;
+  a.kv = m->kv;
+  a.logits = m->logits; a.host_logits = m->logits_pin;
+  a.host_err = m->tok_pin + PP_MAX_T;
+  a.spin_limit = spin_limit();
+  m->pp_epoch = 0;
+  return WGPT_OK;
+}
+
+// The prompt's forward in one launch, logits into logits_pin. *done: it has run to its end; where it has not (a wait that
+// expired, sums that the split operands may have spoilt) the caller runs the launches of forward_blocks, and so does every later
+// call.
+static int prefill_persistent(Model* m, const int32_t* tokens, int T, bool* done) {
+  const unsigned n = prefill_epochs(m->L);
+  if (m->pp_epoch > 0x7fffffffu - 2 * n) {
+    WGPT_HIP(hipMemsetAsync(m->pp.flags, 0, PP_FLAGS * sizeof(unsigned), rt().stream));
+    m->pp_epoch = 0;
+  }
+  memcpy(m->tok_pin, tokens, sizeof(int32_t) * (size_t)T);  // (every earlier use has completed: each call ends with a synchronisation)
+  m->tok_pin[PP_MAX_T] = 0;
+  PrefillArgs a = m->pp;
+  a.T = T;
+  a.ebase = m->pp_epoch;
+  LAUNCH(launch_prefill_persistent(a, m->p.weight_dtype == 1, rt().stream));
+  m->pp_epoch += n;
+  WGPT_HIP(hipEventRecord(m->ev1, rt().stream));
+  WGPT_HIP(hipStreamSynchronize(rt().stream));
+  *done = m->tok_pin[PP_MAX_T] == 0;
+  if (!*done) m->pp_rows = 0;
+  return WGPT_OK;
+}
+
 static void destroy_model(Model* m) {
   if (m->token_graph_exec) (void)hipGraphExecDestroy(m->token_graph_exec);
   if (m->token_graph) (void)hipGraphDestroy(m->token_graph);
@@ -677,6 +735,7 @@ int wgpt_model_finalize(wgpt_model h) {
   const size_t part_bytes = gemm_workspace_floats((int)T, 4 * (int)d) * f;  // partial sums of the prefill products
   const size_t att_ws = attention_workspace_bytes((int)T, 0, m->H, m->hs);
   void* block_buf = nullptr;
+  m->pp_rows = m->p.flags & WGPT_FLAG_TAPS ? 0 : std::min(m->maxT, prefill_persistent_rows(m->d, m->H, m->hs, m->V, i8, rt().compute_units));
   // everything in one allocation: each costs a model's load tenths of a millisecond
   const struct { void** dst; size_t bytes; } bufs[] = {
       {(void**)&m->kv, (size_t)m->L * 2 * m->ctx * d * f},
@@ -690,7 +749,8 @@ int wgpt_model_finalize(wgpt_model h) {
       {(void**)&m->u_dev, (size_t)m->ctx * sizeof(double)}, {(void**)&m->part, part_bytes},
       {(void**)&m->att_ws, att_ws > part_bytes ? att_ws : 0},
       {(void**)&m->taps, m->p.flags & WGPT_FLAG_TAPS ? (size_t)(2 + 6 * m->L) * T * d * f : 0},
-      {&block_buf, (size_t)4 * d * d * (i8 ? 1 : f)}};
+      {(void**)&m->pp.layers, m->pp_rows ? sizeof(PrefillLayer) * m->L : 0}, {(void**)&m->pp.flags, m->pp_rows ? PP_FLAGS * sizeof(unsigned) : 0},
+      {(void**)&m->pp.q, prefill_exchange_floats(m->pp_rows, (int)d) * f}, {&block_buf, (size_t)4 * d * d * (i8 ? 1 : f)}};
   const auto room = [](size_t bytes) { return (bytes + 16 + 255) / 256 * 256; };
   size_t total = 0;
   for (const auto& b : bufs) total += room(b.bytes);
@@ -708,8 +768,10 @@ int wgpt_model_finalize(wgpt_model h) {
     m->pin[0] = m->pin[1] = m->pin[2] = m->pin[3] = 0;
   }
   if (!m->logits_pin) WGPT_HIP(hipHostMalloc((void**)&m->logits_pin, sizeof(float) * ((size_t)m->V + 1), hipHostMallocDefault));
-  if (!m->u_pin) WGPT_HIP(hipHostMalloc((void**)&m->u_pin, (sizeof(double) + sizeof(int32_t)) * (size_t)m->ctx, hipHostMallocDefault));
+  if (!m->u_pin)
+    WGPT_HIP(hipHostMalloc((void**)&m->u_pin, (sizeof(double) + sizeof(int32_t)) * (size_t)m->ctx + (PP_MAX_T + 1) * sizeof(int32_t), hipHostMallocDefault));
   m->ids_pin = reinterpret_cast<int32_t*>(m->u_pin + m->ctx);
+  m->tok_pin = m->ids_pin + m->ctx;
   WGPT_HIP(hipMemsetAsync(m->pos_dev, 0, sizeof(int), rt().stream));
   WGPT_HIP(hipMemsetAsync(m->kv, 0, (size_t)m->L * 2 * m->ctx * d * f, rt().stream));
   if (!m->ev0) WGPT_HIP(hipEventCreate(&m->ev0));
@@ -719,6 +781,7 @@ int wgpt_model_finalize(wgpt_model h) {
   m->weights_moved = true;
   if ((rc = block_linear_weights(m, block_buf))) return rc;
   WGPT_HIP(hipStreamSynchronize(rt().stream));  // (its errors are this call's)
+  if (m->pp_rows && (rc = setup_prefill(m))) return rc;
   m->decode_mode = m->persist_ok ? 1 : 0;
   m->pos = 0;
   m->finalized = true;
@@ -736,16 +799,26 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
   if (T > m->maxT) return fail(WGPT_ERR_ARG, "wgpt_prefill: T = %d exceeds max_prefill = %d", T, m->maxT);
   for (int i = 0; i < T; ++i)
     if (tokens[i] < 0 || tokens[i] >= m->V) return fail(WGPT_ERR_ARG, "wgpt_prefill: token id %d at %d outside [0, %d)", tokens[i], i, m->V);
-  WGPT_HIP(hipMemcpyAsync(m->tok_dev, tokens, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, rt().stream));
-  WGPT_HIP(hipStreamSynchronize(rt().stream));
-  WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
   m->pos = 0;
   m->tap_T = 0;
   m->x_rows = 0;
-  int rc = forward_blocks(m, T, 0, true);
-  if (rc) return rc;
-  rc = finish_timed(m, logits);
-  if (rc) return rc;
+  int rc;
+  bool done = false;
+  if (T <= m->pp_rows) {
+    WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
+    if ((rc = prefill_persistent(m, tokens, T, &done))) return rc;
+    if (done) {
+      if (logits) memcpy(logits, m->logits_pin, sizeof(float) * (size_t)m->V);
+      WGPT_HIP(hipEventElapsedTime(&m->last_ms, m->ev0, m->ev1));
+    }
+  }
+  if (!done) {
+    WGPT_HIP(hipMemcpyAsync(m->tok_dev, tokens, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, rt().stream));
+    WGPT_HIP(hipStreamSynchronize(rt().stream));
+    WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
+    if ((rc = forward_blocks(m, T, 0, true))) return rc;
+    if ((rc = finish_timed(m, logits))) return rc;
+  }
   m->pos = T;
   m->tap_T = m->taps ? T : 0;
   m->x_rows = T;
