@@ -1,0 +1,97 @@
+"""Decode steps of shapes that the persistent kernel of fixed widths does not have (csrc/decode_generic.hip) against the CPU
+oracle: widths of no whole segment, more heads than workgroups of a phase, head sizes up to 128, both weight dtypes, contexts on
+both sides of the slices' limits, and what the host does when the launch gives up."""
+import numpy as np
+import pytest
+
+from oracle import ref
+from webgpt_amd import synth
+from webgpt_amd._lib import WgptError
+from webgpt_amd.model import GPT
+
+from helpers import close, make_model, oracle_weights, small_cfg, worst
+
+pytestmark = pytest.mark.gpu
+
+# (width, heads): the smallest, workgroups without columns (72), heads of 4, widths of no whole segment, one to seven segments
+SHAPES = [(8, 1), (72, 2), (200, 5), (256, 64), (384, 32), (576, 12), (768, 8), (1032, 129), (1280, 10), (1600, 50), (1792, 14)]
+
+
+def load(cfg, tensors):
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg))
+    gpt.initialize()
+    return gpt
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head", SHAPES)
+def test_steps_against_oracle_and_launches(device, dtype, d, n_head):
+    """Single steps against the oracle and against a launch per block, from contexts around 64 and 128 positions (where a slice
+    more is taken), then a run of greedy steps in one call; the rows that the steps leave in the cache."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=200, vocab_size=301, dtype=dtype)
+    tensors = make_model(cfg, d)
+    gpt = load(cfg, tensors)
+    gpt.set_decode_mode(1)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    tokens = synth.tokens(5, "prompt", 200, cfg["vocab_size"])
+    for T in (1, 62, 127, 193):
+        gpt.prefill(tokens[:T])
+        for i in range(3):
+            got = gpt.decode(int(tokens[T + i]))
+            want, kv = ref.forward(p, w, tokens[:T + i + 1], want_kv=True)
+            assert close(got, want), (T, i, worst(got, want))
+        for li in range(2):
+            for j, name in enumerate("kv"):
+                rows = gpt.tap(f"kv{li}_{name}")
+                assert close(rows, kv[li, j]), (T, li, name, worst(rows, kv[li, j]))
+    out = {}
+    for mode in (1, 0):
+        gpt.set_decode_mode(mode)
+        gpt.prefill(tokens[:60])
+        out[mode] = gpt.decode_greedy(int(tokens[60]), 9, want_logits=True)
+    assert np.array_equal(out[1][0], out[0][0])
+    assert close(out[1][1], out[0][1]), worst(out[1][1], out[0][1])
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("n_head,n_embd,n_ctx", [(4, 512, 1024), (4, 256, 1024), (3, 96, 2048), (80, 1280, 1152)])
+def test_the_longest_contexts(device, n_head, n_embd, n_ctx):
+    """The last positions that the slices of a head hold in registers (heads of 128, 64 and 32; eighty heads in three slices)."""
+    cfg = small_cfg(n_layer=1, n_head=n_head, n_embd=n_embd, n_ctx=n_ctx, vocab_size=97)
+    tensors = make_model(cfg, 1)
+    gpt = load(cfg, tensors)
+    gpt.set_decode_mode(1)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    tokens = synth.tokens(3, "prompt", n_ctx, cfg["vocab_size"])
+    for T in (509, n_ctx - 2):
+        gpt.prefill(tokens[:T])
+        for i in range(2):
+            got = gpt.decode(int(tokens[T + i]))
+            want = ref.forward(p, w, tokens[:T + i + 1])
+            assert close(got, want), (T, i, worst(got, want))
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_expired_wait_repeats_the_call_with_launches(device, monkeypatch, dtype):
+    """Waits that give up at their first look (forced from the host; every kernel drains): the calls succeed with the results of a
+    launch per block, bit for bit."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 3)
+    monkeypatch.setenv("WEBGPT_AMD_SPIN_LIMIT", "0")
+    monkeypatch.setenv("WEBGPT_AMD_POLL_DELAYS", "0,0,0,0,0,0,0")
+    launches = load(cfg, tensors)  # (its prompts give up as well: the caches are the same)
+    launches.set_decode_mode(0)
+    tokens = synth.tokens(9, "prompt", 20, cfg["vocab_size"])
+    u = np.array([0.3, 0.6, 0.9])
+    calls = [lambda g: g.decode(int(tokens[12])), lambda g: g.decode_greedy(int(tokens[12]), 3), lambda g: g.decode_sample(int(tokens[12]), 3, 5, 0.8, u)]
+    for call in calls:
+        gpt = load(cfg, tensors)
+        for g in (gpt, launches):
+            g.prefill(tokens[:12])
+        assert np.array_equal(call(gpt), call(launches))
+        assert np.array_equal(gpt.decode(int(tokens[16])), launches.decode(int(tokens[16])))
+        with pytest.raises(WgptError, match="not available"):
+            gpt.set_decode_mode(1)
+        gpt.unloadBuffers()
+    launches.unloadBuffers()

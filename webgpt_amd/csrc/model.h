@@ -55,6 +55,7 @@ struct Model {
   // persistent whole-token decode (decode_mode 1): slab-layout weights, exchange buffers
   bool slabs_ok = false;   // pa.slabs / pa.lparams are built (every shape)
   bool persist_ok = false;
+  bool generic = false;    // the persistent kernel is launch_decode_generic's
   PersistentArgs pa{};
   int* perr = nullptr;       // device error word of the persistent kernel
   // pinned host words (hipHostMalloc): [0] the token of a single-step call on its way to the device,

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "common.h"
+#include "decode_generic.h"
 #include "gemm_split.h"
 #include "kernels.h"
 #include "model.h"
@@ -351,14 +352,17 @@ static int setup_persistent(Model* m) {
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   m->slabs_ok = true;
   // The slabs and the folded parameters serve both decode paths (the one-launch-per-block path reads a column of a
-  // slab as one contiguous run of K); what follows is for the persistent kernel and the shapes it is built for.
-  if (m->hs != 64) return WGPT_OK;
+  // slab as one contiguous run of K); what follows is for the persistent kernels: the one of fixed shapes where it has
+  // this one, else the one of any shape.
   if (rt().compute_units < G) return WGPT_OK;
-  if (!persistent_supports(d, m->H, m->ctx, m->p.weight_dtype)) return WGPT_OK;
-  float* colparams;
-  if ((rc = dev_alloc(m, sizeof(float) * (size_t)m->L * PD_GRID * PD_COLP, (void**)&colparams))) return rc;
-  LAUNCH(build_colparams(lparams, m->L, d, i8 ? 1 : 0, colparams, rt().stream));
-  WGPT_HIP(hipStreamSynchronize(rt().stream));
+  m->generic = !(m->hs == 64 && persistent_supports(d, m->H, m->ctx, m->p.weight_dtype));
+  if (m->generic && !decode_generic_supports(d, m->H, m->hs, m->ctx, m->V, rt().compute_units)) return WGPT_OK;
+  float* colparams = nullptr;
+  if (!m->generic) {
+    if ((rc = dev_alloc(m, sizeof(float) * (size_t)m->L * PD_GRID * PD_COLP, (void**)&colparams))) return rc;
+    LAUNCH(build_colparams(lparams, m->L, d, i8 ? 1 : 0, colparams, rt().stream));
+    WGPT_HIP(hipStreamSynchronize(rt().stream));
+  }
   a.slabs = slabs;
   a.lparams = lparams;
   a.colparams = colparams;
@@ -385,16 +389,17 @@ static int setup_persistent(Model* m) {
     // curves are flat within a few percent around them and over context length);
     // wgpt_model_tune_poll_delays searches around them on the GPU at hand,
     // WEBGPT_AMD_POLL_DELAYS="a,b,c,d,e,f,g" overrides them for experiments
-    static const int tuned[6][7] = {{16, 4, 22, 78, 24, 28, 48},    // d = 768
+    static const int tuned[7][7] = {{16, 4, 22, 78, 24, 28, 48},    // d = 768
                                     {36, 0, 26, 82, 40, 40, 4},     // d = 1024
                                     {20, 0, 34, 100, 16, 16, 52},   // d = 1280
                                     {8, 12, 22, 84, 20, 12, 44},    // d = 1600, int8
                                     {32, 0, 48, 96, 4, 20, 40},     // d = 1600, fp32
-                                    {20, 4, 22, 78, 16, 16, 32}};   // d = 384: 51.1 us per token against 55.0 with d = 768's
+                                    {20, 4, 22, 78, 16, 16, 32},    // d = 384: 51.1 us per token against 55.0 with d = 768's
+                                    {12, 4, 22, 48, 12, 12, 32}};   // the kernel of any shape
     // growth of [2] and [3] per 1024 positions of context (the best values at contexts of 100, 350, 650 and 900
     // positions lie on a line: 117M 80, 88, 88, 104 for [3]; int8 88, 104, 128, 136)
-    static const int slopes[6][2] = {{11, 28}, {0, 46}, {9, 70}, {20, 61}, {0, 0}, {11, 28}};
-    const int row = d <= 384 ? 5 : d <= 768 ? 0 : d == 1024 ? 1 : d == 1280 ? 2 : i8 ? 3 : 4;
+    static const int slopes[7][2] = {{11, 28}, {0, 46}, {9, 70}, {20, 61}, {0, 0}, {11, 28}, {0, 0}};
+    const int row = m->generic ? 6 : d <= 384 ? 5 : d <= 768 ? 0 : d == 1024 ? 1 : d == 1280 ? 2 : i8 ? 3 : 4;
     const int* dflt = tuned[row];
     for (int i = 0; i < 7; ++i) a.delay[i] = dflt[i];
     a.att_slope[0] = slopes[row][0];
@@ -412,7 +417,7 @@ static int setup_persistent(Model* m) {
   }
   a.spin_limit = spin_limit();
   // context length from which a launch uses twice the attention slices per head (WEBGPT_AMD_SHORT_KEYS for tuning)
-  a.short_keys = PD_SHORT_KEYS;
+  a.short_keys = m->generic ? m->ctx : PD_SHORT_KEYS;
   if (const char* e = getenv("WEBGPT_AMD_SHORT_KEYS")) {
     char* end = nullptr;
     const long v = strtol(e, &end, 10);
@@ -433,6 +438,10 @@ static int setup_persistent(Model* m) {
   }
   m->persist_ok = true;
   return WGPT_OK;
+}
+
+static hipError_t launch_steps(Model* m, const PersistentArgs& a) {
+  return m->generic ? launch_decode_generic(a, rt().stream) : launch_decode_persistent(a, rt().stream);
 }
 
 // Runs `steps` greedy decode steps from position m->pos with the persistent kernel.
@@ -478,7 +487,7 @@ static int decode_persistent(Model* m, int steps, int top_k = 1, double temperat
   const int short_steps = a.short_keys - m->pos;
   if (short_steps > 0 && short_steps < steps) {
     a.nsteps = short_steps;
-    LAUNCH(launch_decode_persistent(a, rt().stream));
+    LAUNCH(launch_steps(m, a));
     a.ebase += per_step * (unsigned)short_steps;
     a.pos0 += short_steps;
     a.tok = a.out_tok + short_steps - 1;
@@ -491,9 +500,9 @@ static int decode_persistent(Model* m, int steps, int top_k = 1, double temperat
   if (host_results) {  // (the last launch of the call only)
     m->pin[1] = -1;  // every earlier use of the word has completed: each call ends with a synchronisation
     a.host_done = &m->pin[1];
-    if (persistent_writes_host_logits(m->d, m->p.weight_dtype) && a.rows_per_wg <= 4 * m->d) a.host_logits = m->logits_pin;
+    if (m->generic || (persistent_writes_host_logits(m->d, m->p.weight_dtype) && a.rows_per_wg <= 4 * m->d)) a.host_logits = m->logits_pin;
   }
-  LAUNCH(launch_decode_persistent(a, rt().stream));
+  LAUNCH(launch_steps(m, a));
   m->res_host_done = a.host_done != nullptr;
   m->res_host_ids = a.host_ids != nullptr;
   m->res_host_logits = a.host_logits != nullptr;
@@ -501,7 +510,7 @@ static int decode_persistent(Model* m, int steps, int top_k = 1, double temperat
   return WGPT_OK;
 }
 
-// After the stream has drained: did a bounded wait of the persistent kernel expire?
+// After the stream has drained: did a bounded wait of the persistent kernel expire? (decode_mode is 0 if so.)
 static int check_persistent(Model* m) {
 #ifdef WGPT_TRACE
   if (const char* path = getenv("WGPT_TRACE_FILE")) {
@@ -515,6 +524,12 @@ static int check_persistent(Model* m) {
 #endif
   // the error word came back with the call's results (read_back)
   const int herr = m->pin[1];
+  if (herr != 0 && m->generic) {  // its callers repeat the call with a launch per block, as they would have run it
+    (void)hipMemset(m->perr, 0, sizeof(int));
+    m->persist_ok = false;
+    m->decode_mode = 0;
+    return WGPT_OK;
+  }
   if (herr != 0) {
     (void)hipMemset(m->perr, 0, sizeof(int));
     m->persist_ok = false;  // do not trust the exchange buffers again
@@ -845,7 +860,10 @@ int wgpt_decode(wgpt_model h, int32_t token, float* logits) {
   if (rc) return rc;
   rc = finish_timed(m, logits);
   if (rc) return rc;
-  if (m->decode_mode == 1 && (rc = check_persistent(m))) return rc;
+  if (m->decode_mode == 1) {
+    if ((rc = check_persistent(m))) return rc;
+    if (m->decode_mode != 1) return wgpt_decode(h, token, logits);
+  }
   m->pos += 1;
   return WGPT_OK;
 }
@@ -886,6 +904,7 @@ int wgpt_decode_greedy(wgpt_model h, int32_t token, int steps, int32_t* out_toke
   if (persistent) {
     int rc = check_persistent(m);
     if (rc) return rc;
+    if (m->decode_mode != 1) return wgpt_decode_greedy(h, token, steps, out_tokens, logits);
   }
   m->pos += steps;
   return WGPT_OK;
@@ -910,8 +929,8 @@ int wgpt_decode_sample(wgpt_model h, int32_t token, int steps, int top_k, double
     return fail(WGPT_ERR_STATE, "wgpt_decode_sample: %d steps from position %d exceed the context of %d", steps, m->pos, m->ctx);
   const bool persistent = m->decode_mode == 1;
   const int k = top_k < m->V ? top_k : m->V;
-  // up to PD_TOPK candidates the persistent kernel selects and samples itself, all steps in one launch
-  const bool in_kernel = persistent && k <= PD_TOPK;
+  // up to PD_TOPK candidates the persistent kernel selects and samples itself, all steps in one launch (that of any shape one)
+  const bool in_kernel = persistent && k <= (m->generic ? 1 : PD_TOPK);
   if (!in_kernel) {  // (that launch brings the token and the draws along)
     m->pin[0] = token;  // every earlier use of the pinned words has completed: each call ends with a synchronisation
     memcpy(m->u_pin, u, sizeof(double) * (size_t)steps);
@@ -948,7 +967,10 @@ int wgpt_decode_sample(wgpt_model h, int32_t token, int steps, int top_k, double
     m->pos = pos_before;
     return rc;
   }
-  if (persistent && (rc = check_persistent(m))) return rc;
+  if (persistent) {
+    if ((rc = check_persistent(m))) return rc;
+    if (m->decode_mode != 1) return wgpt_decode_sample(h, token, steps, top_k, temperature, u, out_tokens, logits);
+  }
   m->pos = pos_before + steps;
   return WGPT_OK;
 }
@@ -1178,7 +1200,7 @@ int wgpt_model_set_decode_mode(wgpt_model h, int mode) {
   if (mode != 0 && mode != 1) return fail(WGPT_ERR_ARG, "wgpt_model_set_decode_mode: unknown mode %d", mode);
   if (mode == 1 && !m->persist_ok)
     return fail(WGPT_ERR_STATE, "wgpt_model_set_decode_mode: the persistent decode path is not available for this model "
-                                "(needs head size 64, a supported width and 256 compute units)");
+                                "(needs 256 compute units, heads of at most 128, a width of at most 1792 and a context that its registers hold)");
   m->decode_mode = mode;
   return WGPT_OK;
 }
