@@ -26,7 +26,7 @@ static int grow_scratch(int slot, size_t bytes, void** out) {
       s.ptr = nullptr;
       s.bytes = 0;
     }
-    hipError_t e = hipMalloc(&s.ptr, bytes + 16);
+    hipError_t e = device_malloc(&s.ptr, bytes + 16);
     if (e != hipSuccess) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu) for scratch: %s", bytes, hipGetErrorString(e));
     s.bytes = bytes;
   }
@@ -312,12 +312,15 @@ int wgpt_embed(const int32_t* idx, int T, int d, int V, wgpt_buf wte, wgpt_buf w
   const float* pp = F(wpe, (size_t)T * d, "wgpt_embed(wpe)");
   float* po = F(out, (size_t)T * d, "wgpt_embed(out)");
   if (!pe || !pp || !po) return WGPT_ERR_ARG;
-  void* didx;
-  int rc = grow_scratch(2, sizeof(int32_t) * (size_t)T, &didx);
-  if (rc) return rc;
-  WGPT_HIP(hipMemcpyAsync(didx, idx, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, rt().stream));
-  // idx is caller memory that may change once this returns: finish the copy first.
-  WGPT_HIP(hipStreamSynchronize(rt().stream));
+  // idx is caller memory that may change once this returns: the kernel reads a pinned copy (a copy to the device and the wait
+  // for it cost 20 us more), or the copy to the device has ended.
+  void* didx = stage_ids(idx, (size_t)T);
+  if (!didx) {
+    int rc = grow_scratch(2, sizeof(int32_t) * (size_t)T, &didx);
+    if (rc) return rc;
+    WGPT_HIP(hipMemcpyAsync(didx, idx, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, rt().stream));
+    WGPT_HIP(hipStreamSynchronize(rt().stream));
+  }
   hipError_t e = launch_embed((const int32_t*)didx, T, d, 0, pe, pp, po, rt().stream);
   if (e != hipSuccess) return fail(WGPT_ERR_HIP, "embed launch: %s", hipGetErrorString(e));
   return WGPT_OK;

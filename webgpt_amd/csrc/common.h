@@ -28,6 +28,13 @@ Runtime& rt();
 // least `need` bytes. Returns nullptr (and records the error) otherwise.
 void* resolve(wgpt_buf h, size_t need, const char* what);
 
+// hipMalloc that gives the freed buffers back which wgpt_free has kept before it reports that memory has run out.
+hipError_t device_malloc(void** out, size_t bytes);
+
+// Pinned words through which `count` token ids pass to a launch on the library's stream that is made before the next call; the
+// words are not written again before that launch has ended. null: too many for it.
+int32_t* stage_ids(const int32_t* ids, size_t count);
+
 // Frees the grow-only scratch buffers of the block entry points.
 void release_scratch();
 // Looks up this device's address of the fixed workspace of wgpt_matmul_bias_noalloc; called by wgpt_init

@@ -36,7 +36,7 @@ static Model* find_model(wgpt_model h) {
 
 static int dev_alloc(Model* m, size_t bytes, void** out) {
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes + 16);
+  hipError_t e = device_malloc(&p, bytes + 16);
   if (e != hipSuccess) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   m->allocs.push_back(p);
   *out = p;
