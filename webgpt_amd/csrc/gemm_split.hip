@@ -16,6 +16,7 @@
 #include "gemm_split.h"
 
 #include <cmath>
+#include <type_traits>
 
 #include "kernels.h"
 #include "split_bf16.h"
@@ -447,10 +448,13 @@ __device__ __forceinline__ void lds_barrier() {  // orders LDS accesses only: lo
 }
 
 // KG groups of NWN waves; a group takes every KG-th step of 32 k. Its waves own 32 * NB columns each, for all rows of the
-// tile: W goes straight from memory into registers, A through LDS, split once per workgroup on its way in; the products of a
-// step have the splitting of the next one between them. Half the traffic from L2 of the kernel above per product (a
-// compute unit takes 58 KB/us from there): 1024x4096x1024 in 128x128 tiles 54.4 us = 158 TFLOP/s, where 64x64 tiles of the
-// other take 61; 32x64 tiles for 65 to 128 rows: 100x3072x768 10.9 us against 12.5.
+// tile: W goes straight from memory into registers, A through LDS, split once per workgroup on its way in. A step is two halves of
+// 16 k; between the products of a half stand the reads of the next half's A from LDS and the splitting of its W, so that no product
+// waits for either: with the reads of a step in front of its products, where all waves of a compute unit make them at once,
+// the matrix cores stood still for a third of the time (cold weights, us before and now: 943x3072x768 in 96x128 tiles 32.5, 29.9,
+// in 128x128 tiles 37.9, 32.9; 512x3072x1024 in 64x128 27.5, 23.9; 512x1024x1024 in 32x64 13.2, 11.2). A step of 128x128 takes 1.04 us
+// with all units at work and 0.85 with 32 of them, its products 0.64 at the matrix cores' rate. 96x128 tiles are for row counts
+// of which 128 leave units idle: 943x2304x768 180 workgroups, 26.6 us, where 144 of 128x128 take 31.0 and 64x64 tiles of the kernel above 37.4.
 template <int MB, int NB, int NWN, int KG, bool I8, bool BLK, int OCC, int D>
 __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmArgs a) {
   constexpr int R = 32;
@@ -458,8 +462,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
   constexpr int MT = MB * R, GT = NWN * 64, Q = 4;
   constexpr int CH = MT + 2;               // units of 16 bytes between chunks of eight k: conflict-free writes and reads
   constexpr int BUF = 3 * 4 * CH;          // units of one buffer: planes x chunks
-  constexpr int AV = MT * 4 / GT;          // runs of eight k that a thread stages per step
-  static_assert(AV >= 1 && MT * 4 % GT == 0, "staging");
+  constexpr int AV = (MT * 4 + GT - 1) / GT;          // runs of eight k that a thread stages per step
   extern __shared__ __attribute__((aligned(16))) float gs_lds[];
   int m0, n0, slice;
   if (!tile_of(a, m0, n0, slice)) return;
@@ -468,6 +471,8 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = wave / NWN, wn = wave % NWN, gt = threadIdx.x % GT;
   const int r = lane & 31, kg = lane >> 5;
+  // the v-th run of this thread among the tile's MT * 4; where the last ones do not reach all threads, the others repeat one
+  const auto run_of = [&](int v) { return gt + v * GT < MT * 4 ? gt + v * GT : gt + (v - 1) * GT; };
   u32x4* abuf = reinterpret_cast<u32x4*>(gs_lds) + grp * 2 * BUF;
   const int full = a.K >> 5;
   const int s0 = (int)((long)full * slice / a.S), s1 = (int)((long)full * (slice + 1) / a.S);
@@ -482,7 +487,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
   }
 #pragma unroll
   for (int v = 0; v < AV; ++v) {
-    const int row = (gt + v * GT) >> 2, c = gt & 3;
+    const int u = run_of(v), row = u >> 2, c = u & 3;
     xo[v] = 4 * ((m0 + row < a.M ? m0 + row : a.M - 1) * a.lda + c * 8);
     xl[v] = c * CH + row;
   }
@@ -496,7 +501,7 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
   static_assert(D % 2 == 0, "the buffer of a step is a constant of the unrolled loop");
   WRaw<R, I8, BLK> w[D][NB];
   f32x4 x[D][AV][2];
-  Split8 ws[2][2][NB];
+  Split8 ws[2][NB], xs[2][MB];  // of the two halves of a step
   const auto clamp_step = [&](int i) { const int t = s0 + i * KG + grp; return t < s1 ? t : s1 - 1; };
   const auto fetch_w = [&](int u, int i) {
     const int t = clamp_step(i);
@@ -523,25 +528,28 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
       d[8 * CH] = p.lo;
     }
   };
-  const auto convert = [&](int u, int c) {
+  const auto convert = [&](int u, int h) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int j = 0; j < NB; ++j) ws[c][s][j] = w[u][j].get(s, nn[j]);
+    for (int j = 0; j < NB; ++j) ws[h][j] = w[u][j].get(h, nn[j]);
   };
-  const auto multiply = [&](int buf, int c) {
-    Split8 xs[2][MB];
+  const auto read = [&](int buf, int h) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int i = 0; i < MB; ++i) {
+      const u32x4* p = abuf + buf * BUF + (2 * h + kg) * CH + i * R + r;
+      xs[h][i].hi = p[0];
+      xs[h][i].mid = p[4 * CH];
+      xs[h][i].lo = p[8 * CH];
+    }
+  };
+  constexpr int NMF = MB * NB * (I8 ? 3 : 6), VW = NB * (I8 ? 14 : 46), VA = AV * 48;  // matrix and vector instructions of half a step
+  const auto interleave = [&](auto vector) {
+    constexpr int NVAL = decltype(vector)::value / NMF + 1;
+    __builtin_amdgcn_sched_group_barrier(0x100, 3 * MB, 0);
 #pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        const u32x4* p = abuf + buf * BUF + (2 * s + kg) * CH + i * R + r;
-        xs[s][i].hi = p[0];
-        xs[s][i].mid = p[4 * CH];
-        xs[s][i].lo = p[8 * CH];
-      }
-#pragma unroll
-    for (int s = 0; s < 2; ++s) split_products<R, MB, NB, I8>(ws[c][s], xs[s], acc);
+    for (int m = 0; m < NMF; ++m) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, NVAL, 0);
+    }
   };
   if (rounds > 0) {
 #pragma unroll
@@ -552,36 +560,36 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
     stage(0, 0);
     fetch_x(0, D);
     convert(0, 0);
-    fetch_w(0, D);
     lds_barrier();
+    read(0, 0);
     for (int i = 0; i < rounds; i += D) {
 #pragma unroll
       for (int u = 0; u < D; ++u) {
         if (u > 0 && i + u >= rounds) break;
-        // the products of step i + u; between them, so that the vector units work while the matrix units do, the
-        // splitting of the next step's W and A
-        multiply(u & 1, u & 1);
-        convert((u + 1) % D, (u + 1) & 1);
+        // Half a step's products, between them the second half's operands and the splitting of the next step's A ..
+        read(u & 1, 1);
+        split_products<R, MB, NB, I8>(ws[0], xs[0], acc);
+        convert(u, 1);
         stage((u + 1) % D, (u + 1) & 1);
-        fetch_w((u + 1) % D, i + u + 1 + D);
+        fetch_w(u, i + u + D);
         fetch_x((u + 1) % D, i + u + 1 + D);
-        constexpr int NMF = MB * NB * 2 * (I8 ? 3 : 6), NVAL = (NB * 2 * (I8 ? 14 : 46) + AV * 48) / NMF + 1;
-        __builtin_amdgcn_sched_group_barrier(0x100, 3 * MB, 0);
-#pragma unroll
-        for (int m = 0; m < NMF; ++m) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, NVAL, 0);
-          if (m == 1) __builtin_amdgcn_sched_group_barrier(0x100, 3 * MB, 0);
-        }
+        interleave(std::integral_constant<int, VW + VA>());
         lds_barrier();
+        // .. the other half's, and the next step's first operands
+        read((u + 1) & 1, 0);
+        split_products<R, MB, NB, I8>(ws[1], xs[1], acc);
+        convert((u + 1) % D, 0);
+        interleave(std::integral_constant<int, VW>());
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
   if ((a.K & 31) && slice == a.S - 1) {  // the last, partial step: group 0
+    lds_barrier();
     if (grp == 0) {
 #pragma unroll
       for (int v = 0; v < AV; ++v) {
-        const int row = (gt + v * GT) >> 2, m = m0 + row < a.M ? m0 + row : a.M - 1;
+        const int u = run_of(v), row = u >> 2, m = m0 + row < a.M ? m0 + row : a.M - 1;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int k = full * 32 + (gt & 3) * 8 + 4 * h;
@@ -595,8 +603,12 @@ __global__ __launch_bounds__(NWN * KG * 64, OCC) void gemm_split_tile(SplitGemmA
     }
     lds_barrier();
     if (grp == 0) {
-      convert(0, 0);
-      multiply(0, 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        convert(0, h);
+        read(0, h);
+        split_products<R, MB, NB, I8>(ws[h], xs[h], acc);
+      }
     }
     lds_barrier();
   }
@@ -638,25 +650,27 @@ __global__ __launch_bounds__(256) void block_weights_i8(int K, int N, const sign
 // ---- launches ----
 // A launch takes about fixed + rounds * (one + more * (ceil(workgroups / 256) - 1)) us, where a workgroup needs
 // ceil(steps of its slice / kpar) rounds: a compute unit that gets a second workgroup determines the launch. The numbers
-// are least-squares fits to launches on MI355X (8 to 943 rows, 384 to 6400 columns, K from 384 to 6400, 1 to 8 slices):
-// 2700 of them for rows of W (6-13 % rms), 5700 for blocked W (8-19 %). The shape that they choose is within 1.4 % of the best
-// one (geometric mean; 2.9 % where K may be sliced).
+// are least-squares fits to launches on MI355X (8 to 1024 rows, 384 to 6400 columns, K from 384 to 6400, 1 to 8 slices; 39800 of
+// them, those within 1.5 or 2 times the best shape's time). The shape that they choose is within 1.0 to 1.7 % of the best one
+// (geometric mean). Zeros: a form of W for which the shape is not needed (without it the choice is no worse, or 0.1 %) or not built.
 struct Shape {
   int mtile, ntile, kpar;  // tile; steps of 32 k that a workgroup works on at a time
   struct Fit { float fixed, one, more; } f32, i8, f32_blk, i8_blk;
 };
 constexpr Shape SHAPES[] = {
-    {16, 16, 8, {2.78f, 0.77f, 0.92f}, {2.99f, 0.52f, 0.60f}, {3.37f, 0.57f, 0.74f}, {3.11f, 0.45f, 0.62f}},    // gemm_split_rows<16, 1, 1, 8>
-    {16, 32, 8, {3.11f, 0.90f, 1.31f}, {3.10f, 0.68f, 0.82f}, {3.51f, 0.71f, 0.98f}, {3.31f, 0.51f, 0.72f}},    // gemm_split_rows<16, 1, 2, 8>
-    {32, 32, 8, {3.09f, 1.27f, 1.75f}, {3.39f, 1.26f, 1.29f}, {3.46f, 1.07f, 1.55f}, {3.44f, 0.78f, 1.38f}},    // gemm_split_rows<32, 1, 1, 8>
-    {64, 64, 4, {4.56f, 1.45f, 2.06f}, {5.30f, 1.05f, 1.56f}, {4.63f, 1.38f, 1.82f}, {4.71f, 0.95f, 1.51f}},    // gemm_split_rows<32, 2, 2, 4>
-    {64, 64, 8, {4.58f, 2.58f, 4.77f}, {5.05f, 2.11f, 3.49f}, {4.35f, 2.39f, 4.31f}, {4.34f, 1.73f, 3.71f}},    // gemm_split_rows<32, 2, 2, 8>
-    {32, 64, 4, {4.70f, 1.03f, 2.41f}, {4.84f, 0.87f, 1.04f}, {4.64f, 0.88f, 1.16f}, {4.29f, 0.49f, 0.73f}},    // gemm_split_tile<1, 1, 2, 4>
-    {128, 128, 2, {7.97f, 2.00f, 4.69f}, {8.00f, 1.56f, 3.06f}, {7.74f, 2.27f, 3.73f}, {8.61f, 1.22f, 2.48f}},  // gemm_split_tile<4, 1, 4, 2>
-    {64, 128, 2, {0, 0, 0}, {0, 0, 0}, {5.36f, 1.24f, 2.09f}, {5.45f, 0.67f, 0.96f}},                         // gemm_split_tile<2, 1, 4, 2>
+    {16, 16, 8, {2.74f, 0.85f, 0.90f}, {3.61f, 0.50f, 0.53f}, {3.34f, 0.56f, 0.78f}, {3.62f, 0.39f, 0.57f}},  // gemm_split_rows<16, 1, 1, 8>
+    {16, 32, 8, {3.36f, 0.94f, 1.11f}, {3.58f, 0.70f, 0.87f}, {3.84f, 0.68f, 0.95f}, {3.68f, 0.47f, 0.70f}},  // gemm_split_rows<16, 1, 2, 8>
+    {32, 32, 8, {3.35f, 1.24f, 1.55f}, {3.68f, 1.14f, 1.26f}, {3.63f, 1.10f, 1.51f}, {3.83f, 0.73f, 1.27f}},  // gemm_split_rows<32, 1, 1, 8>
+    {64, 64, 4, {5.17f, 1.38f, 1.78f}, {5.53f, 1.10f, 1.47f}, {4.85f, 1.33f, 1.89f}, {0, 0, 0}},              // gemm_split_rows<32, 2, 2, 4>
+    {64, 64, 8, {4.72f, 2.68f, 3.90f}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}},                                      // gemm_split_rows<32, 2, 2, 8>
+    {32, 64, 4, {5.10f, 0.93f, 1.14f}, {5.50f, 0.72f, 0.90f}, {4.76f, 0.74f, 1.12f}, {4.74f, 0.39f, 0.70f}},  // gemm_split_tile<1, 1, 2, 4>
+    {128, 128, 2, {8.59f, 1.98f, 3.36f}, {10.50f, 1.40f, 2.32f}, {7.98f, 1.85f, 3.54f}, {0, 0, 0}},           // gemm_split_tile<4, 1, 4, 2>
+    {64, 128, 2, {0, 0, 0}, {0, 0, 0}, {5.95f, 1.05f, 1.98f}, {6.67f, 0.57f, 0.99f}},                         // gemm_split_tile<2, 1, 4, 2>
+    {96, 128, 2, {0, 0, 0}, {0, 0, 0}, {6.96f, 1.57f, 2.82f}, {0, 0, 0}},                                     // gemm_split_tile<3, 1, 4, 2>
 };
 constexpr int NSHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
-constexpr int NSHAPES_ROWS = NSHAPES - 1;  // with rows of W the last one is never the best
+constexpr const Shape::Fit& fit_of(const Shape& sh, bool i8, bool blocked) { return blocked ? (i8 ? sh.i8_blk : sh.f32_blk) : i8 ? sh.i8 : sh.f32; }
+constexpr bool built(int kind, bool i8, bool blocked) { return fit_of(SHAPES[kind], i8, blocked).fixed > 0; }
 
 constexpr size_t rows_lds(int R, int MB, int NB, int NW) { return (size_t)NW * MB * NB * R * R * sizeof(float); }
 constexpr size_t tile_lds(int MB, int NB, int NWN, int KG) {
@@ -682,12 +696,22 @@ hipError_t launch_shape(int kind, const SplitGemmArgs& a, hipStream_t s) {
     case 0: return launch_kernel(gemm_split_rows<16, 1, 1, 8, I8, BLK>, a, 512, rows_lds(16, 1, 1, 8), s);
     case 1: return launch_kernel(gemm_split_rows<16, 1, 2, 8, I8, BLK>, a, 512, rows_lds(16, 1, 2, 8), s);
     case 2: return launch_kernel(gemm_split_rows<32, 1, 1, 8, I8, BLK>, a, 512, rows_lds(32, 1, 1, 8), s);
-    case 3: return launch_kernel(gemm_split_rows<32, 2, 2, 4, I8, BLK>, a, 256, rows_lds(32, 2, 2, 4), s);
-    case 4: return launch_kernel(gemm_split_rows<32, 2, 2, 8, I8, BLK>, a, 512, rows_lds(32, 2, 2, 8), s);
+    case 3:
+      if constexpr (built(3, I8, BLK)) return launch_kernel(gemm_split_rows<32, 2, 2, 4, I8, BLK>, a, 256, rows_lds(32, 2, 2, 4), s);
+      break;
+    case 4:
+      if constexpr (built(4, I8, BLK)) return launch_kernel(gemm_split_rows<32, 2, 2, 8, I8, BLK>, a, 512, rows_lds(32, 2, 2, 8), s);
+      break;
     case 5: return launch_kernel(gemm_split_tile<1, 1, 2, 4, I8, BLK, 2, 2>, a, 512, tile_lds(1, 1, 2, 4), s);
-    case 6: return launch_kernel(gemm_split_tile<4, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(4, 1, 4, 2), s);
+    case 6:
+      if constexpr (built(6, I8, BLK)) return launch_kernel(gemm_split_tile<4, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(4, 1, 4, 2), s);
+      break;
     case 7:
-      if constexpr (BLK) return launch_kernel(gemm_split_tile<2, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(2, 1, 4, 2), s);
+      if constexpr (built(7, I8, BLK)) return launch_kernel(gemm_split_tile<2, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(2, 1, 4, 2), s);
+      break;
+    case 8:
+      if constexpr (built(8, I8, BLK)) return launch_kernel(gemm_split_tile<3, 1, 4, 2, I8, BLK, 2, 2>, a, 512, tile_lds(3, 1, 4, 2), s);
+      break;
   }
   return hipErrorInvalidValue;
 }
@@ -698,9 +722,10 @@ SplitPlan plan_gemm_split(int M, int N, int K, bool i8, bool blocked, bool with_
   SplitPlan best = {0, 1};
   double best_t = 1e30;
   const int steps = (K + 31) / 32;
-  for (int c = 0; c < (blocked ? NSHAPES : NSHAPES_ROWS); ++c) {
+  for (int c = 0; c < NSHAPES; ++c) {
     const Shape& sh = SHAPES[c];
-    const Shape::Fit& f = blocked ? (i8 ? sh.i8_blk : sh.f32_blk) : i8 ? sh.i8 : sh.f32;
+    const Shape::Fit& f = fit_of(sh, i8, blocked);
+    if (!built(c, i8, blocked)) continue;
     const double tiles = (double)((M + sh.mtile - 1) / sh.mtile) * ((N + sh.ntile - 1) / sh.ntile);
     for (int S = 1; S <= (may_slice ? 8 : 1); ++S) {
       if (S > 1 && steps < 4 * S) break;
