@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import ref
-from webgpt_amd import _lib, synth
+from webgpt_amd import _lib, blocks, synth
 from webgpt_amd.model import GPT
 
 from helpers import close, make_model, oracle_weights, small_cfg, worst
@@ -44,6 +44,27 @@ def test_prompts_against_oracle(device, dtype, d, n_head):
         rows, exp = gpt.tap("residual", T), taps[ref.tap_names(2).index("block1_r2")]
         assert close(rows, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T
     gpt.unloadBuffers()
+
+
+def test_memory_as_it_was_left(device):
+    """A model in memory full of NaN: rows of the last row group beyond the prompt hold nothing that ends the launch early, so the
+    logits are those of the same model in other memory, bit for bit (launches round in another order)."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=256, n_ctx=64, vocab_size=301, dtype="int8")
+    tensors, tokens = make_model(cfg, 5), synth.tokens(13, "left", 0, cfg["vocab_size"])
+
+    def run():
+        gpt = load(cfg, tensors)
+        got = [gpt.prefill(tokens[:T]) for T in (13, 16, 1)]
+        gpt.unloadBuffers()
+        return got
+
+    want = run()
+    nan = np.full(8 << 20, np.nan, np.float32)
+    junk = [blocks.init_tensor(nan, [nan.size]) for _ in range(16)]  # (twice what the library keeps of freed buffers)
+    for b in junk:
+        b.destroy()
+    for a, b in zip(want, run()):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("dtype", ["f32", "int8"])

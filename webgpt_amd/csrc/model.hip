@@ -621,6 +621,8 @@ static int setup_prefill(Model* m) {
   PrefillArgs& a = m->pp;
   WGPT_HIP(hipMemcpyAsync((void*)a.layers, layers.data(), sizeof(PrefillLayer) * (size_t)m->L, hipMemcpyHostToDevice, rt().stream));
   WGPT_HIP(hipMemsetAsync(a.flags, 0, PP_FLAGS * sizeof(unsigned), rt().stream));
+  // (rows of the last row group beyond the prompt are multiplied too: what memory holds by chance would count as spoilt sums)
+  WGPT_HIP(hipMemsetAsync(a.q, 0, prefill_exchange_floats(m->pp_rows, m->d) * sizeof(float), rt().stream));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   a.L = m->L; a.H = m->H; a.hs = m->hs; a.d = m->d; a.ctx = m->ctx; a.V = m->V;
   a.scale = (float)(1.0 / std::sqrt((double)m->hs));
