@@ -50,7 +50,7 @@ def test_memory_as_it_was_left(device):
     """A model in memory full of NaN: rows of the last row group beyond the prompt hold nothing that ends the launch early, so the
     logits are those of the same model in other memory, bit for bit (launches round in another order)."""
     cfg = small_cfg(n_layer=2, n_head=4, n_embd=256, n_ctx=64, vocab_size=301, dtype="int8")
-    tensors, tokens = make_model(cfg, 5), synth.tokens(13, "left", 0, cfg["vocab_size"])
+    tensors, tokens = make_model(cfg, 5), synth.tokens(5, "prompt", 16, cfg["vocab_size"])
 
     def run():
         gpt = load(cfg, tensors)
