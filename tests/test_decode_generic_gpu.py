@@ -72,6 +72,32 @@ def test_the_longest_contexts(device, n_head, n_embd, n_ctx):
     gpt.unloadBuffers()
 
 
+# vocabularies: fewer rows than workgroups, one row and some two, more than the 256 of a workgroup that registers hold
+@pytest.mark.parametrize("vocab_size,repeat", [(5, 5), (301, 301), (301, 7), (5003, 5003), (70001, 70001), (70001, 3)])
+def test_sampled_steps_select_what_the_oracle_selects(device, vocab_size, repeat):
+    """Ids of sampled calls against the oracle's selection from the logits of single steps, whose arithmetic is the same; with a
+    table of a few different rows the candidates are ties within and between workgroups, which the lowest index wins."""
+    cfg = small_cfg(n_layer=1, n_head=2, n_embd=72, n_ctx=64, vocab_size=vocab_size)
+    tensors = make_model(cfg, 2)
+    wte = tensors["transformer.wte.weight"]
+    tensors["transformer.wte.weight"] = np.ascontiguousarray(wte[np.arange(vocab_size) % repeat])
+    gpt = load(cfg, tensors)
+    gpt.set_decode_mode(1)
+    tokens = synth.tokens(4, "prompt", 9, vocab_size)
+    rng = np.random.default_rng(3)
+    for top_k in (2, 3, 4, 5, 8):
+        for steps in (1, 11):  # draws that travel with the launch, and in device memory
+            u = rng.random(steps)
+            gpt.prefill(tokens[:8])
+            got = gpt.decode_sample(int(tokens[8]), steps, top_k, 0.8, u)
+            gpt.prefill(tokens[:8])
+            token = int(tokens[8])
+            for i in range(steps):
+                token = ref.sample_topk(gpt.decode(token), min(top_k, vocab_size), 0.8, float(u[i]))[0]
+                assert token == got[i], (top_k, steps, i)
+    gpt.unloadBuffers()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "int8"])
 def test_expired_wait_repeats_the_call_with_launches(device, monkeypatch, dtype):
     """Waits that give up at their first look (forced from the host; every kernel drains): the calls succeed with the results of a

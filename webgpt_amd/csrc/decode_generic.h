@@ -10,7 +10,7 @@ constexpr int DG_SPLIT = 8;  // most slices of the context per head
 
 // Shapes that launch_decode_generic takes.
 bool decode_generic_supports(int d, int H, int hs, int ctx, int V, int compute_units);
-// a.nsteps greedy steps; a.top_k, a.u and a.colparams are not used. Epochs as persistent_epochs_per_step says.
+// a.nsteps steps, greedy or sampled as a.top_k says; a.colparams is not used. Epochs as persistent_epochs_per_step says.
 hipError_t launch_decode_generic(const PersistentArgs& a, hipStream_t s);
 
 }  // namespace wgpt

@@ -14,7 +14,10 @@
 //   - attention: a workgroup per (head, slice of the context); the slices are merged by the waves of the projection;
 //   - rows pass between workgroups as {value, epoch} words, written and polled at device scope; a word validates itself;
 //   - weights of a phase, keys and values are requested before the wait in front of it;
-//   - at the end of a step every workgroup finds the arg-max of all workgroups' candidates, so a step needs no broadcast.
+//   - at the end of a step every workgroup finds the arg-max of all workgroups' candidates, so a step needs no broadcast. With
+//     top_k up to PD_TOPK a workgroup's candidates are its top_k first logits and every wave samples from the first of all (us per
+//     token at top_k 2 and 8, before with a launch and a selection for each: 4 x 576 of 5003 tokens 77 -> 61.5 and 67, 3 x 64
+//     57 -> 44.5 and 52, 6 x 1280 of 50257 210 -> 191.5 and 196). Above eight the words would outgrow a poll of four a thread.
 //
 // No word is overwritten while somebody may still wait for its epoch: an exchange is written again only by a workgroup that has
 // seen, through the exchanges between, the results of everyone who reads it. The candidates, which workgroups without
@@ -27,6 +30,7 @@
 #include <type_traits>
 
 #include "persistent_common.h"
+#include "select_key.h"
 
 namespace wgpt {
 namespace {
@@ -98,6 +102,38 @@ __device__ __forceinline__ float across_keys(float v, int lpk, Op op) {
 }
 __device__ __forceinline__ float dot4(const f32x4& a, const f32x4& b) { return (a[0] * b[0] + a[1] * b[1]) + (a[2] * b[2] + a[3] * b[3]); }
 
+template <int CTRL, int ROWS>
+__device__ __forceinline__ sel_key dpp_first(sel_key v) {  // (lanes without a source get 0, which is no key)
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROWS, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, ROWS, 0xf, false);
+  const sel_key o = (sel_key)hi << 32 | lo;
+  return o > v ? o : v;
+}
+// The first key of the wave, wave-uniform; 0: none.
+__device__ __forceinline__ sel_key wave_first(sel_key v) {
+  v = dpp_first<0x111, 0xf>(v);
+  v = dpp_first<0x112, 0xf>(v);
+  v = dpp_first<0x114, 0xf>(v);
+  v = dpp_first<0x118, 0xf>(v);
+  v = dpp_first<0x142, 0xa>(v);
+  v = dpp_first<0x143, 0xc>(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)v, 63), hi = __builtin_amdgcn_readlane((int)(unsigned)(v >> 32), 63);
+  return (sel_key)hi << 32 | lo;
+}
+// The k first of the wave's keys, N a lane, in order: lane r has the r-th, the others 0.
+template <int N>
+__device__ __forceinline__ sel_key wave_firsts(const sel_key (&keys)[N], int k, int lane) {
+  sel_key mine = 0, last = ~(sel_key)0;
+  for (int r = 0; r < k; ++r) {
+    sel_key best = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) best = keys[i] < last && keys[i] > best ? keys[i] : best;
+    last = wave_first(best);
+    if (lane == r) mine = last;
+  }
+  return mine;
+}
+
 // Four consecutive k of one column.
 template <bool I8>
 struct Weight {
@@ -162,8 +198,8 @@ __device__ __forceinline__ void nap(int units) {  // about 64 clocks each
   for (int i = 0; i < units; ++i) __builtin_amdgcn_s_sleep(1);
 }
 
-// NS: segments of a row. R: key rows of a lane, 8 for heads of more than 64.
-template <bool I8, int NS, int R>
+// NS: segments of a row. R: key rows of a lane, 8 for heads of more than 64. SAMPLE: tokens are sampled from the top_k first logits.
+template <bool I8, int NS, int R, bool SAMPLE>
 __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
   constexpr int CWA = (3 * NS + NW - 1) / NW, CWD = (4 * NS + NW - 1) / NW;  // columns of a wave, segments of a wave of the 4d-long row
   constexpr int PW = Weight<I8>::BYTES;
@@ -173,6 +209,7 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
   __shared__ float out[4 * NS];
   __shared__ float best_v[NW];
   __shared__ int best_i[NW], bail;
+  __shared__ sel_key firsts[NW * PD_TOPK];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wg = blockIdx.x;
   ConstArgs* const a0 = fresh_args();
   const int d = a0->d, H = a0->H, hs = d / H, L = a0->L, V = a0->V;
@@ -576,14 +613,44 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
 #pragma unroll
         for (int i = 0; i < RV; ++i)
           if (v + i < v1) {
-            if (besti == 0x7fffffff || z[i] > best) best = z[i], besti = v + i;
-            if (ends && lane == 0) run[v + i - v0] = z[i];
+            if (!SAMPLE && (besti == 0x7fffffff || z[i] > best)) best = z[i], besti = v + i;
+            if ((SAMPLE || ends) && lane == 0) run[v + i - v0] = z[i];
           }
       }
-      if (lane == 0) best_v[wave] = best, best_i[wave] = besti;
+      if (!SAMPLE && lane == 0) best_v[wave] = best, best_i[wave] = besti;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the step's keys and values are where others read them)
       __syncthreads();
-      if (tid == 0) {
+      if constexpr (SAMPLE) {
+        if (wave == 0) {
+          const int k = fresh_args()->top_k, n = v1 - v0;
+          sel_key mine = 0;
+          if (n <= 256) {
+            sel_key keys[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int j = lane + 64 * i;
+              keys[i] = j < n ? make_key(run[j], v0 + j) : 0;
+            }
+            mine = wave_firsts(keys, k, lane);
+          } else {
+            sel_key last = ~(sel_key)0;
+            for (int r = 0; r < k; ++r) {
+              sel_key best = 0;
+              for (int j = lane; j < n; j += 64) {
+                const sel_key key = make_key(run[j], v0 + j);
+                best = key < last && key > best ? key : best;
+              }
+              last = wave_first(best);
+              if (lane == r) mine = last;
+            }
+          }
+          if (lane < k) {  // the r-th of all workgroups side by side
+            const u32x4 pk = {(unsigned)mine, ep + 1, (unsigned)(mine >> 32), ep + 1};
+            u64* to = fresh_args()->bufAM + 2 * (size_t)G * (PD_TOPK * (step & 1) + lane) + 2 * wg;
+            asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(to), "v"(pk) : "memory");
+          }
+        }
+      } else if (tid == 0) {
         for (int u = 1; u < NW; ++u) {
           const float v = best_v[u];
           const int i = best_i[u];
@@ -601,33 +668,77 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
       if (ends && wg) return;
     }
     if (!ends) request_A(0);
-    // ---- the arg-max of all workgroups (lowest index of equal ones) ----
-    if (wave < G / 64) {
+    if constexpr (SAMPLE) {
+      // ---- the top_k first of all workgroups' candidates, cpuSoftmax in float64 and sampleFromDistribution (globals.js:47-74) ----
+      const int k = fresh_args()->top_k;
+      const double rnd = fresh_args()->u ? fresh_args()->u[step] : fresh_args()->u_arg[step];
       nap(fresh_args()->delay[6]);
-      int off[1] = {16 * opaque(tid)};
-      u32x4 v[1];
-      wt.words(buffer_of(fresh_args()->bufAM + 2 * (size_t)G * (step & 1), 16 * (size_t)G), off, v, ep + 1);
-      float best = __uint_as_float(v[0][0]);
-      int besti = (int)v[0][2];
+      const auto gather = [&](auto per_thread) {
+        constexpr int N = decltype(per_thread)::value;
+        int off[N];
+        u32x4 v[N];
+        sel_key keys[N];
+        const int t = opaque(tid);
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(best, o);
-        const int oi = __shfl_xor(besti, o);
-        if (oi != 0x7fffffff && (besti == 0x7fffffff || ov > best || (ov == best && oi < besti))) best = ov, besti = oi;
+        for (int i = 0; i < N; ++i) off[i] = 16 * (t + NT * i < G * k ? t + NT * i : t);
+        wt.words(buffer_of(fresh_args()->bufAM + 2 * (size_t)G * PD_TOPK * (step & 1), 16 * (size_t)G * PD_TOPK), off, v, ep + 1);
+#pragma unroll
+        for (int i = 0; i < N; ++i) keys[i] = t + NT * i < G * k ? (sel_key)v[i][2] << 32 | v[i][0] : 0;
+        const sel_key mine = wave_firsts(keys, k, lane);
+        if (lane < PD_TOPK) firsts[wave * PD_TOPK + lane] = mine;
+      };
+      if (k <= 2) gather(Count<1>());
+      else if (k <= 4) gather(Count<2>());
+      else gather(Count<4>());
+      __syncthreads();
+      if (bail) return;
+      static_assert(NW * PD_TOPK == 64 && 4 * NT == PD_TOPK * G, "a key per lane, four words a thread");
+      const sel_key all[1] = {firsts[lane]};
+      const sel_key mine = wave_firsts(all, k, lane);
+      // lane r: the r-th; sums in the reference's order on every lane
+      const unsigned first = __builtin_amdgcn_readfirstlane((unsigned)(mine >> 32));
+      const double mx = (double)key_value((sel_key)first << 32);
+      const double e = exp(((double)key_value(mine) - mx) / fresh_args()->temperature);
+      double sum = 0.0;
+      for (int r = 0; r < k; ++r) sum += wave_read(e, r);
+      const double p = e / sum;
+      double cum = 0.0;
+      int pick = -1;
+      for (int r = 0; r < k && pick < 0; ++r) {
+        cum += wave_read(p, r);
+        if (rnd < cum) pick = r;
       }
-      if (lane == 0) best_v[wave] = best, best_i[wave] = besti;
-    }
-    __syncthreads();
-    if (bail) return;
-    {
-      float best = best_v[0];
-      int besti = best_i[0];
-      for (int u = 1; u < G / 64; ++u) {
-        const float v = best_v[u];
-        const int i = best_i[u];
-        if (i != 0x7fffffff && (besti == 0x7fffffff || v > best || (v == best && i < besti))) best = v, besti = i;
+      tok = __builtin_amdgcn_readfirstlane(__shfl(key_index(mine), pick < 0 ? k - 1 : pick));
+      tok = tok >= 0 && tok < V ? tok : 0;
+    } else {
+      // ---- the arg-max of all workgroups (lowest index of equal ones) ----
+      if (wave < G / 64) {
+        nap(fresh_args()->delay[6]);
+        int off[1] = {16 * opaque(tid)};
+        u32x4 v[1];
+        wt.words(buffer_of(fresh_args()->bufAM + 2 * (size_t)G * (step & 1), 16 * (size_t)G), off, v, ep + 1);
+        float best = __uint_as_float(v[0][0]);
+        int besti = (int)v[0][2];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+          const float ov = __shfl_xor(best, o);
+          const int oi = __shfl_xor(besti, o);
+          if (oi != 0x7fffffff && (besti == 0x7fffffff || ov > best || (ov == best && oi < besti))) best = ov, besti = oi;
+        }
+        if (lane == 0) best_v[wave] = best, best_i[wave] = besti;
       }
-      tok = __builtin_amdgcn_readfirstlane(besti < V ? besti : 0);
+      __syncthreads();
+      if (bail) return;
+      {
+        float best = best_v[0];
+        int besti = best_i[0];
+        for (int u = 1; u < G / 64; ++u) {
+          const float v = best_v[u];
+          const int i = best_i[u];
+          if (i != 0x7fffffff && (besti == 0x7fffffff || v > best || (v == best && i < besti))) best = v, besti = i;
+        }
+        tok = __builtin_amdgcn_readfirstlane(besti < V ? besti : 0);
+      }
     }
     ep += 1;
     if (wg == 0 && tid == 0) {
@@ -643,20 +754,21 @@ constexpr size_t MAX_LDS = 128 * 1024;
 
 size_t run_bytes(int V) { const size_t n = 4 * (size_t)((V + G - 1) / G); return n > RUN_LDS ? n : RUN_LDS; }
 
-template <bool I8, int NS, int R>
+template <bool I8, int NS, int R, bool SAMPLE>
 hipError_t launch_r(const PersistentArgs& a, hipStream_t s) {
   static bool enabled = false;  // dynamic LDS size already raised
   if (!enabled) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(decode_generic_kernel<I8, NS, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(decode_generic_kernel<I8, NS, R, SAMPLE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
     if (e != hipSuccess) return e;
     enabled = true;
   }
-  decode_generic_kernel<I8, NS, R><<<G, NT, run_bytes(a.V), s>>>(a);
+  decode_generic_kernel<I8, NS, R, SAMPLE><<<G, NT, run_bytes(a.V), s>>>(a);
   return hipGetLastError();
 }
 template <bool I8, int NS>
 hipError_t launch_ns(const PersistentArgs& a, hipStream_t s) {
-  return a.d / a.H <= 64 ? launch_r<I8, NS, 4>(a, s) : launch_r<I8, NS, 8>(a, s);
+  if (a.top_k > 1) return a.d / a.H <= 64 ? launch_r<I8, NS, 4, true>(a, s) : launch_r<I8, NS, 8, true>(a, s);
+  return a.d / a.H <= 64 ? launch_r<I8, NS, 4, false>(a, s) : launch_r<I8, NS, 8, false>(a, s);
 }
 template <bool I8>
 hipError_t launch_any(const PersistentArgs& a, hipStream_t s) {
@@ -678,7 +790,7 @@ bool decode_generic_supports(int d, int H, int hs, int ctx, int V, int compute_u
 }
 
 hipError_t launch_decode_generic(const PersistentArgs& a, hipStream_t s) {
-  if (!decode_generic_supports(a.d, a.H, a.d / a.H, a.ctx, a.V, G) || a.nsteps < 1 || a.pos0 + a.nsteps > a.ctx) return hipErrorInvalidValue;
+  if (!decode_generic_supports(a.d, a.H, a.d / a.H, a.ctx, a.V, G) || a.nsteps < 1 || a.top_k < 1 || a.top_k > PD_TOPK || a.top_k > a.V || a.pos0 + a.nsteps > a.ctx) return hipErrorInvalidValue;
   return a.weight_dtype == 1 ? launch_any<true>(a, s) : launch_any<false>(a, s);
 }
 

@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "gemm_split.h"
+#include "select_key.h"
 
 namespace wgpt {
 
@@ -1315,26 +1316,6 @@ __global__ __launch_bounds__(WG) void vocab_gemv_ln_kernel(int V, int d, const f
 //     u is the caller's uniform draw in [0, 1) (the reference's Math.random()).
 // The chosen id goes to tok[0] (input of the next decode step) and out[slot]; ids/probs
 // (optional) receive the k selected indices and their probabilities.
-// A logit and its index as one number whose order is the selection's: larger value first, lower index among equals
-// (-0 and 0 are equal; NaN comes last).
-typedef unsigned long long sel_key;
-__device__ __forceinline__ unsigned order_bits(float v) {
-  const unsigned b = __float_as_uint(v + 0.0f);
-  return v != v ? 0u : (b & 0x80000000u ? ~b : b | 0x80000000u);
-}
-__device__ __forceinline__ sel_key make_key(float v, int i) { return (sel_key)order_bits(v) << 32 | (0xffffffffu - (unsigned)i); }
-__device__ __forceinline__ float key_value(sel_key k) {
-  const unsigned b = (unsigned)(k >> 32);
-  return b == 0u ? NAN : __uint_as_float(b & 0x80000000u ? b & 0x7fffffffu : ~b);
-}
-__device__ __forceinline__ int key_index(sel_key k) { return (int)(0xffffffffu - (unsigned)k); }
-
-// x[lane] of the wave, lane uniform
-__device__ __forceinline__ double wave_read(double x, int lane) {
-  const unsigned long long b = __double_as_longlong(x);
-  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
-  return __longlong_as_double((unsigned long long)hi << 32 | lo);
-}
 
 // One workgroup. A bound below which the k largest logits cannot lie is the k-th largest of the threads' maxima, or a little
 // less; the logits not below it are k candidates or some more (normal logits, V = 50257, k = 40: about 60), and only they are

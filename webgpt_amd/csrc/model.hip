@@ -284,6 +284,9 @@ static unsigned spin_limit() {
   return 1u << 18;
 }
 
+// Words of PersistentArgs::bufAM: the kernel of any shape has two sets of candidates in turn.
+static size_t candidate_words(const Model* m) { return (size_t)(m->generic ? 4 : 2) * PD_TOPK * PD_GRID; }
+
 // Prepares the decode paths: slab-layout copies of the linear weights and the per-layer parameter blocks
 // (any shape), then, for the shapes the persistent whole-token kernel is built for, its per-workgroup
 // parameter blocks and exchange buffers. Leaves m->persist_ok false (and the per-block path in charge) for
@@ -368,7 +371,7 @@ static int setup_persistent(Model* m) {
   a.colparams = colparams;
   a.wte = m->wte; a.wpe = m->wpe; a.lnf_g = m->lnf_g; a.lnf_b = m->lnf_b;
   a.kv = m->kv;
-  const size_t words = (size_t)3 * d + attw + d + hid + d + 2 * PD_TOPK * G;
+  const size_t words = (size_t)3 * d + attw + d + hid + d + candidate_words(m);
   unsigned long long* buf;
   if ((rc = dev_alloc(m, words * sizeof(unsigned long long), (void**)&buf))) return rc;
   WGPT_HIP(hipMemsetAsync(buf, 0, words * sizeof(unsigned long long), rt().stream));
@@ -474,7 +477,7 @@ static int decode_persistent(Model* m, int steps, int top_k = 1, double temperat
   if (m->epoch > 0x7fffffffu - per_step * (unsigned)steps - 8u) {
     // epoch counter about to leave the positive ints (the kernel's error word is the epoch of the wait that
     // expired, as an int; negative values are its other codes): start over from clean exchange buffers
-    const size_t words = (size_t)(a.bufAM + 2 * PD_TOPK * PD_GRID - a.bufQKV);
+    const size_t words = (size_t)(a.bufAM + candidate_words(m) - a.bufQKV);
     WGPT_HIP(hipMemsetAsync(a.bufQKV, 0, words * sizeof(unsigned long long), rt().stream));
     m->epoch = 0;
   }
@@ -931,8 +934,8 @@ int wgpt_decode_sample(wgpt_model h, int32_t token, int steps, int top_k, double
     return fail(WGPT_ERR_STATE, "wgpt_decode_sample: %d steps from position %d exceed the context of %d", steps, m->pos, m->ctx);
   const bool persistent = m->decode_mode == 1;
   const int k = top_k < m->V ? top_k : m->V;
-  // up to PD_TOPK candidates the persistent kernel selects and samples itself, all steps in one launch (that of any shape one)
-  const bool in_kernel = persistent && k <= (m->generic ? 1 : PD_TOPK);
+  // up to PD_TOPK candidates the persistent kernel selects and samples itself, all steps in one launch
+  const bool in_kernel = persistent && k <= PD_TOPK;
   if (!in_kernel) {  // (that launch brings the token and the draws along)
     m->pin[0] = token;  // every earlier use of the pinned words has completed: each call ends with a synchronisation
     memcpy(m->u_pin, u, sizeof(double) * (size_t)steps);
