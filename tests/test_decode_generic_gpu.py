@@ -121,3 +121,21 @@ def test_expired_wait_repeats_the_call_with_launches(device, monkeypatch, dtype)
             gpt.set_decode_mode(1)
         gpt.unloadBuffers()
     launches.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_rows_whose_variance_overflows(device, dtype):
+    """Finite residual values of 1e28: a row's variance is infinite, its quotients are zeros and the LayerNorm's result is beta."""
+    cfg = small_cfg(n_layer=2, n_head=5, n_embd=200, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    tensors["transformer.wpe.weight"] = tensors["transformer.wpe.weight"] * np.float32(1e30)
+    gpt = load(cfg, tensors)
+    gpt.set_decode_mode(1)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    tokens = synth.tokens(5, "prompt", 20, cfg["vocab_size"])
+    with np.errstate(all="ignore"):
+        gpt.prefill(tokens[:17])
+        for i in range(17, 20):
+            got, want = gpt.decode(int(tokens[i])), ref.forward(p, w, tokens[:i + 1])
+            assert np.isfinite(want).all() and close(got, want), i
+    gpt.unloadBuffers()

@@ -123,3 +123,21 @@ def test_values_that_are_not_finite(device, dtype, what):
         assert close(got[ok], want[ok])
     gpt.unloadBuffers()
     launches.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("name", ["wpe.weight", "h.1.attn.c_proj.bias", "h.1.mlp.c_proj.bias"])
+def test_rows_whose_variance_overflows(device, dtype, name):
+    """Finite residual values of 1e28 from the first, the last and the final LayerNorm on: a row's variance is infinite, its quotients
+    are zeros and the LayerNorm's result is beta."""
+    cfg = small_cfg(n_layer=2, n_head=5, n_embd=200, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    tensors["transformer." + name] = tensors["transformer." + name] * np.float32(1e30)
+    gpt = load(cfg, tensors)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (1, 20, 64):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        with np.errstate(all="ignore"):
+            got, want = gpt.prefill(tokens), ref.forward(p, w, tokens)
+        assert np.isfinite(want).all() and close(got, want), T
+    gpt.unloadBuffers()

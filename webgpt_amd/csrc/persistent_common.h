@@ -60,10 +60,12 @@ __device__ __forceinline__ float gelu_ref(float x) {  // instructions.js:718-727
   r = x > 10.0f ? x : r;
   return r;
 }
-// x / s with r = 1 / s at hand, rounded once (but for results under the smallest normal number)
+// x / s with r = 1 / s at hand, rounded once (but for results under the smallest normal number), x finite. s infinite: 0, as the
+// division gives it (the standard deviation of values from about 2^64 on; with r = 0 the finite number in its place changes nothing,
+// where 0 * s would be no number).
 __device__ __forceinline__ float quotient(float x, float s, float r) {
   const float q = x * r;
-  return __builtin_fmaf(__builtin_fmaf(-q, s, x), r, q);
+  return __builtin_fmaf(__builtin_fmaf(-q, fminf(s, 3.402823466e+38f), x), r, q);
 }
 
 // v, opaque to the optimiser: addresses built on the result are not kept in registers from one phase to the next.

@@ -314,9 +314,9 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
     for (int v = 0; v < NW; ++v) {
       const float2 c = cnt[v];
       const float e = p[v].x * c.y - mean;
-      m2 += p[v].y + c.x * (e * e);
+      m2 += p[v].y + (c.x * e) * e;  // (0 for a wave without elements, also where e * e overflows)
     }
-    const float stdev = sqrtf(quotient(m2, fd, rd) + 1e-5f), rstd = 1.0f / stdev;
+    const float stdev = sqrtf(m2 / fd + 1e-5f), rstd = 1.0f / stdev;  // (m2 may be infinite)
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const int k8 = (s1 + s) * 4 + kg;
