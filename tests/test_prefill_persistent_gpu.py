@@ -8,7 +8,7 @@ from oracle import ref
 from webgpt_amd import _lib, blocks, synth
 from webgpt_amd.model import GPT
 
-from helpers import close, make_model, oracle_weights, small_cfg, worst
+from helpers import close, make_model, oracle_weights, pack_words, small_cfg, worst
 
 pytestmark = pytest.mark.gpu
 
@@ -140,4 +140,42 @@ def test_rows_whose_variance_overflows(device, dtype, name):
         with np.errstate(all="ignore"):
             got, want = gpt.prefill(tokens), ref.forward(p, w, tokens)
         assert np.isfinite(want).all() and close(got, want), T
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("n_head", [1, 4])
+def test_sixteen_keys_whose_scores_overflow(device, dtype, n_head):
+    """Scores of minus infinity for all keys of the first row group, whose weights are then zero, and finite ones for all others:
+    a LayerNorm that passes the sign of the first sixteen rows' first element and zeros for the others, keys that are 1e20 of it."""
+    d, T = 64, 40
+    cfg = small_cfg(n_layer=1, n_head=n_head, n_embd=d, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    wte, wpe = np.zeros((90, d), np.float32), np.zeros((64, d), np.float32)
+    wte[:, 3] = np.arange(90)  # (token 0, which the prompt repeats, has no embedding)
+    wpe[:16, 0], wpe[:16, 1] = 1, -1
+    tensors.update({"transformer.wte.weight": wte, "transformer.wpe.weight": wpe, "transformer.h.0.ln_1.bias": np.zeros(d, np.float32)})
+    bias = tensors["transformer.h.0.attn.c_attn.bias"].copy()
+    bias[:d], bias[d:2 * d] = -1e20, 0
+    tensors["transformer.h.0.attn.c_attn.bias"] = bias
+    name = "transformer.h.0.attn.c_attn.weight"
+    if dtype == "f32":
+        W = tensors[name].copy()
+        W[:, :2 * d] = 0
+        W[0, d:2 * d] = 1e20
+        tensors[name] = W
+    else:
+        q = np.random.default_rng(3).integers(-127, 128, (d, 3 * d)).astype(np.int8)
+        q[:, :2 * d] = 0
+        q[0, d:2 * d] = 127
+        tensors[name + ".q"] = pack_words(q)
+        scale = tensors[name + ".scale"].copy()
+        scale[d:2 * d] = 1e20
+        tensors[name + ".scale"] = scale
+    gpt = load(cfg, tensors)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    tokens = np.zeros(T, np.int32)
+    with np.errstate(all="ignore"):
+        got, want = gpt.prefill(tokens), ref.forward(p, w, tokens)
+    assert np.isfinite(want).all() and close(got, want), worst(got, want)
     gpt.unloadBuffers()

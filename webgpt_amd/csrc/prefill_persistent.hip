@@ -498,9 +498,10 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
               m = fmaxf(m, p[e]);
             }
             m = quad_max(m);
+            const float base = m == -INFINITY ? 0.f : m;  // (scores of -inf only: weights of 0, which other waves' keys outweigh)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              p[e] = wave * PP_ROWS + 4 * kg + e <= row ? expf(p[e] - m) : 0.f;
+              p[e] = wave * PP_ROWS + 4 * kg + e <= row ? expf(p[e] - base) : 0.f;
               l += p[e];
             }
             l = quad_sum(l);
