@@ -139,3 +139,21 @@ def test_rows_whose_variance_overflows(device, dtype):
             got, want = gpt.decode(int(tokens[i])), ref.forward(p, w, tokens[:i + 1])
             assert np.isfinite(want).all() and close(got, want), i
     gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_rows_of_one_huge_value(device, dtype):
+    """All elements of a row 2^120: its LayerNorm is beta, at a width that leaves lanes without elements, whose zeros are 2^128 standard
+    deviations from the mean."""
+    cfg = small_cfg(n_layer=2, n_head=2, n_embd=40, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    tensors["transformer.wpe.weight"] = np.full_like(tensors["transformer.wpe.weight"], 2.0 ** 120)
+    gpt = load(cfg, tensors)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    gpt.set_decode_mode(1)
+    tokens = synth.tokens(5, "prompt", 20, cfg["vocab_size"])
+    gpt.prefill(tokens[:17])
+    for i in range(17, 20):
+        got, want = gpt.decode(int(tokens[i])), ref.forward(p, w, tokens[:i + 1])
+        assert np.isfinite(want).all() and close(got, want), i
+    gpt.unloadBuffers()

@@ -179,3 +179,20 @@ def test_sixteen_keys_whose_scores_overflow(device, dtype, n_head):
         got, want = gpt.prefill(tokens), ref.forward(p, w, tokens)
     assert np.isfinite(want).all() and close(got, want), worst(got, want)
     gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("name", ["wpe.weight", "h.1.attn.c_proj.bias"])
+def test_rows_of_one_huge_value(device, dtype, name):
+    """All elements of a row 2^120: its LayerNorm is beta, at a width that leaves lanes without elements, whose zeros are 2^128 standard
+    deviations from the mean."""
+    cfg = small_cfg(n_layer=2, n_head=2, n_embd=40, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    tensors["transformer." + name] = np.full_like(tensors["transformer." + name], 2.0 ** 120)
+    gpt = load(cfg, tensors)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (1, 20, 64):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        got, want = gpt.prefill(tokens), ref.forward(p, w, tokens)
+        assert np.isfinite(want).all() and close(got, want), T
+    gpt.unloadBuffers()

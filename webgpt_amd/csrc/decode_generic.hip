@@ -335,12 +335,14 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
     }
     const float stdev = sqrtf(wave_total(q) / fd + 1e-5f), rstd = 1.0f / stdev;
 #pragma unroll
-    for (int s = 0; s < NS; ++s)
+    for (int s = 0; s < NS; ++s) {
+      const float r = SEG * s + e0l < d ? rstd : 0.f;  // (beyond d the weights are zero, and so is x, whatever the mean)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float v = quotient(x[s][e] - mean, stdev, rstd);
-        x[s][e] = affine ? gam[s][e] * v + bet[s][e] : v;  // (beyond d the weights are zero)
+        const float v = quotient(x[s][e] - mean, stdev, r);
+        x[s][e] = affine ? gam[s][e] * v + bet[s][e] : v;
       }
+    }
   };
   const auto columns = [&](const f32x4 (&x)[NS], int nc, auto cw) {  // products to `out`
     float sums[decltype(cw)::value];

@@ -277,7 +277,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
   };
   // LayerNorm of the wave's slice (instructions.js:451-550); all waves take part.
   const auto normalise = [&](f32x4 (&x)[NS][2]) {
-    const int ol = opaque(lane), r = ol & 15, kg = ol >> 4;
+    const int ol = opaque(lane), row = ol & 15, kg = ol >> 4;
     float sum = 0.f;
 #pragma unroll
     for (int s = 0; s < NS; ++s)
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       }
     }
     q = quad_sum(q);
-    if (kg == 0) stat[wave][r] = make_float2(sum, q);
+    if (kg == 0) stat[wave][row] = make_float2(sum, q);
     if (tid < LN / 4) {
       lnp[tid] = gamma;
       lnp[LN / 4 + tid] = beta;
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
     float2 p[NW];
 #pragma unroll
     for (int v = 0; v < NW; ++v) {
-      p[v] = stat[v][r];
+      p[v] = stat[v][row];
       total += p[v].x;
     }
     const float fd = (float)d, rd = 1.0f / fd, mean = quotient(total, fd, rd);
@@ -320,12 +320,16 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const int k8 = (s1 + s) * 4 + kg;
-      const f32x4* lg = lnp + 2 * (s < n1 && k8 < K81 ? k8 : 0);  // (beyond the slice x is finite and its weights are zero)
+      // beyond the slice the weights are zero and x becomes zero too, whatever the mean: an entry behind the row, of zeros (a row that
+      // fills all entries has nothing beyond a slice)
+      const bool in = s < n1 && k8 < K81;
+      const f32x4* lg = lnp + 2 * (in ? k8 : K81);
+      const float r = in ? rstd : 0.f;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const f32x4 g = lg[h], be = lg[LN / 4 + h];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[s][h][i] = g[i] * quotient(x[s][h][i] - mean, stdev, rstd) + be[i];
+        for (int i = 0; i < 4; ++i) x[s][h][i] = g[i] * quotient(x[s][h][i] - mean, stdev, r) + be[i];
       }
     }
   };
