@@ -9,7 +9,7 @@ from webgpt_amd import synth
 from webgpt_amd._lib import WgptError
 from webgpt_amd.model import GPT
 
-from helpers import close, make_model, oracle_weights, small_cfg, worst
+from helpers import close, make_model, oracle_weights, pack_words, small_cfg, worst
 
 pytestmark = pytest.mark.gpu
 
@@ -156,4 +156,31 @@ def test_rows_of_one_huge_value(device, dtype):
     for i in range(17, 20):
         got, want = gpt.decode(int(tokens[i])), ref.forward(p, w, tokens[:i + 1])
         assert np.isfinite(want).all() and close(got, want), i
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("inputs,product", [("ln_1.bias", "attn.c_attn"), ("attn.c_attn.bias", "attn.c_proj"), ("ln_2.bias", "mlp.c_fc"), ("mlp.c_fc.bias", "mlp.c_proj")])
+def test_int8_sums_beyond_the_range_of_fp32(device, inputs, product):
+    """Inputs of 1e35 in front of one product, whose column scales bring its results back to about 1e2: the sums of 127 x 1e35 and less are infinite
+    before the scale meets them. Of c_attn only the values' columns (the scores stay small)."""
+    d = 200
+    cfg = small_cfg(n_layer=2, n_head=5, n_embd=d, n_ctx=64, vocab_size=90, dtype="int8")
+    tensors = make_model(cfg, 5)
+    p, rng = "transformer.h.0.", np.random.default_rng(3)
+    K, N = (4 * d if product == "mlp.c_proj" else d), {"attn.c_attn": 3 * d, "mlp.c_fc": 4 * d}.get(product, d)
+    q, scale = rng.integers(1, 128, (K, N)).astype(np.int8), np.full(N, 127e-37, np.float32)
+    if product == "attn.c_attn":
+        q[:, :2 * d] = 0
+    tensors[p + inputs] = np.full_like(tensors[p + inputs], 1e35)
+    if inputs == "attn.c_attn.bias":
+        tensors[p + inputs][:2 * d] = 0
+    tensors[p + product + ".weight.q"], tensors[p + product + ".weight.scale"] = pack_words(q), scale
+    gpt = load(cfg, tensors)
+    gpt.set_decode_mode(1)
+    w, prm = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    tokens = synth.tokens(5, "prompt", 20, cfg["vocab_size"])
+    gpt.prefill(tokens[:17])
+    for i in range(17, 20):
+        got, want = gpt.decode(int(tokens[i])), ref.forward(prm, w, tokens[:i + 1])
+        assert np.isfinite(want).all() and close(got, want), (i, worst(got, want))
     gpt.unloadBuffers()

@@ -206,7 +206,7 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
   constexpr int NP = (NS * SEG / 2 + NT - 1) / NT;                           // pairs of words of a row per thread
   extern __shared__ __attribute__((aligned(16))) float run[];                // this workgroup's logits
   __shared__ __attribute__((aligned(16))) float row[NS * SEG], part[NW][8], heads[NW][136];
-  __shared__ float out[4 * NS];
+  __shared__ float out[4 * NS], far_out[I8 ? 4 * NS : 1], far_part[I8 ? NW : 1][8];
   __shared__ float best_v[NW];
   __shared__ int best_i[NW], bail;
   __shared__ sel_key firsts[NW * PD_TOPK];
@@ -344,40 +344,85 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
       }
     }
   };
+  // int8: a column's scale meets its finished sum, which may leave the range of fp32 where the scaled products and the result
+  // do not (inputs of 1e35, scales of 1e-34). A wave with a sum that is not finite takes its sums again, of inputs times DOWN (4 d products
+  // of up to 127 times the largest float stay finite), for those who finish such columns.
+  constexpr float DOWN = 0x1p-24f, UP = 0x1p24f;
+  const auto sums_of = [&](auto& sums, auto take, auto keep) {
+    take(1.f);
+    keep(false);
+    if constexpr (I8) {
+      float all = 0.f;
+#pragma unroll
+      for (const float v : sums) all += fabsf(v);
+      if (__builtin_expect(!(all < INFINITY), 0)) {
+        take(DOWN);
+        keep(true);
+      }
+    }
+    __syncthreads();
+  };
   const auto columns = [&](const f32x4 (&x)[NS], int nc, auto cw) {  // products to `out`
     float sums[decltype(cw)::value];
+    sums_of(
+        sums,
+        [&](float f) {
 #pragma unroll
-    for (int j = 0; j < cw(); ++j) {
-      sums[j] = 0.f;
+          for (int j = 0; j < cw(); ++j) {
+            sums[j] = 0.f;
 #pragma unroll
-      for (int s = 0; s < NS; ++s) sums[j] += dot4(w[j * NS + s].value(), x[s]);
-    }
-    wave_sums(sums);
+            for (int s = 0; s < NS; ++s) sums[j] += dot4(w[j * NS + s].value(), f * x[s]);
+          }
+          wave_sums(sums);
+        },
+        [&](bool far) {
 #pragma unroll
-    for (int j = 0; j < cw(); ++j)
-      if (lane == 0 && wave + NW * j < nc) out[wave + NW * j] = sums[j];
-    __syncthreads();
+          for (int j = 0; j < cw(); ++j)
+            if (lane == 0 && wave + NW * j < nc) (far ? far_out : out)[wave + NW * j] = sums[j];
+        });
   };
-  const auto segments = [&](const auto& x, int waves, auto cw) {  // this thread's column of a projection
+  const auto segments = [&](const auto& x, auto cw) {  // partial sums of the projections to `part`
     float sums[NS];
+    sums_of(
+        sums,
+        [&](float f) {
 #pragma unroll
-    for (int c = 0; c < NS; ++c) {
-      sums[c] = 0.f;
+          for (int c = 0; c < NS; ++c) {
+            sums[c] = 0.f;
 #pragma unroll
-      for (int j = 0; j < cw(); ++j) sums[c] += dot4(w[c * cw() + j].value(), x[j]);
-    }
-    wave_sums(sums);
+            for (int j = 0; j < cw(); ++j) sums[c] += dot4(w[c * cw() + j].value(), f * x[j]);
+          }
+          wave_sums(sums);
+        },
+        [&](bool far) {
 #pragma unroll
-    for (int c = 0; c < NS; ++c)
-      if (lane == 0) part[wave][c] = sums[c];
-    __syncthreads();
-    float v = 0.f;
-    if (tid < ncC)
-      for (int u = 0; u < waves; ++u) v += part[u][tid];
-    return v;
+          for (int c = 0; c < NS; ++c)
+            if (lane == 0) (far ? far_part : part)[wave][c] = sums[c];
+        });
   };
-  const auto finished = [&](float v) {
-    if constexpr (I8) v *= scale / 127.0f;
+  // This thread's column of `out`, or of a projection whose partial sums the first `waves` waves have.
+  const auto finished_column = [&] {
+    float v = out[tid];
+    if constexpr (I8) {
+      const float s = scale / 127.0f;
+      if (__builtin_expect(fabsf(v) < INFINITY, 1)) v *= s;
+      else v = far_out[tid] * s * UP;
+    }
+    return v + bias;
+  };
+  const auto finished_parts = [&](int waves) {
+    float v = 0.f;
+    for (int u = 0; u < waves; ++u) v += part[u][tid];
+    if constexpr (I8) {
+      const float s = scale / 127.0f;
+      if (__builtin_expect(fabsf(v) < INFINITY, 1)) {
+        v *= s;
+      } else {
+        v = 0.f;
+        for (int u = 0; u < waves; ++u) v += fabsf(part[u][tid]) < INFINITY ? part[u][tid] * DOWN : far_part[u][tid];
+        v = v * s * UP;
+      }
+    }
     return v + bias;
   };
 
@@ -414,7 +459,7 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
         f32x4 x[NS];
         normalised(x, I8);
         columns(x, ncA, Count<CWA>());
-        if (tid < ncA) publish(fresh_args()->bufQKV + cA + tid, finished(out[tid]), ep + 1);
+        if (tid < ncA) publish(fresh_args()->bufQKV + cA + tid, finished_column(), ep + 1);
       }
       // ---- attention of (head, slice) ----
       if (attends) {
@@ -533,10 +578,10 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
           if (slices <= 2) merge(Count<2>());
           else merge(Count<DG_SPLIT>());
         }
-        const float v = segments(x, S, Count<1>());
+        segments(x, Count<1>());
         if (bail) return;
         if (tid < ncC) {
-          res += finished(v);
+          res += finished_parts(S);
           publish(fresh_args()->bufR1 + cC + tid, res, ep + 3);
         }
       }
@@ -549,7 +594,7 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
         f32x4 x[NS];
         normalised(x, I8);
         columns(x, ncD, Count<CWD>());
-        if (tid < ncD) publish(fresh_args()->bufH + cD + tid, gelu_ref(finished(out[tid])), ep + 4);
+        if (tid < ncD) publish(fresh_args()->bufH + cD + tid, gelu_ref(finished_column()), ep + 4);
       }
       // ---- mlp c_proj + residual ----
       if (ncC) {
@@ -566,10 +611,10 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
         wt.words(buffer_of(fresh_args()->bufH, 32 * (size_t)d), off, v, ep + 4);
 #pragma unroll
         for (int i = 0; i < 4 * CWD; ++i) x[i >> 2][i & 3] = __uint_as_float(v[i >> 1][2 * (i & 1)]);
-        const float y = segments(x, SH < NW ? SH : NW, Count<CWD>());
+        segments(x, Count<CWD>());
         if (bail) return;
         if (tid < ncC) {
-          res += finished(y);
+          res += finished_parts(SH < NW ? SH : NW);
           publish(fresh_args()->bufR2 + cC + tid, res, ep + 5);
         }
       }
