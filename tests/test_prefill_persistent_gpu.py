@@ -126,6 +126,33 @@ def test_values_that_are_not_finite(device, dtype, what):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_a_spoilt_prompt_is_no_matter_of_the_next_ones(device, dtype):
+    """Prompts before and behind one with a value that is not finite: the same bits (launches round in another order), also where the row
+    group holds rows that the spoilt one has left. Behind several spoilt ones prompts are tried again after a while."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=90, dtype=dtype)
+    tensors = make_model(cfg, 5)
+    tensors["transformer.wpe.weight"] = tensors["transformer.wpe.weight"].copy()
+    tensors["transformer.wpe.weight"][37, 5] = np.inf
+    tokens = synth.tokens(5, "prompt", 50, cfg["vocab_size"])
+    launches = load(cfg, tensors, flags=_lib.FLAG_TAPS)
+    gpt = load(cfg, tensors)
+    lengths = (35, 12, 37, 1)
+    alone = {T: gpt.prefill(tokens[:T]) for T in lengths}
+    assert not all(np.array_equal(alone[T], launches.prefill(tokens[:T])) for T in lengths)
+    with np.errstate(all="ignore"):
+        for T in lengths:
+            gpt.prefill(tokens)
+            for again in lengths[:lengths.index(T) + 1]:
+                assert np.array_equal(gpt.prefill(tokens[:again]), alone[again]), (T, again)
+        for _ in range(5):
+            gpt.prefill(tokens)
+        got = [gpt.prefill(tokens[:35]) for _ in range(8)]
+    assert all(close(g, alone[35]) for g in got) and np.array_equal(got[-1], alone[35])
+    gpt.unloadBuffers()
+    launches.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
 @pytest.mark.parametrize("name", ["wpe.weight", "h.1.attn.c_proj.bias", "h.1.mlp.c_proj.bias"])
 def test_rows_whose_variance_overflows(device, dtype, name):
     """Finite residual values of 1e28 from the first, the last and the final LayerNorm on: a row's variance is infinite, its quotients

@@ -75,6 +75,8 @@ struct Model {
   int pp_rows = 0;
   PrefillArgs pp{};
   unsigned pp_epoch = 0;       // last epoch of its earlier launches
+  int pp_spoilt = 0;           // launches in a row that gave up on their prompt's values, and
+  int pp_skip = 0;             // the prompts that are not tried on account of them
   int32_t* tok_pin = nullptr;  // pinned (behind ids_pin's): [PP_MAX_T] the prompt, then the word that a launch leaves its error in
 
   // decode with one launch per block (decode_mode 0): the token's launches read the cache position from pos_dev and

@@ -624,8 +624,6 @@ static int setup_prefill(Model* m) {
   PrefillArgs& a = m->pp;
   WGPT_HIP(hipMemcpyAsync((void*)a.layers, layers.data(), sizeof(PrefillLayer) * (size_t)m->L, hipMemcpyHostToDevice, rt().stream));
   WGPT_HIP(hipMemsetAsync(a.flags, 0, PP_FLAGS * sizeof(unsigned), rt().stream));
-  // (rows of the last row group beyond the prompt are multiplied too: what memory holds by chance would count as spoilt sums)
-  WGPT_HIP(hipMemsetAsync(a.q, 0, prefill_exchange_floats(m->pp_rows, m->d) * sizeof(float), rt().stream));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   a.L = m->L; a.H = m->H; a.hs = m->hs; a.d = m->d; a.ctx = m->ctx; a.V = m->V;
   a.scale = (float)(1.0 / std::sqrt((double)m->hs));
@@ -639,12 +637,14 @@ static int setup_prefill(Model* m) {
   a.host_err = m->tok_pin + PP_MAX_T;
   a.spin_limit = spin_limit();
   m->pp_epoch = 0;
+  m->pp_spoilt = m->pp_skip = 0;
   return WGPT_OK;
 }
 
-// The prompt's forward in one launch, logits into logits_pin. *done: it has run to its end; where it has not (a wait that
-// expired, sums that the split operands may have spoilt) the caller runs the launches of forward_blocks, and so does every later
-// call.
+// The prompt's forward in one launch, logits into logits_pin. *done: it has run to its end; where it has not, the caller runs
+// the launches of forward_blocks. After a wait that expired every later call runs them too: workgroups may not have been on the
+// device together. Sums that the split operands may have spoilt are this prompt's own, and the next one is tried again; of a
+// model whose prompts are spoilt one after the other only every second, fourth .. 64th is.
 static int prefill_persistent(Model* m, const int32_t* tokens, int T, bool* done) {
   const unsigned n = prefill_epochs(m->L);
   if (m->pp_epoch > 0x7fffffffu - 2 * n) {
@@ -660,8 +660,11 @@ static int prefill_persistent(Model* m, const int32_t* tokens, int T, bool* done
   m->pp_epoch += n;
   WGPT_HIP(hipEventRecord(m->ev1, rt().stream));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
-  *done = m->tok_pin[PP_MAX_T] == 0;
-  if (!*done) m->pp_rows = 0;
+  const int why = m->tok_pin[PP_MAX_T];
+  *done = why == 0;
+  m->pp_spoilt = *done ? 0 : std::min(m->pp_spoilt + 1, 7);
+  m->pp_skip = *done ? 0 : (1 << (m->pp_spoilt - 1)) - 1;
+  if (why == PP_ERR_WAIT) m->pp_rows = 0;
   return WGPT_OK;
 }
 
@@ -824,7 +827,9 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
   m->x_rows = 0;
   int rc;
   bool done = false;
-  if (T <= m->pp_rows) {
+  if (T <= m->pp_rows && m->pp_skip > 0) {
+    --m->pp_skip;
+  } else if (T <= m->pp_rows) {
     WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
     if ((rc = prefill_persistent(m, tokens, T, &done))) return rc;
     if (done) {

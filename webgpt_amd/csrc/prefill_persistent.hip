@@ -167,7 +167,8 @@ __device__ __forceinline__ f32x4 products(const WSlice8<false> (&w)[N], const Op
     for (int e = 0; e < 8; ++e) acc[e & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w[i].v[e]), x.v[i].v[e >> 2][e & 3], acc[e & 3], 0, 0, 0);
   return (acc[0] + acc[1]) + (acc[2] + acc[3]);
 }
-// int8 sums that the split may have spoilt, as in gemm_split.hip: not finite, from 2^124 on, under 2^-60 but zero.
+// int8 sums that the split may have spoilt, as in gemm_split.hip: not finite, from 2^124 on, under 2^-60 but zero. (Of the prompt's rows
+// only: those of the last row group beyond it hold what earlier prompts or other owners of the memory have left.)
 template <bool I8>
 __device__ __forceinline__ bool spoilt(const f32x4& v) {
   bool bad = false;
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
     const auto tile = [&](WSlice<I8, NS>& wt, int t) {
       const f32x4 v = products(wt.s, xs);
       if (t + RING < tiles) request_w(wt, W, N, cp, nc, t + RING);
-      bad = bad || spoilt<I8>(v);
+      bad = bad || (em < T && spoilt<I8>(v));
       red[(wave * tiles + t) * 64 + opaque(lane)] = v;
     };
 #pragma unroll 1
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
           for (int t = 0; t < TM; ++t)
             if (t0 + t < tilesC) {
-              bad = bad || spoilt<I8>(sum[t]);
+              bad = bad || (em < T && spoilt<I8>(sum[t]));
               red[(wave * tilesC + t0 + t) * 64 + lane] = sum[t];
             }
         }
