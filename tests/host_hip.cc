@@ -9,7 +9,7 @@
 
 extern "C" {
 int host_hip_launches = 0, host_hip_fail_at = 0;
-int host_hip_allocs = 0, host_hip_alloc_fail_at = 0;
+int host_hip_allocs = 0, host_hip_alloc_fail_at = 0, host_hip_frees = 0;
 int host_hip_unwaited = 0;  // launches since the last wait for the stream
 
 static dim3 cfg_grid, cfg_block;
@@ -54,7 +54,7 @@ static hipError_t allocate(void** p, size_t n) {
   return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipMalloc(void** p, size_t n) { return allocate(p, n); }
-hipError_t hipFree(void* p) { return free(p), hipSuccess; }
+hipError_t hipFree(void* p) { return ++host_hip_frees, free(p), hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return allocate(p, n); }
 hipError_t hipHostFree(void* p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }

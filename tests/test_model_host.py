@@ -104,3 +104,39 @@ for i in range(1, total + 1):
     _lib.call("wgpt_decode_sample", m, 1, 2, 12, 1.0, np.zeros(2).ctypes.data_as(C.POINTER(C.c_double)), tokens.ctypes.data_as(C.POINTER(C.c_int32)), None)
     _lib.call("wgpt_model_destroy", m)
 """)
+
+
+def test_buffers_of_a_window_that_grows(host_hip):
+    """Nineteen buffers a window, given back behind it, as a forward from blocks has them: a window of a token more finds its memory among
+    that of the shorter ones, also when those of many lengths have been left behind, and what is held stays within its bound."""
+    run(host_hip, "f32", """
+frees = C.c_int.in_dll(hip, "host_hip_frees")
+own = allocs.value
+
+def window(T, d=128):
+    before = allocs.value
+    hs = []
+    for n in [d] * 12 + [4 * d] * 5 + [3 * d, 5003]:
+        h = C.c_uint64(0)
+        _lib.call("wgpt_alloc", 4 * T * n, C.byref(h))
+        hs.append(h)
+    for h in hs:
+        _lib.call("wgpt_free", h)
+    return allocs.value - before
+
+assert [window(64) for _ in range(3)] == [19, 0, 0]
+made = sum(window(T) for T in range(65, 1000))
+assert made <= 19 * 16 * 4, made              # four octaves
+assert sum(window(T) for T in range(900, 700, -1)) <= 19 * 8
+big = [C.c_uint64(0) for _ in range(300)]      # a pass that does not fit keeps what it can
+for _ in range(3):
+    before = allocs.value
+    for h in big:
+        _lib.call("wgpt_alloc", 1 << 20, C.byref(h))
+    made = allocs.value - before
+    for h in big:
+        _lib.call("wgpt_free", h)
+assert made < 300 - 128, made
+assert [window(10) for _ in range(60)][-1] == 0  # and makes room when nobody asks for it any more
+assert allocs.value - frees.value - own <= 256, (allocs.value, frees.value)
+""")

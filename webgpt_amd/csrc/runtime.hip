@@ -2,7 +2,6 @@
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
-#include <map>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -32,43 +31,69 @@ Runtime& rt() {
 
 struct Buffer {
   void* ptr;
-  size_t bytes;
+  size_t bytes, block;    // as asked for, and as allocated
   bool uploaded = false;  // the host has written to it
 };
 
 // ---- device memory of freed buffers, for the next ones ----
 // A forward assembled from blocks frees and allocates a buffer per block; the driver's calls, and the wait for the stream that a
 // free needs, cost it 3 us a buffer: 59 of the 430 us of two layers of 117M at 100 tokens. A block that is handed out again is used by
-// the library's one stream behind what still uses it. At most POOL_BYTES in POOL_BLOCKS blocks are kept; they are given back when
-// memory runs out and by wgpt_shutdown. Buffers that the host has written to, weights above all, come and go with a model and are not
+// the library's one stream behind what still uses it. Blocks come in sixteen sizes an octave, so that a window which grows by a token
+// finds those of the shorter one. At most POOL_BYTES in POOL_BLOCKS blocks are kept. Where there is no room for another, those that nobody
+// has asked for in the last POOL_AGE frees go (sizes that a program has left behind; with none of them the new one goes: to give up
+// the oldest of a pass that does not fit would take them from the next pass). All are given back when memory runs out and by wgpt_shutdown.
+// Buffers that the host has written to, weights above all, come and go with a model and are not
 // kept: with 214 MB of them here the driver took longer for the first results of the next model (first pass of two layers of 117M behind
 // another model's 1.04 ms in the mean, 0.90 without them, 0.87 with nothing kept at all).
-constexpr size_t POOL_BYTES = (size_t)256 << 20, POOL_BLOCKS = 256;
+constexpr size_t POOL_BYTES = (size_t)256 << 20, POOL_BLOCKS = 256, POOL_AGE = 2 * POOL_BLOCKS;
 struct Pool {
+  struct Block {
+    size_t size;
+    void* ptr;
+    size_t since;  // `frees` when it was kept
+  };
   std::mutex lock;
-  std::multimap<size_t, void*> blocks;  // by size
-  size_t bytes = 0;
+  std::vector<Block> blocks;  // the oldest first
+  size_t bytes = 0, frees = 0;
 };
 static Pool& pool() {
   static Pool p;
   return p;
 }
-static size_t block_size(size_t bytes) { return (bytes + 255) / 256 * 256; }
+// 16 bytes of slack so that a float4 access to the last elements of a buffer whose element count is a multiple of 4 never leaves
+// the allocation.
+static size_t plain_size(size_t bytes) { return (bytes + 16 + 255) / 256 * 256; }
+// The size of a block of so many bytes: theirs to the next sixteenth of the power of two below (6 % more at most), nothing more where
+// they are one or where the block will not be kept.
+static size_t block_size(size_t bytes) {
+  size_t step = 256;
+  while (32 * step <= bytes && bytes <= POOL_BYTES) step *= 2;
+  return (bytes + step - 1) / step * step + 256;
+}
 static void* pool_take(size_t size) {
   Pool& p = pool();
   std::lock_guard<std::mutex> g(p.lock);
-  const auto it = p.blocks.find(size);
-  if (it == p.blocks.end()) return nullptr;
-  void* ptr = it->second;
-  p.blocks.erase(it);
-  p.bytes -= size;
-  return ptr;
+  for (auto it = p.blocks.rbegin(); it != p.blocks.rend(); ++it)
+    if (it->size == size) {
+      void* ptr = it->ptr;
+      p.blocks.erase(std::next(it).base());
+      p.bytes -= size;
+      return ptr;
+    }
+  return nullptr;
 }
 static bool pool_keep(size_t size, void* ptr) {
   Pool& p = pool();
   std::lock_guard<std::mutex> g(p.lock);
-  if (p.bytes + size > POOL_BYTES || p.blocks.size() >= POOL_BLOCKS) return false;
-  p.blocks.emplace(size, ptr);
+  ++p.frees;
+  const auto full = [&] { return p.bytes + size > POOL_BYTES || p.blocks.size() >= POOL_BLOCKS; };
+  while (full() && !p.blocks.empty() && p.frees - p.blocks[0].since > POOL_AGE) {  // (hipFree waits for the device)
+    (void)hipFree(p.blocks[0].ptr);
+    p.bytes -= p.blocks[0].size;
+    p.blocks.erase(p.blocks.begin());
+  }
+  if (full()) return false;
+  p.blocks.push_back({size, ptr, p.frees});
   p.bytes += size;
   return true;
 }
@@ -76,7 +101,7 @@ static bool pool_release() {  // (hipFree waits for the device)
   Pool& p = pool();
   std::lock_guard<std::mutex> g(p.lock);
   const bool some = !p.blocks.empty();
-  for (const auto& b : p.blocks) (void)hipFree(b.second);
+  for (const auto& b : p.blocks) (void)hipFree(b.ptr);
   p.blocks.clear();
   p.bytes = 0;
   return some;
@@ -245,17 +270,19 @@ int wgpt_alloc(size_t bytes, wgpt_buf* out) {
   if (!out) return fail(WGPT_ERR_ARG, "wgpt_alloc: out is NULL");
   if (bytes == 0) return fail(WGPT_ERR_ARG, "wgpt_alloc: zero-sized buffer");
   void* p = nullptr;
-  // 16 bytes of slack so that a float4 access to the last elements of a buffer whose
-  // element count is a multiple of 4 never leaves the allocation.
-  const size_t size = block_size(bytes + 16);
-  if (size < bytes) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): size overflow", bytes);
+  size_t size = block_size(bytes);
+  if (size < bytes || plain_size(bytes) < bytes) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): size overflow", bytes);
   p = pool_take(size);
   if (!p) {
-    const hipError_t e = device_malloc(&p, size);
+    hipError_t e = device_malloc(&p, size);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      e = device_malloc(&p, size = plain_size(bytes));
+    }
     if (e != hipSuccess) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   }
   wgpt_buf h = g_next_handle++;
-  registry()[h] = Buffer{p, bytes, false};
+  registry()[h] = Buffer{p, bytes, size, false};
   *out = h;
   return WGPT_OK;
 }
@@ -264,7 +291,7 @@ int wgpt_free(wgpt_buf buf) {
   WGPT_REQUIRE_INIT();
   auto it = registry().find(buf);
   if (it == registry().end()) return fail(WGPT_ERR_ARG, "wgpt_free: unknown buffer handle %llu", (unsigned long long)buf);
-  if (it->second.uploaded || !pool_keep(block_size(it->second.bytes + 16), it->second.ptr)) {
+  if (it->second.uploaded || !pool_keep(it->second.block, it->second.ptr)) {
     WGPT_HIP(hipStreamSynchronize(rt().stream));
     WGPT_HIP(hipFree(it->second.ptr));
   }
