@@ -130,7 +130,9 @@ typedef struct {
 
 enum {
   WGPT_FLAG_TAPS = 1, /* keep the activation taps of the last wgpt_prefill for wgpt_model_tap */
-  WGPT_FLAG_TUNE_DELAYS = 2 /* wgpt_model_finalize ends with wgpt_model_tune_poll_delays(m, 2, ...) */
+  /* wgpt_model_finalize ends with wgpt_model_tune_poll_delays(m, 2, ...) where the persistent decode kernel has the model (the one of
+   * any shape from a context of 4 on; a trial of it that gives up leaves the model loaded, with decode mode 0) */
+  WGPT_FLAG_TUNE_DELAYS = 2
 };
 
 int wgpt_model_create(const wgpt_params* params, wgpt_model* out);

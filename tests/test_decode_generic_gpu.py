@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import ref
-from webgpt_amd import synth
+from webgpt_amd import _lib, synth
 from webgpt_amd._lib import WgptError
 from webgpt_amd.model import GPT
 
@@ -184,3 +184,25 @@ def test_int8_sums_beyond_the_range_of_fp32(device, inputs, product):
         got, want = gpt.decode(int(tokens[i])), ref.forward(prm, w, tokens[:i + 1])
         assert np.isfinite(want).all() and close(got, want), (i, worst(got, want))
     gpt.unloadBuffers()
+
+
+def test_expired_wait_in_a_search_of_delays(device, monkeypatch):
+    """A search whose trials give up says so; where it is a part of loading the model, the model is loaded. Both decode with launches."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=90)
+    tensors = make_model(cfg, 3)
+    monkeypatch.setenv("WEBGPT_AMD_SPIN_LIMIT", "0")
+    monkeypatch.setenv("WEBGPT_AMD_POLL_DELAYS", "0,0,0,0,0,0,0")
+    tokens, rows = synth.tokens(9, "prompt", 20, cfg["vocab_size"]), []
+    for flags in (0, _lib.FLAG_TUNE_DELAYS):
+        gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg), flags=flags)
+        gpt.initialize()
+        if not flags:
+            with pytest.raises(WgptError, match="a wait of a trial launch expired"):
+                gpt.tune_poll_delays(1)
+        with pytest.raises(WgptError, match="not available"):
+            gpt.set_decode_mode(1)
+        gpt.prefill(tokens[:12])
+        rows.append(gpt.decode(int(tokens[12])))
+        gpt.unloadBuffers()
+    assert np.array_equal(rows[0], rows[1])
+    assert close(rows[0], ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens[:13]))

@@ -140,3 +140,22 @@ assert made < 300 - 128, made
 assert [window(10) for _ in range(60)][-1] == 0  # and makes room when nobody asks for it any more
 assert allocs.value - frees.value - own <= 256, (allocs.value, frees.value)
 """)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_search_of_poll_delays_at_finalize(host_hip, dtype):
+    """WGPT_FLAG_TUNE_DELAYS is for models whose context is long enough for a trial; the others load as they do without it."""
+    run(host_hip, dtype, """
+for ctx in (1, 2, 3, 4, 5, 24):
+    cfg["n_ctx"] = ctx
+    tensors = make_model(cfg, 1)
+    p = _lib.Params(**synth.model_params(cfg), weight_dtype=int(sys.argv[2] == "int8"), flags=_lib.FLAG_TUNE_DELAYS)
+    m = C.c_uint64(0)
+    _lib.call("wgpt_model_create", C.byref(p), C.byref(m))
+    for n, t in tensors.items():
+        _lib.call("wgpt_model_set_tensor", m, n.encode(), np.ascontiguousarray(t).ctypes.data, t.nbytes)
+    _lib.call("wgpt_model_finalize", m)
+    again = refused("wgpt_model_tune_poll_delays", m, 0, None, None, None)
+    assert (again is not None) == (ctx < 4) and (again is None or "context too short" in again), (ctx, again)
+    _lib.call("wgpt_model_destroy", m)
+""")

@@ -284,6 +284,8 @@ static unsigned spin_limit() {
   return 1u << 18;
 }
 
+constexpr int TUNE_MIN_CTX = 4;  // shortest context with a position at three tenths of it
+
 // Words of PersistentArgs::bufAM: the kernel of any shape has two sets of candidates in turn.
 static size_t candidate_words(const Model* m) { return (size_t)(m->generic ? 4 : 2) * PD_TOPK * PD_GRID; }
 
@@ -808,7 +810,12 @@ int wgpt_model_finalize(wgpt_model h) {
   m->decode_mode = m->persist_ok ? 1 : 0;
   m->pos = 0;
   m->finalized = true;
-  if ((m->p.flags & WGPT_FLAG_TUNE_DELAYS) && m->persist_ok) return wgpt_model_tune_poll_delays(h, 2, nullptr, nullptr, nullptr);
+  // (the kernel of any shape also has models with contexts that are too short for a trial)
+  if ((m->p.flags & WGPT_FLAG_TUNE_DELAYS) && m->persist_ok && !(m->generic && m->ctx < TUNE_MIN_CTX)) {
+    rc = wgpt_model_tune_poll_delays(h, 2, nullptr, nullptr, nullptr);
+    if (rc && m->generic && !m->persist_ok) return WGPT_OK;  // a wait expired: the model is loaded and decodes with launches
+    return rc;
+  }
   return WGPT_OK;
 }
 
@@ -1018,7 +1025,7 @@ int wgpt_model_tune_poll_delays(wgpt_model h, int rounds, int32_t* chosen, float
   // 5 ms) that the event clock's granularity does not matter
   const int pa = m->ctx * 3 / 10, pb = m->ctx * 3 / 4;
   int steps = m->ctx - pb < 8 ? m->ctx - pb : 8;
-  if (steps < 1 || pa < 1) return fail(WGPT_ERR_STATE, "wgpt_model_tune_poll_delays: context too short");
+  if (m->ctx < TUNE_MIN_CTX) return fail(WGPT_ERR_STATE, "wgpt_model_tune_poll_delays: context too short");
   const auto timed_pair = [&](int n) {
     const float a = timed_trial(m, pa, n);
     if (a < 0) return -1.f;
@@ -1028,7 +1035,10 @@ int wgpt_model_tune_poll_delays(wgpt_model h, int rounds, int32_t* chosen, float
   const auto failed = [&](const int* restore) -> int {
     for (int i = 0; i < 7; ++i) m->pa.delay[i] = restore[i];
     m->pos = 0;
-    if (m->pin[1] != 0) { (void)check_persistent(m); return WGPT_ERR_DEVICE; }
+    if (m->pin[1] != 0) {
+      const int rc = check_persistent(m);
+      return rc ? rc : fail(WGPT_ERR_DEVICE, "wgpt_model_tune_poll_delays: a wait of a trial launch expired; the model decodes with a launch per block from now on");
+    }
     return fail(WGPT_ERR_DEVICE, "wgpt_model_tune_poll_delays: a trial launch failed");
   };
   int start[7];
