@@ -98,6 +98,31 @@ def test_sampled_steps_select_what_the_oracle_selects(device, vocab_size, repeat
     gpt.unloadBuffers()
 
 
+@pytest.mark.parametrize("start", [2**31 - 1, 2**31 - 1 - 60, 2**31 - 1 - 200])
+def test_epochs_restart_below_their_limit(device, monkeypatch, start):
+    """The counter starts over, from cleared exchange buffers and both sets of candidates, in front of the first, the second or a later
+    call: ids and logits of greedy and sampled calls are those of one from 0 on."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=301)
+    tensors, tokens, out = make_model(cfg, 3), synth.tokens(3, "prompt", 12, 301), []
+    u = np.random.default_rng(3).random(5)
+    for s in (0, start):
+        monkeypatch.setenv("WEBGPT_AMD_EPOCH_START", str(s))
+        gpt = load(cfg, tensors)
+        gpt.set_decode_mode(1)
+        gpt.prefill(tokens[:11])
+        ids, rows = [int(tokens[11])], []
+        for _ in range(4):
+            more, last = gpt.decode_greedy(ids[-1], 4, want_logits=True)
+            ids += [int(t) for t in more]
+            rows.append(last)
+            ids += [int(t) for t in gpt.decode_sample(ids[-1], 5, 8, 0.8, u)]
+            rows.append(gpt.decode(ids[-1]))
+        gpt.set_decode_mode(1)  # (no wait has expired)
+        out.append((ids, rows))
+        gpt.unloadBuffers()
+    assert out[0][0] == out[1][0] and all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
+
+
 @pytest.mark.parametrize("dtype", ["f32", "int8"])
 def test_expired_wait_repeats_the_call_with_launches(device, monkeypatch, dtype):
     """Waits that give up at their first look (forced from the host; every kernel drains): the calls succeed with the results of a

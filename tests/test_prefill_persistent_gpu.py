@@ -87,6 +87,19 @@ def test_expired_wait_falls_back_to_launches(device, monkeypatch, dtype):
     launches.unloadBuffers()
 
 
+@pytest.mark.parametrize("start", [2**31 - 1, 2**31 - 1 - 22, 2**31 - 1 - 33])
+def test_epochs_restart_below_their_limit(device, monkeypatch, start):
+    """Eleven epochs a prompt: the counter starts over in front of the first, second or third prompt, with the bits of one from 0 on."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=90)
+    tensors, tokens, rows = make_model(cfg, 3), synth.tokens(3, "prompt", 64, 90), []
+    for s in (0, start):
+        monkeypatch.setenv("WEBGPT_AMD_EPOCH_START", str(s))
+        gpt = load(cfg, tensors)
+        rows.append([gpt.prefill(tokens[:T]) for T in (40, 64, 12, 33, 64)])
+        gpt.unloadBuffers()
+    assert all(np.array_equal(a, b) for a, b in zip(*rows))
+
+
 @pytest.mark.parametrize("dtype", ["f32", "int8"])
 @pytest.mark.parametrize("what", ["value", "scale", "weight"])
 def test_values_that_are_not_finite(device, dtype, what):

@@ -284,6 +284,16 @@ static unsigned spin_limit() {
   return 1u << 18;
 }
 
+// WEBGPT_AMD_EPOCH_START: tests start the epoch counters just below their limits to run the restarts there.
+static unsigned epoch_start() {
+  if (const char* e = getenv("WEBGPT_AMD_EPOCH_START")) {
+    char* end = nullptr;
+    const unsigned long v = strtoul(e, &end, 10);
+    if (end != e && v <= 0x7fffffffu) return (unsigned)v;
+  }
+  return 0;
+}
+
 constexpr int TUNE_MIN_CTX = 4;  // shortest context with a position at three tenths of it
 
 // Words of PersistentArgs::bufAM: the kernel of any shape has two sets of candidates in turn.
@@ -434,13 +444,7 @@ static int setup_persistent(Model* m) {
   if ((rc = dev_alloc(m, sizeof(unsigned long long) * 512 * G, (void**)&a.trace))) return rc;
   WGPT_HIP(hipMemsetAsync(a.trace, 0, sizeof(unsigned long long) * 512 * G, rt().stream));
 #endif
-  m->epoch = 0;
-  // WEBGPT_AMD_EPOCH_START: tests start the counter just below its limit to run the restart above
-  if (const char* e = getenv("WEBGPT_AMD_EPOCH_START")) {
-    char* end = nullptr;
-    const unsigned long v = strtoul(e, &end, 10);
-    if (end != e && v <= 0x7fffffffu) m->epoch = (unsigned)v;
-  }
+  m->epoch = epoch_start();
   m->persist_ok = true;
   return WGPT_OK;
 }
@@ -638,7 +642,7 @@ static int setup_prefill(Model* m) {
   a.logits = m->logits; a.host_logits = m->logits_pin;
   a.host_err = m->tok_pin + PP_MAX_T;
   a.spin_limit = spin_limit();
-  m->pp_epoch = 0;
+  m->pp_epoch = epoch_start();
   m->pp_spoilt = m->pp_skip = 0;
   return WGPT_OK;
 }
