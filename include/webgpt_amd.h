@@ -188,6 +188,10 @@ int wgpt_model_decode_bytes(wgpt_model m, int t, uint64_t* bytes);
 /* Selects the decode implementation: 0 = one kernel per block, 1 = persistent
  * whole-token kernel. Default is the fastest available. */
 int wgpt_model_set_decode_mode(wgpt_model m, int mode);
+/* How the model runs, for those who time or test it: *prefill: 1 the last wgpt_prefill ran to its end as one persistent launch,
+ * 0 with a launch per block (longer than the kernel takes, WGPT_FLAG_TAPS, a launch that gave up), -1 there was none; *decode: the decode
+ * mode in use, 0 also after a wait of the persistent kernel that expired. Either may be NULL. */
+int wgpt_model_routes(wgpt_model m, int* prefill, int* decode);
 /* The persistent decode kernel waits a fixed time after publishing before it first looks for the other workgroups'
  * values (seven delays, one per exchange; a table per model width is built in, measured on one MI355X). This searches
  * around the current row on the GPU the model lives on: `rounds` passes of coordinate descent (0 = only measure), each

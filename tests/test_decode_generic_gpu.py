@@ -44,11 +44,13 @@ def test_steps_against_oracle_and_launches(device, dtype, d, n_head):
             for j, name in enumerate("kv"):
                 rows = gpt.tap(f"kv{li}_{name}")
                 assert close(rows, kv[li, j]), (T, li, name, worst(rows, kv[li, j]))
+    assert gpt.routes()[1] == 1  # (no call was repeated with launches)
     out = {}
     for mode in (1, 0):
         gpt.set_decode_mode(mode)
         gpt.prefill(tokens[:60])
         out[mode] = gpt.decode_greedy(int(tokens[60]), 9, want_logits=True)
+        assert gpt.routes()[1] == mode
     assert np.array_equal(out[1][0], out[0][0])
     assert close(out[1][1], out[0][1]), worst(out[1][1], out[0][1])
     gpt.unloadBuffers()
@@ -69,6 +71,7 @@ def test_the_longest_contexts(device, n_head, n_embd, n_ctx):
             got = gpt.decode(int(tokens[T + i]))
             want = ref.forward(p, w, tokens[:T + i + 1])
             assert close(got, want), (T, i, worst(got, want))
+    assert gpt.routes()[1] == 1
     gpt.unloadBuffers()
 
 
@@ -95,6 +98,7 @@ def test_sampled_steps_select_what_the_oracle_selects(device, vocab_size, repeat
             for i in range(steps):
                 token = ref.sample_topk(gpt.decode(token), min(top_k, vocab_size), 0.8, float(u[i]))[0]
                 assert token == got[i], (top_k, steps, i)
+    assert gpt.routes()[1] == 1
     gpt.unloadBuffers()
 
 
@@ -117,7 +121,7 @@ def test_epochs_restart_below_their_limit(device, monkeypatch, start):
             rows.append(last)
             ids += [int(t) for t in gpt.decode_sample(ids[-1], 5, 8, 0.8, u)]
             rows.append(gpt.decode(ids[-1]))
-        gpt.set_decode_mode(1)  # (no wait has expired)
+        assert gpt.routes()[1] == 1
         out.append((ids, rows))
         gpt.unloadBuffers()
     assert out[0][0] == out[1][0] and all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
@@ -141,6 +145,7 @@ def test_expired_wait_repeats_the_call_with_launches(device, monkeypatch, dtype)
         for g in (gpt, launches):
             g.prefill(tokens[:12])
         assert np.array_equal(call(gpt), call(launches))
+        assert gpt.routes() == (0, 0)
         assert np.array_equal(gpt.decode(int(tokens[16])), launches.decode(int(tokens[16])))
         with pytest.raises(WgptError, match="not available"):
             gpt.set_decode_mode(1)
@@ -163,6 +168,7 @@ def test_rows_whose_variance_overflows(device, dtype):
         for i in range(17, 20):
             got, want = gpt.decode(int(tokens[i])), ref.forward(p, w, tokens[:i + 1])
             assert np.isfinite(want).all() and close(got, want), i
+    assert gpt.routes()[1] == 1
     gpt.unloadBuffers()
 
 
@@ -181,6 +187,7 @@ def test_rows_of_one_huge_value(device, dtype):
     for i in range(17, 20):
         got, want = gpt.decode(int(tokens[i])), ref.forward(p, w, tokens[:i + 1])
         assert np.isfinite(want).all() and close(got, want), i
+    assert gpt.routes()[1] == 1
     gpt.unloadBuffers()
 
 
@@ -208,6 +215,7 @@ def test_int8_sums_beyond_the_range_of_fp32(device, inputs, product):
     for i in range(17, 20):
         got, want = gpt.decode(int(tokens[i])), ref.forward(prm, w, tokens[:i + 1])
         assert np.isfinite(want).all() and close(got, want), (i, worst(got, want))
+    assert gpt.routes()[1] == 1
     gpt.unloadBuffers()
 
 

@@ -75,6 +75,7 @@ struct Model {
   int pp_rows = 0;
   PrefillArgs pp{};
   unsigned pp_epoch = 0;       // last epoch of its earlier launches
+  int prefill_route = -1;      // wgpt_model_routes
   int pp_spoilt = 0;           // launches in a row that gave up on their prompt's values, and
   int pp_skip = 0;             // the prompts that are not tried on account of them
   int32_t* tok_pin = nullptr;  // pinned (behind ids_pin's): [PP_MAX_T] the prompt, then the word that a launch leaves its error in

@@ -855,6 +855,7 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
     if ((rc = forward_blocks(m, T, 0, true))) return rc;
     if ((rc = finish_timed(m, logits))) return rc;
   }
+  m->prefill_route = done;
   m->pos = T;
   m->tap_T = m->taps ? T : 0;
   m->x_rows = T;
@@ -1226,6 +1227,14 @@ int wgpt_model_set_decode_mode(wgpt_model h, int mode) {
     return fail(WGPT_ERR_STATE, "wgpt_model_set_decode_mode: the persistent decode path is not available for this model "
                                 "(needs 256 compute units, heads of at most 128, a width of at most 1792 and a context that its registers hold)");
   m->decode_mode = mode;
+  return WGPT_OK;
+}
+
+int wgpt_model_routes(wgpt_model h, int* prefill, int* decode) {
+  Model* m = find_model(h);
+  if (!m) return WGPT_ERR_ARG;
+  if (prefill) *prefill = m->prefill_route;
+  if (decode) *decode = m->decode_mode;
   return WGPT_OK;
 }
 

@@ -297,6 +297,12 @@ class GPT:
     def set_decode_mode(self, mode):
         _lib.call("wgpt_model_set_decode_mode", self._handle, int(mode))
 
+    def routes(self):
+        """(prefill, decode): whether the last prefill ran as one launch (-1: none yet), and the decode mode in use."""
+        prefill, decode = C.c_int(0), C.c_int(0)
+        _lib.call("wgpt_model_routes", self._handle, C.byref(prefill), C.byref(decode))
+        return prefill.value, decode.value
+
     def tune_poll_delays(self, rounds=2):
         """Searches the persistent decode kernel's seven poll delays on this GPU (wgpt_model_tune_poll_delays; needs
         position 0). Returns (delays, ms_per_token_before, ms_per_token_after)."""
