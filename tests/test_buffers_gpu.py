@@ -23,21 +23,37 @@ def test_downloads_of_any_length_and_offset(device, n):
 
 
 def test_buffers_freed_under_launches_that_read_them(device):
-    """Freed at once, handed out again and written while the launches that read them wait their turn on the stream."""
-    n = 1 << 20
-    ins, outs = [], []
-    for i in range(40):
-        a = RNG.standard_normal(n).astype(np.float32)
-        x, y = blocks.init_tensor(a, [n]), blocks.Buffer([n])
-        _lib.call("wgpt_residual", 1, n, x.handle, x.handle, y.handle)
+    """Buffers that the host has not written to (which the library keeps) given back and handed out again at once, and written by a later
+    launch, while the launch that reads them waits its turn on the stream: nothing in between uploads, downloads or waits."""
+    n, rounds = 1 << 20, 100
+    a, b = (RNG.standard_normal(n).astype(np.float32) for _ in range(2))
+    xa, xb = blocks.init_tensor(a, [n]), blocks.init_tensor(b, [n])
+    slow = [blocks.Buffer([16 * n]) for _ in range(2)]
+
+    def add(x, y, out, count=n):
+        _lib.call("wgpt_residual", 1, count, x.handle, y.handle, out.handle)
+
+    outs = []
+    for i in range(rounds):
+        if i % 10 == 0:  # (the launches of ten rounds take the device longer than the host)
+            for _ in range(8):
+                add(slow[0], slow[0], slow[1], 16 * n)
+        first, out = blocks.Buffer([n]), blocks.Buffer([n])
+        add(xa, xb if i % 2 else xa, first)
+        add(first, xb, out)
+        first.destroy()
+        again = blocks.Buffer([n])  # (a block of this size is there: the one that the launch above reads)
+        add(xb, xb, again)
+        again.destroy()
+        outs.append(out)
+        if len(outs) > 12:  # (so are results that nobody has asked for)
+            outs.pop(0).destroy()
+    for i, out in list(zip(range(rounds), [None] * (rounds - len(outs)) + outs)):
+        if out:
+            assert np.array_equal(out.download(), (a + (b if i % 2 else a)) + b), i
+            out.destroy()
+    for x in [xa, xb] + slow:
         x.destroy()
-        ins.append(a)
-        outs.append(y)
-        if i >= 20:
-            outs[i - 20].destroy()
-    for a, y in list(zip(ins, outs))[20:]:
-        assert np.array_equal(y.download(), a + a)
-        y.destroy()
 
 
 def test_ids_of_many_embeddings_under_way(device):
