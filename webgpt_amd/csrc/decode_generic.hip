@@ -356,6 +356,8 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
 #pragma unroll
       for (const float v : sums) all += fabsf(v);
       if (__builtin_expect(!(all < INFINITY), 0)) {
+#pragma unroll
+        for (auto& wt : w) wt.v = opaque(wt.v);  // (unpacked again: the floats would have to be kept for this)
         take(DOWN);
         keep(true);
       }
