@@ -2,8 +2,13 @@
 //
 // A token as one launch per block is 5 L + 3 dependent launches of 4 to 6 us, whatever they move (token_launches, model.hip).
 // us per token with launches and with this kernel, 40 positions and on (layers x width, head size): 4 x 576, 48, 111 -> 59, int8
-// 149 -> 59; 4 x 320, 16, 96 -> 52; 6 x 1280, 128, 251 -> 165 (480 MB of weights, 74 us at the rate of reads); 3 x 64, 16, 73 -> 40. What is left
-// are the five exchanges of a layer, 1 to 2 us each, the two of a step, and the latency of the phases between them.
+// 149 -> 59; 4 x 320, 16, 96 -> 52; 6 x 1280, 128, 251 -> 165 (480 MB of weights, 74 us at the rate of reads); 3 x 64, 16, 73 -> 40.
+// At the widest and at long contexts (four layers, position 100 and 900): 1600, 32, 197 and 205 -> 141 and 148, int8 240 and 248 -> 95 and 102;
+// 1792, 128, 205 and 239 -> 158 and 167, int8 242 and 275 -> 98 and 108; 1288, 92, 175 and 209 -> 124 and 132; 64, 16, 90 -> 57 (800).
+// What is left, as clock stamps of 4 x 576 have it: a layer is 13.7 us, of which 6.4 pass between the last word of an exchange and its readers
+// (0.8 the attention's, 1.0 to 1.7 each other one), 5.3 are the phases (1.9 the attention, 1.2 c_fc, 1.0 c_attn, 0.5 and 0.7 the projections), 2.0
+// workgroups behind the median one; a step's end is 6.3. The compiler spills 144 to 191 scalar registers into vector lanes, and of fp32
+// rows above 1280 7 vector registers (sampled 28) to scratch.
 // Here one workgroup per compute unit stays for all steps and the blocks are phases of it, as in decode_persistent.hip, whose
 // phases are compiled for one width and heads of 64 each. This kernel has its geometry in registers; only the number of 256-wide
 // segments of a row (NS) and the key rows that a wave holds (R) are compile-time, so that weights and keys have registers:
@@ -41,7 +46,11 @@ constexpr int NT = PD_THREADS, NW = NT / 64, G = PD_GRID;
 constexpr int SEG = 256;                          // contraction elements of a slab item
 template <int N>
 using Count = std::integral_constant<int, N>;
-constexpr int POLL = SC1 | (int)0x80000000;       // device scope, volatile
+// Polls: volatile, which makes them system scope (sc0 sc1). A poll sees a word that another XCD's compute unit has stored at device scope
+// because neither the L1 nor a stale line of its own L2 answers it, and it is made again in every round because the loops also hold relaxed
+// atomic loads, across which the compiler moves no read (a loop of nothing but such loads is one load: volatile or not, it is a plain
+// read of memory to the compiler).
+constexpr int POLL = SC1 | (int)0x80000000;
 
 template <int CTRL, int ROWS>
 __device__ __forceinline__ float dpp_add(float v) {
@@ -833,6 +842,7 @@ hipError_t launch_any(const PersistentArgs& a, hipStream_t s) {
 
 bool decode_generic_supports(int d, int H, int hs, int ctx, int V, int compute_units) {
   if (compute_units < G || d % 8 || hs % 4 || hs > 128 || d > 1792 || H * hs != d || H > G || run_bytes(V) > MAX_LDS) return false;
+  // (every width and dtype of this range, at short and long contexts, is faster than with launches: the figures above)
   // a slice's keys fit the registers of its workgroup
   const int lpk = hs <= 16 ? 4 : hs <= 32 ? 8 : hs <= 64 ? 16 : 32, most = H * DG_SPLIT <= G ? DG_SPLIT : G / H;
   return ctx <= most * (hs <= 64 ? 4 : 8) * NW * (64 / lpk);

@@ -410,7 +410,9 @@ static int setup_persistent(Model* m) {
                                     {8, 12, 22, 84, 20, 12, 44},    // d = 1600, int8
                                     {32, 0, 48, 96, 4, 20, 40},     // d = 1600, fp32
                                     {20, 4, 22, 78, 16, 16, 32},    // d = 384: 51.1 us per token against 55.0 with d = 768's
-                                    {12, 4, 22, 48, 12, 12, 32}};   // the kernel of any shape
+                                    // the kernel of any shape: a search around them gains nothing at widths of 64, 320, 576, 1280 and
+                                    // 1792, contexts of 512 and 1024, and 0.5 % at 1600, int8
+                                    {12, 4, 22, 48, 12, 12, 32}};
     // growth of [2] and [3] per 1024 positions of context (the best values at contexts of 100, 350, 650 and 900
     // positions lie on a line: 117M 80, 88, 88, 104 for [3]; int8 88, 104, 128, 136)
     static const int slopes[7][2] = {{11, 28}, {0, 46}, {9, 70}, {20, 61}, {0, 0}, {11, 28}, {0, 0}};

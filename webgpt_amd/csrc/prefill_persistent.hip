@@ -3,10 +3,12 @@
 // A launch per block costs a short prompt 3 to 5 us of fixed time for each of its 7 or 8 dependent launches a layer, more than
 // its operations and bytes (117M, 13 tokens: 86 launches in 0.50 ms for 340 MB of weights, 52 us at the rate of reads).
 // Calls of wgpt_prefill with launches and with this kernel, ms: 117M 1 token 0.50 -> 0.42, 13 0.55 -> 0.42, 64 0.67 -> 0.47,
-// 128 0.79 -> 0.58; 345M 100 1.72 -> 1.44; 774M 64 2.59 -> 2.12; 1.5B int8 16 2.54 -> 2.20; toy 64 0.28 -> 0.17. A layer of 117M is
-// 28 us at 13 rows: five hops of 1.5 to 2 us (stores to the common level 0.4, flag to reader 0.5, weights in front of the look
-// at it), 5.6 the second MLP product (a compute unit reads all hidden rows for four columns), 4.2 the attention, 1 to 1.4 each
-// other product; 42 us at 128 rows, 24 of them in products at two thirds of the matrix units' rate.
+// 128 0.79 -> 0.58; 345M 100 1.72 -> 1.44; 774M 64 2.59 -> 2.12; 1.5B int8 16 2.54 -> 2.20; toy 64 0.28 -> 0.17. Clock stamps of a layer of
+// 117M, which is 30 us with them at 13 rows and 43 at 128: from the last flag to the end of a wait 0.3 to 1.4 us (0.4 to 1.4 at 128 rows), sums,
+// epilogue, stores and the flag 0.8 to 1.1 a phase (0.6 to 1.2), loads with LayerNorm and products c_attn 2.5 (7.3), attention 2.7 (4.0), c_proj
+// 2.1 (2.4), c_fc 3.1 (8.6), the second MLP product 5.7 (9.1; at 13 rows a compute unit reads all hidden rows for four columns), the last workgroup 0.6
+// to 2.4 behind the median. The matrix units are busy for 11 % of the launch at 13 rows and 31 % at 128: 14 us a layer of the 27 in its products.
+// The compiler spills 218 to 329 scalar registers into vector lanes.
 // Here one workgroup per compute unit stays for the whole forward and the blocks are phases of it:
 //
 //   - workgroups form a grid of row groups (16 rows of the prompt, the rows of a matrix instruction) times column groups;
@@ -30,7 +32,9 @@
 // values, which later row groups read too, have rows of their own in the cache.
 //
 // Every wait is bounded. A wait that expires, and sums that the split may have spoilt (spoilt, gemm_split.hip), end the launch
-// early with a word for the host, which then runs the prompt with a launch per block.
+// early with a word for the host, which then runs the prompt with a launch per block. A flag is looked at with relaxed atomic loads at device
+// scope, and the rows behind it are read with device-scope loads (sc1) that the compiler cannot move above them; they were stored
+// at that scope and had arrived (s_waitcnt) before the flag was raised.
 #include "prefill_persistent.h"
 
 #include "persistent_common.h"
