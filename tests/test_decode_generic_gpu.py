@@ -239,3 +239,28 @@ def test_expired_wait_in_a_search_of_delays(device, monkeypatch):
         gpt.unloadBuffers()
     assert np.array_equal(rows[0], rows[1])
     assert close(rows[0], ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens[:13]))
+
+
+@pytest.mark.parametrize("vocab_size", [301, 5003])
+def test_logits_that_are_no_numbers_hide_no_others(device, vocab_size):
+    """Every second token's embedding is NaN, and so is its logit: greedy steps choose among the others, as the selection for sampling does."""
+    cfg = small_cfg(n_layer=2, n_head=4, n_embd=128, n_ctx=64, vocab_size=vocab_size)
+    tensors = make_model(cfg, 3)
+    wte = tensors["transformer.wte.weight"].copy()
+    wte[2::2] = np.nan
+    tensors["transformer.wte.weight"] = wte
+    gpt = load(cfg, tensors)
+    gpt.set_decode_mode(1)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    history = [int(t) // 2 * 2 - 1 for t in synth.tokens(9, "prompt", 12, vocab_size) if t > 1]
+    gpt.prefill(history[:-1])
+    got = [int(t) for t in gpt.decode_greedy(history[-1], 4)]
+    gpt.prefill(history[:-1])
+    sampled = [int(t) for t in gpt.decode_sample(history[-1], 4, 1, 0.8, np.full(4, 0.5))]
+    assert gpt.routes()[1] == 1
+    with np.errstate(all="ignore"):
+        for t in got:
+            assert t == int(np.nanargmax(ref.forward(p, w, np.array(history, np.int32))))
+            history.append(t)
+    assert sampled == got
+    gpt.unloadBuffers()

@@ -671,7 +671,7 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
 #pragma unroll
         for (int i = 0; i < RV; ++i)
           if (v + i < v1) {
-            if (!SAMPLE && (besti == 0x7fffffff || z[i] > best)) best = z[i], besti = v + i;
+            if (!SAMPLE && (z[i] > best || (besti == 0x7fffffff && z[i] == z[i]))) best = z[i], besti = v + i;  // (NaN: never)
             if ((SAMPLE || ends) && lane == 0) run[v + i - v0] = z[i];
           }
       }
