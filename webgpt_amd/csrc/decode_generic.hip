@@ -211,6 +211,7 @@ __device__ __forceinline__ void nap(int units) {  // about 64 clocks each
 template <bool I8, int NS, int R, bool SAMPLE>
 __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
   constexpr int CWA = (3 * NS + NW - 1) / NW, CWD = (4 * NS + NW - 1) / NW;  // columns of a wave, segments of a wave of the 4d-long row
+  constexpr int FULL = NS == 7 ? 5 : NS - 1;                                 // segments that every width of this instantiation fills (launch_any)
   constexpr int PW = Weight<I8>::BYTES;
   constexpr int NP = (NS * SEG / 2 + NT - 1) / NT;                           // pairs of words of a row per thread
   extern __shared__ __attribute__((aligned(16))) float run[];                // this workgroup's logits
@@ -340,12 +341,12 @@ __global__ __launch_bounds__(NT, 2) void decode_generic_kernel(PersistentArgs) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const float e0 = x[s][0] - mean, e1 = x[s][1] - mean, e2 = x[s][2] - mean, e3 = x[s][3] - mean;
-      q += SEG * s + e0l < d ? (e0 * e0 + e1 * e1) + (e2 * e2 + e3 * e3) : 0.f;
+      q += s < FULL || SEG * s + e0l < d ? (e0 * e0 + e1 * e1) + (e2 * e2 + e3 * e3) : 0.f;
     }
     const float stdev = sqrtf(wave_total(q) / fd + 1e-5f), rstd = 1.0f / stdev;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const float r = SEG * s + e0l < d ? rstd : 0.f;  // (beyond d the weights are zero, and so is x, whatever the mean)
+      const float r = s < FULL || SEG * s + e0l < d ? rstd : 0.f;  // (beyond d the weights are zero, and so is x, whatever the mean)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float v = quotient(x[s][e] - mean, stdev, r);
