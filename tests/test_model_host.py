@@ -139,6 +139,21 @@ for _ in range(3):
 assert made < 300 - 128, made
 assert [window(10) for _ in range(60)][-1] == 0  # and makes room when nobody asks for it any more
 assert allocs.value - frees.value - own <= 256, (allocs.value, frees.value)
+
+# out of memory: what is kept is given back, then the size that was asked for is enough
+h = C.c_uint64(0)
+_lib.call("wgpt_shutdown")
+_lib.init(0)
+alloc_fail_at.value = allocs.value + 1
+_lib.call("wgpt_alloc", 1000001, C.byref(h))   # nothing kept: a block of fewer bytes
+size = C.c_size_t(0)
+_lib.call("wgpt_buf_size", h, C.byref(size))
+assert size.value == 1000001
+_lib.call("wgpt_free", h)
+before, alloc_fail_at.value = frees.value, allocs.value + 1
+_lib.call("wgpt_alloc", 2000001, C.byref(h))
+assert frees.value == before + 1
+_lib.call("wgpt_free", h)
 """)
 
 
