@@ -1,0 +1,98 @@
+"""Longer prompts, whose products are made of pairs of fp16 values (csrc/gemm_pair.hip), against the CPU oracle: edges of the tiles'
+rows and columns, widths of no whole run of sixteen, both weight dtypes, and models whose weights the pairs cannot take."""
+import numpy as np
+import pytest
+
+from oracle import ref
+from webgpt_amd import _lib, synth
+from webgpt_amd.model import GPT
+
+from helpers import close, make_model, oracle_weights, small_cfg, worst
+
+pytestmark = pytest.mark.gpu
+
+FLAG_TAPS = 1
+
+
+def load(cfg, tensors, flags=0):
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg), flags=flags)
+    gpt.initialize()
+    return gpt
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head", [(512, 8), (520, 13), (576, 12), (1288, 23), (1608, 67)])
+def test_prompts_against_oracle(device, dtype, d, n_head):
+    """Logits, cache rows and residual rows, of one model in turn: a longer prompt's rows are left behind a shorter one's. Widths of
+    sixteen and of eight, heads of 64, 40, 48, 56 and 24. A model that keeps taps runs the other products: other last bits."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=260, vocab_size=301, dtype=dtype)
+    tensors = make_model(cfg, d)
+    gpt, taps = load(cfg, tensors), load(cfg, tensors, FLAG_TAPS)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (129, 257, 160, 193, 161, 192):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        want, all_taps, kv = ref.forward(p, w, tokens, want_taps=True, want_kv=True)
+        got = gpt.prefill(tokens)
+        assert close(got, want), (T, worst(got, want))
+        assert not np.array_equal(got, taps.prefill(tokens)), T
+        for i in range(2):
+            for j, name in enumerate("kv"):
+                assert close(gpt.tap(f"kv{i}_{name}"), kv[i, j]), (T, i, name)
+        rows, exp = gpt.tap("residual", T), all_taps[ref.tap_names(2).index("block1_r2")]
+        # (a sum of five values of the rows' size: near zero its error is theirs)
+        assert close(rows, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T
+    gpt.unloadBuffers()
+    taps.unloadBuffers()
+
+
+def spoil(tensors, how):
+    name = "transformer.h.1.mlp.c_fc.weight"
+    t = {k: v.copy() for k, v in tensors.items()}
+    if how == "infinite":
+        t[name][3, 5] = np.inf
+    elif how == "tiny columns":  # all but one weight of a column 2^-30 of that one
+        t[name][1:, 7] *= np.float32(2.0 ** -30)
+    elif how == "tiny":
+        t[name] *= np.float32(2.0 ** -100)
+    elif how == "gamma":
+        t["transformer.h.0.ln_2.weight"][1:] *= np.float32(2.0 ** -20)
+    elif how == "large":  # a bound beyond what the rows' scales reach
+        t["transformer.h.1.mlp.c_fc.bias"][0] = 2.0 ** 70
+    return t
+
+
+@pytest.mark.parametrize("how", ["infinite", "tiny columns", "tiny", "gamma", "large"])
+def test_weights_beyond_the_pairs(device, how):
+    """Found when the model is loaded: bit for bit the results of the products of a model that keeps taps."""
+    cfg = small_cfg(n_layer=2, n_head=8, n_embd=512, n_ctx=140, vocab_size=101)
+    tensors = spoil(make_model(cfg, 3), how)
+    tokens = synth.tokens(3, "prompt", 140, cfg["vocab_size"])
+    gpt, taps = load(cfg, tensors), load(cfg, tensors, FLAG_TAPS)
+    got, want = gpt.prefill(tokens), taps.prefill(tokens)
+    # (the LayerNorm in front of a product is a pass of its own where there are taps: equal to rounding, not to the last bit)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and close(got[~np.isnan(want)], want[~np.isnan(want)])
+    gpt.unloadBuffers()
+    taps.unloadBuffers()
+
+
+def test_rows_that_are_no_numbers(device):
+    """An embedding that is infinite makes its row's logits and those of the rows behind it NaN, and none of the tiles before it; the next
+    prompt is not affected by what was left in the rows' memory."""
+    cfg = small_cfg(n_layer=2, n_head=8, n_embd=512, n_ctx=300, vocab_size=101)
+    tensors = make_model(cfg, 4)
+    clean = load(cfg, tensors)
+    bad = {k: v.copy() for k, v in tensors.items()}
+    bad["transformer.wte.weight"][100, 9] = np.inf
+    gpt = load(cfg, bad)
+    tokens = [int(t) % 100 for t in synth.tokens(4, "prompt", 299, cfg["vocab_size"])]
+    spoilt = list(tokens)
+    spoilt[150] = 100
+    want = clean.prefill(tokens[:200])[:100]
+    assert np.isnan(gpt.prefill(spoilt)[:100]).all()
+    assert np.isnan(gpt.tap("residual", 299)[151:]).any(axis=1).all() and np.isfinite(gpt.tap("residual", 299)[:128]).all()
+    for T in (200, 150):
+        got = gpt.prefill(tokens[:T])[:100]
+        assert np.isfinite(got).all() and np.array_equal(got, clean.prefill(tokens[:T])[:100])
+    assert np.array_equal(gpt.prefill(tokens[:200])[:100], want)
+    gpt.unloadBuffers()
+    clean.unloadBuffers()

@@ -12,7 +12,7 @@
 #include <cmath>
 
 #include "kernels.h"
-#include "split_bf16.h"
+#include "pair_f16.h"
 
 namespace wgpt {
 namespace {
@@ -30,8 +30,14 @@ struct AttnSplitArgs {
   int ldkv;
   float* out;
   int ldo;
+  PairRows pairs;
   u32x4 *Q3, *K3, *V3;  // [H][block or tile][KS steps][3 parts][64 lanes]
 };
+
+__device__ __forceinline__ void put(const AttnSplitArgs& a, int row, int h, int dim, float v) {
+  if (a.pairs.rows) put_pair(a.pairs.rows, a.pairs.K16, row, h * a.hs + dim, v * a.pairs.scale);
+  else a.out[(size_t)row * a.ldo + (size_t)h * a.hs + dim] = v;
+}
 
 // Operands of one block of queries or tile of keys: unit (step, part, lane) of 16 bytes holds the eight values that the lane
 // supplies to the step. q and K: row lane % 32, dimensions 16 step + 8 (lane / 32) ..; V: dimension 32 (step / 2) + lane % 32,
@@ -226,7 +232,7 @@ __device__ __forceinline__ void plain_rows(const AttnSplitArgs& a, int h, int q0
       if (tid < a.hs) {
         float o = 0.f;
         for (int g = 0; g < ngrp; ++g) o += red[g * lpk + (tid >> 2)][tid & 3];
-        a.out[(size_t)row[u] * a.ldo + (size_t)h * a.hs + tid] = l[u] < INFINITY ? o / l[u] : NAN;
+        put(a, row[u], h, tid, l[u] < INFINITY ? o / l[u] : NAN);
       }
       __syncthreads();
     }
@@ -382,7 +388,7 @@ __global__ __launch_bounds__(NWV * 64, NWV / 4) void attention_split_kernel(Attn
       lo = fminf(lo, as_lds[w * WAVE_FLOATS + DIMS * AS_MERGE + 2 * ASQ + qi]);
     }
     const float v = num / den;
-    a.out[(size_t)(q0 + qi) * a.ldo + (size_t)h * a.hs + dim] = v;
+    put(a, q0 + qi, h, dim, v);
     // twice the bits, so without the sign: not finite, or under 2^-60 and no zero (far keys: under 2^-20, or zero)
     constexpr unsigned HI = 0xff000000u;
     const bool far = lo < M - AS_FAR;
@@ -416,9 +422,9 @@ size_t attention_split_bytes(int Tq, int pos0, int H, int hs) {
 }
 
 hipError_t launch_attention_split(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc, const float* Vc,
-                                  size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s) {
+                                  size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s, const PairRows* pairs) {
   if (hs > 128 || (hs & 3) || H > 65535) return hipErrorInvalidValue;
-  AttnSplitArgs a{Tq, pos0, H, hs, (Tq + ASQ - 1) / ASQ, (pos0 + Tq + ASQ - 1) / ASQ, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, nullptr, nullptr, nullptr};
+  AttnSplitArgs a{Tq, pos0, H, hs, (Tq + ASQ - 1) / ASQ, (pos0 + Tq + ASQ - 1) / ASQ, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, pairs ? *pairs : PairRows{}, nullptr, nullptr, nullptr};
   const int DB = (hs + 31) / 32;
   const size_t unit = (size_t)2 * DB * 192;
   a.Q3 = static_cast<u32x4*>(ws);

@@ -68,14 +68,20 @@ hipError_t launch_vocab_gemv(int V, int d, const float* x, const float* wte, flo
 // Causal attention of Tq query rows (absolute positions pos0..pos0+Tq-1) against
 // keys/values 0..pos. q row i is at q + i*ldq + h*hs; key row j of head h is at
 // Kc + h*hstride + j*ldkv (likewise values).
-// ws: attention_workspace_bytes of memory (may be null where that is 0).
+// ws: attention_workspace_bytes of memory (may be null where that is 0). pairs: the rows, times its scale, as pairs (pair_f16.h)
+// instead of floats at `out`; Tq from 32 on.
+struct PairRows {
+  void* rows;
+  int K16;
+  float scale;
+};
 size_t attention_workspace_bytes(int Tq, int pos0, int H, int hs);
 hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc,
-                            const float* Vc, size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s);
+                            const float* Vc, size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s, const PairRows* pairs = nullptr);
 // The same on the bf16 matrix cores (attention_split.hip), hs a multiple of 4 up to 128; ws: attention_split_bytes.
 size_t attention_split_bytes(int Tq, int pos0, int H, int hs);
 hipError_t launch_attention_split(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc, const float* Vc,
-                                  size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s);
+                                  size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s, const PairRows* pairs = nullptr);
 // Top-k / temperature / inverse-CDF selection of one token on the device (globals.js:47-74,
 // model.js:81-85); *u is the uniform draw, device memory. tok[0] and out[slot] (optional) get
 // the id, ids[k] / probs[k] (optional) the selected indices and their probabilities.

@@ -9,6 +9,7 @@
 
 #include "../../include/webgpt_amd.h"
 #include "decode_persistent.h"
+#include "gemm_pair.h"
 #include "prefill_persistent.h"
 
 namespace wgpt {
@@ -25,6 +26,14 @@ struct LayerW {
   float *ln1_g = nullptr, *ln1_b = nullptr, *ln2_g = nullptr, *ln2_b = nullptr;
   LinW attn, proj, fc, fc2;  // c_attn [d,3d], c_proj [d,d], c_fc [d,4d], mlp c_proj [4d,d]
   float *attn_b = nullptr, *proj_b = nullptr, *fc_b = nullptr, *fc2_b = nullptr;
+};
+
+// One layer's weights as pairs of fp16 values (int8 ones stay in LinW), what their products' columns are multiplied with, and the
+// scales of the rows: behind the two LayerNorms, the attention and the GELU.
+struct PairLayer {
+  void *wA = nullptr, *wC = nullptr, *wD = nullptr, *wE = nullptr;
+  float *cA = nullptr, *cC = nullptr, *cD = nullptr, *cE = nullptr;
+  float s1 = 1.f, sv = 1.f, s2 = 1.f, sh = 1.f;
 };
 
 struct Model {
@@ -78,6 +87,9 @@ struct Model {
   int prefill_route = -1;      // wgpt_model_routes
   int pp_spoilt = 0;           // launches in a row that gave up on their prompt's values, and
   int pp_skip = 0;             // the prompts that are not tried on account of them
+  // prompts beyond those: products of pairs of fp16 values, where the weights allow (empty: they do not)
+  std::vector<PairLayer> pairs;
+  void *pair_ln = nullptr, *pair_att = nullptr, *pair_h = nullptr;  // rows of up to maxT tokens
   int32_t* tok_pin = nullptr;  // pinned (behind ids_pin's): [PP_MAX_T] the prompt, then the word that a launch leaves its error in
 
   // decode with one launch per block (decode_mode 0): the token's launches read the cache position from pos_dev and

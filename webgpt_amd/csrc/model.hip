@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "decode_generic.h"
+#include "gemm_pair.h"
 #include "gemm_split.h"
 #include "kernels.h"
 #include "model.h"
@@ -175,6 +176,61 @@ static int forward_blocks(Model* m, int T, int pos0, bool want_taps) {
     // Only the last row is de-embedded (instructions.js:849-856).
     LAUNCH(launch_vocab_gemv_ln(m->V, d, m->x + (size_t)(T - 1) * d, m->lnf_g, m->lnf_b, m->wte, m->logits, nullptr, s));
   }
+  return WGPT_OK;
+}
+
+// The same forward with products of pairs of fp16 values (gemm_pair.hip); positions 0 .. T - 1, no taps.
+static int forward_pairs(Model* m, int T) {
+  hipStream_t s = rt().stream;
+  const int d = m->d, H = m->H, hs = m->hs, hid = 4 * d;
+  const bool i8 = m->p.weight_dtype == 1;
+  const float scale = (float)(1.0 / std::sqrt((double)hs));  // model.js:321
+  const PairPlan plA = plan_gemm_pair(T, 3 * d, d, i8, false), plC = plan_gemm_pair(T, d, d, i8, true);
+  const PairPlan plD = plan_gemm_pair(T, hid, d, i8, false), plE = plan_gemm_pair(T, d, hid, i8, true);
+  LAUNCH(launch_embed(m->tok_dev, T, d, 0, m->wte, m->wpe, m->x, s));
+  PairLnArgs ln{T, d, 0, m->part, nullptr, m->x, m->layers[0].ln1_g, m->layers[0].ln1_b, m->pairs[0].s1, m->pair_ln};
+  LAUNCH(launch_ln_pair(ln, s));
+  for (int li = 0; li < m->L; ++li) {
+    const LayerW& l = m->layers[li];
+    const PairLayer& p = m->pairs[li];
+    PairGemmArgs g{};
+    g.M = T; g.N = 3 * d; g.K = d;
+    g.A = m->pair_ln; g.W = i8 ? (const void*)l.attn.q : p.wA; g.cscale = p.cA; g.bias = l.attn_b;
+    g.end = PAIR_QKV;
+    g.C = m->qkv; g.ldc = 3 * d;
+    g.Kc = m->kv + ((size_t)li * 2 + 0) * m->ctx * d; g.Vc = m->kv + ((size_t)li * 2 + 1) * m->ctx * d;
+    g.d = d; g.hs = hs; g.ctx = m->ctx;
+    LAUNCH(launch_gemm_pair(plA, g, i8, s));
+    const PairRows rows = {m->pair_att, pair_k16(d), p.sv};
+    LAUNCH(launch_attention(T, 0, H, hs, scale, m->qkv, 3 * d, g.Kc, g.Vc, (size_t)m->ctx * hs, hs, nullptr, d, m->att_ws, s, &rows));
+    // the two projections leave x finished, or slices that the LayerNorm's pass sums
+    const auto project = [&](const PairPlan& pl, int K, const void* A, const LinW& w, const void* wp, const float* cs, const float* bias) {
+      PairGemmArgs c{};
+      c.M = T; c.N = d; c.K = K;
+      c.A = A; c.W = i8 ? (const void*)w.q : wp; c.cscale = cs; c.bias = bias;
+      c.end = pl.S > 1 ? PAIR_PART : PAIR_RESIDUAL;
+      c.C = m->x; c.ldc = d; c.resid = m->x; c.part = m->part;
+      ln.S = pl.S > 1 ? pl.S : 0;
+      ln.bias = bias;
+      return launch_gemm_pair(pl, c, i8, s);
+    };
+    LAUNCH(project(plC, d, m->pair_att, l.proj, p.wC, p.cC, l.proj_b));
+    ln.gamma = l.ln2_g; ln.beta = l.ln2_b; ln.scale = p.s2;
+    LAUNCH(launch_ln_pair(ln, s));
+    PairGemmArgs f{};
+    f.M = T; f.N = hid; f.K = d;
+    f.A = m->pair_ln; f.W = i8 ? (const void*)l.fc.q : p.wD; f.cscale = p.cD; f.bias = l.fc_b;
+    f.end = PAIR_GELU;
+    f.P = m->pair_h; f.pscale = p.sh;
+    LAUNCH(launch_gemm_pair(plD, f, i8, s));
+    LAUNCH(project(plE, hid, m->pair_h, l.fc2, p.wE, p.cE, l.fc2_b));
+    const bool last = li + 1 == m->L;
+    if (last && !ln.S) break;
+    ln.out = last ? nullptr : m->pair_ln;
+    if (!last) ln.gamma = m->layers[li + 1].ln1_g, ln.beta = m->layers[li + 1].ln1_b, ln.scale = m->pairs[li + 1].s1;
+    LAUNCH(launch_ln_pair(ln, s));
+  }
+  LAUNCH(launch_vocab_gemv_ln(m->V, d, m->x + (size_t)(T - 1) * d, m->lnf_g, m->lnf_b, m->wte, m->logits, nullptr, s));
   return WGPT_OK;
 }
 
@@ -617,6 +673,93 @@ static int block_linear_weights(Model* m, void* free_buf) {
   return WGPT_OK;
 }
 
+// Narrowest rows whose products are made of pairs: below, their sums would be further from exact ones than those of three bf16
+// values each (gemm_pair.hip).
+constexpr int PAIR_MIN_D = 512;
+constexpr int PAIR_MIN_T = 64;
+
+// Prepares forward_pairs (before block_linear_weights: it reads the matrices as they came). Leaves m->pairs empty, and forward_blocks
+// in charge, where the weights do not allow it or memory has run out.
+static int setup_pairs(Model* m) {
+  const int d = m->d, hid = 4 * d, L = m->L;
+  const bool i8 = m->p.weight_dtype == 1;
+  m->pairs.clear();
+  if (d < PAIR_MIN_D || (m->p.flags & WGPT_FLAG_TAPS)) return WGPT_OK;
+  const auto room = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+  const struct { int K, N; LinW LayerW::*w; void* PairLayer::*wp; float* PairLayer::*c; } lins[4] = {
+      {d, 3 * d, &LayerW::attn, &PairLayer::wA, &PairLayer::cA}, {d, d, &LayerW::proj, &PairLayer::wC, &PairLayer::cC},
+      {d, hid, &LayerW::fc, &PairLayer::wD, &PairLayer::cD}, {hid, d, &LayerW::fc2, &PairLayer::wE, &PairLayer::cE}};
+  size_t per_layer = 0;
+  for (const auto& t : lins) {
+    if (pair_weights_bytes(t.K, t.N) >= 0x80000000u) return WGPT_OK;
+    per_layer += (i8 ? 0 : room(pair_weights_bytes(t.K, t.N))) + room(sizeof(float) * (size_t)t.N);
+  }
+  const size_t row = room(pair_rows_bytes(m->maxT, d)), rowh = room(pair_rows_bytes(m->maxT, hid));
+  if (rowh >= 0x80000000u) return WGPT_OK;
+  const size_t stats_bytes = room(sizeof(unsigned) * (1 + 4 * (size_t)L));
+  char* base;
+  // (what only the loading needs lies in the rows' memory: they are cleared behind it)
+  const size_t sums_bytes = sizeof(float) * pair_bounds_floats(d, hid), few_bytes = i8 ? 0 : room(sizeof(int) * 9 * (size_t)d * L);
+  const size_t rows_bytes = std::max(2 * row + rowh, room(sums_bytes) + few_bytes);
+  if (dev_alloc(m, per_layer * L + rows_bytes + stats_bytes, (void**)&base)) return WGPT_OK;
+  char* const all = base;
+  const auto take = [&](size_t bytes) { char* p = base; base += bytes; return p; };
+  char* const rows = take(rows_bytes);
+  m->pair_ln = rows;
+  m->pair_att = rows + row;
+  m->pair_h = rows + 2 * row;
+  float* const sums = (float*)rows;
+  int* few = (int*)(rows + room(sums_bytes));
+  unsigned* stats = (unsigned*)take(stats_bytes);  // [0]: what the products cannot take; then the four bounds of each layer
+  WGPT_HIP(hipMemsetAsync(all, 0, per_layer * L + rows_bytes + stats_bytes, rt().stream));
+  std::vector<PairLayer> layers(L);
+  for (int i = 0; i < L; ++i) {
+    const LayerW& l = m->layers[i];
+    for (const auto& t : lins) {
+      const LinW& w = l.*t.w;
+      float* c = layers[i].*t.c = (float*)take(room(sizeof(float) * (size_t)t.N));
+      if (i8) {
+        LAUNCH(launch_pair_scales(t.N, w.s, c, stats, rt().stream));
+      } else {
+        layers[i].*t.wp = take(room(pair_weights_bytes(t.K, t.N)));
+        LAUNCH(launch_pair_weights(t.K, t.N, w.w, layers[i].*t.wp, c, few, stats, rt().stream));
+        few += t.N;
+      }
+    }
+    unsigned* b = stats + 1 + 4 * i;
+    LAUNCH(launch_pair_bounds(d, i8 ? 3 * d / 4 : 3 * d, 2 * d, 3 * d, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
+    LAUNCH(launch_pair_bounds(d, i8 ? hid / 4 : hid, 0, hid, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 3, b + 2, rt().stream));
+  }
+  std::vector<unsigned> host(1 + 4 * (size_t)L);
+  WGPT_HIP(hipMemcpyAsync(host.data(), stats, sizeof(unsigned) * host.size(), hipMemcpyDeviceToHost, rt().stream));
+  WGPT_HIP(hipStreamSynchronize(rt().stream));
+  bool ok = host[0] == 0;
+  for (int i = 0; i < L && ok; ++i) {
+    float* const s[4] = {&layers[i].s1, &layers[i].sv, &layers[i].s2, &layers[i].sh};
+    for (int j = 0; j < 4; ++j) {
+      float bound;
+      memcpy(&bound, &host[1 + 4 * i + j], sizeof bound);
+      ok = ok && (bound == 0.f || (bound > 0x1p-60f && bound < 0x1p60f));
+      int e = 0;
+      if (ok && bound > 0.f) (void)frexpf(bound * 1.001f, &e);  // (the bounds' own roundings, and those of the values)
+      *s[j] = ldexpf(1.f, 15 - e);
+    }
+  }
+  if (!ok) {
+    m->pair_ln = m->pair_att = m->pair_h = nullptr;
+    m->allocs.pop_back();
+    (void)hipFree(all);
+    return WGPT_OK;
+  }
+  for (int i = 0; i < L; ++i) {
+    const float s[4] = {layers[i].s1, layers[i].sv, layers[i].s2, layers[i].sh};
+    for (int j = 0; j < 4; ++j) LAUNCH(launch_pair_rescale(lins[j].N, 1.f / s[j], layers[i].*lins[j].c, rt().stream));
+  }
+  WGPT_HIP(hipMemsetAsync(rows, 0, rows_bytes, rt().stream));
+  m->pairs = std::move(layers);
+  return WGPT_OK;
+}
+
 // Prepares the persistent prefill in the buffers that wgpt_model_finalize has allocated for it; after block_linear_weights.
 static int setup_prefill(Model* m) {
   const bool i8 = m->p.weight_dtype == 1;
@@ -809,6 +952,7 @@ int wgpt_model_finalize(wgpt_model h) {
   if (!m->ev1) WGPT_HIP(hipEventCreate(&m->ev1));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   if ((rc = setup_persistent(m))) return rc;
+  if ((rc = setup_pairs(m))) return rc;
   m->weights_moved = true;
   if ((rc = block_linear_weights(m, block_buf))) return rc;
   WGPT_HIP(hipStreamSynchronize(rt().stream));  // (its errors are this call's)
@@ -854,7 +998,7 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
     WGPT_HIP(hipMemcpyAsync(m->tok_dev, tokens, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, rt().stream));
     WGPT_HIP(hipStreamSynchronize(rt().stream));
     WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
-    if ((rc = forward_blocks(m, T, 0, true))) return rc;
+    if ((rc = T > m->pp_rows && T >= PAIR_MIN_T && !m->pairs.empty() ? forward_pairs(m, T) : forward_blocks(m, T, 0, true))) return rc;
     if ((rc = finish_timed(m, logits))) return rc;
   }
   m->prefill_route = done;
