@@ -1,0 +1,66 @@
+"""The attention of longer prompts (csrc/attention_pair.hip) against the CPU oracle, by what it leaves in the residual stream: every number
+of 32-dimension blocks of a head, heads that fill part of one, both sides of the rule for the waves of a workgroup (16 tiles of 32 keys),
+ends of tiles; a shorter prompt behind a longer one. Heads that it does not take (12 dimensions), and q and keys whose scales do not fit."""
+import numpy as np
+import pytest
+
+from oracle import ref
+from webgpt_amd import synth
+from webgpt_amd.model import GPT
+
+from helpers import close, make_model, oracle_weights, small_cfg, worst
+
+pytestmark = pytest.mark.gpu
+
+
+def load(cfg, tensors, flags=0):
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg), flags=flags)
+    gpt.initialize()
+    return gpt
+
+
+@pytest.mark.parametrize("d,n_head", [(512, 64), (576, 48), (512, 16), (640, 16), (512, 8), (576, 6), (640, 5), (512, 4)])
+def test_rows_against_oracle(device, d, n_head):
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=552, vocab_size=201)
+    tensors = make_model(cfg, d + n_head)
+    gpt, w, p = load(cfg, tensors), oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (545, 512, 513, 130):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        want, all_taps, _ = ref.forward(p, w, tokens, want_taps=True, want_kv=True)
+        got = gpt.prefill(tokens)
+        assert close(got, want), (T, worst(got, want))
+        rows, exp = gpt.tap("residual", T), all_taps[ref.tap_names(2).index("block1_r2")]
+        assert close(rows, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T  # (near zero a sum's error is its terms')
+    gpt.unloadBuffers()
+
+
+def test_sharp_softmax(device):
+    """Scores of hundreds: almost all weights vanish, in other tiles than the largest."""
+    cfg = small_cfg(n_layer=1, n_head=8, n_embd=512, n_ctx=300, vocab_size=201)
+    tensors = make_model(cfg, 5)
+    tensors["transformer.h.0.attn.c_attn.weight"] = tensors["transformer.h.0.attn.c_attn.weight"].copy()
+    tensors["transformer.h.0.attn.c_attn.weight"][:, :1024] *= np.float32(12.0)
+    gpt, taps = load(cfg, tensors), load(cfg, tensors, flags=1)
+    tokens = synth.tokens(6, "prompt", 300, cfg["vocab_size"])
+    want = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens)
+    err = lambda m: float(np.max(np.abs(m.prefill(tokens) - want)))
+    # (scores of 300 lose 300 x 2^-24 to rounding, whoever makes them: no further off than a few times the other kernels')
+    assert err(gpt) <= 4 * err(taps) + 1e-6
+    gpt.unloadBuffers()
+    taps.unloadBuffers()
+
+
+def test_uneven_queries(device):
+    """Most columns of q far below the others: found when the model is loaded, which then runs the other products."""
+    cfg = small_cfg(n_layer=2, n_head=8, n_embd=512, n_ctx=140, vocab_size=101)
+    tensors = make_model(cfg, 3)
+    name = "transformer.h.1.attn.c_attn."
+    for end in ("weight", "bias"):
+        tensors[name + end] = tensors[name + end].copy()
+        tensors[name + end][..., 64:512] *= np.float32(2.0 ** -14)
+    tokens = synth.tokens(3, "prompt", 140, cfg["vocab_size"])
+    gpt, taps = load(cfg, tensors), load(cfg, tensors, flags=1)
+    assert close(gpt.prefill(tokens), taps.prefill(tokens))
+    assert close(gpt.prefill(tokens), ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens))
+    gpt.unloadBuffers()
+    taps.unloadBuffers()

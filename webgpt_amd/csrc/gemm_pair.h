@@ -19,6 +19,7 @@ inline size_t pair_weights_bytes(int K, int N) { return pair_rows_bytes(N, K); }
 enum PairEnd {
   PAIR_PART,      // slice s of K leaves its sums, scaled, at part + s * M * N
   PAIR_QKV,       // + bias; columns below d to C, the others to their rows of the cache
+  PAIR_HEADS,     // + bias; as operands of the attention to heads[] (attention_pair.h), keys and values to their rows of the cache too
   PAIR_RESIDUAL,  // + bias + resid to C
   PAIR_GELU,      // GELU(+ bias), scaled by `pscale`, as pairs to P
 };
@@ -34,6 +35,9 @@ struct PairGemmArgs {
   const float* resid;   // [M, ldc], may alias C
   float *Kc, *Vc;
   int d, hs, ctx;
+  void* heads[3];       // q, keys, values
+  int head_tiles;       // AttnPairArgs::tiles
+  float hscale[3], rhs; // the scales of q, keys, values; 1 / hs
   void* P;
   float pscale;
   float* part;
@@ -64,12 +68,13 @@ hipError_t launch_ln_pair(const PairLnArgs& a, hipStream_t s);
 hipError_t launch_pair_weights(int K, int N, const float* W, void* out, float* cscale, int* few, unsigned* stats, hipStream_t s);
 // cscale[n] = scale[n] / 127 of an int8 matrix; stats[0] as above.
 hipError_t launch_pair_scales(int N, const float* scale, float* cscale, unsigned* stats, hipStream_t s);
-// Largest absolute value that (LayerNorm with gamma and beta) . W + bias can have in columns n0 .. n1 of W [K, ldw] (int8: words of
-// four columns and scales), and that the LayerNorm itself can have: as maxima of floats' bits at *bound and *ln_bound (zeros before).
-// sums: pair_bounds_floats(K, n1 - n0) of memory.
+// Largest absolute value that (LayerNorm with gamma and beta) . W + bias can have in each of `runs` equal runs of the columns of W
+// [K, N] (int8: words of four columns and scales), and that the LayerNorm itself can have: as floats at bound[run] and *ln_bound.
+// Infinite where the run is one of the first `even` and more than one in 64 of its columns have bounds below 2^-10 of the largest.
+// sums: pair_bounds_floats(K, N) of memory.
 size_t pair_bounds_floats(int K, int N);
-hipError_t launch_pair_bounds(int K, int ldw, int n0, int n1, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
-                              const float* gamma, const float* beta, float* sums, unsigned* bound, unsigned* ln_bound, hipStream_t s);
+hipError_t launch_pair_bounds(int K, int N, int runs, int even, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
+                              const float* gamma, const float* beta, float* sums, float* bound, float* ln_bound, hipStream_t s);
 // cscale[n] *= factor (a power of two)
 hipError_t launch_pair_rescale(int N, float factor, float* cscale, hipStream_t s);
 

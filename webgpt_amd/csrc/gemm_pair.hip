@@ -28,6 +28,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "attention_pair.h"
 #include "pair_f16.h"
 #include "persistent_common.h"
 
@@ -46,6 +47,57 @@ __device__ __forceinline__ f32x16 mfma(const u32x4& w, const u32x4& a, const f32
 __device__ __forceinline__ unsigned f16_of_bytes(const unsigned (&v)[2], int q) {
   const unsigned x = __builtin_amdgcn_perm(0x64646464u, v[q >> 1] ^ 0x80808080u, q & 1 ? 0x04030402u : 0x04010400u);
   return __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, x) - f16x2{(_Float16)1152.f, (_Float16)1152.f});
+}
+
+// A lane's four values in a row become one value of each of its quad's four: element `lane % 4` of lanes 0 .. 3.
+__device__ __forceinline__ f32x4 transpose_quad(f32x4 v) {
+  const auto swap = [](float& a, float& b, bool odd, auto perm) {
+    const float got = __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(odd ? a : b), decltype(perm)::value, 0xf, 0xf, false));
+    (odd ? a : b) = got;
+  };
+  const bool o1 = threadIdx.x & 1, o2 = threadIdx.x & 2;
+  float e[4] = {v[0], v[1], v[2], v[3]};
+  const std::integral_constant<int, 0xB1> by1;
+  const std::integral_constant<int, 0x4E> by2;
+  swap(e[0], e[1], o1, by1);
+  swap(e[2], e[3], o1, by1);
+  swap(e[0], e[2], o2, by2);
+  swap(e[1], e[3], o2, by2);
+  return f32x4{e[0], e[1], e[2], e[3]};
+}
+__device__ __forceinline__ unsigned ror8(unsigned v) { return __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, false); }  // from lane ^ 8
+// Values of a q/k/v product, of row r of a block of rows and columns n8 + 4 half .. + 3: to the operands of attention_pair.hip, and keys
+// and values to the cache too. The eight columns at n8 are a wave's, of one head (d and hs are multiples of 8), so all but the lane's place
+// in them is scalar: with head, dimension and unit found by every lane the product of 512 x 3072 x 1024 took 20.2 us instead of 18.7.
+// The other half of a lane's unit is with the lane 32 on (q and keys: eight dimensions of a row) or 8 on (values: eight keys):
+// one of the two keeps the hi, the other the lo, and each writes 16 bytes.
+__device__ __forceinline__ void put_heads(const PairGemmArgs& a, int block, int r, int half, int n8, const f32x4& v) {
+  const int which = n8 < a.d ? 0 : n8 < 2 * a.d ? 1 : 2, e = n8 - which * a.d;
+  const int h = __builtin_amdgcn_readfirstlane(div_by(e, a.hs, a.rhs)), dim = e - h * a.hs;
+  if (which && block * 32 + r < a.M) {
+    float* const rows = (which == 2 ? a.Vc : a.Kc) + ((size_t)h * a.ctx + block * 32) * a.hs + dim;
+    *reinterpret_cast<f32x4*>(rows + (r * a.hs + 4 * half)) = v;
+  }
+  f32x4 x = v * (which == 0 ? a.hscale[0] : which == 1 ? a.hscale[1] : a.hscale[2]);
+  u32x4* const units = static_cast<u32x4*>(which == 0 ? a.heads[0] : which == 1 ? a.heads[1] : a.heads[2]) +
+                       (size_t)(h * a.head_tiles + block) * (pair_attn_steps(a.hs) * 128);
+  unsigned hi[2], lo[2];
+  if (which == 2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = fabsf(x[i]) < INFINITY ? x[i] : 0.f;
+    x = transpose_quad(x);  // four keys of a dimension
+    pair_f16(x[0], x[1], hi[0], lo[0]);
+    pair_f16(x[2], x[3], hi[1], lo[1]);
+    const bool low = r & 8;
+    const unsigned g0 = ror8(low ? hi[0] : lo[0]), g1 = ror8(low ? hi[1] : lo[1]);
+    units[(dim >> 5) * 256 + (dim & 31) + ((r >> 4) * 128 + (low ? 64 : 0) + ((r >> 2) & 1) * 32 + 4 * half + (r & 3))] =
+        low ? u32x4{g0, g1, lo[0], lo[1]} : u32x4{hi[0], hi[1], g0, g1};
+  } else {
+    pair_f16(x[0], x[1], hi[0], lo[0]);
+    pair_f16(x[2], x[3], hi[1], lo[1]);
+    const auto s0 = __builtin_amdgcn_permlane32_swap(hi[0], lo[0], false, false), s1 = __builtin_amdgcn_permlane32_swap(hi[1], lo[1], false, false);
+    units[(dim >> 4) * 128 + ((dim >> 3) & 1) * 32 + (64 * half + r)] = u32x4{s0[0], s1[0], s0[1], s1[1]};
+  }
 }
 
 // MB x NB blocks of 32 rows and 32 columns. Two workgroups to a compute unit (three of the small tiles), which fill each other's waits.
@@ -202,6 +254,11 @@ __global__ __launch_bounds__(256, MB * NB <= 4 ? 3 : 2) void gemm_pair_kernel(Pa
       const auto s0 = __builtin_amdgcn_permlane32_swap(h[0], l[0], false, false), s1 = __builtin_amdgcn_permlane32_swap(h[1], l[1], false, false);
       if (m < a.M && n < a.N)
         static_cast<u32x4*>(a.P)[pair_unit(m, n & ~7, (a.N + 15) >> 4) + 64 * half] = u32x4{s0[0], s1[0], s0[1], s1[1]};
+      continue;
+    }
+    if (a.end == PAIR_HEADS) {
+      const int n8 = (ni * NB + j) * 32 + 8 * wave;
+      if (mi * MB + b / NB < a.row_blocks && n8 < a.N) put_heads(a, mi * MB + b / NB, r, half, n8, v);  // (rows beyond the last have their place in its block)
       continue;
     }
     if (m >= a.M || n >= a.N) continue;
@@ -388,20 +445,20 @@ __global__ __launch_bounds__(256) void pair_scales_kernel(int N, const float* __
   if (!in_range(scale[n])) atomicAdd(stats, 1u);
 }
 
-// |LN(x) . w + b| <= sqrt(K) |gamma w| + |beta . w + b|: the two sums of a chunk of a column at sums[chunk][column - n0]
-__global__ __launch_bounds__(256) void pair_bounds_kernel(int K, int ldw, int n0, int n1, const float* __restrict__ W, const int32_t* __restrict__ Wq,
+// |LN(x) . w + b| <= sqrt(K) |gamma w| + |beta . w + b|: the two sums of a chunk of a column at sums[chunk][column]
+__global__ __launch_bounds__(256) void pair_bounds_kernel(int K, int N, const float* __restrict__ W, const int32_t* __restrict__ Wq,
                                                           const float* __restrict__ wscale, const float* __restrict__ gamma, const float* __restrict__ beta,
                                                           float2* sums) {
   __shared__ float2 sh[8][32];
-  const ColumnChunk t(K, n0);
+  const ColumnChunk t(K, 0);
   float s = 0.f, d = 0.f;
-  if (t.n < n1) {
+  if (t.n < N) {
     const float ws = Wq ? wscale[t.n] / 127.0f : 1.f;
 #pragma unroll
     for (int i = 0; i < CHUNK / 8; ++i) {
       const int k = t.k0 + 8 * i + t.p;
       if (k >= t.k1) break;
-      const float w = Wq ? (float)((int)(Wq[(size_t)k * ldw + (t.n >> 2)] << (24 - 8 * (t.n & 3))) >> 24) * ws : W[(size_t)k * ldw + t.n];
+      const float w = Wq ? (float)((int)(Wq[(size_t)k * (N >> 2) + (t.n >> 2)] << (24 - 8 * (t.n & 3))) >> 24) * ws : W[(size_t)k * N + t.n];
       const float g = gamma[k] * w;
       s += g * g;
       d += beta[k] * w;
@@ -409,24 +466,43 @@ __global__ __launch_bounds__(256) void pair_bounds_kernel(int K, int ldw, int n0
   }
   sh[t.p][t.c] = make_float2(s, d);
   __syncthreads();
-  if (t.p || t.n >= n1) return;
+  if (t.p || t.n >= N) return;
 #pragma unroll
   for (int i = 1; i < 8; ++i) s += sh[i][t.c].x, d += sh[i][t.c].y;
-  sums[(size_t)blockIdx.y * (n1 - n0) + (t.n - n0)] = make_float2(s, d);
+  sums[(size_t)blockIdx.y * N + t.n] = make_float2(s, d);
 }
-__global__ __launch_bounds__(256) void pair_bounds_end(int K, int n0, int n1, const float* __restrict__ bias, const float2* __restrict__ sums, unsigned* bound) {
-  const int n = n0 + (int)blockIdx.x * 256 + threadIdx.x;
-  if (n >= n1) return;
-  float s = 0.f, d = 0.f;
-  for (int i = 0; i * CHUNK < K; ++i) {
-    const float2 p = sums[(size_t)i * (n1 - n0) + (n - n0)];
-    s += p.x, d += p.y;
+// A workgroup per run of n columns.
+__global__ __launch_bounds__(1024) void pair_bounds_end(int K, int N, int n, int even, const float* __restrict__ bias, float2* sums, float* bound) {
+  __shared__ unsigned most;
+  __shared__ int low;
+  if (threadIdx.x == 0) most = 0u, low = 0;
+  __syncthreads();
+  const int n0 = (int)blockIdx.x * n;
+  float top = 0.f;
+  for (int c = n0 + threadIdx.x; c < n0 + n; c += 1024) {
+    float s = 0.f, d = 0.f;
+    for (int i = 0; i * CHUNK < K; ++i) {
+      const float2 p = sums[(size_t)i * N + c];
+      s += p.x, d += p.y;
+    }
+    float b = sqrtf((float)K * s) + fabsf(d + bias[c]);
+    b = b < INFINITY ? b : INFINITY;
+    sums[c].x = b;  // (this thread's own)
+    top = fmaxf(top, b);
   }
-  const float b = sqrtf((float)K * s) + fabsf(d + bias[n]);
-  atomicMax(bound, b < INFINITY ? __float_as_uint(b) : __float_as_uint(INFINITY));
+  atomicMax(&most, __float_as_uint(top));
+  __syncthreads();
+  top = __uint_as_float(most);
+  if ((int)blockIdx.x < even) {
+    int few = 0;
+    for (int c = n0 + threadIdx.x; c < n0 + n; c += 1024) few += sums[c].x != 0.f && sums[c].x < 0x1p-10f * top;
+    if (few) atomicAdd(&low, few);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) bound[blockIdx.x] = 64 * low <= n ? top : INFINITY;
 }
 // One workgroup: the largest |LayerNorm|, infinite where too many of gamma are far below the largest one.
-__global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, const float* __restrict__ gamma, const float* __restrict__ beta, unsigned* bound) {
+__global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, const float* __restrict__ gamma, const float* __restrict__ beta, float* bound) {
   __shared__ float sh[2][256];
   __shared__ int low;
   float g = 0.f, b = 0.f;
@@ -446,7 +522,7 @@ __global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, const float* 
   atomicAdd(&low, n);
   __syncthreads();
   const float v = sqrtf((float)d) * g + b;
-  if (threadIdx.x == 0) atomicMax(bound, v < INFINITY && 64 * low <= d ? __float_as_uint(v) : __float_as_uint(INFINITY));
+  if (threadIdx.x == 0) *bound = v < INFINITY && 64 * low <= d ? v : INFINITY;
 }
 __global__ __launch_bounds__(256) void pair_rescale_kernel(int N, float factor, float* cscale) {
   const int n = (int)blockIdx.x * 256 + threadIdx.x;
@@ -550,11 +626,11 @@ hipError_t launch_pair_scales(int N, const float* scale, float* cscale, unsigned
   return hipGetLastError();
 }
 size_t pair_bounds_floats(int K, int N) { return (size_t)2 * ((K + CHUNK - 1) / CHUNK) * N; }
-hipError_t launch_pair_bounds(int K, int ldw, int n0, int n1, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
-                              const float* gamma, const float* beta, float* sums, unsigned* bound, unsigned* ln_bound, hipStream_t s) {
+hipError_t launch_pair_bounds(int K, int N, int runs, int even, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
+                              const float* gamma, const float* beta, float* sums, float* bound, float* ln_bound, hipStream_t s) {
   float2* const p = reinterpret_cast<float2*>(sums);
-  pair_bounds_kernel<<<dim3((n1 - n0 + 31) / 32, (K + CHUNK - 1) / CHUNK), 256, 0, s>>>(K, ldw, n0, n1, W, Wq, wscale, gamma, beta, p);
-  pair_bounds_end<<<(n1 - n0 + 255) / 256, 256, 0, s>>>(K, n0, n1, bias, p, bound);
+  pair_bounds_kernel<<<dim3((N + 31) / 32, (K + CHUNK - 1) / CHUNK), 256, 0, s>>>(K, N, W, Wq, wscale, gamma, beta, p);
+  pair_bounds_end<<<runs, 1024, 0, s>>>(K, N, N / runs, even, bias, p, bound);
   pair_ln_bound_kernel<<<1, 256, 0, s>>>(K, gamma, beta, ln_bound);
   return hipGetLastError();
 }

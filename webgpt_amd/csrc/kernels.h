@@ -69,7 +69,7 @@ hipError_t launch_vocab_gemv(int V, int d, const float* x, const float* wte, flo
 // keys/values 0..pos. q row i is at q + i*ldq + h*hs; key row j of head h is at
 // Kc + h*hstride + j*ldkv (likewise values).
 // ws: attention_workspace_bytes of memory (may be null where that is 0). pairs: the rows, times its scale, as pairs (pair_f16.h)
-// instead of floats at `out`; Tq from 32 on.
+// instead of floats at `out`, for head sizes that attention_pair.hip does not take.
 struct PairRows {
   void* rows;
   int K16;

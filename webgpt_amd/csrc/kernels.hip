@@ -664,7 +664,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 template <int NWV>
 __global__ __launch_bounds__(NWV * 64) void attention_mfma_kernel(int Tq, int pos0, float scale, const float* __restrict__ q, int ldq,
                                                              const float* __restrict__ Kc, const float* __restrict__ Vc,
-                                                             size_t hstride, int ldkv, float* __restrict__ out, int ldo, PairRows pairs) {
+                                                             size_t hstride, int ldkv, float* __restrict__ out, int ldo) {
   extern __shared__ __attribute__((aligned(16))) float am_lds[];
   const int h = blockIdx.x, q0 = blockIdx.y * AMQ;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -804,9 +804,7 @@ __global__ __launch_bounds__(NWV * 64) void attention_mfma_kernel(int Tq, int po
       num += am_lds[w * AM_WAVE_FLOATS + dim * AMOST + qi] * f;
       den += am_lds[w * AM_WAVE_FLOATS + AHS * AMOST + AMQ + qi] * f;
     }
-    if (q0 + qi >= Tq) continue;
-    if (pairs.rows) put_pair(pairs.rows, pairs.K16, q0 + qi, h * AHS + dim, num / den * pairs.scale);
-    else out[(size_t)(q0 + qi) * ldo + h * AHS + dim] = num / den;
+    if (q0 + qi < Tq) out[(size_t)(q0 + qi) * ldo + h * AHS + dim] = num / den;
   }
 }
 
@@ -1747,9 +1745,8 @@ size_t attention_workspace_bytes(int Tq, int pos0, int H, int hs) {
 hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const float* q, int ldq, const float* Kc,
                             const float* Vc, size_t hstride, int ldkv, float* out, int ldo, void* ws, hipStream_t s, const PairRows* pairs) {
   if (ws && attention_splits(Tq, pos0, H, hs)) return launch_attention_split(Tq, pos0, H, hs, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, ws, s, pairs);
-  const PairRows rows = pairs ? *pairs : PairRows{};
   // a block of 32 queries per workgroup on the matrix cores
-  if (hs == AHS && Tq >= AMQ) {
+  if (!pairs && hs == AHS && Tq >= AMQ) {
     static_assert(AHS * AMOST + 2 * AMQ <= AM_WAVE_FLOATS, "merge area must fit a wave's tile area");
     // eight waves once the longest query block has more than eight key tiles
     const bool wide = cdiv(pos0 + Tq, AMK) > 8;
@@ -1764,8 +1761,8 @@ hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const 
       if (e != hipSuccess) return e;
       enabled = true;
     }
-    if (wide) attention_mfma_kernel<8><<<dim3(H, cdiv(Tq, AMQ)), 512, lds, s>>>(Tq, pos0, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, rows);
-    else attention_mfma_kernel<4><<<dim3(H, cdiv(Tq, AMQ)), 256, lds, s>>>(Tq, pos0, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, rows);
+    if (wide) attention_mfma_kernel<8><<<dim3(H, cdiv(Tq, AMQ)), 512, lds, s>>>(Tq, pos0, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo);
+    else attention_mfma_kernel<4><<<dim3(H, cdiv(Tq, AMQ)), 256, lds, s>>>(Tq, pos0, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo);
     return hipGetLastError();
   }
   // enough (head, query block) workgroups to fill the GPU; else one workgroup per query row
@@ -1778,7 +1775,7 @@ hipError_t launch_attention(int Tq, int pos0, int H, int hs, float scale, const 
   if (lpk > 64 || hs > 256 || (hs & 3)) return hipErrorInvalidValue;
   const size_t smem = sizeof(float) * (size_t)(pos0 + Tq);
   if (smem > 48 * 1024) return hipErrorInvalidValue;
-  attention_kernel<<<dim3(H, Tq), WG, smem, s>>>(pos0, hs, lpk, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, rows);
+  attention_kernel<<<dim3(H, Tq), WG, smem, s>>>(pos0, hs, lpk, scale, q, ldq, Kc, Vc, hstride, ldkv, out, ldo, pairs ? *pairs : PairRows{});
   return hipGetLastError();
 }
 

@@ -29,11 +29,11 @@ struct LayerW {
 };
 
 // One layer's weights as pairs of fp16 values (int8 ones stay in LinW), what their products' columns are multiplied with, and the
-// scales of the rows: behind the two LayerNorms, the attention and the GELU.
+// scales of the rows: behind the two LayerNorms, the attention (its values' too) and the GELU, and of q and the keys.
 struct PairLayer {
   void *wA = nullptr, *wC = nullptr, *wD = nullptr, *wE = nullptr;
   float *cA = nullptr, *cC = nullptr, *cD = nullptr, *cE = nullptr;
-  float s1 = 1.f, sv = 1.f, s2 = 1.f, sh = 1.f;
+  float s1 = 1.f, sv = 1.f, s2 = 1.f, sh = 1.f, sq = 1.f, sk = 1.f;
 };
 
 struct Model {
@@ -90,6 +90,7 @@ struct Model {
   // prompts beyond those: products of pairs of fp16 values, where the weights allow (empty: they do not)
   std::vector<PairLayer> pairs;
   void *pair_ln = nullptr, *pair_att = nullptr, *pair_h = nullptr;  // rows of up to maxT tokens
+  void* pair_heads[3] = {};  // the attention's operands (null: heads that it does not take)
   int32_t* tok_pin = nullptr;  // pinned (behind ids_pin's): [PP_MAX_T] the prompt, then the word that a launch leaves its error in
 
   // decode with one launch per block (decode_mode 0): the token's launches read the cache position from pos_dev and

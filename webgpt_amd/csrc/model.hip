@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "common.h"
+#include "attention_pair.h"
 #include "decode_generic.h"
 #include "gemm_pair.h"
 #include "gemm_split.h"
@@ -183,7 +184,7 @@ static int forward_blocks(Model* m, int T, int pos0, bool want_taps) {
 static int forward_pairs(Model* m, int T) {
   hipStream_t s = rt().stream;
   const int d = m->d, H = m->H, hs = m->hs, hid = 4 * d;
-  const bool i8 = m->p.weight_dtype == 1;
+  const bool i8 = m->p.weight_dtype == 1, heads = m->pair_heads[0];
   const float scale = (float)(1.0 / std::sqrt((double)hs));  // model.js:321
   const PairPlan plA = plan_gemm_pair(T, 3 * d, d, i8, false), plC = plan_gemm_pair(T, d, d, i8, true);
   const PairPlan plD = plan_gemm_pair(T, hid, d, i8, false), plE = plan_gemm_pair(T, d, hid, i8, true);
@@ -196,13 +197,21 @@ static int forward_pairs(Model* m, int T) {
     PairGemmArgs g{};
     g.M = T; g.N = 3 * d; g.K = d;
     g.A = m->pair_ln; g.W = i8 ? (const void*)l.attn.q : p.wA; g.cscale = p.cA; g.bias = l.attn_b;
-    g.end = PAIR_QKV;
+    g.end = heads ? PAIR_HEADS : PAIR_QKV;
     g.C = m->qkv; g.ldc = 3 * d;
+    for (int j = 0; j < 3; ++j) g.heads[j] = m->pair_heads[j];
+    g.head_tiles = pair_attn_tiles(m->maxT);
+    g.hscale[0] = p.sq; g.hscale[1] = p.sk; g.hscale[2] = p.sv; g.rhs = 1.0f / (float)hs;
     g.Kc = m->kv + ((size_t)li * 2 + 0) * m->ctx * d; g.Vc = m->kv + ((size_t)li * 2 + 1) * m->ctx * d;
     g.d = d; g.hs = hs; g.ctx = m->ctx;
     LAUNCH(launch_gemm_pair(plA, g, i8, s));
-    const PairRows rows = {m->pair_att, pair_k16(d), p.sv};
-    LAUNCH(launch_attention(T, 0, H, hs, scale, m->qkv, 3 * d, g.Kc, g.Vc, (size_t)m->ctx * hs, hs, nullptr, d, m->att_ws, s, &rows));
+    if (heads) {
+      const AttnPairArgs at{T, H, hs, g.head_tiles, g.heads[0], g.heads[1], g.heads[2], scale / p.sq / p.sk, m->pair_att, pair_k16(d), 0};
+      LAUNCH(launch_attention_pair(at, s));
+    } else {
+      const PairRows rows = {m->pair_att, pair_k16(d), p.sv};
+      LAUNCH(launch_attention(T, 0, H, hs, scale, m->qkv, 3 * d, g.Kc, g.Vc, (size_t)m->ctx * hs, hs, nullptr, d, m->att_ws, s, &rows));
+    }
     // the two projections leave x finished, or slices that the LayerNorm's pass sums
     const auto project = [&](const PairPlan& pl, int K, const void* A, const LinW& w, const void* wp, const float* cs, const float* bias) {
       PairGemmArgs c{};
@@ -696,11 +705,13 @@ static int setup_pairs(Model* m) {
   }
   const size_t row = room(pair_rows_bytes(m->maxT, d)), rowh = room(pair_rows_bytes(m->maxT, hid));
   if (rowh >= 0x80000000u) return WGPT_OK;
-  const size_t stats_bytes = room(sizeof(unsigned) * (1 + 4 * (size_t)L));
+  const size_t heads = pair_attn_takes(m->hs) ? room(pair_attn_bytes(m->maxT, m->H, m->hs)) : 0;
+  constexpr int NB = 6;  // bounds of a layer: behind LN1, q, keys, values, behind LN2, hidden rows
+  const size_t stats_bytes = room(sizeof(unsigned) * (1 + NB * (size_t)L));
   char* base;
   // (what only the loading needs lies in the rows' memory: they are cleared behind it)
   const size_t sums_bytes = sizeof(float) * pair_bounds_floats(d, hid), few_bytes = i8 ? 0 : room(sizeof(int) * 9 * (size_t)d * L);
-  const size_t rows_bytes = std::max(2 * row + rowh, room(sums_bytes) + few_bytes);
+  const size_t rows_bytes = std::max(2 * row + rowh + 3 * heads, room(sums_bytes) + few_bytes);
   if (dev_alloc(m, per_layer * L + rows_bytes + stats_bytes, (void**)&base)) return WGPT_OK;
   char* const all = base;
   const auto take = [&](size_t bytes) { char* p = base; base += bytes; return p; };
@@ -708,9 +719,10 @@ static int setup_pairs(Model* m) {
   m->pair_ln = rows;
   m->pair_att = rows + row;
   m->pair_h = rows + 2 * row;
+  for (int j = 0; j < 3; ++j) m->pair_heads[j] = heads ? rows + 2 * row + rowh + j * heads : nullptr;
   float* const sums = (float*)rows;
   int* few = (int*)(rows + room(sums_bytes));
-  unsigned* stats = (unsigned*)take(stats_bytes);  // [0]: what the products cannot take; then the four bounds of each layer
+  unsigned* stats = (unsigned*)take(stats_bytes);  // [0]: what the products cannot take; then the bounds of each layer
   WGPT_HIP(hipMemsetAsync(all, 0, per_layer * L + rows_bytes + stats_bytes, rt().stream));
   std::vector<PairLayer> layers(L);
   for (int i = 0; i < L; ++i) {
@@ -726,19 +738,21 @@ static int setup_pairs(Model* m) {
         few += t.N;
       }
     }
-    unsigned* b = stats + 1 + 4 * i;
-    LAUNCH(launch_pair_bounds(d, i8 ? 3 * d / 4 : 3 * d, 2 * d, 3 * d, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
-    LAUNCH(launch_pair_bounds(d, i8 ? hid / 4 : hid, 0, hid, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 3, b + 2, rt().stream));
+    float* b = (float*)stats + 1 + NB * i;
+    LAUNCH(launch_pair_bounds(d, 3 * d, 3, heads ? 2 : 0, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
+    LAUNCH(launch_pair_bounds(d, hid, 1, 0, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 5, b + 4, rt().stream));
   }
-  std::vector<unsigned> host(1 + 4 * (size_t)L);
+  std::vector<unsigned> host(1 + NB * (size_t)L);
   WGPT_HIP(hipMemcpyAsync(host.data(), stats, sizeof(unsigned) * host.size(), hipMemcpyDeviceToHost, rt().stream));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   bool ok = host[0] == 0;
   for (int i = 0; i < L && ok; ++i) {
-    float* const s[4] = {&layers[i].s1, &layers[i].sv, &layers[i].s2, &layers[i].sh};
-    for (int j = 0; j < 4; ++j) {
+    PairLayer& p = layers[i];
+    float* const s[NB] = {&p.s1, &p.sq, &p.sk, &p.sv, &p.s2, &p.sh};
+    for (int j = 0; j < NB; ++j) {
       float bound;
-      memcpy(&bound, &host[1 + 4 * i + j], sizeof bound);
+      memcpy(&bound, &host[1 + NB * i + j], sizeof bound);
+      if (!heads && (j == 1 || j == 2)) continue;
       ok = ok && (bound == 0.f || (bound > 0x1p-60f && bound < 0x1p60f));
       int e = 0;
       if (ok && bound > 0.f) (void)frexpf(bound * 1.001f, &e);  // (the bounds' own roundings, and those of the values)
@@ -746,7 +760,7 @@ static int setup_pairs(Model* m) {
     }
   }
   if (!ok) {
-    m->pair_ln = m->pair_att = m->pair_h = nullptr;
+    m->pair_ln = m->pair_att = m->pair_h = m->pair_heads[0] = nullptr;
     m->allocs.pop_back();
     (void)hipFree(all);
     return WGPT_OK;
