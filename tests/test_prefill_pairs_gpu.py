@@ -96,3 +96,23 @@ def test_rows_that_are_no_numbers(device):
     assert np.array_equal(gpt.prefill(tokens[:200])[:100], want)
     gpt.unloadBuffers()
     clean.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head", [(520, 13), (1024, 16), (1288, 23), (1608, 67)])
+def test_short_prompts_of_weights_beyond_the_pairs(device, dtype, d, n_head):
+    """One column that the pairs cannot take: short prompts run in one launch all the same, on plain values."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=70, vocab_size=101, dtype=dtype)
+    tensors = spoil(make_model(cfg, 8), "tiny columns") if dtype == "f32" else make_model(cfg, 8)
+    if dtype == "int8":
+        name = "transformer.h.1.mlp.c_fc.weight.scale"
+        tensors[name] = tensors[name].copy()
+        tensors[name][7] = 2.0 ** -100
+    gpt, w, p = load(cfg, tensors), oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in (1, 17, 61):
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        want = ref.forward(p, w, tokens)
+        got = gpt.prefill(tokens)
+        assert close(got, want), (T, worst(got, want))
+        assert gpt.routes()[0] == 1, T
+    gpt.unloadBuffers()

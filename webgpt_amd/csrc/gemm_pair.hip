@@ -43,12 +43,6 @@ __device__ __forceinline__ void unrolled(F&& f) { unrolled_(f, std::make_integer
 __device__ __forceinline__ f32x16 mfma(const u32x4& w, const u32x4& a, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
 }
-// int8 values 2 q and 2 q + 1 of eight as fp16: a byte b + 128 under 0x64 is 1024 + b + 128
-__device__ __forceinline__ unsigned f16_of_bytes(const unsigned (&v)[2], int q) {
-  const unsigned x = __builtin_amdgcn_perm(0x64646464u, v[q >> 1] ^ 0x80808080u, q & 1 ? 0x04030402u : 0x04010400u);
-  return __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, x) - f16x2{(_Float16)1152.f, (_Float16)1152.f});
-}
-
 // A lane's four values in a row become one value of each of its quad's four: element `lane % 4` of lanes 0 .. 3.
 __device__ __forceinline__ f32x4 transpose_quad(f32x4 v) {
   const auto swap = [](float& a, float& b, bool odd, auto perm) {
@@ -155,8 +149,7 @@ __global__ __launch_bounds__(256, MB * NB <= 4 ? 3 : 2) void gemm_pair_kernel(Pa
     }
   };
   const auto convert = [&](int u, int o) {
-    const unsigned v[2] = {w[u][o >> 2][0][0], w[u][o >> 2][0][1]};
-    wf[u][o >> 2][o & 3] = f16_of_bytes(v, o & 3);
+    wf[u][o >> 2][o & 3] = f16_of_bytes(w[u][o >> 2][0][(o >> 1) & 1], o & 1);
   };
   // smallest products first
   constexpr int SEC = MB * NB, NMF = SEC * (I8 ? 2 : 3), NCV = I8 ? 4 * NB : 0, CV0 = NMF / 4;

@@ -774,6 +774,8 @@ static int setup_pairs(Model* m) {
   return WGPT_OK;
 }
 
+static bool prefill_pairs(const Model* m) { return !m->pairs.empty() && m->d > PP_PAIR_ABOVE; }
+
 // Prepares the persistent prefill in the buffers that wgpt_model_finalize has allocated for it; after block_linear_weights.
 static int setup_prefill(Model* m) {
   const bool i8 = m->p.weight_dtype == 1;
@@ -784,7 +786,13 @@ static int setup_prefill(Model* m) {
     const void* p[4];
     for (int j = 0; j < 4; ++j) p[j] = i8 ? (const void*)w[j]->q : (const void*)w[j]->w;
     layers[i] = {p[0], p[1], p[2], p[3], w[0]->s, w[1]->s, w[2]->s, w[3]->s, l.attn_b, l.proj_b, l.fc_b, l.fc2_b,
-                 l.ln1_g, l.ln1_b, l.ln2_g, l.ln2_b};
+                 l.ln1_g, l.ln1_b, l.ln2_g, l.ln2_b, 1.f, 1.f, 1.f, 1.f};
+    if (!prefill_pairs(m)) continue;
+    const PairLayer& q = m->pairs[i];
+    PrefillLayer& t = layers[i];
+    if (!i8) t.wA = q.wA, t.wC = q.wC, t.wD = q.wD, t.wE = q.wE;
+    t.sA = q.cA, t.sC = q.cC, t.sD = q.cD, t.sE = q.cE;
+    t.xA = q.s1, t.xC = q.sv, t.xD = q.s2, t.xE = q.sh;
   }
   PrefillArgs& a = m->pp;
   WGPT_HIP(hipMemcpyAsync((void*)a.layers, layers.data(), sizeof(PrefillLayer) * (size_t)m->L, hipMemcpyHostToDevice, rt().stream));
@@ -821,7 +829,8 @@ static int prefill_persistent(Model* m, const int32_t* tokens, int T, bool* done
   PrefillArgs a = m->pp;
   a.T = T;
   a.ebase = m->pp_epoch;
-  LAUNCH(launch_prefill_persistent(a, m->p.weight_dtype == 1, rt().stream));
+  const bool i8 = m->p.weight_dtype == 1;
+  LAUNCH(launch_prefill_persistent(a, prefill_pairs(m) ? (i8 ? PP_PAIR_I8 : PP_PAIR_F32) : i8 ? PP_SPLIT_I8 : PP_PLAIN_F32, rt().stream));
   m->pp_epoch += n;
   WGPT_HIP(hipEventRecord(m->ev1, rt().stream));
   WGPT_HIP(hipStreamSynchronize(rt().stream));

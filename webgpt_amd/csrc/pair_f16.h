@@ -22,6 +22,12 @@ __device__ __forceinline__ void pair_f16(float a, float b, unsigned& hi, unsigne
   lo = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a - (float)h[0], b - (float)h[1]}), f16x2));
 }
 
+// int8 values 2 q and 2 q + 1 of the four of a word as fp16: a byte b + 128 under 0x64 is 1024 + b + 128
+__device__ __forceinline__ unsigned f16_of_bytes(unsigned v, int q) {
+  const unsigned x = __builtin_amdgcn_perm(0x64646464u, v ^ 0x80808080u, q ? 0x04030402u : 0x04010400u);
+  return __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, x) - f16x2{(_Float16)1152.f, (_Float16)1152.f});
+}
+
 // Rows in runs of 16 k: unit ((row / 32 * K16 + k / 16) * 2 + part) * 64 + (k / 8 % 2) * 32 + row % 32 of 16 bytes holds eight
 // consecutive k of one part of a row, so that an operand of a 32x32x16 matrix instruction is one load of 1 KB of a wave.
 __host__ __device__ __forceinline__ size_t pair_unit(int row, int k, int K16) {

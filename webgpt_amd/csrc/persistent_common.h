@@ -21,6 +21,7 @@ __device__ __forceinline__ f32x4 load4(__amdgpu_buffer_rsrc_t b, int o, int so =
 }
 __device__ __forceinline__ unsigned ld_flag(const unsigned* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void st_agent(float* p, const f32x4& v) { asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory"); }
+__device__ __forceinline__ void st_agent2(float* p, const u32x2& v) { asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory"); }
 
 __device__ __forceinline__ void pair16(float v, float& a, float& b) {
   const unsigned u = __float_as_uint(v);

@@ -16,11 +16,21 @@ constexpr int PP_MAX_GROUPS = 8;  // a wave of the attention takes the keys of o
 constexpr int PP_MAX_T = PP_ROWS * PP_MAX_GROUPS;
 constexpr int PP_FLAGS = PP_MAX_GROUPS * PP_GRID + 64;  // words of PrefillArgs::flags, the launch's error word among them
 
-// One layer's weights in the order of launch_block_weights, and its small parameters (device pointers).
+// What the products are made of: fp32 values, int8 weights and rows of three bf16 values each, or rows (and fp32 weights) that are
+// pairs of fp16 values as those of gemm_pair.hip.
+// Pairs are for rows above PP_PAIR_ABOVE: logits of 6 layers of 512, 90 tokens, 2.8e-7 from 64-bit arithmetic with them against 2.7e-7; 8
+// layers of 576, 100 tokens, 2.8e-7 against 2.9e-7.
+constexpr int PP_PAIR_ABOVE = 512;
+enum PrefillMode { PP_PLAIN_F32 = 0, PP_SPLIT_I8 = 1, PP_PAIR_F32 = 2, PP_PAIR_I8 = 3 };
+
+// One layer's weights in the order of launch_block_weights (PP_PAIR_F32: of launch_pair_weights), and its small parameters
+// (device pointers).
 struct PrefillLayer {
   const void *wA, *wC, *wD, *wE;                            // c_attn, attention c_proj, c_fc, mlp c_proj
-  const float *sA, *sC, *sD, *sE, *bA, *bC, *bD, *bE;       // int8 column scales (null for fp32), biases
+  // int8 column scales, or what the columns of pairs are multiplied with (null for plain fp32); biases
+  const float *sA, *sC, *sD, *sE, *bA, *bC, *bD, *bE;
   const float *ln1g, *ln1b, *ln2g, *ln2b;
+  float xA, xC, xD, xE;  // scales of the rows that the four products read, as pairs
 };
 
 struct PrefillArgs {
@@ -54,7 +64,7 @@ inline size_t prefill_exchange_floats(int T, int d) { return (size_t)8 * prefill
 inline unsigned prefill_epochs(int L) { return 5u * (unsigned)L + 1u; }
 // The longest prompt that the kernel takes of such a model, 0: none (compute_units of the device at hand).
 int prefill_persistent_rows(int d, int H, int hs, int V, bool i8, int compute_units);
-hipError_t launch_prefill_persistent(PrefillArgs a, bool i8, hipStream_t s);
+hipError_t launch_prefill_persistent(PrefillArgs a, PrefillMode mode, hipStream_t s);
 
 }  // namespace wgpt
 

@@ -2,12 +2,14 @@
 //
 // A launch per block costs a short prompt 3 to 5 us of fixed time for each of its 7 or 8 dependent launches a layer, more than
 // its operations and bytes (117M, 13 tokens: 86 launches in 0.50 ms for 340 MB of weights, 52 us at the rate of reads).
-// Calls of wgpt_prefill with launches and with this kernel, ms: 117M 1 token 0.50 -> 0.42, 13 0.55 -> 0.42, 64 0.67 -> 0.47,
-// 128 0.79 -> 0.58; 345M 100 1.72 -> 1.44; 774M 64 2.59 -> 2.12; 1.5B int8 16 2.54 -> 2.20; toy 64 0.28 -> 0.17. Clock stamps of a layer of
-// 117M, which is 30 us with them at 13 rows and 43 at 128: from the last flag to the end of a wait 0.3 to 1.4 us (0.4 to 1.4 at 128 rows), sums,
+// Calls of wgpt_prefill with launches, with this kernel on plain values (three bf16 values each beside int8 weights), and on pairs of
+// fp16 values, ms: 117M 1 token 0.50, 0.37, 0.35, 13 0.55, 0.39, 0.37, 45 0.45 (plain), 0.41, 128 0.79, 0.56, 0.48; toy 64 0.28, 0.17 (plain).
+// Twelve layers, plain and pairs: 345M 100 tokens 0.71, 0.59, 774M 64 0.71, 0.62, 128 1.01, 0.85; 24 of 1.5B int8, 16 tokens 1.10, 0.99, 128
+// 1.90, 1.71. Clock stamps of a layer of 117M on plain values, which is 30 us with them at 13 rows and 43 at 128: from the last flag to the end of a wait 0.3 to 1.4 us (0.4 to 1.4 at 128 rows), sums,
 // epilogue, stores and the flag 0.8 to 1.1 a phase (0.6 to 1.2), loads with LayerNorm and products c_attn 2.5 (7.3), attention 2.7 (4.0), c_proj
 // 2.1 (2.4), c_fc 3.1 (8.6), the second MLP product 5.7 (9.1; at 13 rows a compute unit reads all hidden rows for four columns), the last workgroup 0.6
-// to 2.4 behind the median. The matrix units are busy for 11 % of the launch at 13 rows and 31 % at 128: 14 us a layer of the 27 in its products.
+// to 2.4 behind the median. The matrix units were busy for 11 % of the launch at 13 rows and 31 % at 128, 14 us a layer of the 27 in its
+// products; on pairs they are for 3 us of those at 128.
 // The compiler spills 218 to 329 scalar registers into vector lanes.
 // Here one workgroup per compute unit stays for the whole forward and the blocks are phases of it:
 //
@@ -15,8 +17,10 @@
 //     a linear layer's output columns are dealt to the column groups. The workgroups of one column group are on one XCD, so
 //     the weights that they share come out of its L2;
 //   - inside a workgroup the eight waves split the contraction; a wave multiplies its slice of the 16 rows with its slice of
-//     all columns of the workgroup on the bf16 matrix cores (fp32 values as exact sums of three bf16 values, split_bf16.h,
-//     the products and their order those of gemm_split.hip), and the partial tiles meet in LDS;
+//     all columns of the workgroup on the matrix cores, and the partial tiles meet in LDS. Weights and rows are the pairs of fp16
+//     values and the scales of gemm_pair.hip where the model has them and its rows are wide enough (PP_PAIR_ABOVE); the attention's
+//     output and the hidden rows travel as pairs. Else fp32 values are multiplied as they are, and beside int8 weights rows are
+//     exact sums of three bf16 values (split_bf16.h, gemm_split.hip);
 //   - LayerNorm is applied to the rows in registers on their way in (statistics of a row: each wave about its own mean,
 //     merged through LDS), GELU, bias and residual are epilogues, and a workgroup keeps the residual stream of its columns;
 //   - rows pass from phase to phase through memory with write-through stores at device scope; a workgroup that has finished a
@@ -37,8 +41,8 @@
 // at that scope and had arrived (s_waitcnt) before the flag was raised.
 #include "prefill_persistent.h"
 
+#include "pair_f16.h"
 #include "persistent_common.h"
-#include "split_bf16.h"
 
 namespace wgpt {
 namespace {
@@ -83,10 +87,13 @@ struct Flags {
   }
 };
 
-// Eight consecutive k of one column: floats, or bytes.
-template <bool I8>
+constexpr bool is_i8(int mode) { return mode & 1; }
+constexpr bool is_pair(int mode) { return mode & 2; }
+
+// Eight consecutive k of one column: floats, the hi and lo halves of pairs, or bytes.
+template <int MODE>
 struct WSlice8 {
-  unsigned v[I8 ? 2 : 8];
+  unsigned v[is_i8(MODE) ? 2 : 8];
   __device__ __forceinline__ u32x4 bf16() const {
     u32x4 h;
 #pragma unroll
@@ -96,45 +103,58 @@ struct WSlice8 {
     }
     return h;
   }
+  __device__ __forceinline__ u32x4 f16() const { return u32x4{f16_of_bytes(v[0], 0), f16_of_bytes(v[0], 1), f16_of_bytes(v[1], 0), f16_of_bytes(v[1], 1)}; }
 };
-// The same for NS steps of 32 k, in the order of launch_block_weights.
-template <bool I8, int NS>
+// The same for NS steps of 32 k, in the order of launch_block_weights, or of pair_unit.
+template <int MODE, int NS>
 struct WSlice {
-  WSlice8<I8> s[NS];
+  WSlice8<MODE> s[NS];
   // Column n of N (nok: there is one) from step `step` on, cnt steps of them; a lane's place in the step is its kg, the step's
   // a scalar offset.
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int N, int K8, int n, bool nok, int step, int cnt, int kg) {
-    const int o = nok ? (I8 ? 8 : 32) * kg * N + (I8 ? 8 : 16) * n : OUT;
+    constexpr bool I8 = is_i8(MODE), UNITS = MODE == PP_PAIR_F32;
+    const int place = UNITS ? ((n >> 5) * ((K8 + 1) >> 1) + (kg >> 1)) * 2048 + (kg & 1) * 512 + (n & 31) * 16 : (I8 ? 8 : 32) * kg * N + (I8 ? 8 : 16) * n;
+    const int o = nok ? place : OUT, stride = UNITS ? 4096 : (I8 ? 32 : 128) * N;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      const int left = i < cnt ? K8 - 4 * (step + i) : 0, so = (I8 ? 32 : 128) * N * (i < cnt ? step + i : 0);
+      const int left = i < cnt ? K8 - 4 * (step + i) : 0, so = stride * (i < cnt ? step + i : 0);
       const int oi = kg < left ? o : OUT;
       if constexpr (I8) {
         const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(b, oi, so, 0);
         s[i].v[0] = x[0], s[i].v[1] = x[1];
       } else {
-        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(b, oi, so, 0), y = __builtin_amdgcn_raw_buffer_load_b128(b, oi, so + 16 * N, 0);
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(b, oi, so, 0), y = __builtin_amdgcn_raw_buffer_load_b128(b, oi, so + (UNITS ? 1024 : 16 * N), 0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[i].v[e] = x[e], s[i].v[4 + e] = y[e];
       }
     }
   }
 };
+// The memory of a weight matrix [K, N].
+template <int MODE>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t weights_of(const void* W, int K, int N) {
+  return buffer_of(W, MODE == PP_PAIR_F32 ? (size_t)((N + 31) >> 5) * ((K + 15) >> 4) * 2048 : (size_t)K * N * (is_i8(MODE) ? 1 : 4));
+}
 
-// Eight k of one row as the products take them.
-template <bool I8>
+// Eight k of one row as the products take them, from two runs of four floats, or from the hi and lo halves of pairs.
+template <int MODE>
 struct Operand {
+  u32x4 hi, lo;
+  __device__ __forceinline__ void set(const f32x4 (&x)[2]) { hi = __builtin_bit_cast(u32x4, x[0]), lo = __builtin_bit_cast(u32x4, x[1]); }
+};
+template <>
+struct Operand<PP_SPLIT_I8> {
   Split8 v;
   __device__ __forceinline__ void set(const f32x4 (&x)[2]) { v = split8(x[0], x[1]); }
 };
 template <>
-struct Operand<false> {
+struct Operand<PP_PLAIN_F32> {
   f32x4 v[2];
   __device__ __forceinline__ void set(const f32x4 (&x)[2]) { v[0] = x[0], v[1] = x[1]; }
 };
-template <bool I8, int N>
+template <int MODE, int N>
 struct Operands {
-  Operand<I8> v[N];
+  Operand<MODE> v[N];
   __device__ __forceinline__ void set(const f32x4 (&x)[N][2]) {
 #pragma unroll
     for (int i = 0; i < N; ++i) v[i].set(x[i]);
@@ -143,13 +163,45 @@ struct Operands {
 __device__ __forceinline__ f32x4 mfma(const u32x4& w, const u32x4& x, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
 }
-// Products of N steps of 32 k. int8: a weight is one bf16 value, a row's the sum of three (the products of gemm_split.hip).
+__device__ __forceinline__ f32x4 mfma_f16(const u32x4& w, const u32x4& x, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, x), c, 0, 0, 0);
+}
+// Products of N steps of 32 k. Pairs: all four products (with the three of gemm_pair.hip the logits of 12 layers of 117M at 128 tokens
+// were 3.3e-7 from 64-bit arithmetic; 3.1e-7 with four, and 3.1e-7 with plain values; at 117M's other lengths and from 576 to
+// 1600 columns four are as close as plain values or closer).
+// Else, int8: a weight is one bf16 value, a row's the sum of three (the products of gemm_split.hip).
 // fp32: fp32 matrix instructions, which round after every product; four sums and their tree keep the chains short: the logits
 // of 8 layers of 117M are 3.3e-7 from 64-bit arithmetic (one chain in two 4.5e-7; the launches of gemm_split.hip 3.8e-7). (Six
 // bf16 products for an fp32 one take a third of the matrix units' time of these eight instructions, but eleven vector
 // instructions for every two weights and rows: c_fc of 13 rows of 768 2.1 us of its phase, 1.5 with these.)
 template <int N>
-__device__ __forceinline__ f32x4 products(const WSlice8<true> (&w)[N], const Operands<true, N>& x) {
+__device__ __forceinline__ f32x4 products(const WSlice8<PP_PAIR_F32> (&w)[N], const Operands<PP_PAIR_F32, N>& x) {
+  f32x4 acc[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const u32x4 hi = {w[i].v[0], w[i].v[1], w[i].v[2], w[i].v[3]}, lo = {w[i].v[4], w[i].v[5], w[i].v[6], w[i].v[7]};
+    acc[0] = mfma_f16(lo, x.v[i].lo, acc[0]);
+    acc[1] = mfma_f16(hi, x.v[i].lo, acc[1]);
+    acc[0] = mfma_f16(lo, x.v[i].hi, acc[0]);
+    acc[2 + (i & 1)] = mfma_f16(hi, x.v[i].hi, acc[2 + (i & 1)]);
+  }
+  return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
+template <int N>
+__device__ __forceinline__ f32x4 products(const WSlice8<PP_PAIR_I8> (&w)[N], const Operands<PP_PAIR_I8, N>& x) {
+  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const u32x4 wv = w[i].f16();
+    acc[0] = mfma_f16(wv, x.v[i].lo, acc[0]);
+    acc[1] = mfma_f16(wv, x.v[i].hi, acc[1]);
+  }
+  return acc[0] + acc[1];
+}
+template <int N>
+__device__ __forceinline__ f32x4 products(const WSlice8<PP_SPLIT_I8> (&w)[N], const Operands<PP_SPLIT_I8, N>& x) {
   f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -161,7 +213,7 @@ __device__ __forceinline__ f32x4 products(const WSlice8<true> (&w)[N], const Ope
   return acc[0] + acc[1];
 }
 template <int N>
-__device__ __forceinline__ f32x4 products(const WSlice8<false> (&w)[N], const Operands<false, N>& x) {
+__device__ __forceinline__ f32x4 products(const WSlice8<PP_PLAIN_F32> (&w)[N], const Operands<PP_PLAIN_F32, N>& x) {
   f32x4 acc[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -173,10 +225,10 @@ __device__ __forceinline__ f32x4 products(const WSlice8<false> (&w)[N], const Op
 }
 // int8 sums that the split may have spoilt, as in gemm_split.hip: not finite, from 2^124 on, under 2^-60 but zero. (Of the prompt's rows
 // only: those of the last row group beyond it hold what earlier prompts or other owners of the memory have left.)
-template <bool I8>
+template <int MODE>
 __device__ __forceinline__ bool spoilt(const f32x4& v) {
   bool bad = false;
-  if constexpr (I8) {
+  if constexpr (MODE == PP_SPLIT_I8) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float m = fabsf(v[i]);
@@ -206,11 +258,27 @@ __device__ __forceinline__ ConstLayer* fresh_layer(int li) {
 // or a few channels of the L2, the same ones for every workgroup: the second MLP product of 128 rows of 768 took 19.8 us, 12.4
 // in this order and with requests two chunks ahead.)
 __device__ __forceinline__ int row_offset(int r, int k) { return ((k >> 2) * PP_ROWS + r) * 4; }
+// Four values of a row of the attention's output or the hidden rows to their readers: as pairs, where these take pairs (made by every
+// reader, 96 values a lane at 13 rows of 3072 would be 0.9 us of the phase), with hi and lo in the place of the two runs of four.
+template <int MODE>
+__device__ __forceinline__ void put_row(float* rows, int r, int k, const f32x4& v, float scale) {
+  if constexpr (is_pair(MODE)) {
+    unsigned hi[2], lo[2];
+    pair_f16(v[0] * scale, v[1] * scale, hi[0], lo[0]);
+    pair_f16(v[2] * scale, v[3] * scale, hi[1], lo[1]);
+    float* const p = rows + row_offset(r, k & ~7) + ((k >> 1) & 2);
+    st_agent2(p, u32x2{hi[0], hi[1]});
+    st_agent2(p + 4 * PP_ROWS, u32x2{lo[0], lo[1]});
+  } else {
+    st_agent(rows + row_offset(r, k), v);
+  }
+}
 
 // HJ: head sizes up to 16 HJ.
-template <bool I8, int NS, int HJ>
+template <int MODE, int NS, int HJ>
 __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
+  constexpr bool I8 = is_i8(MODE), PAIR = is_pair(MODE), SCALED = I8 || PAIR;  // (columns have factors)
   constexpr int LN = 256 * NS;  // the widest row of this instantiation
   constexpr int CH = NS < 3 ? NS : 3;  // steps of a chunk of the 4d-long contraction
   __shared__ int bail;
@@ -245,20 +313,20 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
   // What the next phase needs first is requested when this one has raised its flag, in front of the wait for the others'. (A phase
   // earlier, behind the requests for the rows, the weights were in the way of the stores and flags of the phase: 117M, 13 tokens
   // 0.495 ms against 0.415.)
-  WSlice<I8, NS> w_next;                    // weights of its first tile
+  WSlice<MODE, NS> w_next;                    // weights of its first tile
   f32x4 bias_next[2], scale_next[2];        // of this thread's columns
   constexpr int RING = I8 || NS < 6 ? 2 : 1;  // tiles whose weights are on their way
-  const auto request_w = [&](WSlice<I8, NS>& to, const void* W, int N, int cp, int nc, int t) {
+  const auto request_w = [&](WSlice<MODE, NS>& to, const void* W, int N, int cp, int nc, int t) {
     const int o = opaque(lane), n = 16 * t + (o & 15);
-    to.load(buffer_of(W, (size_t)d * N * (I8 ? 1 : 4)), N, K81, cg * cp + n, n < nc, s1, n1, o >> 4);
+    to.load(weights_of<MODE>(W, d, N), N, K81, cg * cp + n, n < nc, s1, n1, o >> 4);
   };
   const auto request_cols = [&](const float* b, const float* s, int N, int cp, int nc) {
-    const __amdgpu_buffer_rsrc_t bb = buffer_of(b, 4 * (size_t)N), sb = buffer_of(I8 ? s : b, 4 * (size_t)N);
+    const __amdgpu_buffer_rsrc_t bb = buffer_of(b, 4 * (size_t)N), sb = buffer_of(SCALED ? s : b, 4 * (size_t)N);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int n = 16 * (et + NW * i) + (4 * (opaque(tid) >> 4) & 12), o = n < nc ? 4 * (cg * cp + n) : OUT;
       bias_next[i] = load4<0>(bb, o);
-      if constexpr (I8) scale_next[i] = load4<0>(sb, o);
+      if constexpr (SCALED) scale_next[i] = load4<0>(sb, o);
     }
   };
   // Gamma and beta of the next LayerNorm: a float4 of each per thread, on their way while the workgroup waits for the rows.
@@ -280,8 +348,8 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       x[i][1] = load4<SC1>(b, o, so + 16 * PP_ROWS);
     }
   };
-  // LayerNorm of the wave's slice (instructions.js:451-550); all waves take part.
-  const auto normalise = [&](f32x4 (&x)[NS][2]) {
+  // LayerNorm of the wave's slice (instructions.js:451-550), as pairs where the products take them; all waves take part.
+  const auto normalise = [&](f32x4 (&x)[NS][2], float scale) {
     const int ol = opaque(lane), row = ol & 15, kg = ol >> 4;
     float sum = 0.f;
 #pragma unroll
@@ -336,17 +404,27 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[s][h][i] = g[i] * quotient(x[s][h][i] - mean, stdev, r) + be[i];
       }
+      if constexpr (PAIR) {
+        u32x4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          unsigned a, b;
+          pair_f16(x[s][i >> 1][2 * (i & 1)] * scale, x[s][i >> 1][2 * (i & 1) + 1] * scale, a, b);
+          hi[i] = a, lo[i] = b;
+        }
+        x[s][0] = __builtin_bit_cast(f32x4, hi), x[s][1] = __builtin_bit_cast(f32x4, lo);
+      }
     }
   };
   // Products of the wave's slice of a d-long contraction with the workgroup's columns; partial tiles to `red`.
-  const auto multiply = [&](const f32x4 (&x)[NS][2], WSlice<I8, NS> (&w)[RING], const void* W, int N, int cp, int nc, int tiles) {
-    Operands<I8, NS> xs;
+  const auto multiply = [&](const f32x4 (&x)[NS][2], WSlice<MODE, NS> (&w)[RING], const void* W, int N, int cp, int nc, int tiles) {
+    Operands<MODE, NS> xs;
     xs.set(x);
     bool bad = false;
-    const auto tile = [&](WSlice<I8, NS>& wt, int t) {
+    const auto tile = [&](WSlice<MODE, NS>& wt, int t) {
       const f32x4 v = products(wt.s, xs);
       if (t + RING < tiles) request_w(wt, W, N, cp, nc, t + RING);
-      bad = bad || (em < T && spoilt<I8>(v));
+      bad = bad || (em < T && spoilt<MODE>(v));
       red[(wave * tiles + t) * 64 + opaque(lane)] = v;
     };
 #pragma unroll 1
@@ -363,7 +441,8 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
     for (int i = 0; i < NW; ++i) u[i] = p[i * tiles * 64];
     f32x4 v = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
-    if constexpr (I8) {
+    if constexpr (PAIR) v *= scale[slot];
+    else if constexpr (I8) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] *= scale[slot][e] / 127.0f;
     }
@@ -394,13 +473,13 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
     request_cols(ly->bD, ly->sD, 4 * d, cpD, ncD);
   };
   // The phase takes over what was requested for it; the weights of its second tile.
-  const auto take = [&](WSlice<I8, NS> (&w)[RING], f32x4 (&bias)[2], f32x4 (&scale)[2], const void* W, int N, int cp, int nc) {
+  const auto take = [&](WSlice<MODE, NS> (&w)[RING], f32x4 (&bias)[2], f32x4 (&scale)[2], const void* W, int N, int cp, int nc) {
     w[0] = w_next;
     if (RING > 1) request_w(w[RING - 1], W, N, cp, nc, 1);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       bias[i] = bias_next[i];
-      if constexpr (I8) scale[i] = scale_next[i];
+      if constexpr (SCALED) scale[i] = scale_next[i];
     }
   };
 
@@ -415,7 +494,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       // ---- c_attn: LN1, q/k/v; keys and values to their rows of the cache ----
       if (tilesA) {
         f32x4 x[NS][2], bias[2], scale[2];
-        WSlice<I8, NS> w[RING];
+        WSlice<MODE, NS> w[RING];
         ConstArgs* a = fresh_args();
         if (li == 0) {  // the embedding (instructions.js:795-821)
           const int ol = opaque(lane), m = rg * PP_ROWS + (ol & 15), row = m < T ? m : T - 1;
@@ -435,7 +514,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
         }
         ConstLayer* ly = fresh_layer(li);
         take(w, bias, scale, ly->wA, 3 * d, cpA, ncA);
-        normalise(x);
+        normalise(x, ly->xA);
         multiply(x, w, ly->wA, 3 * d, cpA, ncA, tilesA);
         __syncthreads();
         if (bail) return;
@@ -552,7 +631,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] /= l;
-            st_agent(a->att + (size_t)rg * PP_ROWS * d + row_offset(qr, h * hs + c), v);
+            put_row<MODE>(a->att + (size_t)rg * PP_ROWS * d, qr, h * hs + c, v, PAIR ? fresh_layer(li)->xC : 1.f);
           }
           if (h + a->cols < H) __syncthreads();
         }
@@ -567,7 +646,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
           fl.wait(h1 - h0 + 1, ep + 2, lane, [&](int i) { return fl.word(rg, (h0 + i) % cols); });
         }
         f32x4 x[NS][2], bias[2], scale[2];
-        WSlice<I8, NS> w[RING];
+        WSlice<MODE, NS> w[RING];
         load_rows(x, a->att, K81, s1, n1);
         ConstLayer* ly = fresh_layer(li);
         take(w, bias, scale, ly->wC, d, cpC, ncC);
@@ -583,22 +662,22 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       request_D(li);
 
       // ---- c_fc: LN2, GELU ----
-      WSlice<I8, CH> we;  // the second MLP product's first weights
+      WSlice<MODE, CH> we;  // the second MLP product's first weights
       const auto request_E = [&] {
         ConstLayer* ly = fresh_layer(li);
         const int ol = opaque(lane), r = ol & 15;
-        we.load(buffer_of(ly->wE, (size_t)4 * d * d * (I8 ? 1 : 4)), d, K84, cg * cpC + r, r < ncC, s4, n4, ol >> 4);
+        we.load(weights_of<MODE>(ly->wE, 4 * d, d), d, K84, cg * cpC + r, r < ncC, s4, n4, ol >> 4);
         request_cols(ly->bE, ly->sE, d, cpC, ncC);
       };
       if (tilesD) {
         f32x4 x[NS][2], bias[2], scale[2];
-        WSlice<I8, NS> w[RING];
+        WSlice<MODE, NS> w[RING];
         ConstArgs* a = fresh_args();
         if (n1 > 0) wait_cols(cpC, a->rcpC, 32 * s1, last_col(s1, n1, d), ep + 3);
         load_rows(x, a->x1, K81, s1, n1);
         ConstLayer* ly = fresh_layer(li);
         take(w, bias, scale, ly->wD, 4 * d, cpD, ncD);
-        normalise(x);
+        normalise(x, ly->xD);
         multiply(x, w, ly->wD, 4 * d, cpD, ncD, tilesD);
         __syncthreads();
         if (bail) return;
@@ -610,7 +689,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
           f32x4 v = finished(tilesD, i, bias, scale);
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = gelu_ref(v[e]);
-          st_agent(h + row_offset(er, cg * cpD + n), v);
+          put_row<MODE>(h, er, cg * cpD + n, v, PAIR ? ly->xE : 1.f);
         }
         raise(ep + 4);
       }
@@ -620,7 +699,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       if (tilesC) {
         ConstArgs* a = fresh_args();
         constexpr int TM = 2;  // tiles of a pass over the slice
-        const __amdgpu_buffer_rsrc_t b = buffer_of(fresh_layer(li)->wE, (size_t)4 * d * d * (I8 ? 1 : 4));
+        const __amdgpu_buffer_rsrc_t b = weights_of<MODE>(fresh_layer(li)->wE, 4 * d, d);
         const float* hidden = a->h;
         const int ol = opaque(lane), r = ol & 15, kg = ol >> 4;
         if (n4 > 0) wait_cols(cpD, a->rcpD, 32 * s4, last_col(s4, n4, 4 * d), ep + 4);
@@ -631,9 +710,9 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           bias[i] = bias_next[i];
-          if constexpr (I8) scale[i] = scale_next[i];
+          if constexpr (SCALED) scale[i] = scale_next[i];
         }
-        WSlice<I8, CH> w[2] = {we, we};
+        WSlice<MODE, CH> w[2] = {we, we};
         bool bad = false;
 #pragma unroll 1
         for (int t0 = 0; t0 < tilesC; t0 += TM) {
@@ -649,7 +728,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
           for (int t = 0; t < TM; ++t) sum[t] = f32x4{0.f, 0.f, 0.f, 0.f};
           const auto chunk = [&](f32x4 (&xc)[CH][2], int c) {
-            Operands<I8, CH> xs;
+            Operands<MODE, CH> xs;
             xs.set(xc);
             load_rows(xc, hidden, K84, s4 + c + 2 * CH, n4 - c - 2 * CH);
             sum[0] += products(w[0].s, xs);
@@ -667,7 +746,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
 #pragma unroll
           for (int t = 0; t < TM; ++t)
             if (t0 + t < tilesC) {
-              bad = bad || (em < T && spoilt<I8>(sum[t]));
+              bad = bad || (em < T && spoilt<MODE>(sum[t]));
               red[(wave * tilesC + t0 + t) * 64 + lane] = sum[t];
             }
         }
@@ -780,29 +859,32 @@ size_t lds_bytes(const PrefillArgs& a) {
   return need > 84 * 1024 ? need : 84 * 1024;  // more than half of a compute unit's, so that exactly one workgroup lives on each
 }
 
-template <bool I8, int NS, int HJ>
+template <int MODE, int NS, int HJ>
 hipError_t launch_hj(const PrefillArgs& a, hipStream_t s) {
   const size_t lds = lds_bytes(a);
   static bool enabled = false;  // dynamic LDS size already raised
   if (!enabled) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_persistent_kernel<I8, NS, HJ>), hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_persistent_kernel<MODE, NS, HJ>), hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS);
     if (e != hipSuccess) return e;
     enabled = true;
   }
-  prefill_persistent_kernel<I8, NS, HJ><<<PP_GRID, NT, lds, s>>>(a);
+  prefill_persistent_kernel<MODE, NS, HJ><<<PP_GRID, NT, lds, s>>>(a);
   return hipGetLastError();
 }
-template <bool I8, int NS>
+template <int MODE, int NS>
 hipError_t launch_ns(const PrefillArgs& a, hipStream_t s) {
-  return a.hs <= 64 ? launch_hj<I8, NS, 4>(a, s) : launch_hj<I8, NS, 8>(a, s);
+  return a.hs <= 64 ? launch_hj<MODE, NS, 4>(a, s) : launch_hj<MODE, NS, 8>(a, s);
 }
-template <bool I8>
+template <int MODE>
 hipError_t launch_any(const PrefillArgs& a, hipStream_t s) {
-  if (a.d <= 512) return launch_ns<I8, 2>(a, s);
-  if (a.d <= 768) return launch_ns<I8, 3>(a, s);
-  if (a.d <= 1024) return launch_ns<I8, 4>(a, s);
-  if (a.d <= 1280) return launch_ns<I8, 5>(a, s);
-  return launch_ns<I8, 7>(a, s);
+  if (a.d <= PP_PAIR_ABOVE) {
+    if constexpr (is_pair(MODE)) return hipErrorInvalidValue;
+    else return launch_ns<MODE, 2>(a, s);
+  }
+  if (a.d <= 768) return launch_ns<MODE, 3>(a, s);
+  if (a.d <= 1024) return launch_ns<MODE, 4>(a, s);
+  if (a.d <= 1280) return launch_ns<MODE, 5>(a, s);
+  return launch_ns<MODE, 7>(a, s);
 }
 
 }  // namespace
@@ -820,10 +902,16 @@ int prefill_persistent_rows(int d, int H, int hs, int V, bool i8, int compute_un
   return !i8 && d > 1280 ? 64 : PP_MAX_T;
 }
 
-hipError_t launch_prefill_persistent(PrefillArgs a, bool i8, hipStream_t s) {
+hipError_t launch_prefill_persistent(PrefillArgs a, PrefillMode mode, hipStream_t s) {
   if (a.T < 1 || a.T > PP_MAX_T || a.T > a.ctx) return hipErrorInvalidValue;
   cut(a);
-  return i8 ? launch_any<true>(a, s) : launch_any<false>(a, s);
+  switch (mode) {
+    case PP_PLAIN_F32: return launch_any<PP_PLAIN_F32>(a, s);
+    case PP_SPLIT_I8: return launch_any<PP_SPLIT_I8>(a, s);
+    case PP_PAIR_F32: return launch_any<PP_PAIR_F32>(a, s);
+    case PP_PAIR_I8: return launch_any<PP_PAIR_I8>(a, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace wgpt
