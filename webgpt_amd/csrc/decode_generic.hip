@@ -111,38 +111,6 @@ __device__ __forceinline__ float across_keys(float v, int lpk, Op op) {
 }
 __device__ __forceinline__ float dot4(const f32x4& a, const f32x4& b) { return (a[0] * b[0] + a[1] * b[1]) + (a[2] * b[2] + a[3] * b[3]); }
 
-template <int CTRL, int ROWS>
-__device__ __forceinline__ sel_key dpp_first(sel_key v) {  // (lanes without a source get 0, which is no key)
-  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROWS, 0xf, false);
-  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, ROWS, 0xf, false);
-  const sel_key o = (sel_key)hi << 32 | lo;
-  return o > v ? o : v;
-}
-// The first key of the wave, wave-uniform; 0: none.
-__device__ __forceinline__ sel_key wave_first(sel_key v) {
-  v = dpp_first<0x111, 0xf>(v);
-  v = dpp_first<0x112, 0xf>(v);
-  v = dpp_first<0x114, 0xf>(v);
-  v = dpp_first<0x118, 0xf>(v);
-  v = dpp_first<0x142, 0xa>(v);
-  v = dpp_first<0x143, 0xc>(v);
-  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)v, 63), hi = __builtin_amdgcn_readlane((int)(unsigned)(v >> 32), 63);
-  return (sel_key)hi << 32 | lo;
-}
-// The k first of the wave's keys, N a lane, in order: lane r has the r-th, the others 0.
-template <int N>
-__device__ __forceinline__ sel_key wave_firsts(const sel_key (&keys)[N], int k, int lane) {
-  sel_key mine = 0, last = ~(sel_key)0;
-  for (int r = 0; r < k; ++r) {
-    sel_key best = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) best = keys[i] < last && keys[i] > best ? keys[i] : best;
-    last = wave_first(best);
-    if (lane == r) mine = last;
-  }
-  return mine;
-}
-
 // Four consecutive k of one column.
 template <bool I8>
 struct Weight {

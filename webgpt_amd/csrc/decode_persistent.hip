@@ -28,6 +28,8 @@
 // the launch drains.
 #include "decode_persistent.h"
 
+#include "select_key.h"
+
 #include <cstdio>
 #include <type_traits>
 
@@ -57,6 +59,11 @@ __device__ __forceinline__ void publish3(u64* p, float v0, float v1, float v2, u
   pk.z = __float_as_uint(v2);
   pk.w = epoch;
   asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(pk) : "memory");
+}
+
+// Two words side by side.
+__device__ __forceinline__ void publish2(u64* p, unsigned v0, unsigned v1, unsigned epoch) {
+  publish3(p, __uint_as_float(v0), __uint_as_float(epoch), __uint_as_float(v1), epoch);
 }
 
 // Streaming (non-temporal) 128-bit load: weights are read once per token and must
@@ -183,8 +190,8 @@ struct Shared {
   int bail;
   float red[32];
   float red_idx[NW];
-  float cand_v[NW * PD_TOPK];  // per-wave top-k candidates of the vocabulary phase
-  int cand_i[NW * PD_TOPK];
+  sel_key cand[NW * PD_TOPK];    // per-wave top-k candidates of the vocabulary phase
+  sel_key firsts[NW * PD_TOPK];  // and of the words of all workgroups that a wave has taken
 };
 __shared__ Shared sh;
 
@@ -320,7 +327,7 @@ struct WideLoads<7> {
 // whether the two halves of a load are from the same moment; a naturally aligned 8-byte half is never torn.
 template <int N>
 __device__ __forceinline__ void poll_words(const u64* __restrict__ buf, unsigned epoch, float* dst, int* err, int delay,
-                                           unsigned spin_limit) {
+                                           unsigned spin_limit, int n = N) {
   static_assert(N % 2 == 0, "words are polled in pairs");
   constexpr int NPAIR = N / 2;
   constexpr int NP = (NPAIR + NT - 1) / NT;
@@ -330,22 +337,22 @@ __device__ __forceinline__ void poll_words(const u64* __restrict__ buf, unsigned
   const u64* src[NP];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    const bool mine = i * NT + NT <= NPAIR || t + i * NT < NPAIR;
+    const bool mine = (i * NT + NT <= NPAIR || t + i * NT < NPAIR) && (n == N || t + i * NT < n / 2);
     if (mine) pending |= 1u << i;
-    src[i] = buf + 2 * (mine ? t + i * NT : NPAIR - 1);  // (a thread without a pair re-reads the last one)
+    src[i] = buf + 2 * (mine ? t + i * NT : n / 2 - 1);  // (a thread without a pair re-reads the last one)
   }
   unsigned spins = 0;
   nap(delay);
   while (pending) {
     static_for<(NP + CH - 1) / CH>([&](auto CI) {
-      constexpr int c0 = decltype(CI)::value * CH, n = NP - c0 < CH ? NP - c0 : CH;
-      u32x4 pk[n];
-      const u64* ps[n];
+      constexpr int c0 = decltype(CI)::value * CH, nl = NP - c0 < CH ? NP - c0 : CH;
+      u32x4 pk[nl];
+      const u64* ps[nl];
 #pragma unroll
-      for (int i = 0; i < n; ++i) ps[i] = src[c0 + i];
-      WideLoads<n>::run(pk, ps);
+      for (int i = 0; i < nl; ++i) ps[i] = src[c0 + i];
+      WideLoads<nl>::run(pk, ps);
 #pragma unroll
-      for (int i = 0; i < n; ++i)
+      for (int i = 0; i < nl; ++i)
         if ((pending & (1u << (c0 + i))) && pk[i].y == epoch && pk[i].w == epoch) {
           *reinterpret_cast<float2*>(dst + 2 * (t + (c0 + i) * NT)) = make_float2(__uint_as_float(pk[i].x), __uint_as_float(pk[i].z));
           pending &= ~(1u << (c0 + i));
@@ -1009,19 +1016,6 @@ constexpr int NOCAND = 0x7fffffff;
 __device__ __forceinline__ bool cand_before(float ov, int oi, float cv, int ci) {
   return oi != NOCAND && (ci == NOCAND || ov > cv || (ov == cv && oi < ci));
 }
-// The first candidate of the wave in that order, as wave-uniform values.
-__device__ __forceinline__ void wave_first(float& v, int& i) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(v, off);
-    const int oi = __shfl_xor(i, off);
-    if (cand_before(ov, oi, v, i)) {
-      v = ov;
-      i = oi;
-    }
-  }
-}
-
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
@@ -1799,8 +1793,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
             cvv = tv[j];
             cii = ti[j];
           }
-        sh.cand_v[wave * PD_TOPK + lane] = cvv;
-        sh.cand_i[wave * PD_TOPK + lane] = cii;
+        sh.cand[wave * PD_TOPK + lane] = cii != NOCAND ? make_key(cvv, cii) : 0;
       }
       __syncthreads();
       ++ep;
@@ -1821,27 +1814,10 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
       if (SAMPLE) {
         // the workgroup's K best of its waves' candidates (one per lane of wave 0), published in order
         if (wave == 0) {
-          float cv = sh.cand_v[lane];
-          int ci = sh.cand_i[lane];
-          float wv = -INFINITY;
-          int wi = NOCAND;
-          for (int r = 0; r < K; ++r) {
-            float fv = cv;
-            int fi = ci;
-            wave_first(fv, fi);
-            if (lane == r) {
-              wv = fv;
-              wi = fi;
-            }
-            if (ci == fi) {  // indices are unique: the owner retires its candidate
-              cv = -INFINITY;
-              ci = NOCAND;
-            }
-          }
-          if (lane < PD_TOPK) {
-            publish(a.bufAM + 2 * (wg * PD_TOPK + lane), wv, ep);
-            publish(a.bufAM + 2 * (wg * PD_TOPK + lane) + 1, __int_as_float(wi), ep);
-          }
+          static_assert(NW * PD_TOPK == 64, "a candidate per lane");
+          const sel_key all[1] = {sh.cand[lane]};
+          const sel_key mine = wave_firsts(all, K, lane);
+          if (lane < K) publish2(a.bufAM + 2 * (lane * C::G + wg), (unsigned)mine, (unsigned)(mine >> 32), ep);  // the r-th of all side by side
         }
       } else if (tid == 0) {
         float b = sh.red[0];
@@ -1870,7 +1846,32 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
     double ustep = 0.0;
     if (SAMPLE) {
       ustep = a.u ? a.u[step] : a.u_arg[step];
-      poll_words<2 * PD_TOPK * C::G>(a.bufAM, ep, attp, a.err, a.delay[6], a.spin_limit);
+      // A thread takes its words of the K first of all workgroups, and a wave selects from its threads' (K = 2: a word per thread;
+      // with all PD_TOPK places read whatever K, and every wave selecting among the heads of all lists, a step of 117M at top_k 3
+      // was 10 us longer than a greedy one).
+      const auto gather = [&](auto per_thread) {
+        constexpr int N = decltype(per_thread)::value;
+        poll_words<2 * N * NT>(a.bufAM, ep, attp, a.err, a.delay[6], a.spin_limit, 2 * C::G * a.top_k);
+        sel_key mine = 0, last = ~(sel_key)0;
+#pragma unroll 1
+        for (int r = 0; r < a.top_k; ++r) {
+          sel_key best = 0;
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            const int p = opaque(tid) + i * NT;
+            const float2 w = *reinterpret_cast<const float2*>(attp + 2 * p);  // (this thread's own)
+            const sel_key key = p < C::G * a.top_k ? (sel_key)__float_as_uint(w.y) << 32 | __float_as_uint(w.x) : 0;
+            best = key < last && key > best ? key : best;
+          }
+          last = wave_first(best);
+          if (lane == r) mine = last;
+        }
+        if (lane < PD_TOPK) sh.firsts[wave * PD_TOPK + lane] = mine;
+      };
+      static_assert(PD_TOPK * C::G == 4 * NT, "up to four words of candidates for a thread");
+      if constexpr (LROWS == 0) gather(std::integral_constant<int, 4>{});
+      else if (a.top_k <= 2) gather(std::integral_constant<int, 1>{});
+      else gather(std::integral_constant<int, 4>{});
     } else {
       poll_words<2 * C::G>(a.bufAM, ep, attp, a.err, a.delay[6], a.spin_limit);
     }
@@ -1881,61 +1882,23 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
     if (SAMPLE) {
       // Every wave of every workgroup selects the same K candidates in order (selectTopK), applies
       // cpuSoftmax in float64 and sampleFromDistribution with the step's draw (globals.js:47-74).
-      // A workgroup's list arrives in order, so a lane only ever looks at the heads of its G/64 lists.
       const int K = a.top_k;
-      constexpr int LPL = C::G / 64;  // workgroup lists per lane
-      static_assert(C::G % 64 == 0, "workgroup lists are dealt to lanes evenly");
-      float hv[LPL];
-      int hi[LPL], hp[LPL];
-#pragma unroll
-      for (int jj = 0; jj < LPL; ++jj) {
-        const int c = (lane + 64 * jj) * PD_TOPK;
-        hp[jj] = 0;
-        hv[jj] = attp[2 * c];
-        hi[jj] = __float_as_int(attp[2 * c + 1]);
-      }
-      float myv = -INFINITY;  // lane r keeps the r-th selection
-      int myi = NOCAND;
-      for (int r = 0; r < K; ++r) {
-        float fv = -INFINITY;
-        int fi = NOCAND;
-#pragma unroll
-        for (int jj = 0; jj < LPL; ++jj)
-          if (cand_before(hv[jj], hi[jj], fv, fi)) {
-            fv = hv[jj];
-            fi = hi[jj];
-          }
-        wave_first(fv, fi);
-        if (lane == r) {
-          myv = fv;
-          myi = fi;
-        }
-        // the owner moves on to the next entry of that list
-#pragma unroll
-        for (int jj = 0; jj < LPL; ++jj)
-          if (hi[jj] == fi && fi != NOCAND) {
-            ++hp[jj];
-            const int c = (lane + 64 * jj) * PD_TOPK + hp[jj];
-            hv[jj] = hp[jj] < K ? attp[2 * c] : -INFINITY;
-            hi[jj] = hp[jj] < K ? __float_as_int(attp[2 * c + 1]) : NOCAND;
-          }
-      }
+      const sel_key all[1] = {sh.firsts[lane]};
+      const sel_key mine = wave_firsts(all, K, lane);  // lane r: the r-th
+      const unsigned first = __builtin_amdgcn_readfirstlane((unsigned)(mine >> 32));
       // lane r: exp((x_r - max) / temperature); then the sums in the reference's order on every lane
-      const float first = __shfl(myv, 0);
-      const double mye = myi != NOCAND ? exp(((double)myv - (double)first) / a.temperature) : 0.0;
+      const double e = exp(((double)key_value(mine) - (double)key_value((sel_key)first << 32)) / a.temperature);
       double sum = 0.0;
-      for (int r = 0; r < K; ++r) sum = sum + __shfl(mye, r);
+      for (int r = 0; r < K; ++r) sum += wave_read(e, r);
+      const double p = e / sum;
       double cum = 0.0;
-      int pick = NOCAND, lastsel = 0;
-      for (int r = 0; r < K; ++r) {
-        const int si = __shfl(myi, r);
-        if (si != NOCAND) {
-          cum += __shfl(mye, r) / sum;
-          lastsel = si;
-          if (pick == NOCAND && ustep < cum) pick = si;
-        }
+      int pick = -1;
+      for (int r = 0; r < K && pick < 0; ++r) {
+        cum += wave_read(p, r);
+        if (ustep < cum) pick = r;
       }
-      tok = pick != NOCAND ? pick : lastsel;
+      tok = __builtin_amdgcn_readlane(key_index(mine), pick < 0 ? K - 1 : pick);
+      tok = tok >= 0 && tok < a.V ? tok : 0;
       if (wg == 0 && tid == 0) {
         a.out_tok[step] = tok;
         if (a.host_ids) a.host_ids[step] = tok;
