@@ -267,12 +267,21 @@ __global__ __launch_bounds__(256, MB * NB <= 4 ? 3 : 2) void gemm_pair_kernel(Pa
   }
 }
 
-// A wave per row, four rows a workgroup. Each lane holds eight values in G runs of 512. (layernorm_kernel's steps; memory and its
-// latency bound it: a row is read once, with the sums of its slices in flight together.)
-template <int G>
+// W = 1: a wave per row, four rows a workgroup. W = 4: a workgroup per row. Each lane holds eight values in G runs of 512 W.
+// (layernorm_kernel's steps; memory and its latency bound it: a row is read once, with the sums of its slices in flight together.)
+template <int G, int W>
 __global__ __launch_bounds__(256) void ln_pair_kernel(PairLnArgs a) {
-  const int row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  __shared__ float sh[8];
+  constexpr int RUN = 512 * W;
+  const int row = W > 1 ? (int)blockIdx.x : (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = W > 1 ? threadIdx.x : threadIdx.x & 63;
   if (row >= a.M) return;
+  const auto row_sum = [&](float v, float* to) {
+    v = wave_sum(v);
+    if constexpr (W == 1) return v;
+    if ((lane & 63) == 0) to[lane >> 6] = v;
+    __syncthreads();
+    return (to[0] + to[1]) + (to[2] + to[3]);
+  };
   // (loads of a lane beyond the row, or of a slice too many, ask for nothing and give zeros: under a branch each would be waited for)
   const size_t row_bytes = 4 * (size_t)a.d;
   float* const xr = a.x + (size_t)row * a.d;
@@ -282,7 +291,7 @@ __global__ __launch_bounds__(256) void ln_pair_kernel(PairLnArgs a) {
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) v[g][h] = load4<0>(xb, 2048 * g + 32 * lane + 16 * h);
+    for (int h = 0; h < 2; ++h) v[g][h] = load4<0>(xb, 4 * RUN * g + 32 * lane + 16 * h);
   if (a.S > 0) {
     const __amdgpu_buffer_rsrc_t sb = buffer_of(a.bias, row_bytes);
     f32x4 p[G][2][PAIR_MAX_SLICES], bias[G][2];
@@ -290,7 +299,7 @@ __global__ __launch_bounds__(256) void ln_pair_kernel(PairLnArgs a) {
     for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int o = 2048 * g + 32 * lane + 16 * h;
+        const int o = 4 * RUN * g + 32 * lane + 16 * h;
 #pragma unroll
         for (int s = 0; s < PAIR_MAX_SLICES; ++s) p[g][h][s] = load4<0>(buffer_of(a.part + ((size_t)s * a.M + row) * a.d, s < a.S ? row_bytes : 0), o);
         bias[g][h] = load4<0>(sb, o);
@@ -300,7 +309,7 @@ __global__ __launch_bounds__(256) void ln_pair_kernel(PairLnArgs a) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         v[g][h] += ((p[g][h][0] + p[g][h][1]) + (p[g][h][2] + p[g][h][3])) + bias[g][h];
-        const int k = 512 * g + 8 * lane + 4 * h;
+        const int k = RUN * g + 8 * lane + 4 * h;
         if (k < a.d) *reinterpret_cast<f32x4*>(xr + k) = v[g][h];
       }
   }
@@ -308,26 +317,26 @@ __global__ __launch_bounds__(256) void ln_pair_kernel(PairLnArgs a) {
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      ga[g][h] = load4<0>(gb, 2048 * g + 32 * lane + 16 * h);
-      be[g][h] = load4<0>(bb, 2048 * g + 32 * lane + 16 * h);
+      ga[g][h] = load4<0>(gb, 4 * RUN * g + 32 * lane + 16 * h);
+      be[g][h] = load4<0>(bb, 4 * RUN * g + 32 * lane + 16 * h);
       sum += (v[g][h][0] + v[g][h][1]) + (v[g][h][2] + v[g][h][3]);
     }
   if (!a.out) return;
-  const float mean = wave_sum(sum) / (float)a.d;
+  const float mean = row_sum(sum, sh) / (float)a.d;
   float q = 0.f;
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      if (512 * g + 8 * lane + 4 * h < a.d) {
+      if (RUN * g + 8 * lane + 4 * h < a.d) {
         const f32x4 e = v[g][h] - mean;
         q += (e[0] * e[0] + e[1] * e[1]) + (e[2] * e[2] + e[3] * e[3]);
       }
-  const float stdev = sqrtf(wave_sum(q) / (float)a.d + 1e-5f), rstd = 1.0f / stdev;
+  const float stdev = sqrtf(row_sum(q, sh + 4) / (float)a.d + 1e-5f), rstd = 1.0f / stdev;
   u32x4* out = static_cast<u32x4*>(a.out);
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    const int k = 512 * g + 8 * lane;
+    const int k = RUN * g + 8 * lane;
     if (k >= a.d) continue;
     u32x4 hi, lo;
 #pragma unroll
@@ -594,14 +603,20 @@ hipError_t launch_gemm_pair(const PairPlan& p, PairGemmArgs a, bool i8, hipStrea
 }
 
 hipError_t launch_ln_pair(const PairLnArgs& a, hipStream_t s) {
+  // Few rows leave compute units without one of four waves' rows: a workgroup per row, us at 200 x 1280 6.1 -> 5.0, 300 x 1600 (four slices)
+  // 7.6 -> 6.3, 500 x 1280 6.8 -> 6.4; 500 x 1600 6.4 either way, 512 x 1024 6.0 -> 6.2, 943 x 768 6.3 -> 7.0, 1000 x 1280 6.8 -> 7.5.
+  if (a.M <= 400 && a.d <= 2048) {
+    ln_pair_kernel<1, 4><<<(unsigned)a.M, 256, 0, s>>>(a);
+    return hipGetLastError();
+  }
   const unsigned grid = (unsigned)(a.M + 3) / 4;
   switch ((a.d + 511) / 512) {
-    case 1: ln_pair_kernel<1><<<grid, 256, 0, s>>>(a); break;
-    case 2: ln_pair_kernel<2><<<grid, 256, 0, s>>>(a); break;
-    case 3: ln_pair_kernel<3><<<grid, 256, 0, s>>>(a); break;
-    case 4: ln_pair_kernel<4><<<grid, 256, 0, s>>>(a); break;
+    case 1: ln_pair_kernel<1, 1><<<grid, 256, 0, s>>>(a); break;
+    case 2: ln_pair_kernel<2, 1><<<grid, 256, 0, s>>>(a); break;
+    case 3: ln_pair_kernel<3, 1><<<grid, 256, 0, s>>>(a); break;
+    case 4: ln_pair_kernel<4, 1><<<grid, 256, 0, s>>>(a); break;
     case 5:
-    case 6: ln_pair_kernel<6><<<grid, 256, 0, s>>>(a); break;
+    case 6: ln_pair_kernel<6, 1><<<grid, 256, 0, s>>>(a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
