@@ -1852,6 +1852,8 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
       const auto gather = [&](auto per_thread) {
         constexpr int N = decltype(per_thread)::value;
         poll_words<2 * N * NT>(a.bufAM, ep, attp, a.err, a.delay[6], a.spin_limit, 2 * C::G * a.top_k);
+        // (read from LDS for each of the top_k: kept in registers, behind the weights that are on their way, they cost the int8 shape
+        // four more spilled ones and 4.5 % of a token)
         sel_key mine = 0, last = ~(sel_key)0;
 #pragma unroll 1
         for (int r = 0; r < a.top_k; ++r) {
