@@ -99,6 +99,34 @@ def test_rows_that_are_no_numbers(device):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head", [(512, 8), (768, 12), (640, 5)])
+def test_shorter_prompt_behind_a_longer_one(device, dtype, d, n_head):
+    """A gain of 64 that c_attn's row makes up for: the rows that the longer prompt's last layer left behind are far beyond what the first
+    one's values can be, and the shorter prompt has the results of a fresh model."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=300, vocab_size=301, dtype=dtype)
+    tensors = {k: v.copy() for k, v in make_model(cfg, 6).items()}
+    for i in range(2):
+        p = f"transformer.h.{i}."
+        tensors[p + "ln_1.weight"][5] = 64.0
+        if dtype == "f32":
+            tensors[p + "attn.c_attn.weight"][5] /= 64.0
+        else:
+            tensors[p + "attn.c_attn.weight.q"][5] = 0x01FF01FF  # (-1, 1, -1, 1)
+    tokens = synth.tokens(7, "prompt", 300, cfg["vocab_size"])
+    fresh, gpt = load(cfg, tensors), load(cfg, tensors)
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    gpt.prefill(tokens)
+    for T in (150, 131):
+        want, got = fresh.prefill(tokens[:T]), gpt.prefill(tokens[:T])
+        assert np.array_equal(got, want) and close(got, ref.forward(p, w, tokens[:T])), T
+        gpt.prefill(tokens)
+        fresh.unloadBuffers()
+        fresh = load(cfg, tensors)
+    gpt.unloadBuffers()
+    fresh.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
 @pytest.mark.parametrize("d,n_head", [(520, 13), (1024, 16), (1288, 23), (1608, 67)])
 def test_short_prompts_of_weights_beyond_the_pairs(device, dtype, d, n_head):
     """One column that the pairs cannot take: short prompts run in one launch all the same, on plain values."""

@@ -15,7 +15,7 @@ __host__ __device__ inline int pair_attn_steps(int hs) { return 2 * ((hs + 31) /
 // Bytes of the operands of up to T rows of H heads of q, keys or values: [H][block or tile][steps][2 parts][64 lanes] units of 16
 // bytes, the eight values that the lane supplies to the step. q and keys: row lane % 32, dimensions 16 step + 8 (lane / 32) ..;
 // values: dimension 32 (step / 2) + lane % 32, and of the sixteen keys of step % 2 the eight 4 (lane / 32) .. + 3 and + 8 .. + 11.
-// Dimensions beyond the head size are zeros (once); rows beyond the last hold anything, values of them anything finite.
+// Dimensions beyond the head size are zeros (once); rows beyond the last of its block or tile hold anything, values of them zeros.
 inline int pair_attn_tiles(int T) { return (T + PAIR_ATTN_ROWS - 1) / PAIR_ATTN_ROWS; }
 inline size_t pair_attn_bytes(int T, int H, int hs) {
   return (size_t)H * pair_attn_tiles(T) * pair_attn_steps(hs) * 2048;

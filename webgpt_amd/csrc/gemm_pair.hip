@@ -68,7 +68,8 @@ __device__ __forceinline__ unsigned ror8(unsigned v) { return __builtin_amdgcn_m
 __device__ __forceinline__ void put_heads(const PairGemmArgs& a, int block, int r, int half, int n8, const f32x4& v) {
   const int which = n8 < a.d ? 0 : n8 < 2 * a.d ? 1 : 2, e = n8 - which * a.d;
   const int h = __builtin_amdgcn_readfirstlane(div_by(e, a.hs, a.rhs)), dim = e - h * a.hs;
-  if (which && block * 32 + r < a.M) {
+  const bool row = block * 32 + r < a.M;
+  if (which && row) {
     float* const rows = (which == 2 ? a.Vc : a.Kc) + ((size_t)h * a.ctx + block * 32) * a.hs + dim;
     *reinterpret_cast<f32x4*>(rows + (r * a.hs + 4 * half)) = v;
   }
@@ -77,8 +78,10 @@ __device__ __forceinline__ void put_heads(const PairGemmArgs& a, int block, int 
                        (size_t)(h * a.head_tiles + block) * (pair_attn_steps(a.hs) * 128);
   unsigned hi[2], lo[2];
   if (which == 2) {
+    // (finite in fp16: a row's values are no numbers or within the bound; the rows beyond the last come from what another layer of an
+    // earlier, longer prompt has left in A, for which that bound does not hold)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = fabsf(x[i]) < INFINITY ? x[i] : 0.f;
+    for (int i = 0; i < 4; ++i) x[i] = row && fabsf(x[i]) < INFINITY ? x[i] : 0.f;
     x = transpose_quad(x);  // four keys of a dimension
     pair_f16(x[0], x[1], hi[0], lo[0]);
     pair_f16(x[2], x[3], hi[1], lo[1]);
