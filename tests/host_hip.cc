@@ -1,5 +1,6 @@
 // The HIP calls that libwebgpt_amd.so makes, on host memory: allocations and copies are the host's, a kernel launch does
-// nothing but count, and launch `host_hip_fail_at` (from 1; 0: none) or allocation `host_hip_alloc_fail_at` fails instead. Loaded in front of the library
+// nothing but count, and launch `host_hip_fail_at` (from 1; 0: none) or allocation `host_hip_alloc_fail_at` fails instead; the error
+// stays until hipGetLastError has been asked. Loaded in front of the library
 // (RTLD_GLOBAL) it takes the place of the HIP runtime in that process, so that the library's host code can be tested
 // without a GPU, its error paths among them.
 #include <cstdlib>
@@ -50,8 +51,8 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
 hipError_t hipGetSymbolAddress(void** p, const void*) { return *p = symbol, hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 static hipError_t allocate(void** p, size_t n) {
-  if (++host_hip_allocs == host_hip_alloc_fail_at) return hipErrorOutOfMemory;
-  return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
+  if (++host_hip_allocs == host_hip_alloc_fail_at || !(*p = malloc(n))) return last = hipErrorOutOfMemory;
+  return hipSuccess;
 }
 hipError_t hipMalloc(void** p, size_t n) { return allocate(p, n); }
 hipError_t hipFree(void* p) { return ++host_hip_frees, free(p), hipSuccess; }

@@ -106,6 +106,34 @@ for i in range(1, total + 1):
 """)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+def test_finalize_without_memory_for_the_pairs(host_hip, dtype):
+    """Of a model whose products can be made of pairs of fp16 values: the one allocation of theirs may fail, and the model runs without them;
+    behind every other failure a second call succeeds."""
+    run(host_hip, dtype, """
+cfg.update(n_embd=520, n_head=13, n_ctx=140, n_layer=1)
+tensors = make_model(cfg, 1)
+m = model()
+at = allocs.value
+_lib.call("wgpt_model_finalize", m)
+total, without = allocs.value - at, 0
+_lib.call("wgpt_model_destroy", m)
+tokens = np.zeros(140, np.int32)
+for i in range(1, total + 1):
+    m = model()
+    alloc_fail_at.value = allocs.value + i
+    why = refused("wgpt_model_finalize", m)
+    alloc_fail_at.value = 0
+    without += why is None
+    if why:
+        assert refused("wgpt_model_finalize", m) is None, (i, why)
+    for T in (140, 2):
+        _lib.call("wgpt_prefill", m, tokens.ctypes.data_as(C.POINTER(C.c_int32)), T, None)
+    _lib.call("wgpt_model_destroy", m)
+assert without == 1, (without, total)
+""")
+
+
 def test_buffers_of_a_window_that_grows(host_hip):
     """Nineteen buffers a window, given back behind it, as a forward from blocks has them: a window of a token more finds its memory among
     that of the shorter ones, also when those of many lengths have been left behind, and what is held stays within its bound."""

@@ -28,7 +28,8 @@ Runtime& rt();
 // least `need` bytes. Returns nullptr (and records the error) otherwise.
 void* resolve(wgpt_buf h, size_t need, const char* what);
 
-// hipMalloc that gives the freed buffers back which wgpt_free has kept before it reports that memory has run out.
+// hipMalloc that gives the freed buffers back which wgpt_free has kept before it reports that memory has run out. An error is its
+// result alone: HIP would hand it to the next launch that asks for the last one too.
 hipError_t device_malloc(void** out, size_t bytes);
 
 // Pinned words through which `count` token ids pass to a launch on the library's stream that is made before the next call; the
@@ -41,10 +42,14 @@ void release_scratch();
 // with `device` current.
 int setup_noalloc_scratch(int device);
 
+// (The error is reported here: HIP keeps it until it is asked for, and the launches of a later call would ask.)
 #define WGPT_HIP(call)                                                                      \
   do {                                                                                      \
     hipError_t e_ = (call);                                                                 \
-    if (e_ != hipSuccess) return ::wgpt::fail(WGPT_ERR_HIP, "%s: %s", #call, hipGetErrorString(e_)); \
+    if (e_ != hipSuccess) {                                                                 \
+      (void)hipGetLastError();                                                              \
+      return ::wgpt::fail(WGPT_ERR_HIP, "%s: %s", #call, hipGetErrorString(e_));            \
+    }                                                                                       \
   } while (0)
 
 #define WGPT_REQUIRE_INIT()                                                                  \

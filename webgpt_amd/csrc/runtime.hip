@@ -108,10 +108,8 @@ static bool pool_release() {  // (hipFree waits for the device)
 }
 hipError_t device_malloc(void** out, size_t bytes) {
   hipError_t e = hipMalloc(out, bytes);
-  if (e == hipErrorOutOfMemory && pool_release()) {
-    (void)hipGetLastError();
-    e = hipMalloc(out, bytes);
-  }
+  if (e == hipErrorOutOfMemory && pool_release()) e = hipMalloc(out, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
   return e;
 }
 
@@ -275,10 +273,7 @@ int wgpt_alloc(size_t bytes, wgpt_buf* out) {
   p = pool_take(size);
   if (!p) {
     hipError_t e = device_malloc(&p, size);
-    if (e == hipErrorOutOfMemory) {
-      (void)hipGetLastError();
-      e = device_malloc(&p, size = plain_size(bytes));
-    }
+    if (e == hipErrorOutOfMemory) e = device_malloc(&p, size = plain_size(bytes));
     if (e != hipSuccess) return fail(WGPT_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   }
   wgpt_buf h = g_next_handle++;
