@@ -75,6 +75,34 @@ def test_weights_beyond_the_pairs(device, how):
     taps.unloadBuffers()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head,T", [(512, 8, 140), (520, 13, 140), (520, 13, 60), (1024, 16, 60)])
+@pytest.mark.parametrize("how", ["dead unit", "value column", "value head"])
+def test_one_wide_column(device, dtype, d, n_head, T, how):
+    """A bound far beyond the others', in the rows that c_proj or the second MLP product reads: what the others' values hold is not lost.
+    A hidden unit that its bias keeps at zero; values that c_proj's rows make up for."""
+    cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=140, vocab_size=101, dtype=dtype)
+    tensors = {k: v.copy() for k, v in make_model(cfg, 3).items()}
+    p = "transformer.h.1."
+    if how == "dead unit":
+        tensors[p + "mlp.c_fc.bias"][0] = -1e9
+    else:
+        cols, up = slice(2 * d + 3, 2 * d + 4) if how == "value column" else slice(2 * d, 2 * d + d // n_head), 24
+        rows = slice(cols.start - 2 * d, cols.stop - 2 * d)
+        tensors[p + "attn.c_attn.bias"][cols] *= np.float32(2.0 ** up)
+        if dtype == "f32":
+            tensors[p + "attn.c_attn.weight"][:, cols] *= np.float32(2.0 ** up)
+            tensors[p + "attn.c_proj.weight"][rows] *= np.float32(2.0 ** -up)
+        else:  # (no row of int8 weights is that small: without the column)
+            tensors[p + "attn.c_attn.weight.scale"][cols] *= np.float32(2.0 ** up)
+            tensors[p + "attn.c_proj.weight.q"][rows] = 0
+    gpt, tokens = load(cfg, tensors), synth.tokens(3, "prompt", T, cfg["vocab_size"])
+    want = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens)
+    got = gpt.prefill(tokens)
+    assert close(got, want), worst(got, want)
+    gpt.unloadBuffers()
+
+
 def test_rows_that_are_no_numbers(device):
     """An embedding that is infinite makes its row's logits and those of the rows behind it NaN, and none of the tiles before it; the next
     prompt is not affected by what was left in the rows' memory."""

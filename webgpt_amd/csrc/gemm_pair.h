@@ -70,10 +70,13 @@ hipError_t launch_pair_weights(int K, int N, const float* W, void* out, float* c
 hipError_t launch_pair_scales(int N, const float* scale, float* cscale, unsigned* stats, hipStream_t s);
 // Largest absolute value that (LayerNorm with gamma and beta) . W + bias can have in each of `runs` equal runs of the columns of W
 // [K, N] (int8: words of four columns and scales), and that the LayerNorm itself can have: as floats at bound[run] and *ln_bound.
-// Infinite where the run is one of the first `even` and more than one in 64 of its columns have bounds below 2^-10 of the largest.
+// Infinite where a column of the run has a bound, but zero, below spread.least of the largest: one scale does not fit both.
 // sums: pair_bounds_floats(K, N) of memory.
+struct PairSpread {
+  float least[3];
+};
 size_t pair_bounds_floats(int K, int N);
-hipError_t launch_pair_bounds(int K, int N, int runs, int even, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
+hipError_t launch_pair_bounds(int K, int N, int runs, PairSpread spread, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
                               const float* gamma, const float* beta, float* sums, float* bound, float* ln_bound, hipStream_t s);
 // cscale[n] *= factor (a power of two)
 hipError_t launch_pair_rescale(int N, float factor, float* cscale, hipStream_t s);

@@ -12,8 +12,10 @@
 // fp16's range: a matrix of rows has one scale, a power of two from a bound that its values cannot leave. Behind a LayerNorm a
 // normalised value is at most sqrt(d), so a row times gamma plus beta, its product with a column (Cauchy), GELU of that and
 // averages of it (attention) are bounded by the weights alone (launch_pair_bounds). A column of weights has a scale of its own.
-// Values 17 bits below the bound lose relative precision, not absolute: 2^-40 of the bound. Models whose weights span more than that
-// (more than one in 64 of a column, or of gamma), or leave 2^-80 .. 2^80, or are not finite, are counted when they are loaded and
+// Values 17 bits below the bound lose relative precision, not absolute: 2^-40 of the bound. A value behind a LayerNorm is about the root of
+// the width below its column's bound, an average of T such values the root of T further, and columns below the widest one by the difference:
+// how far they may be (PairSpread, model.hip) is where the error of their pairs begins to grow. Models with wider rows, whose weights span more than 2^17
+// (more than one in 64 of a column) or of gamma 2^10, or leave 2^-80 .. 2^80, or are not finite, are found when they are loaded and
 // keep the six products. A LayerNorm's row is finite or nothing but NaN, so no sum has to be taken again.
 //
 // The four waves of a workgroup split K: each holds the whole tile, its operands come straight from memory in loads of 1 KB,
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(256) void pair_bounds_kernel(int K, int N, const fl
   sums[(size_t)blockIdx.y * N + t.n] = make_float2(s, d);
 }
 // A workgroup per run of n columns.
-__global__ __launch_bounds__(1024) void pair_bounds_end(int K, int N, int n, int even, const float* __restrict__ bias, float2* sums, float* bound) {
+__global__ __launch_bounds__(1024) void pair_bounds_end(int K, int N, int n, PairSpread spread, const float* __restrict__ bias, float2* sums, float* bound) {
   __shared__ unsigned most;
   __shared__ int low;
   if (threadIdx.x == 0) most = 0u, low = 0;
@@ -498,13 +500,11 @@ __global__ __launch_bounds__(1024) void pair_bounds_end(int K, int N, int n, int
   atomicMax(&most, __float_as_uint(top));
   __syncthreads();
   top = __uint_as_float(most);
-  if ((int)blockIdx.x < even) {
-    int few = 0;
-    for (int c = n0 + threadIdx.x; c < n0 + n; c += 1024) few += sums[c].x != 0.f && sums[c].x < 0x1p-10f * top;
-    if (few) atomicAdd(&low, few);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) bound[blockIdx.x] = 64 * low <= n ? top : INFINITY;
+  const float least = spread.least[blockIdx.x] * top;
+  for (int c = n0 + threadIdx.x; c < n0 + n; c += 1024)
+    if (sums[c].x != 0.f && sums[c].x < least) low = 1;
+  __syncthreads();
+  if (threadIdx.x == 0) bound[blockIdx.x] = low ? INFINITY : top;
 }
 // One workgroup: the largest |LayerNorm|, infinite where too many of gamma are far below the largest one.
 __global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, const float* __restrict__ gamma, const float* __restrict__ beta, float* bound) {
@@ -637,11 +637,11 @@ hipError_t launch_pair_scales(int N, const float* scale, float* cscale, unsigned
   return hipGetLastError();
 }
 size_t pair_bounds_floats(int K, int N) { return (size_t)2 * ((K + CHUNK - 1) / CHUNK) * N; }
-hipError_t launch_pair_bounds(int K, int N, int runs, int even, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
+hipError_t launch_pair_bounds(int K, int N, int runs, PairSpread spread, const float* W, const int32_t* Wq, const float* wscale, const float* bias,
                               const float* gamma, const float* beta, float* sums, float* bound, float* ln_bound, hipStream_t s) {
   float2* const p = reinterpret_cast<float2*>(sums);
   pair_bounds_kernel<<<dim3((N + 31) / 32, (K + CHUNK - 1) / CHUNK), 256, 0, s>>>(K, N, W, Wq, wscale, gamma, beta, p);
-  pair_bounds_end<<<runs, 1024, 0, s>>>(K, N, N / runs, even, bias, p, bound);
+  pair_bounds_end<<<runs, 1024, 0, s>>>(K, N, N / runs, spread, bias, p, bound);
   pair_ln_bound_kernel<<<1, 256, 0, s>>>(K, gamma, beta, ln_bound);
   return hipGetLastError();
 }

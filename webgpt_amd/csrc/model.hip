@@ -686,6 +686,10 @@ static int block_linear_weights(Model* m, void* free_buf) {
 // values each (gemm_pair.hip).
 constexpr int PAIR_MIN_D = 512;
 constexpr int PAIR_MIN_T = 64;
+// What the bounds of a matrix's columns may be of the largest one, so that its scale serves them all. Error of pairs of normal values 0, 6, 8, 10 and 12
+// bits below the others, widths of 512 and 1600: rows of q, keys and the hidden layer 5.0e-8, 5.0e-8, 5.2e-8, 8.1e-8, 2.8e-7; averages of 300 to 1024 values
+// 0, 5, 6, 8 and 10 bits below: 7.4e-8, 7.6e-8, 1.1e-7, 3.3e-7, 1.3e-6.
+constexpr float PAIR_ROWS_LEAST = 0x1p-8f, PAIR_VALUES_LEAST = 0x1p-5f;
 
 // Prepares forward_pairs (before block_linear_weights: it reads the matrices as they came). Leaves m->pairs empty, and forward_blocks
 // in charge, where the weights do not allow it or memory has run out.
@@ -739,8 +743,9 @@ static int setup_pairs(Model* m) {
       }
     }
     float* b = (float*)stats + 1 + NB * i;
-    LAUNCH(launch_pair_bounds(d, 3 * d, 3, heads ? 2 : 0, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
-    LAUNCH(launch_pair_bounds(d, hid, 1, 0, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 5, b + 4, rt().stream));
+    const float qk = heads ? PAIR_ROWS_LEAST : 0.f;
+    LAUNCH(launch_pair_bounds(d, 3 * d, 3, {{qk, qk, PAIR_VALUES_LEAST}}, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
+    LAUNCH(launch_pair_bounds(d, hid, 1, {{PAIR_ROWS_LEAST}}, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 5, b + 4, rt().stream));
   }
   std::vector<unsigned> host(1 + NB * (size_t)L);
   WGPT_HIP(hipMemcpyAsync(host.data(), stats, sizeof(unsigned) * host.size(), hipMemcpyDeviceToHost, rt().stream));
