@@ -77,15 +77,19 @@ def test_weights_beyond_the_pairs(device, how):
 
 @pytest.mark.parametrize("dtype", ["f32", "int8"])
 @pytest.mark.parametrize("d,n_head,T", [(512, 8, 140), (520, 13, 140), (520, 13, 60), (1024, 16, 60)])
-@pytest.mark.parametrize("how", ["dead unit", "value column", "value head"])
+@pytest.mark.parametrize("how", ["dead unit", "value column", "value head", "ln_1 beta", "ln_2 beta", "ln_2 gamma"])
 def test_one_wide_column(device, dtype, d, n_head, T, how):
-    """A bound far beyond the others', in the rows that c_proj or the second MLP product reads: what the others' values hold is not lost.
-    A hidden unit that its bias keeps at zero; values that c_proj's rows make up for."""
+    """A bound far beyond the others', in the rows that a product reads: what the others' values hold is not lost. A hidden unit that its
+    bias keeps at zero; values that c_proj's rows make up for; a channel of a LayerNorm that nothing reads."""
     cfg = small_cfg(n_layer=2, n_head=n_head, n_embd=d, n_ctx=140, vocab_size=101, dtype=dtype)
     tensors = {k: v.copy() for k, v in make_model(cfg, 3).items()}
     p = "transformer.h.1."
     if how == "dead unit":
         tensors[p + "mlp.c_fc.bias"][0] = -1e9
+    elif how.startswith("ln"):
+        reader = "attn.c_attn.weight" if how.startswith("ln_1") else "mlp.c_fc.weight"
+        tensors[p + how[:4] + (".bias" if how.endswith("beta") else ".weight")][0] = 1e9
+        tensors[p + reader + (".q" if dtype == "int8" else "")][0] = 0
     else:
         cols, up = slice(2 * d + 3, 2 * d + 4) if how == "value column" else slice(2 * d, 2 * d + d // n_head), 24
         rows = slice(cols.start - 2 * d, cols.stop - 2 * d)

@@ -70,10 +70,10 @@ hipError_t launch_pair_weights(int K, int N, const float* W, void* out, float* c
 hipError_t launch_pair_scales(int N, const float* scale, float* cscale, unsigned* stats, hipStream_t s);
 // Largest absolute value that (LayerNorm with gamma and beta) . W + bias can have in each of `runs` equal runs of the columns of W
 // [K, N] (int8: words of four columns and scales), and that the LayerNorm itself can have: as floats at bound[run] and *ln_bound.
-// Infinite where a column of the run has a bound, but zero, below spread.least of the largest: one scale does not fit both.
-// sums: pair_bounds_floats(K, N) of memory.
+// Infinite where a column of the run, or a channel of the LayerNorm, has a bound, but zero, below spread.least, or .ln, of the largest: one
+// scale does not fit both. sums: pair_bounds_floats(K, N) of memory.
 struct PairSpread {
-  float least[3];
+  float ln, least[3];
 };
 size_t pair_bounds_floats(int K, int N);
 hipError_t launch_pair_bounds(int K, int N, int runs, PairSpread spread, const float* W, const int32_t* Wq, const float* wscale, const float* bias,

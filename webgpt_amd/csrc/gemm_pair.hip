@@ -14,8 +14,8 @@
 // averages of it (attention) are bounded by the weights alone (launch_pair_bounds). A column of weights has a scale of its own.
 // Values 17 bits below the bound lose relative precision, not absolute: 2^-40 of the bound. A value behind a LayerNorm is about the root of
 // the width below its column's bound, an average of T such values the root of T further, and columns below the widest one by the difference:
-// how far they may be (PairSpread, model.hip) is where the error of their pairs begins to grow. Models with wider rows, whose weights span more than 2^17
-// (more than one in 64 of a column) or of gamma 2^10, or leave 2^-80 .. 2^80, or are not finite, are found when they are loaded and
+// how far they may be, a LayerNorm's channels too (PairSpread, model.hip), is where the error of their pairs begins to grow. Models with wider rows,
+// or whose weights span more than 2^17 (more than one in 64 of a column), or leave 2^-80 .. 2^80, or are not finite, are found when they are loaded and
 // keep the six products. A LayerNorm's row is finite or nothing but NaN, so no sum has to be taken again.
 //
 // The four waves of a workgroup split K: each holds the whole tile, its operands come straight from memory in loads of 1 KB,
@@ -506,10 +506,12 @@ __global__ __launch_bounds__(1024) void pair_bounds_end(int K, int N, int n, Pai
   __syncthreads();
   if (threadIdx.x == 0) bound[blockIdx.x] = low ? INFINITY : top;
 }
-// One workgroup: the largest |LayerNorm|, infinite where too many of gamma are far below the largest one.
-__global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, const float* __restrict__ gamma, const float* __restrict__ beta, float* bound) {
+// One workgroup: the largest |LayerNorm|, infinite where a channel can only be far below it, but zero: with one gain, or one bias, far
+// above the others', one scale does not fit both.
+__global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, float least, const float* __restrict__ gamma, const float* __restrict__ beta, float* bound) {
   __shared__ float sh[2][256];
   __shared__ int low;
+  const float root = sqrtf((float)d);
   float g = 0.f, b = 0.f;
   bool odd = false;
   for (int k = threadIdx.x; k < d; k += 256) {
@@ -522,12 +524,13 @@ __global__ __launch_bounds__(256) void pair_ln_bound_kernel(int d, const float* 
   if (threadIdx.x == 0) low = 0;
   __syncthreads();
   for (int i = 0; i < 256; ++i) g = fmaxf(g, sh[0][i]), b = fmaxf(b, sh[1][i]);
-  int n = 0;
-  for (int k = threadIdx.x; k < d; k += 256) n += gamma[k] != 0.f && fabsf(gamma[k]) < 0x1p-10f * g;
-  atomicAdd(&low, n);
+  const float v = root * g + b;
+  for (int k = threadIdx.x; k < d; k += 256) {
+    const float own = root * fabsf(gamma[k]) + fabsf(beta[k]);
+    if (own != 0.f && own < least * v) low = 1;
+  }
   __syncthreads();
-  const float v = sqrtf((float)d) * g + b;
-  if (threadIdx.x == 0) *bound = v < INFINITY && 64 * low <= d ? v : INFINITY;
+  if (threadIdx.x == 0) *bound = v < INFINITY && !low ? v : INFINITY;
 }
 __global__ __launch_bounds__(256) void pair_rescale_kernel(int N, float factor, float* cscale) {
   const int n = (int)blockIdx.x * 256 + threadIdx.x;
@@ -642,7 +645,7 @@ hipError_t launch_pair_bounds(int K, int N, int runs, PairSpread spread, const f
   float2* const p = reinterpret_cast<float2*>(sums);
   pair_bounds_kernel<<<dim3((N + 31) / 32, (K + CHUNK - 1) / CHUNK), 256, 0, s>>>(K, N, W, Wq, wscale, gamma, beta, p);
   pair_bounds_end<<<runs, 1024, 0, s>>>(K, N, N / runs, spread, bias, p, bound);
-  pair_ln_bound_kernel<<<1, 256, 0, s>>>(K, gamma, beta, ln_bound);
+  pair_ln_bound_kernel<<<1, 256, 0, s>>>(K, spread.ln, gamma, beta, ln_bound);
   return hipGetLastError();
 }
 hipError_t launch_pair_rescale(int N, float factor, float* cscale, hipStream_t s) {

@@ -744,8 +744,8 @@ static int setup_pairs(Model* m) {
     }
     float* b = (float*)stats + 1 + NB * i;
     const float qk = heads ? PAIR_ROWS_LEAST : 0.f;
-    LAUNCH(launch_pair_bounds(d, 3 * d, 3, {{qk, qk, PAIR_VALUES_LEAST}}, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
-    LAUNCH(launch_pair_bounds(d, hid, 1, {{PAIR_ROWS_LEAST}}, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 5, b + 4, rt().stream));
+    LAUNCH(launch_pair_bounds(d, 3 * d, 3, {PAIR_ROWS_LEAST, {qk, qk, PAIR_VALUES_LEAST}}, l.attn.w, l.attn.q, l.attn.s, l.attn_b, l.ln1_g, l.ln1_b, sums, b + 1, b, rt().stream));
+    LAUNCH(launch_pair_bounds(d, hid, 1, {PAIR_ROWS_LEAST, {PAIR_ROWS_LEAST}}, l.fc.w, l.fc.q, l.fc.s, l.fc_b, l.ln2_g, l.ln2_b, sums, b + 5, b + 4, rt().stream));
   }
   std::vector<unsigned> host(1 + NB * (size_t)L);
   WGPT_HIP(hipMemcpyAsync(host.data(), stats, sizeof(unsigned) * host.size(), hipMemcpyDeviceToHost, rt().stream));
