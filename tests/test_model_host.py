@@ -134,6 +134,27 @@ assert without == 1, (without, total)
 """)
 
 
+@pytest.mark.parametrize("d,n_head,max_prefill,pairs", [(512, 8, 128, 0), (512, 8, 129, 1), (520, 13, 16, 1), (528, 4, 63, 0), (528, 4, 64, 1)])
+def test_memory_of_the_pairs(host_hip, d, n_head, max_prefill, pairs):
+    """A model whose prompts never read the pairs does not hold them: they all run in the persistent launch and on plain values (512 columns, 128
+    tokens), or there is none (heads of 132) and they are too short."""
+    run(host_hip, "f32", f"""
+cfg.update(n_embd={d}, n_head={n_head}, n_ctx=140, n_layer=1)
+made = []
+for flags in (0, _lib.FLAG_TAPS):  # (with taps: no pairs)
+    p = _lib.Params(**dict(synth.model_params(cfg)), max_prefill={max_prefill}, flags=flags)
+    m = C.c_uint64(0)
+    _lib.call("wgpt_model_create", C.byref(p), C.byref(m))
+    for n, t in make_model(cfg, 1).items():
+        _lib.call("wgpt_model_set_tensor", m, n.encode(), np.ascontiguousarray(t).ctypes.data, t.nbytes)
+    at = allocs.value
+    _lib.call("wgpt_model_finalize", m)
+    made.append(allocs.value - at)
+    _lib.call("wgpt_model_destroy", m)
+assert made[0] - made[1] == {pairs}, made
+""")
+
+
 def test_buffers_of_a_window_that_grows(host_hip):
     """Nineteen buffers a window, given back behind it, as a forward from blocks has them: a window of a token more finds its memory among
     that of the shorter ones, also when those of many lengths have been left behind, and what is held stays within its bound."""

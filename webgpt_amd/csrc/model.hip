@@ -698,6 +698,9 @@ static int setup_pairs(Model* m) {
   const bool i8 = m->p.weight_dtype == 1;
   m->pairs.clear();
   if (d < PAIR_MIN_D || (m->p.flags & WGPT_FLAG_TAPS)) return WGPT_OK;
+  // (a copy of the weights: only where prompts of this model get to read it)
+  const bool launches = m->maxT > m->pp_rows && m->maxT >= PAIR_MIN_T, persistent = m->pp_rows > 0 && d > PP_PAIR_ABOVE;
+  if (!launches && !persistent) return WGPT_OK;
   const auto room = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
   const struct { int K, N; LinW LayerW::*w; void* PairLayer::*wp; float* PairLayer::*c; } lins[4] = {
       {d, 3 * d, &LayerW::attn, &PairLayer::wA, &PairLayer::cA}, {d, d, &LayerW::proj, &PairLayer::wC, &PairLayer::cC},
