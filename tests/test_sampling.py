@@ -248,3 +248,38 @@ def test_decode_sample_rejects_bad_arguments(device):
         assert len(gpt.decode_sample(4, 2, 3, 1.0, [0.1, 0.9])) == 2     # still usable afterwards
     finally:
         gpt.unloadBuffers()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab_size", [301, 5003])
+@pytest.mark.parametrize("d,dtype", [(384, "f32"), (768, "f32"), (1024, "f32"), (1280, "f32"), (1600, "int8")])
+def test_logits_that_are_no_numbers_hide_no_others(device, d, dtype, vocab_size):
+    """Every second token's embedding is NaN, and so is its logit: greedy steps of the kernel of the fixed shapes choose
+    among the others, and the candidates of a sampled step are the ones of the selection on its own."""
+    from oracle import ref
+    from webgpt_amd.model import GPT
+    cfg = small_cfg(n_layer=1, n_head=d // 64, n_embd=d, n_ctx=48, vocab_size=vocab_size, dtype=dtype)
+    tensors = make_model(cfg, 3)
+    wte = tensors["transformer.wte.weight"].copy()
+    wte[2::2] = np.nan
+    tensors["transformer.wte.weight"] = wte
+    gpt = GPT(None, "char", tensors=tensors, params=synth.model_params(cfg))
+    gpt.initialize()
+    history = [int(t) // 2 * 2 - 1 for t in synth.tokens(9, "prompt", 12, vocab_size) if t > 1]
+    w, p = oracle_weights(tensors, cfg), synth.model_params(cfg)
+    picks = {}
+    for mode in (1, 0):
+        gpt.set_decode_mode(mode)
+        gpt.prefill(history[:-1])
+        seen = list(history)
+        with np.errstate(all="ignore"):
+            for t in gpt.decode_greedy(history[-1], 4) if mode else ():
+                assert int(t) == int(np.nanargmax(ref.forward(p, w, np.array(seen, np.int32)))), mode
+                seen.append(int(t))
+        for top_k in (2, 5, 8):
+            gpt.prefill(history[:-1])
+            picks[mode, top_k] = [int(t) for t in gpt.decode_sample(history[-1], 6, top_k, 0.8, np.array([0.0, 0.4, 0.7, 0.9, 0.99, 0.999]))]
+            assert all(t < 2 or t % 2 for t in picks[mode, top_k]), (mode, top_k)
+    assert all(picks[1, k] == picks[0, k] for k in (2, 5, 8)), picks
+    assert gpt.routes()[1] == 0
+    gpt.unloadBuffers()

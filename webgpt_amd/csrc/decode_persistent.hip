@@ -1010,11 +1010,11 @@ __device__ __forceinline__ float column_sum(const float* part, int c) {
 #define TRACE5(k) do {} while (0)
 #endif
 
-// Order of selectTopK (globals.js:66-74): larger logit first, lower index first among equals;
-// index INT_MAX marks an empty candidate.
+// Order of selectTopK (globals.js:66-74): larger logit first, lower index first among equals (NaN behind all numbers, for indices that come
+// in ascending order); index INT_MAX marks an empty candidate.
 constexpr int NOCAND = 0x7fffffff;
 __device__ __forceinline__ bool cand_before(float ov, int oi, float cv, int ci) {
-  return oi != NOCAND && (ci == NOCAND || ov > cv || (ov == cv && oi < ci));
+  return oi != NOCAND && (ci == NOCAND || ov > cv || (ov == cv && oi < ci) || (cv != cv && ov == ov));
 }
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
@@ -1670,7 +1670,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
             const float s = wave_sum(acc);
             if (vb + r < v1) {
               if (lane == 0) a.logits[vb + r] = s;
-              if (s > best || besti == 0x7fffffff) {
+              if (s > best || (besti == NOCAND && s == s)) {  // (NaN: never)
                 best = s;
                 besti = vb + r;
               }
@@ -1705,7 +1705,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
             a.logits[row] = s;
             if (to_host) xs1[row - v0] = s;  // (free since the last layer's second MLP product)
           }
-          if (s > best || besti == 0x7fffffff) {
+          if (s > best || (besti == NOCAND && s == s)) {  // (NaN: never)
             best = s;
             besti = row;
           }
@@ -1925,7 +1925,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
           bi = oi;
         }
       }
-      tok = bi;  // every wave of every workgroup holds the same result
+      tok = bi < a.V ? bi : 0;  // every wave of every workgroup holds the same result
       if (wg == 0 && tid == 0) {
         a.out_tok[step] = tok;
         if (a.host_ids) a.host_ids[step] = tok;
