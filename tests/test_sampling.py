@@ -254,8 +254,8 @@ def test_decode_sample_rejects_bad_arguments(device):
 @pytest.mark.parametrize("vocab_size", [301, 5003])
 @pytest.mark.parametrize("d,dtype", [(384, "f32"), (768, "f32"), (1024, "f32"), (1280, "f32"), (1600, "int8")])
 def test_logits_that_are_no_numbers_hide_no_others(device, d, dtype, vocab_size):
-    """Every second token's embedding is NaN, and so is its logit: greedy steps of the kernel of the fixed shapes choose
-    among the others, and the candidates of a sampled step are the ones of the selection on its own."""
+    """Every second token's embedding is NaN, and so is its logit: greedy steps of the kernel of the fixed shapes, and those with a launch per block,
+    choose among the others, and the candidates of a sampled step are the ones of the selection on its own."""
     from oracle import ref
     from webgpt_amd.model import GPT
     cfg = small_cfg(n_layer=1, n_head=d // 64, n_embd=d, n_ctx=48, vocab_size=vocab_size, dtype=dtype)
@@ -273,7 +273,7 @@ def test_logits_that_are_no_numbers_hide_no_others(device, d, dtype, vocab_size)
         gpt.prefill(history[:-1])
         seen = list(history)
         with np.errstate(all="ignore"):
-            for t in gpt.decode_greedy(history[-1], 4) if mode else ():
+            for t in gpt.decode_greedy(history[-1], 4):
                 assert int(t) == int(np.nanargmax(ref.forward(p, w, np.array(seen, np.int32)))), mode
                 seen.append(int(t))
         for top_k in (2, 5, 8):

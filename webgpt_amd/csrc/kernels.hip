@@ -1503,7 +1503,7 @@ __global__ __launch_bounds__(1024) void argmax_kernel(int V, const float* __rest
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int i = i0 + u * 1024;
-      if (i < V && (v[u] > best || besti == 0x7fffffff)) {
+      if (i < V && (v[u] > best || (besti == 0x7fffffff && v[u] == v[u]))) {  // (NaN: never)
         best = v[u];
         besti = i;
       }
@@ -1526,8 +1526,9 @@ __global__ __launch_bounds__(1024) void argmax_kernel(int V, const float* __rest
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    tok[0] = bi[0];
-    if (out) out[slot] = bi[0];
+    const int first = bi[0] < V ? bi[0] : 0;
+    tok[0] = first;
+    if (out) out[slot] = first;
   }
 }
 
