@@ -788,22 +788,24 @@ static bool prefill_pairs(const Model* m) { return !m->pairs.empty() && m->d > P
 static int setup_prefill(Model* m) {
   const bool i8 = m->p.weight_dtype == 1;
   std::vector<PrefillLayer> layers(m->L);
+  std::vector<PrefillScales> scales(m->L);
   for (int i = 0; i < m->L; ++i) {
     const LayerW& l = m->layers[i];
     const LinW* w[4] = {&l.attn, &l.proj, &l.fc, &l.fc2};
     const void* p[4];
     for (int j = 0; j < 4; ++j) p[j] = i8 ? (const void*)w[j]->q : (const void*)w[j]->w;
     layers[i] = {p[0], p[1], p[2], p[3], w[0]->s, w[1]->s, w[2]->s, w[3]->s, l.attn_b, l.proj_b, l.fc_b, l.fc2_b,
-                 l.ln1_g, l.ln1_b, l.ln2_g, l.ln2_b, 1.f, 1.f, 1.f, 1.f};
+                 l.ln1_g, l.ln1_b, l.ln2_g, l.ln2_b};
     if (!prefill_pairs(m)) continue;
     const PairLayer& q = m->pairs[i];
     PrefillLayer& t = layers[i];
     if (!i8) t.wA = q.wA, t.wC = q.wC, t.wD = q.wD, t.wE = q.wE;
     t.sA = q.cA, t.sC = q.cC, t.sD = q.cD, t.sE = q.cE;
-    t.xA = q.s1, t.xC = q.sv, t.xD = q.s2, t.xE = q.sh;
+    scales[i] = {q.s1, q.sv, q.s2, q.sh};
   }
   PrefillArgs& a = m->pp;
   WGPT_HIP(hipMemcpyAsync((void*)a.layers, layers.data(), sizeof(PrefillLayer) * (size_t)m->L, hipMemcpyHostToDevice, rt().stream));
+  WGPT_HIP(hipMemcpyAsync((void*)(a.layers + m->L), scales.data(), sizeof(PrefillScales) * (size_t)m->L, hipMemcpyHostToDevice, rt().stream));
   WGPT_HIP(hipMemsetAsync(a.flags, 0, PP_FLAGS * sizeof(unsigned), rt().stream));
   WGPT_HIP(hipStreamSynchronize(rt().stream));
   a.L = m->L; a.H = m->H; a.hs = m->hs; a.d = m->d; a.ctx = m->ctx; a.V = m->V;
@@ -954,7 +956,7 @@ int wgpt_model_finalize(wgpt_model h) {
       {(void**)&m->u_dev, (size_t)m->ctx * sizeof(double)}, {(void**)&m->part, part_bytes},
       {(void**)&m->att_ws, att_ws > part_bytes ? att_ws : 0},
       {(void**)&m->taps, m->p.flags & WGPT_FLAG_TAPS ? (size_t)(2 + 6 * m->L) * T * d * f : 0},
-      {(void**)&m->pp.layers, m->pp_rows ? sizeof(PrefillLayer) * m->L : 0}, {(void**)&m->pp.flags, m->pp_rows ? PP_FLAGS * sizeof(unsigned) : 0},
+      {(void**)&m->pp.layers, m->pp_rows ? (sizeof(PrefillLayer) + sizeof(PrefillScales)) * m->L : 0}, {(void**)&m->pp.flags, m->pp_rows ? PP_FLAGS * sizeof(unsigned) : 0},
       {(void**)&m->pp.q, prefill_exchange_floats(m->pp_rows, (int)d) * f}, {&block_buf, (size_t)4 * d * d * (i8 ? 1 : f)}};
   const auto room = [](size_t bytes) { return (bytes + 16 + 255) / 256 * 256; };
   size_t total = 0;

@@ -113,11 +113,10 @@ struct WSlice {
   // a scalar offset.
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int N, int K8, int n, bool nok, int step, int cnt, int kg) {
     constexpr bool I8 = is_i8(MODE), UNITS = MODE == PP_PAIR_F32;
-    const int place = UNITS ? ((n >> 5) * ((K8 + 1) >> 1) + (kg >> 1)) * 2048 + (kg & 1) * 512 + (n & 31) * 16 : (I8 ? 8 : 32) * kg * N + (I8 ? 8 : 16) * n;
-    const int o = nok ? place : OUT, stride = UNITS ? 4096 : (I8 ? 32 : 128) * N;
+    const int o = nok ? (UNITS ? ((n >> 5) * ((K8 + 1) >> 1) + (kg >> 1)) * 2048 + (kg & 1) * 512 + (n & 31) * 16 : (I8 ? 8 : 32) * kg * N + (I8 ? 8 : 16) * n) : OUT;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      const int left = i < cnt ? K8 - 4 * (step + i) : 0, so = stride * (i < cnt ? step + i : 0);
+      const int left = i < cnt ? K8 - 4 * (step + i) : 0, so = UNITS ? 4096 * (i < cnt ? step + i : 0) : (I8 ? 32 : 128) * N * (i < cnt ? step + i : 0);
       const int oi = kg < left ? o : OUT;
       if constexpr (I8) {
         const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(b, oi, so, 0);
@@ -132,8 +131,8 @@ struct WSlice {
 };
 // The memory of a weight matrix [K, N].
 template <int MODE>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t weights_of(const void* W, int K, int N) {
-  return buffer_of(W, MODE == PP_PAIR_F32 ? (size_t)((N + 31) >> 5) * ((K + 15) >> 4) * 2048 : (size_t)K * N * (is_i8(MODE) ? 1 : 4));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t weights_of(const void* W, size_t K, int N) {
+  return buffer_of(W, MODE == PP_PAIR_F32 ? (size_t)((N + 31) >> 5) * ((K + 15) >> 4) * 2048 : K * N * (is_i8(MODE) ? 1 : 4));
 }
 
 // Eight k of one row as the products take them, from two runs of four floats, or from the hi and lo halves of pairs.
@@ -251,6 +250,13 @@ __device__ __forceinline__ ConstLayer* fresh_layer(int li) {
   ConstLayer* p = (ConstLayer*)(size_t)fresh_args()->layers + li;
   asm volatile("" : "+s"(p));
   return p;
+}
+typedef const __attribute__((address_space(4))) PrefillScales ConstScales;
+template <int MODE>
+__device__ __forceinline__ float row_scale(int li, float PrefillScales::*of) {
+  if constexpr (!is_pair(MODE)) return 1.f;
+  ConstArgs* a = fresh_args();
+  return ((ConstScales*)((ConstLayer*)(size_t)a->layers + a->L) + li)->*of;
 }
 
 // Rows travel between the workgroups of a row group in the order in which their readers load them, [K / 8][2][16 rows][4]: a
@@ -514,7 +520,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
         }
         ConstLayer* ly = fresh_layer(li);
         take(w, bias, scale, ly->wA, 3 * d, cpA, ncA);
-        normalise(x, ly->xA);
+        normalise(x, row_scale<MODE>(li, &PrefillScales::A));
         multiply(x, w, ly->wA, 3 * d, cpA, ncA, tilesA);
         __syncthreads();
         if (bail) return;
@@ -631,7 +637,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] /= l;
-            put_row<MODE>(a->att + (size_t)rg * PP_ROWS * d, qr, h * hs + c, v, PAIR ? fresh_layer(li)->xC : 1.f);
+            put_row<MODE>(a->att + (size_t)rg * PP_ROWS * d, qr, h * hs + c, v, row_scale<MODE>(li, &PrefillScales::C));
           }
           if (h + a->cols < H) __syncthreads();
         }
@@ -666,7 +672,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       const auto request_E = [&] {
         ConstLayer* ly = fresh_layer(li);
         const int ol = opaque(lane), r = ol & 15;
-        we.load(weights_of<MODE>(ly->wE, 4 * d, d), d, K84, cg * cpC + r, r < ncC, s4, n4, ol >> 4);
+        we.load(weights_of<MODE>(ly->wE, (size_t)4 * d, d), d, K84, cg * cpC + r, r < ncC, s4, n4, ol >> 4);
         request_cols(ly->bE, ly->sE, d, cpC, ncC);
       };
       if (tilesD) {
@@ -677,7 +683,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
         load_rows(x, a->x1, K81, s1, n1);
         ConstLayer* ly = fresh_layer(li);
         take(w, bias, scale, ly->wD, 4 * d, cpD, ncD);
-        normalise(x, ly->xD);
+        normalise(x, row_scale<MODE>(li, &PrefillScales::D));
         multiply(x, w, ly->wD, 4 * d, cpD, ncD, tilesD);
         __syncthreads();
         if (bail) return;
@@ -689,7 +695,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
           f32x4 v = finished(tilesD, i, bias, scale);
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = gelu_ref(v[e]);
-          put_row<MODE>(h, er, cg * cpD + n, v, PAIR ? ly->xE : 1.f);
+          put_row<MODE>(h, er, cg * cpD + n, v, row_scale<MODE>(li, &PrefillScales::E));
         }
         raise(ep + 4);
       }
@@ -699,7 +705,7 @@ __global__ __launch_bounds__(NT, 2) void prefill_persistent_kernel(PrefillArgs) 
       if (tilesC) {
         ConstArgs* a = fresh_args();
         constexpr int TM = 2;  // tiles of a pass over the slice
-        const __amdgpu_buffer_rsrc_t b = weights_of<MODE>(fresh_layer(li)->wE, 4 * d, d);
+        const __amdgpu_buffer_rsrc_t b = weights_of<MODE>(fresh_layer(li)->wE, (size_t)4 * d, d);
         const float* hidden = a->h;
         const int ol = opaque(lane), r = ol & 15, kg = ol >> 4;
         if (n4 > 0) wait_cols(cpD, a->rcpD, 32 * s4, last_col(s4, n4, 4 * d), ep + 4);
