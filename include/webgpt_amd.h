@@ -192,6 +192,9 @@ int wgpt_model_set_decode_mode(wgpt_model m, int mode);
  * 0 with a launch per block (longer than the kernel takes, WGPT_FLAG_TAPS, a launch that gave up), -1 there was none; *decode: the decode
  * mode in use, 0 also after a wait of the persistent kernel that expired. Either may be NULL. */
 int wgpt_model_routes(wgpt_model m, int* prefill, int* decode);
+/* *pairs: 1 the products of the last wgpt_prefill were made of pairs of fp16 values (weights from 512 columns on that these can hold), 0 they
+ * were not, -1 there was none. */
+int wgpt_model_pairs(wgpt_model m, int* pairs);
 /* The persistent decode kernel waits a fixed time after publishing before it first looks for the other workgroups'
  * values (seven delays, one per exchange; a table per model width is built in, measured on one MI355X). This searches
  * around the current row on the GPU the model lives on: `rounds` passes of coordinate descent (0 = only measure), each

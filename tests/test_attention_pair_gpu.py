@@ -28,7 +28,7 @@ def test_rows_against_oracle(device, d, n_head):
         tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
         want, all_taps, _ = ref.forward(p, w, tokens, want_taps=True, want_kv=True)
         got = gpt.prefill(tokens)
-        assert close(got, want), (T, worst(got, want))
+        assert close(got, want) and gpt.pairs() == 1, (T, worst(got, want))
         rows, exp = gpt.tap("residual", T), all_taps[ref.tap_names(2).index("block1_r2")]
         assert close(rows, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T  # (near zero a sum's error is its terms')
     gpt.unloadBuffers()
@@ -46,6 +46,7 @@ def test_sharp_softmax(device):
     err = lambda m: float(np.max(np.abs(m.prefill(tokens) - want)))
     # (scores of 300 lose 300 x 2^-24 to rounding, whoever makes them: no further off than a few times the other kernels')
     assert err(gpt) <= 4 * err(taps) + 1e-6
+    assert gpt.pairs() == 1
     gpt.unloadBuffers()
     taps.unloadBuffers()
 
@@ -60,7 +61,7 @@ def test_uneven_queries(device):
         tensors[name + end][..., 64:512] *= np.float32(2.0 ** -14)
     tokens = synth.tokens(3, "prompt", 140, cfg["vocab_size"])
     gpt, taps = load(cfg, tensors), load(cfg, tensors, flags=1)
-    assert close(gpt.prefill(tokens), taps.prefill(tokens))
+    assert close(gpt.prefill(tokens), taps.prefill(tokens)) and gpt.pairs() == 0
     assert close(gpt.prefill(tokens), ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens))
     gpt.unloadBuffers()
     taps.unloadBuffers()

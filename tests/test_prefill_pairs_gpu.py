@@ -35,6 +35,7 @@ def test_prompts_against_oracle(device, dtype, d, n_head):
         got = gpt.prefill(tokens)
         assert close(got, want), (T, worst(got, want))
         assert not np.array_equal(got, taps.prefill(tokens)), T
+        assert gpt.pairs() == 1 and taps.pairs() == 0, T
         for i in range(2):
             for j, name in enumerate("kv"):
                 assert close(gpt.tap(f"kv{i}_{name}"), kv[i, j]), (T, i, name)
@@ -63,12 +64,13 @@ def spoil(tensors, how):
 
 @pytest.mark.parametrize("how", ["infinite", "tiny columns", "tiny", "gamma", "large"])
 def test_weights_beyond_the_pairs(device, how):
-    """Found when the model is loaded: bit for bit the results of the products of a model that keeps taps."""
+    """Found when the model is loaded, which then runs the products of a model that keeps taps."""
     cfg = small_cfg(n_layer=2, n_head=8, n_embd=512, n_ctx=140, vocab_size=101)
     tensors = spoil(make_model(cfg, 3), how)
     tokens = synth.tokens(3, "prompt", 140, cfg["vocab_size"])
     gpt, taps = load(cfg, tensors), load(cfg, tensors, FLAG_TAPS)
     got, want = gpt.prefill(tokens), taps.prefill(tokens)
+    assert gpt.pairs() == 0
     # (the LayerNorm in front of a product is a pass of its own where there are taps: equal to rounding, not to the last bit)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and close(got[~np.isnan(want)], want[~np.isnan(want)])
     gpt.unloadBuffers()
@@ -104,6 +106,47 @@ def test_one_wide_column(device, dtype, d, n_head, T, how):
     want = ref.forward(synth.model_params(cfg), oracle_weights(tensors, cfg), tokens)
     got = gpt.prefill(tokens)
     assert close(got, want), worst(got, want)
+    assert gpt.pairs() == 0
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head,rows", [(1608, 67, (513, 401, 400)), (1600, 25, (513, 400))])
+def test_many_rows_of_wide_models(device, dtype, d, n_head, rows):
+    """Both sides of the rule for the LayerNorm's workgroups (a row each up to 400 rows) at widths beyond three runs of 512."""
+    cfg = small_cfg(n_layer=1, n_head=n_head, n_embd=d, n_ctx=520, vocab_size=97, dtype=dtype)
+    tensors = make_model(cfg, d)
+    gpt, w, p = load(cfg, tensors), oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in rows:
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        want, taps, _ = ref.forward(p, w, tokens, want_taps=True, want_kv=True)
+        got = gpt.prefill(tokens)
+        assert close(got, want) and gpt.pairs() == 1, (T, worst(got, want))
+        rows_got, exp = gpt.tap("residual", T), taps[ref.tap_names(1).index("block0_r2")]
+        assert close(rows_got, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T  # (near zero a sum's error is its terms')
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head,rows", [(768, 12, (961, 960, 943, 865)), (744, 6, (513, 385, 289)), (1000, 10, (300, 193)), (1600, 25, (300, 129)),
+                                           (1240, 31, (943, 300)), (2056, 257, (513,)), (512, 8, (257, 140))])
+def test_prompts_without_the_pairs(device, dtype, d, n_head, rows):
+    """A gain that the pairs' scale does not fit: products of three bf16 values each, LayerNorm, GELU and cache rows with them, at the edges of
+    their larger tiles."""
+    cfg = small_cfg(n_layer=1, n_head=n_head, n_embd=d, n_ctx=1024, vocab_size=97, dtype=dtype)
+    tensors = {k: v.copy() for k, v in make_model(cfg, d).items()}
+    tensors["transformer.h.0.ln_2.weight"][3] = 2.0 ** -20
+    tensors["transformer.h.0.ln_2.bias"][3] = 0.0
+    gpt, w, p = load(cfg, tensors), oracle_weights(tensors, cfg), synth.model_params(cfg)
+    for T in rows:
+        tokens = synth.tokens(T, "prompt", T, cfg["vocab_size"])
+        want, taps, kv = ref.forward(p, w, tokens, want_taps=True, want_kv=True)
+        got = gpt.prefill(tokens)
+        assert close(got, want) and gpt.pairs() == 0, (T, worst(got, want))
+        for j, name in enumerate("kv"):
+            assert close(gpt.tap(f"kv0_{name}"), kv[0, j]), (T, name)
+        rows_got, exp = gpt.tap("residual", T), taps[ref.tap_names(1).index("block0_r2")]
+        assert close(rows_got, exp, atol=1e-4 * float(np.sqrt(np.mean(exp ** 2)))), T  # (near zero a sum's error is its terms')
     gpt.unloadBuffers()
 
 
@@ -151,6 +194,7 @@ def test_shorter_prompt_behind_a_longer_one(device, dtype, d, n_head):
     for T in (150, 131):
         want, got = fresh.prefill(tokens[:T]), gpt.prefill(tokens[:T])
         assert np.array_equal(got, want) and close(got, ref.forward(p, w, tokens[:T])), T
+        assert gpt.pairs() == 1, T
         gpt.prefill(tokens)
         fresh.unloadBuffers()
         fresh = load(cfg, tensors)
@@ -174,5 +218,18 @@ def test_short_prompts_of_weights_beyond_the_pairs(device, dtype, d, n_head):
         want = ref.forward(p, w, tokens)
         got = gpt.prefill(tokens)
         assert close(got, want), (T, worst(got, want))
-        assert gpt.routes()[0] == 1, T
+        assert gpt.routes()[0] == 1 and gpt.pairs() == 0, T
+    gpt.unloadBuffers()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "int8"])
+@pytest.mark.parametrize("d,n_head,pairs", [(512, 8, 0), (520, 13, 1)])
+def test_which_prompts_run_on_pairs(device, dtype, d, n_head, pairs):
+    """The persistent launch from 520 columns on, the others from 512 and 129 tokens."""
+    cfg = small_cfg(n_layer=1, n_head=n_head, n_embd=d, n_ctx=140, vocab_size=101, dtype=dtype)
+    gpt = load(cfg, make_model(cfg, 8))
+    assert gpt.pairs() == -1
+    for T, route, on in ((1, 1, pairs), (128, 1, pairs), (129, 0, 1), (64, 1, pairs)):
+        gpt.prefill(synth.tokens(T, "prompt", T, cfg["vocab_size"]))
+        assert (gpt.routes()[0], gpt.pairs()) == (route, on), T
     gpt.unloadBuffers()

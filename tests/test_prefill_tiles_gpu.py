@@ -1,5 +1,6 @@
-"""Prompts whose products run in the larger tiles (csrc/gemm_split.hip, plan_gemm_split) against the CPU oracle: rows on both sides
-of their edges, widths that are no multiple of 128 or of a step of 32, both weight dtypes."""
+"""Long prompts against the CPU oracle: rows on both sides of the edges of the larger tiles, widths that are no multiple of 128 or of a step
+of 32, both weight dtypes. Widths of 512 and more run on pairs (csrc/gemm_pair.hip), 456 in the tiles of csrc/gemm_split.hip, which
+test_prefill_pairs_gpu.py holds the others to as well."""
 import numpy as np
 import pytest
 

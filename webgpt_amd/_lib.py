@@ -74,6 +74,7 @@ _SIGNATURES = {
     "wgpt_model_decode_bytes": ([_u64, _int, C.POINTER(_u64)], True),
     "wgpt_model_set_decode_mode": ([_u64, _int], True),
     "wgpt_model_routes": ([_u64, C.POINTER(_int), C.POINTER(_int)], True),
+    "wgpt_model_pairs": ([_u64, C.POINTER(_int)], True),
     "wgpt_model_tune_poll_delays": ([_u64, _int, _ip, _fp, _fp], True),
     "wgpt_model_poll_delays": ([_u64, _ip], True),
     "wgpt_model_destroy": ([_u64], True),

@@ -85,6 +85,7 @@ struct Model {
   PrefillArgs pp{};
   unsigned pp_epoch = 0;       // last epoch of its earlier launches
   int prefill_route = -1;      // wgpt_model_routes
+  int prefill_on_pairs = -1;   // wgpt_model_pairs
   int pp_spoilt = 0;           // launches in a row that gave up on their prompt's values, and
   int pp_skip = 0;             // the prompts that are not tried on account of them
   // prompts beyond those: products of pairs of fp16 values, where the weights allow (empty: they do not)

@@ -1016,7 +1016,7 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
   m->tap_T = 0;
   m->x_rows = 0;
   int rc;
-  bool done = false;
+  bool done = false, pairs = prefill_pairs(m);
   if (T <= m->pp_rows && m->pp_skip > 0) {
     --m->pp_skip;
   } else if (T <= m->pp_rows) {
@@ -1031,10 +1031,12 @@ int wgpt_prefill(wgpt_model h, const int32_t* tokens, int T, float* logits) {
     WGPT_HIP(hipMemcpyAsync(m->tok_dev, tokens, sizeof(int32_t) * (size_t)T, hipMemcpyHostToDevice, rt().stream));
     WGPT_HIP(hipStreamSynchronize(rt().stream));
     WGPT_HIP(hipEventRecord(m->ev0, rt().stream));
-    if ((rc = T > m->pp_rows && T >= PAIR_MIN_T && !m->pairs.empty() ? forward_pairs(m, T) : forward_blocks(m, T, 0, true))) return rc;
+    pairs = T > m->pp_rows && T >= PAIR_MIN_T && !m->pairs.empty();
+    if ((rc = pairs ? forward_pairs(m, T) : forward_blocks(m, T, 0, true))) return rc;
     if ((rc = finish_timed(m, logits))) return rc;
   }
   m->prefill_route = done;
+  m->prefill_on_pairs = pairs;
   m->pos = T;
   m->tap_T = m->taps ? T : 0;
   m->x_rows = T;
@@ -1414,6 +1416,13 @@ int wgpt_model_routes(wgpt_model h, int* prefill, int* decode) {
   if (!m) return WGPT_ERR_ARG;
   if (prefill) *prefill = m->prefill_route;
   if (decode) *decode = m->decode_mode;
+  return WGPT_OK;
+}
+
+int wgpt_model_pairs(wgpt_model h, int* pairs) {
+  Model* m = find_model(h);
+  if (!m) return WGPT_ERR_ARG;
+  if (pairs) *pairs = m->prefill_on_pairs;
   return WGPT_OK;
 }
 

@@ -31,7 +31,7 @@ void* g_lib = nullptr;
   X(wgpt_model_decode_bytes) X(wgpt_model_set_decode_mode) X(wgpt_model_destroy) X(wgpt_synth_normal)   \
   X(wgpt_synth_tokens) X(wgpt_synth_int8_packed) X(wgpt_synth_uniform) X(wgpt_synth_tensor_id)   \
   X(wgpt_decode_sample) X(wgpt_sample_topk) X(wgpt_matmul_bias_noalloc) X(wgpt_softmax_t) X(wgpt_transpose)   \
-  X(wgpt_model_tune_poll_delays) X(wgpt_model_poll_delays) X(wgpt_model_routes)
+  X(wgpt_model_tune_poll_delays) X(wgpt_model_poll_delays) X(wgpt_model_routes) X(wgpt_model_pairs)
 
 #define DECL(name) decltype(&::name) p_##name = nullptr;
 WGPT_FUNCS(DECL)
@@ -246,6 +246,7 @@ FN(ModelRoutes) {  // (model) -> Float32Array[2]: the last prefill's route, the 
   ((float*)p)[1] = (float)decode;
   return ta;
 }
+FN(ModelPairs) { Args a(env, info); uint64_t m = a.u64(0); if (!a.ok) return nullptr; int on = 0; if (failed(env, p_wgpt_model_pairs(m, &on))) return nullptr; return number(env, on); }
 FN(ModelPosition) { Args a(env, info); uint64_t m = a.u64(0); if (!a.ok) return nullptr; int pos = 0; if (failed(env, p_wgpt_model_position(m, &pos))) return nullptr; return number(env, pos); }
 FN(ModelLastGpuMs) { Args a(env, info); uint64_t m = a.u64(0); if (!a.ok) return nullptr; float ms = 0; if (failed(env, p_wgpt_model_last_gpu_ms(m, &ms))) return nullptr; return number(env, ms); }
 FN(ModelDecodeBytes) { Args a(env, info); uint64_t m = a.u64(0); int t = a.i32(1); if (!a.ok) return nullptr; uint64_t b = 0; if (failed(env, p_wgpt_model_decode_bytes(m, t, &b))) return nullptr; return number(env, (double)b); }
@@ -444,7 +445,7 @@ napi_value InitModule(napi_env env, napi_value exports) {
       {"wgpt_embed", Embed}, {"wgpt_deembed", DeEmbed}, {"wgpt_attention", Attention},
       {"modelCreate", ModelCreate}, {"modelSetTensor", ModelSetTensor}, {"modelFinalize", ModelFinalize},
       {"modelDestroy", ModelDestroy}, {"modelResetCache", ModelResetCache}, {"modelSetDecodeMode", ModelSetDecodeMode},
-      {"modelPosition", ModelPosition}, {"modelRoutes", ModelRoutes}, {"modelLastGpuMs", ModelLastGpuMs}, {"modelDecodeBytes", ModelDecodeBytes},
+      {"modelPosition", ModelPosition}, {"modelRoutes", ModelRoutes}, {"modelPairs", ModelPairs}, {"modelLastGpuMs", ModelLastGpuMs}, {"modelDecodeBytes", ModelDecodeBytes},
       {"modelPollDelays", ModelPollDelays}, {"modelTunePollDelays", ModelTunePollDelays},
       {"prefill", Prefill}, {"decode", Decode}, {"decodeGreedy", DecodeGreedy}, {"decodeSample", DecodeSample}, {"sampleTopK", SampleTopK}, {"modelTap", ModelTap},
       {"synthNormal", SynthNormal}};

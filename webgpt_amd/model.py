@@ -303,6 +303,12 @@ class GPT:
         _lib.call("wgpt_model_routes", self._handle, C.byref(prefill), C.byref(decode))
         return prefill.value, decode.value
 
+    def pairs(self):
+        """Whether the last prefill's products were made of pairs of fp16 values (1, 0; -1: none yet)."""
+        pairs = C.c_int(0)
+        _lib.call("wgpt_model_pairs", self._handle, C.byref(pairs))
+        return pairs.value
+
     def tune_poll_delays(self, rounds=2):
         """Searches the persistent decode kernel's seven poll delays on this GPU (wgpt_model_tune_poll_delays; needs
         position 0). Returns (delays, ms_per_token_before, ms_per_token_after)."""
