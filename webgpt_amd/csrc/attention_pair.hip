@@ -19,6 +19,7 @@
 
 #include <cmath>
 
+#include "exp_neg.h"
 #include "pair_f16.h"
 
 namespace wgpt {
@@ -28,13 +29,6 @@ constexpr int APQ = PAIR_ATTN_ROWS;  // queries per workgroup, keys per tile
 constexpr int AP_MERGE = APQ + 1;    // row stride of a wave's O^T[dim][query] in the merge
 constexpr float AP_UP = 0x1p15f;
 
-// exp(x) for x <= 0 with the rounding of x * log2(e) made up for, times `up`
-__device__ __forceinline__ float exp_neg(float x, float up) {
-  const float t = x * 1.44269504f;
-  const float r = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t));  // log2(e) = 1.44269502162933 + 1.92596303e-8
-  const float e = __builtin_amdgcn_exp2f(t) * up;
-  return fmaf(e, r * 0.693147181f, e);
-}
 __device__ __forceinline__ f32x16 mfma(const u32x4& p, const u32x4& q, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, p), __builtin_bit_cast(f16x8, q), c, 0, 0, 0);
 }
@@ -95,7 +89,7 @@ __global__ __launch_bounds__(NWV * 64, DB < 3 ? 2 : 1) void attention_pair_kerne
       for (int r = 1; r < 16; ++r) top = fmaxf(top, sc[r]);
       top = fmaxf(top, __shfl_xor(top, 32));
       const float mnew = fmaxf(m, top * a.scale);  // (finite: a query sees a key of every tile)
-      const float corr = m > -INFINITY ? exp_neg(m - mnew, 1.f) : 0.f;
+      const float corr = m > -INFINITY ? exp_neg(m - mnew) : 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float w = exp_neg(fmaf(sc[r], a.scale, -mnew), AP_UP);
@@ -144,7 +138,7 @@ __global__ __launch_bounds__(NWV * 64, DB < 3 ? 2 : 1) void attention_pair_kerne
   }
 #pragma unroll
   for (int w = 0; w < NWV; ++w) {
-    f[w] = f[w] > -INFINITY ? exp_neg(f[w] - M, 1.f) : 0.f;
+    f[w] = f[w] > -INFINITY ? exp_neg(f[w] - M) : 0.f;
     den += lds[w * WAVE_FLOATS + DIMS * AP_MERGE + APQ + qi] * f[w];
   }
   if (row >= a.T) return;

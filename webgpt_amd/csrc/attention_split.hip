@@ -11,6 +11,7 @@
 // Bound by what a compute unit takes from L2 (12 KB per 32 keys at head size 64, read by every block of 32 queries).
 #include <cmath>
 
+#include "exp_neg.h"
 #include "kernels.h"
 #include "pair_f16.h"
 
@@ -75,14 +76,6 @@ __global__ void attention_operands(AttnSplitArgs a) {
   dst[0] = s.hi;
   dst[64] = s.mid;
   dst[128] = s.lo;
-}
-
-// exp(x) for x <= 0 with the rounding of x * log2(e) made up for: as exact as expf down to its smallest normal result
-__device__ __forceinline__ float exp_neg(float x) {
-  const float t = x * 1.44269504f;
-  const float r = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t));  // log2(e) = 1.44269502162933 + 1.92596303e-8
-  const float e = __builtin_amdgcn_exp2f(t);
-  return fmaf(e, r * 0.693147181f, e);
 }
 
 __device__ __forceinline__ f32x16 mfma(const u32x4& p, const u32x4& q, f32x16 c) {

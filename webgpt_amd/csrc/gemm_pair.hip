@@ -609,8 +609,10 @@ hipError_t launch_gemm_pair(const PairPlan& p, PairGemmArgs a, bool i8, hipStrea
 }
 
 hipError_t launch_ln_pair(const PairLnArgs& a, hipStream_t s) {
-  // Few rows leave compute units without one of four waves' rows: a workgroup per row, us at 200 x 1280 6.1 -> 5.0, 300 x 1600 (four slices)
-  // 7.6 -> 6.3, 500 x 1280 6.8 -> 6.4; 500 x 1600 6.4 either way, 512 x 1024 6.0 -> 6.2, 943 x 768 6.3 -> 7.0, 1000 x 1280 6.8 -> 7.5.
+  // Few rows leave compute units without one of four waves' rows: a workgroup per row. Passes of a prompt (some of them with slices), us with
+  // a wave and with a workgroup per row, at 150, 300, 400, 500 and 1000 rows: 768 columns 5.1 4.1, 5.4 4.8, 5.4 5.2, 5.9 5.7, 6.0 6.6; 1024 5.1 4.4, 5.2 5.4, 5.8 5.7,
+  // 5.8 6.0, 5.3 6.2; 1280 6.1 4.9, 6.2 5.6, 6.3 5.9, 6.6 6.3, 6.6 7.4; 1600 6.9 5.1, 6.9 5.9, 7.3 6.5, 6.3 6.4, 8.1 8.7; 2048 7.7 5.7, 7.5 6.5, 6.5 6.5, 6.8 7.0,
+  // 8.4 10.2: the sides meet between 300 and 600 rows. (Rows above 2048 would be two runs of a workgroup, which are not built.)
   if (a.M <= 400 && a.d <= 2048) {
     ln_pair_kernel<1, 4><<<(unsigned)a.M, 256, 0, s>>>(a);
     return hipGetLastError();

@@ -685,6 +685,10 @@ static int block_linear_weights(Model* m, void* free_buf) {
 // Narrowest rows whose products are made of pairs: below, their sums would be further from exact ones than those of three bf16
 // values each (gemm_pair.hip).
 constexpr int PAIR_MIN_D = 512;
+// Fewest rows of a prompt that the launches make of pairs. Three layers, us with three bf16 values each and with pairs, heads x head size: fp32 4 x 160
+// 64 rows 196 197, 72 212 207, 128 246 236; 4 x 256 223 213, 252 224, 285 255; 16 x 128 32 rows 310 328, 48 350 328, 64 361 333; int8 4 x 160 64 rows 193 189,
+// 128 240 229; 16 x 128 24 rows 229 238, 32 243 240, 64 260 247. (Fewer rows of wider models would gain too; prompts that short are as a rule the
+// persistent launch's.)
 constexpr int PAIR_MIN_T = 64;
 // What the bounds of a matrix's columns may be of the largest one, so that its scale serves them all. Error of pairs of normal values 0, 6, 8, 10 and 12
 // bits below the others, widths of 512 and 1600: rows of q, keys and the hidden layer 5.0e-8, 5.0e-8, 5.2e-8, 8.1e-8, 2.8e-7; averages of 300 to 1024 values
