@@ -9,7 +9,7 @@
 // epilogue, stores and the flag 0.8 to 1.1 a phase (0.6 to 1.2), loads with LayerNorm and products c_attn 2.5 (7.3), attention 2.7 (4.0), c_proj
 // 2.1 (2.4), c_fc 3.1 (8.6), the second MLP product 5.7 (9.1; at 13 rows a compute unit reads all hidden rows for four columns), the last workgroup 0.6
 // to 2.4 behind the median. The matrix units were busy for 11 % of the launch at 13 rows and 31 % at 128, 14 us a layer of the 27 in its
-// products; on pairs they are for 3 us of those at 128.
+// products; on pairs for 10 % at 128, 4 us a layer.
 // The compiler spills 218 to 329 scalar registers into vector lanes.
 // Here one workgroup per compute unit stays for the whole forward and the blocks are phases of it:
 //
