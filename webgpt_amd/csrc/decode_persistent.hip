@@ -1636,14 +1636,15 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
       input_row<D, true, true>(xv, xs0, lnp, lane);
       float best = -INFINITY;
       int besti = 0x7fffffff;
-      // top_k > 1: this wave's K best rows so far, in order; (lastv, lasti) is the K-th
+      // top_k > 1: this wave's K best rows so far, in order; lastv is the K-th, no number while there are fewer. (Rows come in ascending order, so
+      // one that is no larger than a number there is behind it; the list itself has NaN and empty places in order.)
       const int K = SAMPLE ? a.top_k : 1;
       constexpr int KL = SAMPLE ? PD_TOPK : 1;
-      float tv[KL], lastv = -INFINITY;
-      int ti[KL], lasti = NOCAND;
+      float tv[KL], lastv = NAN;
+      int ti[KL];
 #pragma unroll
       for (int j = 0; j < KL; ++j) {
-        tv[j] = -INFINITY;
+        tv[j] = NAN;
         ti[j] = NOCAND;
       }
       // the last step's logits also go to the caller's pinned memory, through LDS (narrow shapes only)
@@ -1674,7 +1675,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
                 best = s;
                 besti = vb + r;
               }
-              if (SAMPLE && cand_before(s, vb + r, lastv, lasti)) {
+              if (SAMPLE && !(s <= lastv)) {
                 // insert: carry the displaced candidate down the list
                 float cv = s;
                 int ci = vb + r;
@@ -1688,10 +1689,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
                     cv = sv;
                     ci = si;
                   }
-                  if (j == K - 1) {
-                    lastv = tv[j];
-                    lasti = ti[j];
-                  }
+                  if (j == K - 1) lastv = tv[j];
                 }
               }
             }
@@ -1709,7 +1707,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
             best = s;
             besti = row;
           }
-          if (SAMPLE && cand_before(s, row, lastv, lasti)) {
+          if (SAMPLE && !(s <= lastv)) {
             // insert: carry the displaced candidate down the list
             float cv = s;
             int ci = row;
@@ -1723,10 +1721,7 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
                 cv = sv;
                 ci = si;
               }
-              if (j == K - 1) {
-                lastv = tv[j];
-                lasti = ti[j];
-              }
+              if (j == K - 1) lastv = tv[j];
             }
           }
         };
