@@ -83,10 +83,10 @@ def cpu_baseline(cfg, tensors, prompt, budget_s=20.0):
 # on single-token launches of the persistent kernel: bytes, the contexts of the profiled launches, the profile that
 # holds the figures and the first 16 hex digits of the SHA-256 of the kernel's source file when it was profiled.
 MEASURED_TRAFFIC = {
-    "gpt2-117m": (515.8e6, (133, 164), "profiles/decode_persistent_gpt2-117m.md", "238ca3a707727ec6"),
-    "gpt2-345m": (1558.2e6, (555, 586), "profiles/decode_persistent_other_configs.md", "238ca3a707727ec6"),
-    "gpt2-774m": (3178.7e6, (107, 138), "profiles/decode_persistent_other_configs.md", "238ca3a707727ec6"),
-    "gpt2-1.5b-int8": (2116.1e6, (171, 202), "profiles/decode_persistent_other_configs.md", "238ca3a707727ec6"),
+    "gpt2-117m": (515.9e6, (133, 164), "profiles/decode_persistent_gpt2-117m.md", "7fef13125ba3872a"),
+    "gpt2-345m": (1558.1e6, (555, 586), "profiles/decode_persistent_other_configs.md", "7fef13125ba3872a"),
+    "gpt2-774m": (3178.9e6, (107, 138), "profiles/decode_persistent_other_configs.md", "7fef13125ba3872a"),
+    "gpt2-1.5b-int8": (2116.0e6, (171, 202), "profiles/decode_persistent_other_configs.md", "7fef13125ba3872a"),
 }
 KERNEL_SOURCE = os.path.join(ROOT, "webgpt_amd", "csrc", "decode_persistent.hip")
 

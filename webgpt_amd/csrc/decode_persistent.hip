@@ -1866,8 +1866,9 @@ __global__ __launch_bounds__(NT) void decode_persistent_kernel(PersistentArgs a)
         if (lane < PD_TOPK) sh.firsts[wave * PD_TOPK + lane] = mine;
       };
       static_assert(PD_TOPK * C::G == 4 * NT, "up to four words of candidates for a thread");
-      // (Without vocabulary rows in LDS the one form. With the short one beside it 32 tokens of 345M at top_k 2 and 3 took 12.17 and 12.31 ms either way, 16 of
-      // 774M 13.01 and 13.07 instead of 12.99 and 13.03; 16 of 1.5B int8 14.11 and 14.07 instead of 14.23 and 14.16, and 0.7 % less at 8 too, which does not use it.)
+      // (Without vocabulary rows in LDS the one form. With the short one beside it 32 tokens of 345M at top_k 2, 3 and 6 took 12.20, 12.31 and 12.46 ms instead of
+      // 12.18, 12.30 and 12.44, 16 of 774M at 2 and 3 12.99 and 13.05 instead of 12.99 and 13.05, of 1.5B int8 at 2, 3 and 8, which does not use it, 13.98, 13.98 and
+      // 14.14 instead of 14.09, 14.07 and 14.21.)
       if constexpr (LROWS == 0) gather(std::integral_constant<int, 4>{});
       else if (a.top_k <= 2) gather(std::integral_constant<int, 1>{});
       else gather(std::integral_constant<int, 4>{});
